@@ -295,6 +295,21 @@ int pt_mlp_energy_grad(int mode, int n_atoms, const void *G, int ldg, int g_prec
                        const double *scale, const pt_mlp_desc *desc, const void *packed,
                        double *e_atom, void *dEdG, pt_stream_t stream);
 
+/* Several elements' networks in one launch: every job is one call of
+ * pt_mlp_energy_grad (its n_atoms, G, scale, desc, packed, e_atom, dEdG) at
+ * the common mode, ldg and g_precision. */
+typedef struct {
+    int n_atoms;
+    const void *G;
+    const double *scale;
+    const pt_mlp_desc *desc;
+    const void *packed;
+    double *e_atom;
+    void *dEdG;
+} pt_mlp_job;
+int pt_mlp_energy_grad_multi(int mode, int n_jobs, const pt_mlp_job *jobs, int ldg, int g_precision,
+                             pt_stream_t stream);
+
 /* ------------------------------------------------------------------------
  * (c') Training of an atomic MLP (the student surrogate).  No counterpart in
  * the reference runs (its trainer, potentials/nnp/gradient_descent.py:

@@ -87,6 +87,11 @@ class MlpDesc(ctypes.Structure):
     ]
 
 
+class MlpJob(ctypes.Structure):
+    _fields_ = [("n_atoms", _c_int), ("G", _vp), ("scale", _vp), ("desc", ctypes.POINTER(MlpDesc)),
+                ("packed", _vp), ("e_atom", _vp), ("dEdG", _vp)]
+
+
 class PermuteArray(ctypes.Structure):
     _fields_ = [("buf", _vp), ("width", _c_int), ("word_bytes", _c_int)]
 
@@ -122,6 +127,7 @@ _SIGS = {
     "pt_mlp_pack": (_c_int, [_vp, _vp, _vp, _vp]),
     "pt_mlp_energy_grad": (_c_int, [_c_int, _c_int, _vp, _c_int, _c_int, _vp, _vp, _vp, _vp,
                                     _vp, _vp]),
+    "pt_mlp_energy_grad_multi": (_c_int, [_c_int, _c_int, ctypes.POINTER(MlpJob), _c_int, _c_int, _vp]),
     "pt_scaler_workspace_bytes": (_c_size, [_c_int, _c_int]),
     "pt_scaler_partial_fit": (_c_int, [_c_int, _c_int, _vp, _c_int, _c_int, _c_dbl, _vp, _vp, _c_size, _vp]),
     "pt_scaler_extrapolation": (_c_int, [_c_int, _c_int, _vp, _c_int, _c_int, _vp, _c_dbl, _vp, _vp]),

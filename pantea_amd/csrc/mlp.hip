@@ -11,10 +11,11 @@
 //   PT_MLP_BF16   v_mfma_f32_16x16x32_bf16 (BF16 in, FP32 accumulate)
 //   PT_MLP_BF16X3 the same with split operands x = hi + lo (hi*hi + hi*lo +
 //                 lo*hi), giving about 16 mantissa bits per product.
-// One wavefront owns a tile; activations and activation derivatives of
-// each hidden layer go through LDS, weights come from a packed device
-// buffer (both W and W^T layouts, so that every MFMA operand fragment is a
-// contiguous run of K elements) built once by pt_mlp_pack.
+// A workgroup owns a block of rows; layer inputs go through LDS (in the
+// matrix instruction's input type), activation derivatives stay in registers,
+// weights come from a packed device buffer (both W and W^T layouts, so that
+// every MFMA operand fragment is a contiguous run of K elements) built once by
+// pt_mlp_pack.
 //
 // Operand layouts (16x16 output tile, lane l, accumulator element i = 0..3):
 //   A[row = l % 16][k = kc + l / 16 (f64) | kc + 8 (l / 16) + 0..7 (bf16)]
@@ -23,6 +24,7 @@
 //                         or  row = 4 (l / 16) + i (v_mfma_f32_16x16x32_bf16)
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "common.h"
 
@@ -140,24 +142,24 @@ __device__ __forceinline__ void activate(int a, T z, T& y, T& dy) {
     y = z; dy = T(1);
 }
 
-// Activations whose derivative is a function of the output y: the inference
-// kernel then keeps only y and turns it into dy/dz in place once the next
-// layer has read it.
-__host__ __device__ constexpr bool act_from_output(int a) {
-    return a == PT_ACT_IDENTITY || a == PT_ACT_TANH || a == PT_ACT_LOGISTIC || a == PT_ACT_SOFTPLUS ||
-           a == PT_ACT_RELU || a == PT_ACT_EXP;
-}
-
-template <typename T>
-__device__ __forceinline__ T dact_from_output(int a, T y) {
+// The same for N values of one activation (the kind is uniform: one branch for all of them).
+template <typename T, int N>
+__device__ __forceinline__ void activate_n(int a, T (&y)[N], T (&dy)[N]) {
+    auto each = [&](auto kind) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) activate<T>(decltype(kind)::value, y[i], y[i], dy[i]);
+    };
     switch (a) {
-    case PT_ACT_TANH: return T(1) - y * y;
-    case PT_ACT_LOGISTIC: return y * (T(1) - y);
-    case PT_ACT_SOFTPLUS: return -expm1(-y);          // logistic(z) = 1 - e^{-y}
-    case PT_ACT_RELU: return y > T(0) ? T(1) : T(0);   // y = max(z, 0)
-    case PT_ACT_EXP: return -y;                        // y = e^{-z}
+    case PT_ACT_TANH: each(std::integral_constant<int, PT_ACT_TANH>{}); return;
+    case PT_ACT_LOGISTIC: each(std::integral_constant<int, PT_ACT_LOGISTIC>{}); return;
+    case PT_ACT_SOFTPLUS: each(std::integral_constant<int, PT_ACT_SOFTPLUS>{}); return;
+    case PT_ACT_RELU: each(std::integral_constant<int, PT_ACT_RELU>{}); return;
+    case PT_ACT_GAUSSIAN: each(std::integral_constant<int, PT_ACT_GAUSSIAN>{}); return;
+    case PT_ACT_COS: each(std::integral_constant<int, PT_ACT_COS>{}); return;
+    case PT_ACT_EXP: each(std::integral_constant<int, PT_ACT_EXP>{}); return;
+    case PT_ACT_HARMONIC: each(std::integral_constant<int, PT_ACT_HARMONIC>{}); return;
+    default: each(std::integral_constant<int, PT_ACT_IDENTITY>{}); return;
     }
-    return T(1);
 }
 
 // y, dy/dz and d2y/dz2 (the training kernel differentiates the input gradient)
@@ -242,20 +244,27 @@ struct MT { typedef float T; };
 template <>
 struct MT<PT_MLP_F64> { typedef double T; };
 
-struct MlpArgs {
+// One network of a launch: the atoms of one element.
+struct MlpNet {
     MlpShape s;
     int n_atoms;
+    int block0;           // first workgroup of this network
     const void* G;
-    int ldg;
-    int g_f64;
     const double* scale;  // [2][in_dim]: sub, mul
     double scale_add;
     const char* packed;
     double* e_atom;
     void* dEdG;
+};
+
+constexpr int kMlpNets = 4;   // networks per launch (the arguments stay well below the 4 KB limit)
+
+struct MlpArgs {
+    MlpNet net[kMlpNets];
+    int n_net;
+    int ldg;
+    int g_f64;
     int stride;           // LDS row stride (elements)
-    int nbuf;             // LDS buffers per wave
-    int inplace;          // every hidden activation has act_from_output
 };
 
 // C = A(16 x K, LDS row-major, stride) * B, accumulating one 16-column tile.
@@ -316,337 +325,370 @@ __device__ __forceinline__ void gemm_tile(const typename MT<MODE>::T* A, int str
     (void)bt;
 }
 
-// C(16 x 16 nt) += A(16 x K, LDS row-major) * B over the column tiles
-// n0 + 16 t, t < nt <= 2, of one layer.  The A fragment of a k step is read
-// and split once for all tiles, and the weight fragments of all tiles are
-// loaded before their products: the wave waits on weight loads once per k
-// step rather than once per tile and step.  Per tile the products run in the
-// same k order as gemm_tile.  Two tiles per pass: four held the weight
-// fragments of too many tiles at once for four resident waves per SIMD.
+// ---- inference: energies and input gradients ---------------------------------
+//
+// One workgroup of four wavefronts takes ROWS = 16 MTW WR atoms through the
+// whole network.  The wavefronts form a WR x WC grid: WR blocks of MTW row
+// tiles times WC interleaved sets of 16-column tiles (CT tiles each in a
+// hidden layer).  A weight fragment is loaded once for the MTW row tiles of
+// its wavefront, and the MTW products of one fragment are independent chains.
+// Between layers only the next product's input goes through LDS, stored as
+// the matrix instruction takes it (FP64, or the BF16 halves, split once where
+// they are produced); the activation derivatives stay in the registers of the
+// lanes that need them again in the reverse sweep (same C layout).
+//
+// What bounds it: below ~10k atoms the serial chain of one row tile through
+// the layers (13.5 us FP64, 9.0 us BF16x3 for 52-64-64-1; one wavefront doing
+// all columns of 16 rows took 66 and 28 us); above, the weight fragments
+// re-read from L2 by every workgroup and the MFMA issue (98,304 rows: 137 us
+// FP64 = 21 TFLOP/s, 50 us BF16x3; before 245 and 85 us).
 template <int MODE>
-__device__ __forceinline__ void gemm_cols(const typename MT<MODE>::T* A, int stride, int K, const char* packed,
-                                          size_t off_hi, size_t off_lo, int ldb, bool bt, int n0, int nt,
-                                          typename MT<MODE>::T (&acc)[2][4]) {
+struct MlpLds;
+template <>
+struct MlpLds<PT_MLP_F64> {
+    double* x;
+    int stride;
+    static constexpr size_t bytes(int rows, int stride) { return sizeof(double) * (size_t)rows * stride; }
+    __device__ __forceinline__ void put(int r, int k, double v) const { x[r * stride + k] = v; }
+};
+template <int MODE>
+struct MlpLds {
+    unsigned short* hi;
+    unsigned short* lo;
+    int stride;
+    static constexpr size_t bytes(int rows, int stride) { return 2 * sizeof(unsigned short) * (size_t)rows * stride; }
+    __device__ __forceinline__ void put(int r, int k, float v) const {
+        unsigned short h, l;
+        split_bf16(v, h, l);
+        hi[r * stride + k] = h;
+        lo[r * stride + k] = l;
+    }
+};
+
+template <int MODE>
+__device__ __forceinline__ MlpLds<MODE> mlp_lds(char* base, int rows, int stride) {
+    MlpLds<MODE> b;
+    b.stride = stride;
+    if constexpr (MODE == PT_MLP_F64) {
+        b.x = reinterpret_cast<double*>(base);
+    } else {
+        b.hi = reinterpret_cast<unsigned short*>(base);
+        b.lo = b.hi + (size_t)rows * stride;
+    }
+    return b;
+}
+
+// acc[m] += X(rows r0 + 16 m ..) * B(columns n0 ..) for the MTW row tiles of a
+// wavefront, K a multiple of 32.  Every fragment of a K chunk is loaded before
+// the chunk's products.
+template <int MODE, int MTW>
+__device__ __forceinline__ void mlp_gemm(const MlpLds<MODE>& X, int r0, int K, const char* packed, size_t off_hi,
+                                         size_t off_lo, int ldb, bool bt, int n0,
+                                         typename MT<MODE>::T (&acc)[MTW][4]) {
     const int l = wave_lane();
     const int row = l & 15, grp = l >> 4;
     if constexpr (MODE == PT_MLP_F64) {
-        pt_d4 c[2];
+        (void)off_lo;
+        pt_d4 c[MTW];
 #pragma unroll
-        for (int t = 0; t < 2; ++t) c[t] = pt_d4{acc[t][0], acc[t][1], acc[t][2], acc[t][3]};
+        for (int m = 0; m < MTW; ++m) c[m] = pt_d4{0.0, 0.0, 0.0, 0.0};
         const double* W = (const double*)(packed + off_hi);
-#pragma unroll 2
-        for (int k0 = 0; k0 < K; k0 += 4) {
-            const int k = k0 + grp;
-            const double av = A[row * stride + k];
-            double b[2];
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                const int n = n0 + 16 * t + row;
-                b[t] = t < nt ? (bt ? W[(size_t)n * ldb + k] : W[(size_t)k * ldb + n]) : 0.0;
-            }
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-                if (t < nt) c[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, b[t], c[t], 0, 0, 0);
-        }
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            acc[t][0] = c[t][0]; acc[t][1] = c[t][1]; acc[t][2] = c[t][2]; acc[t][3] = c[t][3];
-        }
-    } else {
-        pt_f4 c[2];
-#pragma unroll
-        for (int t = 0; t < 2; ++t) c[t] = pt_f4{acc[t][0], acc[t][1], acc[t][2], acc[t][3]};
-        const unsigned short* Bh = (const unsigned short*)(packed + off_hi);
-        const unsigned short* Bl = (const unsigned short*)(packed + off_lo);
+        // bt == false: B[k][n] = W[k][n] (W is K x ldb);  bt == true: B[k][n] = W[n][k]
+        const double* Wl = bt ? W + (size_t)(n0 + row) * ldb + grp : W + (size_t)grp * ldb + n0 + row;
+        const size_t ks = bt ? 4 : (size_t)4 * ldb;
+        const double* A = X.x + (r0 + row) * X.stride + grp;
         for (int k0 = 0; k0 < K; k0 += 32) {
-            const int kb = k0 + 8 * grp;
-            // B fragments: 8 consecutive k of column n0 + 16 t + row (k-contiguous layout)
-            uint4 vh[2], vl[2];
+            double b[8];
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                vh[t] = make_uint4(0u, 0u, 0u, 0u);
-                vl[t] = vh[t];
-                if (t < nt) {
-                    const size_t bo = (size_t)(n0 + 16 * t + row) * ldb + kb;
-                    vh[t] = *reinterpret_cast<const uint4*>(Bh + bo);
-                    if (MODE == PT_MLP_BF16X3) vl[t] = *reinterpret_cast<const uint4*>(Bl + bo);
-                }
-            }
-            pt_bf8 ah, al;
-            const float* ap = A + row * stride + kb;
+            for (int u = 0; u < 8; ++u) b[u] = Wl[(size_t)(k0 / 4 + u) * ks];
 #pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                unsigned short hi, lo;
-                split_bf16(ap[q], hi, lo);
-                ah[q] = __builtin_bit_cast(__bf16, hi);
-                al[q] = __builtin_bit_cast(__bf16, lo);
-            }
+            for (int u = 0; u < 8; ++u)
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                if (t < nt) {
-                    const pt_bf8 bh = __builtin_bit_cast(pt_bf8, vh[t]);
-                    const pt_bf8 bl = __builtin_bit_cast(pt_bf8, vl[t]);
-                    c[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bh, c[t], 0, 0, 0);
-                    if (MODE == PT_MLP_BF16X3) {
-                        c[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bl, c[t], 0, 0, 0);
-                        c[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh, c[t], 0, 0, 0);
-                    }
+                for (int m = 0; m < MTW; ++m)
+                    c[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(A[16 * m * X.stride + k0 + 4 * u], b[u], c[m], 0, 0, 0);
+        }
+#pragma unroll
+        for (int m = 0; m < MTW; ++m)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[m][i] = c[m][i];
+    } else {
+        (void)bt;
+        pt_f4 c[MTW];
+#pragma unroll
+        for (int m = 0; m < MTW; ++m) c[m] = pt_f4{0.f, 0.f, 0.f, 0.f};
+        // B fragment: 8 consecutive k of column n0 + row, from the k-contiguous layout
+        const size_t bo = (size_t)(n0 + row) * ldb + 8 * grp;
+        const unsigned short* Bh = (const unsigned short*)(packed + off_hi) + bo;
+        const unsigned short* Bl = (const unsigned short*)(packed + off_lo) + bo;
+        const int ao = (r0 + row) * X.stride + 8 * grp;
+        for (int k0 = 0; k0 < K; k0 += 32) {
+            const pt_bf8 bh = __builtin_bit_cast(pt_bf8, *reinterpret_cast<const uint4*>(Bh + k0));
+            const pt_bf8 bl = MODE == PT_MLP_BF16X3 ? __builtin_bit_cast(pt_bf8, *reinterpret_cast<const uint4*>(Bl + k0))
+                                                    : pt_bf8{};
+#pragma unroll
+            for (int m = 0; m < MTW; ++m) {
+                const int o = ao + 16 * m * X.stride + k0;
+                const pt_bf8 ah = __builtin_bit_cast(pt_bf8, *reinterpret_cast<const uint4*>(X.hi + o));
+                c[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bh, c[m], 0, 0, 0);
+                if (MODE == PT_MLP_BF16X3) {
+                    const pt_bf8 al = __builtin_bit_cast(pt_bf8, *reinterpret_cast<const uint4*>(X.lo + o));
+                    c[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bl, c[m], 0, 0, 0);
+                    c[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh, c[m], 0, 0, 0);
                 }
             }
         }
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            acc[t][0] = c[t][0]; acc[t][1] = c[t][1]; acc[t][2] = c[t][2]; acc[t][3] = c[t][3];
-        }
+        for (int m = 0; m < MTW; ++m)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[m][i] = c[m][i];
     }
-    (void)bt;
 }
 
-// Lanes over the cells of a 16-row tile, for elementwise passes: a chunk of 64
-// columns gives lane l column k0 + l of all 16 rows; a last chunk of 32 columns
-// (widths are multiples of 32) gives lanes 32-63 the odd rows, 8 rows each.
-struct TileCols {
-    int k;       // this lane's column
-    int r0;      // first row
-    int rstep;   // row step
-    int nr;      // rows per lane (16 or 8)
-};
-
-__device__ __forceinline__ TileCols tile_cols(int k0, int width) {
-    const int l = wave_lane();
-    if (width - k0 >= kWave) return TileCols{k0 + l, 0, 1, 16};
-    return TileCols{k0 + (l & 31), l >> 5, 2, 8};
+// sum over the 16 lanes of a DPP row (the 16 columns of a C tile), in every lane
+__device__ __forceinline__ float row16_sum(float v) {
+    v += dpp_f32<kDppXor1, 0xF>(v);
+    v += dpp_f32<kDppXor2, 0xF>(v);
+    v += dpp_f32<kDppHalfMirror, 0xF>(v);
+    v += dpp_f32<kDppMirror, 0xF>(v);
+    return v;
+}
+__device__ __forceinline__ double row16_sum(double v) {
+    v += dpp_f64<kDppXor1, 0xF>(v);
+    v += dpp_f64<kDppXor2, 0xF>(v);
+    v += dpp_f64<kDppHalfMirror, 0xF>(v);
+    v += dpp_f64<kDppMirror, 0xF>(v);
+    return v;
 }
 
-template <int MODE>
+// f(0), ..., f(N - 1) with compile-time indices (the layer loops index register arrays)
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+    if constexpr (N > 0) {
+        static_for<N - 1>(f);
+        f(std::integral_constant<int, N - 1>{});
+    }
+}
+
+template <int CT, int WC, int MTW>
+constexpr int mlp_rows() { return 16 * MTW * (4 / WC); }
+
+// HM: most hidden layers; hidden layers have at most 16 CT WC columns (padded).
+template <int MODE, int CT, int WC, int MTW, int HM>
 __global__ __launch_bounds__(256) void k_mlp(MlpArgs a) {
     typedef typename MT<MODE>::T T;
+    constexpr int ROWS = mlp_rows<CT, WC, MTW>();
     extern __shared__ __align__(16) char smem[];
-    const MlpShape& s = a.s;
+    __shared__ T esum[WC][ROWS];
+    int gi = 0;
+    while (gi + 1 < a.n_net && (int)blockIdx.x >= a.net[gi + 1].block0) ++gi;
+    const MlpNet& net = a.net[gi];
+    const MlpShape& s = net.s;
+    const int stride = a.stride;
+    // the two LDS buffers of layer inputs, swapped after each layer
+    MlpLds<MODE> X = mlp_lds<MODE>(smem, ROWS, stride);
+    MlpLds<MODE> Y = mlp_lds<MODE>(smem + MlpLds<MODE>::bytes(ROWS, stride), ROWS, stride);
+    auto swap_xy = [&]() { const MlpLds<MODE> t = X; X = Y; Y = t; };
     const int l = wave_lane();
     const int wv = uniform(threadIdx.x >> 6);
-    const int wpb = blockDim.x >> 6;
-    const int stride = a.stride;
-    T* base = reinterpret_cast<T*>(smem) + (size_t)wv * ((size_t)a.nbuf * 16 * stride + 16);
-    // 16-row buffers: the input in slot 0, hidden output h in slot ys(h)
-    // (slot 1, then slot 0 once the input is dead, then 2, 3, ...).  With
-    // a.inplace the derivative of layer h replaces its output in place after
-    // layer h + 1 has read it (max(2, H) slots); otherwise it has a slot of
-    // its own after those.
-    const int H = s.n_hidden;
-    const int ny = H > 2 ? H : 2;
-    auto ys = [](int h) { return h == 0 ? 1 : (h == 1 ? 0 : h); };
-    T* D[kMaxHidden];                              // activation derivatives
-    for (int h = 0; h < kMaxHidden; ++h)
-        D[h] = base + (size_t)(a.inplace ? ys(h) : ny + h) * 16 * stride;
-    T* gout = base + (size_t)a.nbuf * 16 * stride;  // 16 output derivatives
-    const T* wout = (MODE == PT_MLP_F64) ? (const T*)(a.packed + s.wout64) : (const T*)(a.packed + s.wout32);
-    const T bout = (MODE == PT_MLP_F64) ? (T)((const double*)(a.packed + s.bout64))[0]
-                                        : (T)((const float*)(a.packed + s.bout32))[0];
-
+    const int wc = wv % WC;
+    const int r0 = (wv / WC) * 16 * MTW;     // this wavefront's first row
     const int row = l & 15, grp = l >> 4;
-    const int ntiles = (a.n_atoms + 15) / 16;
-    for (int tile = blockIdx.x * wpb + wv; tile < ntiles; tile += gridDim.x * wpb) {
-        const int a0 = tile * 16;
-        // 1. scaled input -> slot 0 (zero padded): every row's load of a
-        //    column is issued before the first store
-        for (int k0 = 0; k0 < s.in_p; k0 += kWave) {
-            const TileCols tc = tile_cols(k0, s.in_p);
-            const int k = tc.k;
-            const bool col_ok = k < s.in_dim;
-            const double sub = col_ok ? a.scale[k] : 0.0;
-            const double mul = col_ok ? a.scale[s.in_dim + k] : 0.0;
-            for (int j0 = 0; j0 < tc.nr; j0 += 8) {
-                double g[8];
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const int atom = a0 + tc.r0 + (j0 + j) * tc.rstep;
-                    g[j] = 0.0;
-                    if (col_ok && atom < a.n_atoms)
-                        g[j] = a.g_f64 ? ((const double*)a.G)[(size_t)atom * a.ldg + k]
-                                       : (double)((const float*)a.G)[(size_t)atom * a.ldg + k];
-                }
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const int r = tc.r0 + (j0 + j) * tc.rstep;
-                    base[r * stride + k] = (col_ok && a0 + r < a.n_atoms) ? (T)((g[j] - sub) * mul + a.scale_add)
-                                                                         : T(0);
-                }
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
+    const int a0 = ((int)blockIdx.x - net.block0) * ROWS;
+    const char* packed = net.packed;
+    const int H = s.n_hidden;
+    const T* wout = (MODE == PT_MLP_F64) ? (const T*)(packed + s.wout64) : (const T*)(packed + s.wout32);
+    const T bout = (MODE == PT_MLP_F64) ? (T)((const double*)(packed + s.bout64))[0]
+                                        : (T)((const float*)(packed + s.bout32))[0];
+    auto g_at = [&](int atom, int k) {
+        const size_t o = (size_t)atom * a.ldg + k;
+        return a.g_f64 ? ((const double*)net.G)[o] : (double)((const float*)net.G)[o];
+    };
 
-        // 2. hidden layers, 32 columns (two MFMA tiles) at a time
-        int kin = s.in_p;
-        T* xin = base;
-        for (int h = 0; h < H; ++h) {
+    // 1. scaled input, zero padded: 32 columns x 8 rows per step
+    for (int k0 = 0; k0 < s.in_p; k0 += 32) {
+        const int k = k0 + (threadIdx.x & 31);
+        const bool ok = k < s.in_dim;
+        const double sub = ok ? net.scale[k] : 0.0, mul = ok ? net.scale[s.in_dim + k] : 0.0;
+        double g[ROWS / 8];
+#pragma unroll
+        for (int j = 0; j < ROWS / 8; ++j) {
+            const int atom = a0 + (threadIdx.x >> 5) + 8 * j;
+            g[j] = ok && atom < net.n_atoms ? g_at(atom, k) : 0.0;
+        }
+#pragma unroll
+        for (int j = 0; j < ROWS / 8; ++j) {
+            const int r = (threadIdx.x >> 5) + 8 * j;
+            X.put(r, k, ok && a0 + r < net.n_atoms ? (T)((g[j] - sub) * mul + net.scale_add) : T(0));
+        }
+    }
+    __syncthreads();
+
+    // 2. hidden layers; part: this lane's share of the output layer's dot product
+    T D[HM][CT][MTW][4];                     // activation derivatives
+    T part[MTW][4] = {};
+    int kin = s.in_p;
+    static_for<HM>([&](auto hc) {
+        constexpr int h = decltype(hc)::value;
+        if (h < H) {
             const int wp = s.wp[h];
-            const int act = s.act[h];
-            T* yout = base + (size_t)ys(h) * 16 * stride;
-            for (int n0 = 0; n0 < wp; n0 += 32) {
-                const int nt = min(2, (wp - n0) >> 4);
-                T acc[2][4] = {};
-                if (MODE == PT_MLP_F64)
-                    gemm_cols<MODE>(xin, stride, kin, a.packed, s.W64[h], 0, wp, false, n0, nt, acc);
-                else
-                    gemm_cols<MODE>(xin, stride, kin, a.packed, s.WTh[h], s.WTl[h], kin, true, n0, nt, acc);
 #pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    if (t < nt) {
-                        const int col = n0 + 16 * t + row;
-                        const T bias = (MODE == PT_MLP_F64) ? (T)((const double*)(a.packed + s.b64[h]))[col]
-                                                            : (T)((const float*)(a.packed + s.b32[h]))[col];
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const int r = crow<MODE>(grp, i);
-                            T y, dy;
-                            activate<T>(act, acc[t][i] + bias, y, dy);
-                            if (col >= s.w[h]) { y = T(0); dy = T(0); }
-                            yout[r * stride + col] = y;
-                            if (!a.inplace) D[h][r * stride + col] = dy;
-                        }
-                    }
-                }
-            }
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            if (a.inplace && h > 0) {
-                // layer h has read the output of layer h - 1: turn it into its derivative
-                const int wq = s.wp[h - 1], wt = s.w[h - 1], aq = s.act[h - 1];
-                for (int k0 = 0; k0 < wq; k0 += kWave) {
-                    const TileCols tc = tile_cols(k0, wq);
-                    for (int j0 = 0; j0 < tc.nr; j0 += 8) {
-                        T v[8];
-#pragma unroll
-                        for (int j = 0; j < 8; ++j) v[j] = D[h - 1][(tc.r0 + (j0 + j) * tc.rstep) * stride + tc.k];
-#pragma unroll
-                        for (int j = 0; j < 8; ++j)
-                            D[h - 1][(tc.r0 + (j0 + j) * tc.rstep) * stride + tc.k] =
-                                tc.k < wt ? dact_from_output<T>(aq, v[j]) : T(0);
-                    }
-                }
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-            }
-            xin = yout;
-            kin = wp;
-        }
-        T* xlast = xin;
-
-        // 3. output layer (width 1): 4 lanes per atom, lane part takes k = part + 4 j
-        {
-            const int r = l >> 2, part = l & 3;
-            T sum = T(0);
-            for (int j0 = 0; j0 < kin; j0 += 32) {
-                T w[8], x[8];
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const int k = j0 + part + 4 * j;
-                    w[j] = k < kin ? wout[k] : T(0);
-                    x[j] = k < kin ? xlast[r * stride + k] : T(0);
-                }
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    if (j0 + part + 4 * j < kin) sum += x[j] * w[j];
-            }
-            sum += __shfl_xor(sum, 1, kWave);
-            sum += __shfl_xor(sum, 2, kWave);
-            T y, dy;
-            activate<T>(s.act_out, sum + bout, y, dy);
-            if (part == 0) {
-                gout[r] = dy;
-                if (a0 + r < a.n_atoms) a.e_atom[a0 + r] = (double)y;
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        if (!a.dEdG) continue;
-
-        // 4. backward: dZ of the last hidden layer in place in D[h]
-        if (s.n_hidden > 0) {
-            const int h = s.n_hidden - 1;
-            const int wq = s.wp[h], wt = s.w[h], aq = s.act[h];
-            for (int k0 = 0; k0 < wq; k0 += kWave) {
-                const TileCols tc = tile_cols(k0, wq);
-                const T wk = wout[tc.k];
-                for (int j0 = 0; j0 < tc.nr; j0 += 8) {
-                    T v[8], go[8];
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) {
-                        const int r = tc.r0 + (j0 + j) * tc.rstep;
-                        v[j] = D[h][r * stride + tc.k];
-                        go[j] = gout[r];
-                    }
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) {
-                        // in place: the slot still holds the last hidden output
-                        const T dy = !a.inplace ? v[j] : (tc.k < wt ? dact_from_output<T>(aq, v[j]) : T(0));
-                        D[h][(tc.r0 + (j0 + j) * tc.rstep) * stride + tc.k] = dy * go[j] * wk;
-                    }
-                }
-            }
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            for (int hh = h; hh >= 1; --hh) {
-                // dZ_{hh-1} = (dZ_hh . W_hh^T) * D[hh-1]
-                const int wprev = s.wp[hh - 1];
-                for (int n0 = 0; n0 < wprev; n0 += 32) {
-                    const int nt = min(2, (wprev - n0) >> 4);
-                    T acc[2][4] = {};
+            for (int ct = 0; ct < CT; ++ct) {
+                const int n0 = 16 * (wc + WC * ct);
+                T z[MTW][4] = {}, dz[MTW][4] = {};
+                const int col = n0 + row;
+                if (n0 < s.w[h]) {
+                    T acc[MTW][4];
                     if (MODE == PT_MLP_F64)
-                        gemm_cols<MODE>(D[hh], stride, s.wp[hh], a.packed, s.W64[hh], 0, s.wp[hh], true, n0, nt, acc);
+                        mlp_gemm<MODE, MTW>(X, r0, kin, packed, s.W64[h], 0, wp, false, n0, acc);
                     else
-                        gemm_cols<MODE>(D[hh], stride, s.wp[hh], a.packed, s.Wh[hh], s.Wl[hh], s.wp[hh], true, n0,
-                                        nt, acc);
+                        mlp_gemm<MODE, MTW>(X, r0, kin, packed, s.WTh[h], s.WTl[h], kin, true, n0, acc);
+                    const T bias = (MODE == PT_MLP_F64) ? (T)((const double*)(packed + s.b64[h]))[col]
+                                                        : (T)((const float*)(packed + s.b32[h]))[col];
+                    const bool pad = col >= s.w[h];
 #pragma unroll
-                    for (int t = 0; t < 2; ++t)
-                        if (t < nt) {
+                    for (int m = 0; m < MTW; ++m) {
 #pragma unroll
-                            for (int i = 0; i < 4; ++i)
-                                D[hh - 1][crow<MODE>(grp, i) * stride + n0 + 16 * t + row] *= acc[t][i];
-                        }
-                }
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-            }
-        }
-        // 5. dE/dx' = dZ_0 . W_0^T (or wout for a linear model), then chain the scaler
-        for (int n0 = 0; n0 < s.in_p; n0 += 32) {
-            const int nt = min(2, (s.in_p - n0) >> 4);
-            T acc[2][4] = {};
-            if (s.n_hidden > 0) {
-                if (MODE == PT_MLP_F64)
-                    gemm_cols<MODE>(D[0], stride, s.wp[0], a.packed, s.W64[0], 0, s.wp[0], true, n0, nt, acc);
-                else
-                    gemm_cols<MODE>(D[0], stride, s.wp[0], a.packed, s.Wh[0], s.Wl[0], s.wp[0], true, n0, nt, acc);
-            } else {
+                        for (int i = 0; i < 4; ++i) z[m][i] = acc[m][i] + bias;
+                        activate_n<T, 4>(s.act[h], z[m], dz[m]);
 #pragma unroll
-                for (int t = 0; t < 2; ++t)
-                    if (t < nt) {
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) acc[t][i] = gout[crow<MODE>(grp, i)] * wout[n0 + 16 * t + row];
+                        for (int i = 0; i < 4; ++i) { z[m][i] = pad ? T(0) : z[m][i]; dz[m][i] = pad ? T(0) : dz[m][i]; }
                     }
-            }
+                }
+                const T wk = (h == H - 1 && n0 < wp) ? wout[col] : T(0);
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                const int k = n0 + 16 * t + row;
-                if (t < nt && k < s.in_dim) {
-                    const double mk = a.scale[s.in_dim + k];
+                for (int m = 0; m < MTW; ++m)
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        const int atom = a0 + crow<MODE>(grp, i);
-                        if (atom < a.n_atoms) {
-                            const double gk = (double)acc[t][i] * mk;
-                            if (a.g_f64) ((double*)a.dEdG)[(size_t)atom * a.ldg + k] = gk;
-                            else ((float*)a.dEdG)[(size_t)atom * a.ldg + k] = (float)gk;
-                        }
+                        D[h][ct][m][i] = dz[m][i];
+                        if (h == H - 1) part[m][i] += z[m][i] * wk;
+                        else if (n0 < wp) Y.put(r0 + 16 * m + crow<MODE>(grp, i), col, z[m][i]);
                     }
-                }
+            }
+            if (h < H - 1) {
+                __syncthreads();
+                swap_xy();
+                kin = wp;
             }
         }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
+    });
+    if (H == 0) {   // linear model: the scaled input itself
+        for (int n0 = 16 * wc; n0 < s.in_p; n0 += 16 * WC) {
+            const int k = n0 + row;
+            if (k < s.in_dim) {
+                const double sub = net.scale[k], mul = net.scale[s.in_dim + k];
+#pragma unroll
+                for (int m = 0; m < MTW; ++m)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const int atom = a0 + r0 + 16 * m + crow<MODE>(grp, i);
+                        if (atom < net.n_atoms) part[m][i] += (T)((g_at(atom, k) - sub) * mul + net.scale_add) * wout[k];
+                    }
+            }
+        }
+    }
+
+    // 3. output layer (width 1): 16 columns by DPP, the WC column sets through LDS
+    T go[MTW][4];                            // output derivatives of this lane's rows
+#pragma unroll
+    for (int m = 0; m < MTW; ++m)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const T v = row16_sum(part[m][i]);
+            if (row == 0) esum[wc][r0 + 16 * m + crow<MODE>(grp, i)] = v;
+        }
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < MTW; ++m) {
+        T y[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = r0 + 16 * m + crow<MODE>(grp, i);
+            y[i] = esum[0][r];
+#pragma unroll
+            for (int q = 1; q < WC; ++q) y[i] += esum[q][r];
+            y[i] += bout;
+        }
+        activate_n<T, 4>(s.act_out, y, go[m]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = r0 + 16 * m + crow<MODE>(grp, i);
+            if (wc == 0 && row == 0 && a0 + r < net.n_atoms) net.e_atom[a0 + r] = (double)y[i];
+        }
+    }
+    if (!net.dEdG) return;
+
+    // 4. reverse sweep: dZ of layer h goes through LDS, the derivatives come from registers
+    static_for<HM>([&](auto hc) {
+        constexpr int h = HM - 1 - decltype(hc)::value;
+        constexpr int hn = h + 1 < HM ? h + 1 : h;
+        if (h < H) {
+            const int wp = s.wp[h];
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) {
+                const int n0 = 16 * (wc + WC * ct);
+                if (n0 < wp) {
+                    T acc[MTW][4];
+                    if (h == H - 1) {
+                        const T wk = wout[n0 + row];
+#pragma unroll
+                        for (int m = 0; m < MTW; ++m)
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) acc[m][i] = go[m][i] * wk;
+                    } else if (n0 < s.w[h]) {
+                        // dZ_h = (dZ_{h+1} . W_{h+1}^T) * D[h]
+                        const int wn = s.wp[hn];
+                        if (MODE == PT_MLP_F64)
+                            mlp_gemm<MODE, MTW>(X, r0, wn, packed, s.W64[hn], 0, wn, true, n0, acc);
+                        else
+                            mlp_gemm<MODE, MTW>(X, r0, wn, packed, s.Wh[hn], s.Wl[hn], wn, true, n0, acc);
+                    } else {
+#pragma unroll
+                        for (int m = 0; m < MTW; ++m)
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) acc[m][i] = T(0);
+                    }
+#pragma unroll
+                    for (int m = 0; m < MTW; ++m)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            Y.put(r0 + 16 * m + crow<MODE>(grp, i), n0 + row, D[h][ct][m][i] * acc[m][i]);
+                }
+            }
+            __syncthreads();
+            swap_xy();
+        }
+    });
+    // 5. dE/dx' = dZ_0 . W_0^T (or wout for a linear model), then chain the scaler
+    for (int n0 = 16 * wc; n0 < s.in_p; n0 += 16 * WC) {
+        const int k = n0 + row;
+        if (n0 >= s.in_dim) break;
+        T acc[MTW][4];
+        if (H > 0) {
+            if (MODE == PT_MLP_F64)
+                mlp_gemm<MODE, MTW>(X, r0, s.wp[0], packed, s.W64[0], 0, s.wp[0], true, n0, acc);
+            else
+                mlp_gemm<MODE, MTW>(X, r0, s.wp[0], packed, s.Wh[0], s.Wl[0], s.wp[0], true, n0, acc);
+        } else {
+#pragma unroll
+            for (int m = 0; m < MTW; ++m)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[m][i] = go[m][i] * wout[k];
+        }
+        if (k < s.in_dim) {
+            const double mk = net.scale[s.in_dim + k];
+#pragma unroll
+            for (int m = 0; m < MTW; ++m)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int atom = a0 + r0 + 16 * m + crow<MODE>(grp, i);
+                    if (atom < net.n_atoms) {
+                        const double gk = (double)acc[m][i] * mk;
+                        const size_t o = (size_t)atom * a.ldg + k;
+                        if (a.g_f64) ((double*)net.dEdG)[o] = gk;
+                        else ((float*)net.dEdG)[o] = (float)gk;
+                    }
+                }
+        }
     }
 }
 
@@ -1166,26 +1208,56 @@ __global__ void k_adam(int n, double* __restrict__ p, const double* __restrict__
     p[i] = p[i] - lr * (mh / (sqrt(vh) + eps) + wd * p[i]);
 }
 
-template <int MODE>
-int launch_mlp(MlpArgs a, hipStream_t st) {
+template <int MODE, int CT, int WC, int MTW, int HM>
+int launch_mlp_cfg(MlpArgs& a, hipStream_t st) {
     typedef typename MT<MODE>::T T;
-    a.stride = a.s.wmax + (sizeof(T) == 8 ? 1 : 4);
-    a.inplace = 1;
-    for (int h = 0; h < a.s.n_hidden; ++h) a.inplace = a.inplace && act_from_output(a.s.act[h]);
-    const int ny = a.s.n_hidden > 2 ? a.s.n_hidden : 2;
-    a.nbuf = ny + (a.inplace ? 0 : a.s.n_hidden);
-    // nbuf activation buffers of 16 rows plus 16 output derivatives
-    const size_t per_wave = sizeof(T) * ((size_t)a.nbuf * 16 * a.stride + 16);
-    const size_t budget = lds_limit();
-    if (per_wave > budget) {
-        set_error("mlp: layer widths need %zu bytes of LDS per wavefront", per_wave);
+    constexpr int ROWS = mlp_rows<CT, WC, MTW>();
+    int wmax = 0, blocks = 0;
+    for (int g = 0; g < a.n_net; ++g) {
+        wmax = std::max(wmax, a.net[g].s.wmax);
+        a.net[g].block0 = blocks;
+        blocks += (a.net[g].n_atoms + ROWS - 1) / ROWS;
+    }
+    // FP64 rows an odd number of 8-byte words apart; BF16 rows 16 bytes (a fragment) past a multiple of 64
+    a.stride = wmax + (sizeof(T) == 8 ? 1 : 8);
+    const size_t bytes = 2 * MlpLds<MODE>::bytes(ROWS, a.stride);
+    if (bytes + sizeof(T) * WC * ROWS > lds_limit()) {
+        set_error("mlp: layer widths need %zu bytes of LDS per workgroup", bytes);
         return PT_ERR_UNSUPPORTED;
     }
-    const int wpb = (int)std::min<size_t>(4, budget / per_wave);
-    const int ntiles = (a.n_atoms + 15) / 16;
-    const int blocks = std::max(1, std::min((ntiles + wpb - 1) / wpb, 8192));
-    hipLaunchKernelGGL(k_mlp<MODE>, dim3(blocks), dim3(64 * wpb), wpb * per_wave, st, a);
+    hipLaunchKernelGGL((k_mlp<MODE, CT, WC, MTW, HM>), dim3(blocks), dim3(256), bytes, st, a);
     return launch_check("k_mlp");
+}
+
+// Shape of the workgroup by the launch's rows.  Below the lines: 16 rows per
+// workgroup, a column tile per wavefront, for the most wavefronts in flight.
+// Above: 32 rows per workgroup, so that a weight fragment serves two row tiles;
+// narrow FP64 networks (hidden layers of at most two column tiles, which leave
+// wavefronts idle) split 64 rows over the four wavefronts instead.
+// Measured, us per launch (16 rows | the other shape):
+//   52-64-64-1 FP64      12,288 rows 26.9 | 31.5   32,768 rows 58.8 | 53.9   98,304 rows 153 | 137
+//   52-64-64-1 BF16x3    12,288 rows 12.2 | 14.6   32,768 rows 23.0 | 19.2   98,304 rows 58.8 | 50.0
+//   34-16-16-1 FP64      12,288 rows 12.8 | 17.8   32,768 rows 29.4 | 24.5   98,304 rows 78.3 | 65.0
+//   34-16-16-1 BF16x3    32,768 rows 11.4 | 15.7   65,536 rows 21.0 | 19.6   98,304 rows 29.6 | 33.8 (16 rows stay)
+// (64 rows per workgroup for the wide networks, 54.7 us at 98,304 rows in
+// BF16x3, never won.)  One wavefront per 16 rows took 66 / 28 / 32 / 17 us for
+// any size up to 12,288 rows and 245 / 85 / 117 / 42 us at 98,304.
+constexpr long long kMlpWideRows = 20480, kMlpNarrowRows = 24576;
+
+template <int MODE>
+int launch_mlp(MlpArgs& a, hipStream_t st) {
+    int wp = 0, hid = 0;
+    long long n = 0;
+    for (int g = 0; g < a.n_net; ++g) {
+        const MlpShape& s = a.net[g].s;
+        for (int h = 0; h < s.n_hidden; ++h) wp = std::max(wp, s.wp[h]);
+        hid = std::max(hid, s.n_hidden);
+        n += a.net[g].n_atoms;
+    }
+    if (wp > 64) return launch_mlp_cfg<MODE, 2, 4, 1, 3>(a, st);
+    if (MODE == PT_MLP_F64 && wp <= 32 && n >= kMlpNarrowRows) return launch_mlp_cfg<PT_MLP_F64, 2, 1, 1, 3>(a, st);
+    if (hid <= 2 && wp > 32 && n >= kMlpWideRows) return launch_mlp_cfg<MODE, 1, 4, 2, 2>(a, st);
+    return launch_mlp_cfg<MODE, 1, 4, 1, 3>(a, st);
 }
 
 }  // namespace
@@ -1212,33 +1284,51 @@ extern "C" int pt_mlp_pack(const pt_mlp_desc* desc, const double* params, void* 
     return launch_check("pt_mlp_pack");
 }
 
+extern "C" int pt_mlp_energy_grad_multi(int mode, int n_jobs, const pt_mlp_job* jobs, int ldg, int g_precision,
+                                        pt_stream_t stream) {
+    PT_REQUIRE(n_jobs >= 0 && (jobs || n_jobs == 0), "pt_mlp_energy_grad: bad job list");
+    PT_REQUIRE(g_precision == PT_F64 || g_precision == PT_F32, "pt_mlp_energy_grad: bad precision");
+    PT_REQUIRE(mode == PT_MLP_F64 || mode == PT_MLP_BF16 || mode == PT_MLP_BF16X3, "pt_mlp_energy_grad: unknown mode %d",
+               mode);
+    hipStream_t st = (hipStream_t)stream;
+    MlpArgs a{};
+    a.ldg = ldg;
+    a.g_f64 = g_precision == PT_F64;
+    for (int j = 0; j < n_jobs; ++j) {
+        const pt_mlp_job& q = jobs[j];
+        PT_REQUIRE(q.n_atoms >= 0, "pt_mlp_energy_grad: n_atoms < 0");
+        if (q.n_atoms > 0) {
+            PT_REQUIRE(q.G && q.scale && q.desc && q.packed && q.e_atom, "pt_mlp_energy_grad: null argument");
+            MlpNet& t = a.net[a.n_net];
+            if (int rc = make_shape(q.desc, t.s)) return rc;
+            PT_REQUIRE(ldg >= q.desc->in_dim, "pt_mlp_energy_grad: ldg < in_dim");
+            t.n_atoms = q.n_atoms;
+            t.G = q.G;
+            t.scale = q.scale;
+            t.scale_add = q.desc->scale_add;
+            t.packed = (const char*)q.packed;
+            t.e_atom = q.e_atom;
+            t.dEdG = q.dEdG;
+            ++a.n_net;
+        }
+        if (a.n_net == kMlpNets || (j == n_jobs - 1 && a.n_net > 0)) {
+            const int rc = mode == PT_MLP_F64    ? launch_mlp<PT_MLP_F64>(a, st)
+                           : mode == PT_MLP_BF16 ? launch_mlp<PT_MLP_BF16>(a, st)
+                                                 : launch_mlp<PT_MLP_BF16X3>(a, st);
+            if (rc) return rc;
+            a.n_net = 0;
+        }
+    }
+    return PT_OK;
+}
+
 extern "C" int pt_mlp_energy_grad(int mode, int n_atoms, const void* G, int ldg, int g_precision,
                                   const double* scale, const pt_mlp_desc* desc, const void* packed,
                                   double* e_atom, void* dEdG, pt_stream_t stream) {
     PT_REQUIRE(n_atoms >= 0, "pt_mlp_energy_grad: n_atoms < 0");
     if (n_atoms == 0) return PT_OK;
-    PT_REQUIRE(G && scale && desc && packed && e_atom, "pt_mlp_energy_grad: null argument");
-    PT_REQUIRE(g_precision == PT_F64 || g_precision == PT_F32, "pt_mlp_energy_grad: bad precision");
-    MlpArgs a{};
-    if (int rc = make_shape(desc, a.s)) return rc;
-    PT_REQUIRE(ldg >= desc->in_dim, "pt_mlp_energy_grad: ldg < in_dim");
-    a.n_atoms = n_atoms;
-    a.G = G;
-    a.ldg = ldg;
-    a.g_f64 = g_precision == PT_F64;
-    a.scale = scale;
-    a.scale_add = desc->scale_add;
-    a.packed = (const char*)packed;
-    a.e_atom = e_atom;
-    a.dEdG = dEdG;
-    hipStream_t st = (hipStream_t)stream;
-    switch (mode) {
-    case PT_MLP_F64: return launch_mlp<PT_MLP_F64>(a, st);
-    case PT_MLP_BF16: return launch_mlp<PT_MLP_BF16>(a, st);
-    case PT_MLP_BF16X3: return launch_mlp<PT_MLP_BF16X3>(a, st);
-    }
-    set_error("pt_mlp_energy_grad: unknown mode %d", mode);
-    return PT_ERR_ARG;
+    const pt_mlp_job job{n_atoms, G, scale, desc, packed, e_atom, dEdG};
+    return pt_mlp_energy_grad_multi(mode, 1, &job, ldg, g_precision, stream);
 }
 
 extern "C" size_t pt_mlp_param_count(const pt_mlp_desc* desc) {

@@ -14,9 +14,9 @@ Per structure the descriptors G and the centre-only tangents T_a = dG_i/dr_ia
 (a = x, y, z) do not depend on the weights and are built once.  An update
 then runs
 
-    energy:  pt_mlp_energy_grad, pt_reduce_sum_f64, pt_kalman_residual,
+    energy:  pt_mlp_energy_grad_multi, pt_reduce_sum_f64, pt_kalman_residual,
              H = (1/N) sum_i dE_i/dW           pt_mlp_train_grad
-    force:   pt_mlp_energy_grad, pt_acsf_adjoint (self term),
+    force:   pt_mlp_energy_grad_multi, pt_acsf_adjoint (self term),
              pt_kalman_residual, H = dF/dW      pt_mlp_jacobian
     both:    pt_kalman_update (rocBLAS GEMMs + rocSOLVER Cholesky), pt_mlp_pack
 
@@ -36,6 +36,7 @@ import numpy as np
 
 from . import _lib
 from .engine import NeighborList, Reducer, acsf_adjoint, acsf_forward, acsf_tangent, gather_rows
+from .models import energy_grad_multi
 from .potential import NNPSettings, NeuralNetworkPotential
 
 
@@ -196,9 +197,8 @@ class KalmanFilter:
 
     # ---- observations ----------------------------------------------------------------------
     def _energy(self, it: _Item):
-        for e, b, cnt, _ in it.blocks:
-            self.mlps[e].energy_grad(_lib.PT_MLP_F64, cnt, it.G[b:], self.ld, _lib.PT_F64, self.e_atom[b:],
-                                     self.dEdG[b:])
+        energy_grad_multi(_lib.PT_MLP_F64, [(self.mlps[e], cnt, it.G[b:], self.e_atom[b:], self.dEdG[b:])
+                                            for e, b, cnt, _ in it.blocks], self.ld, _lib.PT_F64)
         return self.reducer.sum(self.e_atom[:it.n])
 
     def calculate_loss_energy(self, it: _Item):

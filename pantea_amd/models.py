@@ -179,3 +179,12 @@ class DeviceMLP:
             mode, n_atoms, G.data_ptr(), ldg, g_precision, self.scale.data_ptr(), ctypes.byref(self.desc),
             self.packed.data_ptr(), e_atom.data_ptr(), None if dEdG is None else dEdG.data_ptr(),
             _lib.stream_ptr()), "pt_mlp_energy_grad")
+
+
+def energy_grad_multi(mode: int, jobs, ldg: int, g_precision: int) -> None:
+    """energy_grad of several elements in one launch: ``jobs`` are (mlp, n_atoms, G, e_atom, dEdG)."""
+    arr = (_lib.MlpJob * len(jobs))(*[
+        _lib.MlpJob(n, G.data_ptr(), m.scale.data_ptr(), ctypes.pointer(m.desc), m.packed.data_ptr(), e.data_ptr(),
+                    None if d is None else d.data_ptr()) for m, n, G, e, d in jobs])
+    _lib.check(_lib.load().pt_mlp_energy_grad_multi(mode, len(jobs), arr, ldg, g_precision, _lib.stream_ptr()),
+               "pt_mlp_energy_grad_multi")

@@ -13,7 +13,7 @@ Extensions:
   energy_and_forces(structure, mode)            both from one evaluation
 
 One evaluation = neighbour build (pt_nbr_build) -> per element descriptors
-(pt_acsf_forward) -> scaler + MLP + dE/dG (pt_mlp_energy_grad) -> FP64 energy
+(pt_acsf_forward) -> scaler + MLP + dE/dG (pt_mlp_energy_grad_multi) -> FP64 energy
 sum (pt_reduce_sum_f64) -> adjoint (pt_acsf_adjoint) -> scatter-free force
 gather (pt_force_gather).
 """
@@ -33,7 +33,8 @@ from .atoms import ElementMap
 from .descriptors import (ACSF, G1, G2, G3, G9, CutoffFunction, DescriptorScaler, NeighborElements,
                           ScalerParams)
 from .engine import (NeighborList, Reducer, acsf_adjoint, acsf_forward, force_gather, scatter_rows)
-from .models import MLP_MODES, DeviceMLP, ModelParams, NeuralNetworkModel, UniformInitializer
+from .models import (MLP_MODES, DeviceMLP, ModelParams, NeuralNetworkModel, UniformInitializer,
+                     energy_grad_multi)
 
 # n2p2 / RuNNer keyword codes (settings.py:43-80)
 _CUTOFF_BY_CODE = {"0": "hard", "1": "cos", "2": "tanhu", "3": "tanh", "4": "exp", "5": "poly1", "6": "poly2"}
@@ -241,8 +242,8 @@ class _Evaluation:
     def energy(self, pot):
         for e, b, cnt in self._blocks(pot):
             acsf_forward(self.nl, self.tables[e], self.g_prec, cnt, center_begin=b, out=self.G[b:], ld=self.ld)
-            self.mlps[e].energy_grad(self.mlp_mode, cnt, self.G[b:], self.ld, self.g_prec,
-                                     self.e_atom[b:], self.dEdG[b:])
+        energy_grad_multi(self.mlp_mode, [(self.mlps[e], cnt, self.G[b:], self.e_atom[b:], self.dEdG[b:])
+                                          for e, b, cnt in self._blocks(pot)], self.ld, self.g_prec)
         return self.reducer.sum(self.e_atom)
 
     def forces(self, pot, full: bool):

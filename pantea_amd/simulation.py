@@ -39,6 +39,7 @@ from . import _lib
 from .atoms import ElementMap, host_box
 from .engine import (NeighborList, Reducer, acsf_adjoint, acsf_forward, force_gather, force_gather_transposed,
                      gather_rows, scatter_rows)
+from .models import energy_grad_multi
 from .potential import PRECISION_MODES, NeuralNetworkPotential
 from .units import units
 
@@ -119,9 +120,8 @@ class _ForceField:
             acsf_forward(nl, tab, self.g_prec, cnt, center_begin=b, out=self.G[b:], ld=self.ld)
         mark("acsf_forward", False)
         mark("mlp", True)
-        for e, b, cnt in blocks:
-            self.mlps[e].energy_grad(self.mlp_mode, cnt, self.G[b:], self.ld, self.g_prec, self.e_atom[b:],
-                                     self.dEdG[b:])
+        energy_grad_multi(self.mlp_mode, [(self.mlps[e], cnt, self.G[b:], self.e_atom[b:], self.dEdG[b:])
+                                          for e, b, cnt in blocks], self.ld, self.g_prec)
         mark("mlp", False)
         if with_energy:
             self.energy = self.reducer.sum(self.e_atom)

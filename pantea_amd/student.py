@@ -7,7 +7,7 @@ Pipeline:
   2. ``StudentTrainer``: per snapshot the student's neighbour list and
      descriptors are built once (positions are fixed); every optimisation
      step then runs, per structure,
-        MLP energy + dE/dG          pt_mlp_energy_grad
+        MLP energy + dE/dG          pt_mlp_energy_grad_multi
         E = sum_i E_i               pt_reduce_sum_f64
         F = -J^T dE/dG              pt_acsf_adjoint + pt_force_gather
         delta = dL/dF, dL/dE        pt_train_seeds
@@ -34,6 +34,7 @@ import numpy as np
 from . import _lib
 from .atoms import Structure
 from .engine import NeighborList, Reducer, acsf_adjoint, acsf_forward, acsf_tangent, force_gather, gather_rows
+from .models import energy_grad_multi
 from .potential import PRECISION_MODES, NeuralNetworkPotential
 from .units import units
 
@@ -185,9 +186,8 @@ class StudentTrainer:
     def _energy_forces(self, sn: Snapshot):
         """Student E (device scalar) and F (internal order) of a snapshot."""
         n = sn.n
-        for el, b, cnt in sn.blocks:
-            self.mlps[el].energy_grad(self.mlp_mode, cnt, sn.G[b:], self.ld, self.g_prec, self.e_atom[b:],
-                                      self.dEdG[b:])
+        energy_grad_multi(self.mlp_mode, [(self.mlps[el], cnt, sn.G[b:], self.e_atom[b:], self.dEdG[b:])
+                                          for el, b, cnt in sn.blocks], self.ld, self.g_prec)
         E = self.reducer.sum(self.e_atom[:n])
         for el, b, cnt in sn.blocks:
             acsf_adjoint(sn.nl, self._table(sn, el), self.g_prec, cnt, self.dEdG[b:], self.ld, center_begin=b,
