@@ -263,6 +263,39 @@ int pt_acsf_tangent(int precision, const double *pos4, const double *box,
                     void *T, int ldt, pt_stream_t stream);
 
 /* ------------------------------------------------------------------------
+ * Several tables (or tangent directions) in one launch.  A run is a set of
+ * centres that share a table: n_centers centres center_begin, ... or
+ * centers[] (device), kind = pt_sf_table_kind of the table, its rows of out
+ * (G or T), w and f_self (as in the single-table calls; unused members may be
+ * NULL).  delta == NULL in a center_only tangent means the unit vector of
+ * direction dir (0, 1, 2).  boxes (device, 3 lengths per structure; 0: not
+ * periodic) with box_id (device, a structure index per atom) replaces box for
+ * lists that hold several structures.  rev == NULL: edge_grad in the edges'
+ * own slots (pt_acsf_adjoint), else transposed (pt_acsf_adjoint_transposed).
+ * ---------------------------------------------------------------------- */
+typedef struct {
+    const pt_sf_table *table;
+    int kind;
+    int n_centers;
+    int center_begin;
+    int dir;
+    const int *centers;
+    void *out;
+    const void *w;
+    double *f_self;
+    const double *delta;
+} pt_acsf_run;
+int pt_acsf_forward_multi(int precision, const double *pos4, const double *box, const long long *row_off,
+                          const int *nbr, int max_row, int n_runs, const pt_acsf_run *runs, int ldg,
+                          pt_stream_t stream);
+int pt_acsf_adjoint_multi(int precision, const double *pos4, const double *box, const double *boxes,
+                          const int *box_id, const long long *row_off, const int *nbr, const int *rev, int max_row,
+                          int n_runs, const pt_acsf_run *runs, int ldw, void *edge_grad, pt_stream_t stream);
+int pt_acsf_tangent_multi(int precision, const double *pos4, const double *box, const double *boxes,
+                          const int *box_id, const long long *row_off, const int *nbr, int max_row, int n_runs,
+                          const pt_acsf_run *runs, int center_only, int ldt, pt_stream_t stream);
+
+/* ------------------------------------------------------------------------
  * (c) Atomic MLP of one element on matrix cores: scaler + dense layers +
  * output, and the input gradient.  Replaces _compute_energy_per_atom
  * (potentials/nnp/energy.py:23-39) = scaler (descriptors/scaler.py:206-246)

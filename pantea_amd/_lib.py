@@ -92,6 +92,11 @@ class MlpJob(ctypes.Structure):
                 ("packed", _vp), ("e_atom", _vp), ("dEdG", _vp)]
 
 
+class AcsfRun(ctypes.Structure):
+    _fields_ = [("table", _vp), ("kind", _c_int), ("n_centers", _c_int), ("center_begin", _c_int), ("dir", _c_int),
+                ("centers", _vp), ("out", _vp), ("w", _vp), ("f_self", _vp), ("delta", _vp)]
+
+
 class PermuteArray(ctypes.Structure):
     _fields_ = [("buf", _vp), ("width", _c_int), ("word_bytes", _c_int)]
 
@@ -121,6 +126,12 @@ _SIGS = {
                                  _vp, _c_int, _vp, _c_int, _vp]),
     "pt_acsf_adjoint_transposed": (_c_int, [_c_int, _vp, _vp, _vp, _vp, _vp, _c_int, _c_int, _c_int, _vp, _vp,
                                             _vp, _c_int, _vp, _vp, _vp]),
+    "pt_acsf_forward_multi": (_c_int, [_c_int, _vp, _vp, _vp, _vp, _c_int, _c_int, ctypes.POINTER(AcsfRun), _c_int,
+                                       _vp]),
+    "pt_acsf_adjoint_multi": (_c_int, [_c_int, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _c_int, _c_int,
+                                       ctypes.POINTER(AcsfRun), _c_int, _vp, _vp]),
+    "pt_acsf_tangent_multi": (_c_int, [_c_int, _vp, _vp, _vp, _vp, _vp, _vp, _c_int, _c_int,
+                                       ctypes.POINTER(AcsfRun), _c_int, _c_int, _vp]),
     "pt_force_gather": (_c_int, [_c_int, _vp, _vp, _vp, _c_int, _vp, _vp]),
     "pt_force_gather_transposed": (_c_int, [_c_int, _vp, _vp, _vp, _c_int, _vp, _vp]),
     "pt_mlp_packed_bytes": (_c_size, [_vp]),

@@ -1,6 +1,7 @@
 // (b) ACSF descriptors, their adjoint and their tangent on gfx950.
 //
-// One wavefront (64 lanes) per centre.  The centre's neighbour row is staged
+// One wavefront (64 lanes) per centre, or kTeam wavefronts per centre when a
+// launch has too few centres to fill the chip.  The centre's neighbour row is staged
 // in LDS (relative vectors R_ij = r_i - r_j under the minimum image with r_ij
 // or 1/r_ij, and per mode the cutoff values), compacted to r_ij <= rc_max and
 // r_ij > 0 (atoms/neighbor.py:102-107).  Rows arrive sorted by type, so each
@@ -32,6 +33,7 @@
 // displacement field delta forward: T_is = sum_m dG_is/dr_m . delta_m.
 #include <algorithm>
 #include <cmath>
+#include <cstddef>
 
 #include "common.h"
 
@@ -260,7 +262,7 @@ struct Stage {
     R* D;          // [3][cap] TAN: delta_i - delta_j
     double* DA;    // [cap][3] ADJ: per-edge accumulators (FP64: fast LDS atomics; x, y, z
                    // adjacent so the three adds of an edge share one address)
-    unsigned long long* keep;   // ADJ: the staging ballots, one per 64 row entries
+    unsigned long long* keep;   // ADJ and teams: the staging ballots, one per 64 row entries
     unsigned* queue;
     R* W;          // ADJ, FP64: the group's dE/dG weights (read by broadcast)
 };
@@ -270,27 +272,32 @@ struct Stage {
 // edge positions come back from the staging ballots): the LDS per wave then
 // allows three waves per SIMD in FP64 and four and a half in FP32.
 
-template <typename R, int MODE>
+template <typename R, int MODE, int WPC>
 __host__ __device__ constexpr size_t stage_bytes_per_nbr() {
-    return MODE == MODE_ADJ ? sizeof(double) * 3 + sizeof(R) * 6
+    return MODE == MODE_ADJ ? sizeof(double) * 3 * WPC + sizeof(R) * 6
                             : sizeof(R) * (MODE == MODE_FWD ? 6 : 11);
 }
 
 // cap is a multiple of 4 and >= the row length; the per-wave area is a
 // multiple of 32 bytes
-template <typename R, int MODE>
+// (WPC wavefronts share the stage: each has a queue and, in the adjoint,
+// accumulators of its own -- added in a fixed order at the end, so that the
+// result does not depend on the wavefronts' timing -- and the staging ballots
+// are kept in every mode)
+template <typename R, int MODE, int WPC>
 __host__ __device__ constexpr size_t stage_bytes(int cap) {
-    return ((size_t)cap * stage_bytes_per_nbr<R, MODE>() + queue_len<MODE>() * sizeof(unsigned) +
-            (MODE == MODE_ADJ ? PT_AG_ETA * PT_AG_ANG * sizeof(R) +
-                                    (size_t)((cap + kWave - 1) / kWave) * sizeof(unsigned long long)
-                              : 0) + 31) / 32 * 32;
+    return ((size_t)cap * stage_bytes_per_nbr<R, MODE, WPC>() + WPC * queue_len<MODE>() * sizeof(unsigned) +
+            (MODE == MODE_ADJ ? PT_AG_ETA * PT_AG_ANG * sizeof(R) : 0) +
+            (MODE == MODE_ADJ || WPC > 1 ? (size_t)((cap + kWave - 1) / kWave) * sizeof(unsigned long long) : 0) +
+            31) / 32 * 32;
 }
 
-template <typename R, int MODE>
-__device__ __forceinline__ Stage<R> carve(char* base, int cap) {
+template <typename R, int MODE, int WPC>
+__device__ __forceinline__ Stage<R> carve(char* base, int cap, int sub) {
     Stage<R> s;
     char* p = base;
-    if (MODE == MODE_ADJ) { s.DA = reinterpret_cast<double*>(p); p += 3 * cap * sizeof(double); } else { s.DA = nullptr; }
+    s.DA = nullptr;
+    if (MODE == MODE_ADJ) { s.DA = reinterpret_cast<double*>(p) + 3 * cap * sub; p += 3 * cap * WPC * sizeof(double); }
     s.P = reinterpret_cast<V4<R>*>(p); p += cap * sizeof(V4<R>);
     s.Q = nullptr; s.Q2 = nullptr; s.QF = nullptr;
     if ((MODE == MODE_ADJ)) {
@@ -301,15 +308,15 @@ __device__ __forceinline__ Stage<R> carve(char* base, int cap) {
         s.Q = reinterpret_cast<V4<R>*>(p); p += cap * sizeof(V4<R>);
     }
     if (MODE == MODE_TAN) { s.D = reinterpret_cast<R*>(p); p += 3 * cap * sizeof(R); } else { s.D = nullptr; }
-    s.queue = reinterpret_cast<unsigned*>(p);
-    p += queue_len<MODE>() * sizeof(unsigned);
+    s.queue = reinterpret_cast<unsigned*>(p) + sub * queue_len<MODE>();
+    p += WPC * queue_len<MODE>() * sizeof(unsigned);
     s.W = nullptr;
     s.keep = nullptr;
     if (MODE == MODE_ADJ) {
         s.W = reinterpret_cast<R*>(p);
         p += PT_AG_ETA * PT_AG_ANG * sizeof(R);
-        s.keep = reinterpret_cast<unsigned long long*>(p);
     }
+    if (MODE == MODE_ADJ || WPC > 1) s.keep = reinterpret_cast<unsigned long long*>(p);
     return s;
 }
 
@@ -340,25 +347,83 @@ __device__ __forceinline__ int seg_below(int segv, int t) {
     return __builtin_amdgcn_readlane(segv, t < 0 ? 0 : (t > kSegTypes ? kSegTypes : t));
 }
 
+// One run of a launch: centres that share a descriptor table.
+struct KRun {
+    const pt_sf_table* table;
+    const int* centers;
+    void* out;            // FWD: G, TAN: T (n x ld)
+    const void* w;        // ADJ: dE/dG (n x ld)
+    double* f_self;       // ADJ (n x 3)
+    const double* delta;  // TAN (atoms x 3, internal order); nullptr: the unit vector of dir
+    int n, begin;
+    int item0;            // first work item of the run
+    int dir;
+};
+
+constexpr int kMaxRuns = 8;
+
 struct KArgs {
     const double* pos4;
     BoxArg box;
+    const double* boxes;  // when set: the box lengths of several structures, box_id of each atom
+    const int* box_id;
     const long long* row_off;
     const int* nbr;
-    int n_centers, center_begin;
-    const int* centers;
-    const pt_sf_table* table;
-    void* out;            // FWD: G, TAN: T (n_centers x ld)
     int ld;
-    const void* w;        // ADJ: dE/dG (n_centers x ldw)
-    int ldw;
-    double* f_self;       // ADJ (n_centers x 3)
     void* edge_grad;      // ADJ (n_pairs x 3)
     const int* rev;       // ADJ: when set, edge e's gradient goes to slot rev[e] (the reverse edge)
-    const double* delta;  // TAN (n x 3, internal order)
     int center_only;
     int cap;
+    int n_items, n_runs;
+    KRun run[kMaxRuns];
 };
+
+// A group of the table in registers: lane k holds the group's k-th 32-bit word
+// and its k-th double.  One load each (the fields follow by v_readlane),
+// where reading the fields one by one was a chain of ~35 dependent loads per
+// angular group -- most of a wavefront's latency for a short row.
+struct GroupWords {
+    int w;
+    double d;
+};
+
+template <typename G>
+__device__ __forceinline__ GroupWords group_words(const G* g) {
+    static_assert(sizeof(G) % 8 == 0 && sizeof(G) <= 4 * kWave, "a group fits one word per lane");
+    const int lane = wave_lane();
+    GroupWords r;
+    r.w = lane < (int)(sizeof(G) / 4) ? reinterpret_cast<const int*>(g)[lane] : 0;
+    r.d = lane < (int)(sizeof(G) / 8) ? reinterpret_cast<const double*>(g)[lane] : 0.0;
+    return r;
+}
+
+__device__ __forceinline__ int lane_word(int v, int k) { return __builtin_amdgcn_readlane(v, k); }
+__device__ __forceinline__ float lane_value(float v, int k) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), k));
+}
+__device__ __forceinline__ double lane_value(double v, int k) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(u & 0xffffffffu), k);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(u >> 32), k);
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+
+// word / double index of a field
+#define PT_WORD(type, field) ((int)(offsetof(type, field) / 4))
+#define PT_DBL(type, field) ((int)(offsetof(type, field) / 8))
+
+// all wavefronts of a centre
+template <int WPC>
+__device__ __forceinline__ void centre_sync() {
+    if constexpr (WPC == 1) wave_sync();
+    else __syncthreads();
+}
+
+__device__ __forceinline__ double uniform_f64(double v) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = (unsigned)uniform((int)(unsigned)(u & 0xffffffffu)), hi = (unsigned)uniform((int)(unsigned)(u >> 32));
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
 
 // Uniform description of one angular group inside the kernel.
 template <typename R>
@@ -409,10 +474,11 @@ __device__ __forceinline__ void ang_eval(const AngGroup<R>& X, R cs, R (&v)[PT_A
 
 // All unordered pairs {j, k} of one angular group: screening on r_jk, a
 // per-wave queue of live pairs, and the pair body in full-wave batches.
-template <typename R, int MODE, int CUT, int ANG>
+// The WPC wavefronts of a centre (sub: this one) take the screening steps in turn.
+template <typename R, int MODE, int CUT, int ANG, int WPC>
 __device__ __forceinline__ void angular_group(const Stage<R>& S, const AngGroup<R>& X,
                                               const R (&Win)[PT_AG_ETA][PT_AG_ANG],
-                                              R (&acc)[PT_AG_ETA][PT_AG_ANG], int cap) {
+                                              R (&acc)[PT_AG_ETA][PT_AG_ANG], int cap, int sub) {
     const int lane = wave_lane();
     constexpr int NA = ang_terms<ANG>();
     constexpr bool kPreOut = ANG != ANGK_GEN;   // pre applied outside the pair loop
@@ -444,7 +510,7 @@ __device__ __forceinline__ void angular_group(const Stage<R>& S, const AngGroup<
         }
     }
     if (kWLds) {
-        if (lane == 0) {
+        if (lane == 0 && sub == 0) {
 #pragma unroll
             for (int e = 0; e < PT_AG_ETA; ++e)
 #pragma unroll
@@ -454,7 +520,7 @@ __device__ __forceinline__ void angular_group(const Stage<R>& S, const AngGroup<
     // cutoff values of the group's neighbours
     for (int pass = 0; pass < (X.same ? 1 : 2); ++pass) {
         const int sb = pass == 0 ? X.bj : X.bk, sn = pass == 0 ? X.nj : X.nk;
-        for (int s = sb + lane; s < sb + sn; s += kWave) {
+        for (int s = sb + lane + sub * kWave; s < sb + sn; s += WPC * kWave) {
             R f, df;
             if constexpr ((MODE == MODE_ADJ)) {
                 const R ir = S.P[s].w;
@@ -472,7 +538,7 @@ __device__ __forceinline__ void angular_group(const Stage<R>& S, const AngGroup<
             }
         }
     }
-    wave_sync();
+    centre_sync<WPC>();
 
     // one live pair (ia, ib)
     auto body = [&](const int ia, const int ib) {
@@ -621,7 +687,7 @@ __device__ __forceinline__ void angular_group(const Stage<R>& S, const AngGroup<
     //    index is the diagonal k = (q + d) mod n_long, d = 0 .. n_long-1;
     //  - one segment: k = (q + 1 + d) mod n for d < n/2 -- each unordered
     //    pair once (see below for the last diagonal of an even n).
-    // Pair p = d * nrow + q; each lane advances p by 64 per step.
+    // Pair p = d * nrow + q; each lane advances p by 64 WPC per step.
     const bool jrow = X.nj <= X.nk;
     const int nrow = X.same ? X.nj : (jrow ? X.nj : X.nk);
     const int ncol = X.same ? X.nj : (jrow ? X.nk : X.nj);
@@ -632,16 +698,18 @@ __device__ __forceinline__ void angular_group(const Stage<R>& S, const AngGroup<
     // q < n/2 is taken there
     const int h = X.same ? X.nj / 2 : ncol;
     const int npairs = nrow * h;
-    if (npairs <= 0) return;
+    if (npairs <= 0) return;   // (the same for every wavefront of the centre)
     const int half_d = (X.same && X.nj % 2 == 0) ? h - 1 : -1;   // the doubled diagonal
     const int half_q = X.nj / 2;
-    const int d64 = uniform(kWave / nrow), r64 = uniform(kWave - d64 * nrow);
-    int d = lane / nrow, q = lane - (lane / nrow) * nrow;
+    constexpr int kStep = kWave * WPC;
+    const int d64 = uniform(kStep / nrow), r64 = uniform(kStep - d64 * nrow);
+    const int p0 = WPC == 1 ? lane : lane + sub * kWave;
+    int d = p0 / nrow, q = p0 - (p0 / nrow) * nrow;
     // screen r_jk^2 < rc^2 (loosened by 1e-4 relative); the exact r_jk < rc
     // test is the cutoff's own (it is 0 beyond rc)
     const R rc2 = X.g3 ? X.rc * X.rc * R(1.0001) : R(INFINITY);
     const int sk = X.same ? 1 : 0;
-    int qn = 0, base = 0;
+    int qn = 0, base = WPC == 1 ? 0 : sub * kWave;
     // one batch of up to 64 queued pairs through the body; the rest moves up
     auto drain = [&]() {
         wave_sync();
@@ -700,7 +768,7 @@ __device__ __forceinline__ void angular_group(const Stage<R>& S, const AngGroup<
                 qn += __popcll(b);
                 if (qn >= kWave) drain();
             }
-            base += kWave;
+            base += kStep;
             q += r64;
             d += d64;
             if (q >= nrow) { q -= nrow; ++d; }
@@ -721,33 +789,49 @@ __device__ __forceinline__ void angular_group(const Stage<R>& S, const AngGroup<
 // 1 when the group's terms are exactly zeta {1, 4} x lambda {+1, -1} (any
 // order); qmap[k] then gives the term of canonical slot k = 2 [zeta = 4] +
 // [lambda = -1].
-__device__ __forceinline__ int z14_order(const pt_angular_group* G, int (&qmap)[PT_AG_ANG]) {
-    if (uniform(G->n_ang) != 4) return 0;
+__device__ __forceinline__ int z14_order(const GroupWords& G, int n_ang, int (&qmap)[PT_AG_ANG]) {
     int seen = 0;
 #pragma unroll
+    for (int q = 0; q < 4; ++q) qmap[q] = 0;
+#pragma unroll
     for (int q = 0; q < 4; ++q) {
-        const int iz = uniform(G->izeta[q]);
-        const double lam = G->lam[q];
-        if (!((iz == 1 || iz == 4) && (lam == 1.0 || lam == -1.0))) return 0;
-        const int k = (iz == 4 ? 2 : 0) + (lam < 0.0 ? 1 : 0);
+        const int iz = lane_word(G.w, PT_WORD(pt_angular_group, izeta) + q);
+        const double lam = lane_value(G.d, PT_DBL(pt_angular_group, lam) + q);
+        const bool ok = (iz == 1 || iz == 4) && (lam == 1.0 || lam == -1.0);
+        const int k = ok ? (iz == 4 ? 2 : 0) + (lam < 0.0 ? 1 : 0) : 4;
         seen |= 1 << k;
-        qmap[k] = q;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) qmap[t] = uniform(t == k ? q : qmap[t]);
     }
-    return seen == 15 ? 1 : 0;
+    return n_ang == 4 && uniform(seen) == 15 ? 1 : 0;
 }
 
-template <typename R, int MODE, int KIND>
-__device__ __forceinline__ void acsf_centre(const KArgs& a, char* smem) {
+// Shared between the wavefronts of a centre (beyond the stage).
+template <typename R, int WPC>
+struct Team {
+    R part[WPC][PT_AG_ETA * PT_AG_ANG];   // a group's sums of each wavefront
+    int seg[WPC][16];                     // segment counts of each wavefront's row chunks
+};
+template <typename R>
+struct Team<R, 1> {};
+
+template <typename R, int MODE, int KIND, int WPC>
+__device__ __forceinline__ void acsf_centre(const KArgs& a, char* smem, Team<R, WPC>& T) {
     if (sizeof(R) == 8) exp2_tab_load();
     const int lane = wave_lane();
     const int wv = uniform(threadIdx.x >> 6);
     const int wpb = blockDim.x >> 6;
-    const int c = uniform(xcd_block() * wpb + wv);
-    if (c >= a.n_centers) return;
+    const int sub = WPC == 1 ? 0 : wv;                                    // wavefront of this centre
+    const int item = uniform(WPC == 1 ? xcd_block() * wpb + wv : xcd_block());
+    if (item >= a.n_items) return;
+    int ri = 0;
+    while (ri + 1 < a.n_runs && item >= a.run[ri + 1].item0) ++ri;
+    const KRun& rn = a.run[ri];
+    const int c = item - rn.item0;
     const int cap = a.cap;
-    Stage<R> S = carve<R, MODE>(smem + (size_t)wv * stage_bytes<R, MODE>(cap), cap);
-    const pt_sf_table* __restrict__ tab = a.table;
-    const int i = uniform(a.centers ? a.centers[c] : a.center_begin + c);
+    Stage<R> S = carve<R, MODE, WPC>(WPC == 1 ? smem + (size_t)wv * stage_bytes<R, MODE, WPC>(cap) : smem, cap, sub);
+    const pt_sf_table* __restrict__ tab = rn.table;
+    const int i = uniform(rn.centers ? rn.centers[c] : rn.begin + c);
     const double4 pi = reinterpret_cast<const double4*>(a.pos4)[i];
     const long long off = a.row_off[i];
     const int len = (int)(a.row_off[i + 1] - off);
@@ -755,63 +839,84 @@ __device__ __forceinline__ void acsf_centre(const KArgs& a, char* smem) {
         // the row does not fit the staging slice sized by the caller's max_row:
         // stage nothing and report the centre as NaN (outputs, f_self, the row's edges)
         const R nan = __builtin_nan("");
+        const int t0 = lane + sub * kWave;
         if (MODE != MODE_ADJ) {
-            R* out = (R*)a.out;
-            for (int q = lane; q < a.ld; q += kWave) out[(size_t)c * a.ld + q] = nan;
+            R* out = (R*)rn.out;
+            for (int q = t0; q < a.ld; q += WPC * kWave) out[(size_t)c * a.ld + q] = nan;
         } else {
             if (a.edge_grad) {
                 R* eg = (R*)a.edge_grad;
-                for (int t = lane; t < len; t += kWave) {
+                for (int t = t0; t < len; t += WPC * kWave) {
                     const long long e = a.rev ? (long long)a.rev[off + t] : off + t;
                     if (e >= 0) { eg[3 * e] = nan; eg[3 * e + 1] = nan; eg[3 * e + 2] = nan; }
                 }
             }
-            if (a.f_self && lane < 3) a.f_self[3 * c + lane] = (double)nan;
+            if (rn.f_self && t0 < 3) rn.f_self[3 * c + t0] = (double)nan;
         }
         return;
+    }
+    BoxArg box = a.box;
+    if (a.boxes) {
+        const double* bl = a.boxes + 3 * (size_t)a.box_id[i];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            box.L[d] = uniform_f64(bl[d]);
+            box.half[d] = 0.5 * box.L[d];
+        }
+        box.periodic = uniform((box.L[0] > 0.0) ? 1 : 0);
     }
     const double rcmax = tab->rc_max;
     const R tanh_pre = (R)tab->tanh_pre;
     // |R_ij - R_ik| <= 2 rc_max: the image shift can only act when L/2 < 2 rc_max
     const double lim = 4.0 * rcmax * (1.0 + 1e-9);
-    const bool mic_jk = a.box.periodic && (!(a.box.L[0] > lim) || !(a.box.L[1] > lim) || !(a.box.L[2] > lim));
+    const bool mic_jk = box.periodic && (!(box.L[0] > lim) || !(box.L[1] > lim) || !(box.L[2] > lim));
 
     double dix = 0, diy = 0, diz = 0;
     if (MODE == MODE_TAN) {
-        dix = a.delta[3 * i]; diy = a.delta[3 * i + 1]; diz = a.delta[3 * i + 2];
+        if (rn.delta) {
+            dix = rn.delta[3 * i]; diy = rn.delta[3 * i + 1]; diz = rn.delta[3 * i + 2];
+        } else {
+            dix = rn.dir == 0; diy = rn.dir == 1; diz = rn.dir == 2;
+        }
     }
 
     // segment counts are needed up to one past the largest type the table uses
+    static_assert(PT_MAX_GROUPS <= kWave, "a lane per group");
+    const int n_rg = uniform(tab->n_rg), n_ag = uniform(tab->n_ag);
+    int tg = lane < n_rg ? tab->rg[lane].elem : 0;
+    if (lane < n_ag) tg = max(tg, max(tab->ag[lane].ej, tab->ag[lane].ek));
     int tmax = 0;
-    for (int g = 0; g < uniform(tab->n_rg); ++g) tmax = max(tmax, uniform(tab->rg[g].elem));
-    for (int g = 0; g < uniform(tab->n_ag); ++g)
-        tmax = max(tmax, max(uniform(tab->ag[g].ej), uniform(tab->ag[g].ek)));
+    while (tmax < kSegTypes && __ballot(tg > tmax) != 0ull) ++tmax;
     const int nseg = min(tmax + 1, kSegTypes);
 
     // ---- stage the row ----------------------------------------------------
-    int m = 0;
-    int seg = 0;   // lane q: staged neighbours with type < q
-    for (int t0 = 0; t0 < len; t0 += kWave) {
-        const int t = t0 + lane;
-        bool keep = false;
-        int j = 0;
-        double dx = 0, dy = 0, dz = 0, r = 0, tj = 0;
-        if (t < len) {
-            j = a.nbr[off + t];
-            const double4 pj = reinterpret_cast<const double4*>(a.pos4)[j];
-            dx = pi.x - pj.x; dy = pi.y - pj.y; dz = pi.z - pj.z;
-            r = exact_dist(dx, dy, dz, a.box);
-            tj = pj.w;
-            keep = (r <= rcmax) && (r > 0.0);
+    // one entry of a 64-entry chunk per lane
+    struct Entry {
+        double dx, dy, dz, r, tj;
+        int j;
+        bool in, keep;
+    };
+    auto load = [&](int t0) {
+        Entry e{0, 0, 0, 0, 0, 0, t0 + lane < len, false};
+        if (e.in) {
+            e.j = a.nbr[off + t0 + lane];
+            const double4 pj = reinterpret_cast<const double4*>(a.pos4)[e.j];
+            e.dx = pi.x - pj.x; e.dy = pi.y - pj.y; e.dz = pi.z - pj.z;
+            e.r = exact_dist(e.dx, e.dy, e.dz, box);
+            e.tj = pj.w;
+            e.keep = (e.r <= rcmax) && (e.r > 0.0);
         }
-        const unsigned long long bal = __ballot(keep);
-        if (MODE == MODE_ADJ && lane == 0) S.keep[t0 / kWave] = bal;
-        if (keep) {
+        return e;
+    };
+    int seg = 0;   // lane q: staged neighbours with type < q
+    // kept entries go to the slots m, m + 1, ...
+    auto store = [&](const Entry& e, int t0, unsigned long long bal, int m) {
+        if (e.keep) {
             const int s = m + lanes_below(bal);
             V4<R> pv, qv;
-            pv.x = (R)dx; pv.y = (R)dy; pv.z = (R)dz;
-            pv.w = (R)(1.0 / r);
-            qv.x = (R)r; qv.y = (R)r * (R)r; qv.z = R(0); qv.w = R(0);
+            pv.x = (R)e.dx; pv.y = (R)e.dy; pv.z = (R)e.dz;
+            pv.w = (R)(1.0 / e.r);
+            qv.x = (R)e.r; qv.y = (R)e.r * (R)e.r; qv.z = R(0); qv.w = R(0);
             S.P[s] = pv;
             if constexpr ((MODE == MODE_ADJ)) {
                 // (fc, dfc) are written per group
@@ -822,52 +927,91 @@ __device__ __forceinline__ void acsf_centre(const KArgs& a, char* smem) {
             } else {
                 S.Q[s] = qv;
             }
-            if (MODE == MODE_ADJ) { S.DA[3 * s] = 0.0; S.DA[3 * s + 1] = 0.0; S.DA[3 * s + 2] = 0.0; }
+            if (MODE == MODE_ADJ && WPC == 1) { S.DA[3 * s] = 0.0; S.DA[3 * s + 1] = 0.0; S.DA[3 * s + 2] = 0.0; }
             if (MODE == MODE_TAN) {
                 double ex = dix, ey = diy, ez = diz;
                 if (!a.center_only) {
-                    ex -= a.delta[3 * j]; ey -= a.delta[3 * j + 1]; ez -= a.delta[3 * j + 2];
+                    ex -= rn.delta[3 * e.j]; ey -= rn.delta[3 * e.j + 1]; ez -= rn.delta[3 * e.j + 2];
                 }
                 S.D[s] = (R)ex; S.D[cap + s] = (R)ey; S.D[2 * cap + s] = (R)ez;
             }
-        } else if (MODE == MODE_ADJ && t < len && a.edge_grad) {
+        } else if (MODE == MODE_ADJ && e.in && a.edge_grad) {
             // (a reverse index of -1 would mean an asymmetric list: no slot to write)
-            const long long e = a.rev ? (long long)a.rev[off + t] : off + t;
-            if (e >= 0) {
-                R* eg = (R*)a.edge_grad + 3 * e;
+            const long long k = a.rev ? (long long)a.rev[off + t0 + lane] : off + t0 + lane;
+            if (k >= 0) {
+                R* eg = (R*)a.edge_grad + 3 * k;
                 eg[0] = R(0); eg[1] = R(0); eg[2] = R(0);
             }
         }
-        m += __popcll(bal);
-        const int tk = (int)tj;
+        const int tk = (int)e.tj;
         for (int q = 1; q <= nseg; ++q) {
-            const int cq = __popcll(__ballot(keep && tk < q));
+            const int cq = __popcll(__ballot(e.keep && tk < q));
             seg += lane == q ? cq : 0;
         }
+    };
+    int m = 0;
+    if constexpr (WPC == 1) {
+        for (int t0 = 0; t0 < len; t0 += kWave) {
+            const Entry e = load(t0);
+            const unsigned long long bal = __ballot(e.keep);
+            if (MODE == MODE_ADJ && lane == 0) S.keep[t0 / kWave] = bal;
+            store(e, t0, bal, m);
+            m += __popcll(bal);
+        }
+        m = uniform(m);
+        wave_sync();
+    } else {
+        // chunks in turn; the ballots of all chunks first (a chunk's slots start after
+        // those of the chunks before it), the first chunk of a wavefront stays in registers
+        const Entry e0 = load(sub * kWave);
+        for (int t0 = sub * kWave; t0 < len; t0 += WPC * kWave) {
+            const unsigned long long bal = __ballot(t0 == sub * kWave ? e0.keep : load(t0).keep);
+            if (lane == 0) S.keep[t0 / kWave] = bal;
+        }
+        __syncthreads();
+        for (int t0 = 0; t0 < len; t0 += kWave) {
+            const unsigned long long bal = S.keep[t0 / kWave];
+            if (t0 / kWave % WPC == sub) store(t0 == sub * kWave ? e0 : load(t0), t0, bal, m);
+            m += __popcll(bal);
+        }
+        m = uniform(m);
+        if (MODE == MODE_ADJ)
+            for (int s = lane; s < 3 * m; s += kWave) S.DA[s] = 0.0;
+        if (lane < 16) T.seg[sub][lane] = seg;
+        __syncthreads();
+        seg = 0;
+        if (lane < 16) {
+#pragma unroll
+            for (int k = 0; k < WPC; ++k) seg += T.seg[k][lane];
+        }
     }
-    m = uniform(m);
-    wave_sync();
 
-    R* out = (R*)a.out;
-    const R* w = (const R*)a.w;
+    R* out = (R*)rn.out;
+    const R* w = (const R*)rn.w;
 
     // ---- radial groups -----------------------------------------------------
-    const int n_rg = uniform(tab->n_rg);
-    for (int g = 0; g < n_rg; ++g) {
-        const pt_radial_group* G = &tab->rg[g];
-        const int el = uniform(G->elem);
+    // (a team takes whole groups in turn: no sums across wavefronts)
+    for (int g = sub; g < n_rg; g += WPC) {
+        constexpr int kCol = PT_WORD(pt_radial_group, col), kEta = PT_DBL(pt_radial_group, eta),
+                      kRs = PT_DBL(pt_radial_group, rs), kRc = PT_DBL(pt_radial_group, rc);
+        const GroupWords G = group_words(&tab->rg[g]);
+        const int el = lane_word(G.w, PT_WORD(pt_radial_group, elem));
+        const int cut = lane_word(G.w, PT_WORD(pt_radial_group, cut));
+        const int nfun = lane_word(G.w, PT_WORD(pt_radial_group, n));
         const int b = seg_below(seg, el), e = seg_below(seg, el + 1);
-        const int nfun = uniform(G->n);
-        const int cut = uniform(G->cut);
-        const R rc = (R)G->rc, irc = (R)(1.0 / G->rc);
+        const R gr = (R)G.d;
+        const R rc = lane_value(gr, kRc), irc = lane_value((R)(1.0 / G.d), kRc);
+        const bool mine = lane >= kCol && lane < kCol + nfun;   // lane kCol + q: function q's column
+        R wl = R(0);
+        if (MODE == MODE_ADJ && mine) wl = w[(size_t)c * a.ld + G.w];
         R wgt[PT_RG_MAX], acc[PT_RG_MAX], keta[PT_RG_MAX], eta[PT_RG_MAX], rs[PT_RG_MAX];
 #pragma unroll
         for (int q = 0; q < PT_RG_MAX; ++q) {
             acc[q] = R(0);
-            eta[q] = (q < nfun) ? (R)G->eta[q] : R(0);
+            eta[q] = (q < nfun) ? lane_value(gr, kEta + q) : R(0);
             keta[q] = -eta[q] * M<R>::kexp;
-            rs[q] = (q < nfun) ? (R)G->rs[q] : R(0);
-            wgt[q] = (MODE == MODE_ADJ && q < nfun) ? w[(size_t)c * a.ldw + G->col[q]] : R(0);
+            rs[q] = (q < nfun) ? lane_value(gr, kRs + q) : R(0);
+            wgt[q] = MODE == MODE_ADJ ? lane_value(wl, kCol + q) : R(0);
         }
         for (int s = b + lane; s < e; s += kWave) {
             R r;
@@ -903,65 +1047,73 @@ __device__ __forceinline__ void acsf_centre(const KArgs& a, char* smem) {
             for (int q = 0; q < PT_RG_MAX; ++q)
                 if (q < nfun) {
                     const R v = wave_sum(acc[q]);
-                    if (lane == 0) out[(size_t)c * a.ld + G->col[q]] = v;
+                    wl = lane == kCol + q ? v : wl;
                 }
+            if (mine) out[(size_t)c * a.ld + G.w] = wl;
         }
         wave_sync();
     }
 
     // ---- angular groups ----------------------------------------------------
-    const int n_ag = uniform(tab->n_ag);
     bool bad = false;   // a group outside this kernel's table class
     for (int g = 0; g < n_ag; ++g) {
-        const pt_angular_group* G = &tab->ag[g];
+        typedef pt_angular_group AG;
+        constexpr int kCol = PT_WORD(AG, col), kCells = PT_AG_ETA * PT_AG_ANG;
+        const GroupWords G = group_words(&tab->ag[g]);
+        const R gr = (R)G.d;
         AngGroup<R> X;
-        const int ej = uniform(G->ej), ek = uniform(G->ek);
+        const int ej = lane_word(G.w, PT_WORD(AG, ej)), ek = lane_word(G.w, PT_WORD(AG, ek));
         X.bj = seg_below(seg, ej);
         X.nj = seg_below(seg, ej + 1) - X.bj;
         X.bk = seg_below(seg, ek);
         X.nk = seg_below(seg, ek + 1) - X.bk;
         X.same = ej == ek;
-        X.g3 = uniform(G->kind) == 3;
+        X.g3 = lane_word(G.w, PT_WORD(AG, kind)) == 3;
         X.mic = mic_jk;
-        X.n_eta = uniform(G->n_eta);
-        X.n_ang = uniform(G->n_ang);
-        X.cut = uniform(G->cut);
-        X.rc = (R)G->rc;
-        X.irc = (R)(1.0 / G->rc);
+        X.n_eta = lane_word(G.w, PT_WORD(AG, n_eta));
+        X.n_ang = lane_word(G.w, PT_WORD(AG, n_ang));
+        X.cut = lane_word(G.w, PT_WORD(AG, cut));
+        X.rc = lane_value(gr, PT_DBL(AG, rc));
+        X.irc = lane_value((R)(1.0 / G.d), PT_DBL(AG, rc));
         X.cpre = X.cut == PT_CUT_TANH ? tanh_pre : R(1);
         X.tanh_pre = tanh_pre;
-        X.box = &a.box;
+        X.box = &box;
         // qmap[k]: the table term evaluated in slot k (the identity, or the
         // canonical order of a ZETA {1, 4} x LAMBDA {+1, -1} group)
         int qmap[PT_AG_ANG];
-        const int z14 = (KIND == PT_ACSF_TANH_Z14) ? z14_order(G, qmap) : 0;
+        const int z14 = (KIND == PT_ACSF_TANH_Z14) ? z14_order(G, X.n_ang, qmap) : 0;
         if (!z14) {
 #pragma unroll
             for (int q = 0; q < PT_AG_ANG; ++q) qmap[q] = q;
         }
+        // lane kCol + cell holds the cell's column, its weight (adjoint) and its sum (forward, tangent)
+        const int cell = lane - kCol;
+        const bool mine = cell >= 0 && cell < kCells && cell / PT_AG_ANG < X.n_eta && cell % PT_AG_ANG < X.n_ang && G.w >= 0;
+        R wl = R(0);
+        if (MODE == MODE_ADJ && mine) wl = w[(size_t)c * a.ld + G.w];
+        const unsigned long long owned = __ballot(mine);
         R W[PT_AG_ETA][PT_AG_ANG], acc[PT_AG_ETA][PT_AG_ANG];
+        const R keta_l = (R)(-G.d * M<R>::kexp);
 #pragma unroll
         for (int e = 0; e < PT_AG_ETA; ++e) {
-            X.keta[e] = (e < X.n_eta) ? (R)(-G->eta[e] * M<R>::kexp) : R(0);
+            X.keta[e] = (e < X.n_eta) ? lane_value(keta_l, PT_DBL(AG, eta) + e) : R(0);
 #pragma unroll
             for (int q = 0; q < PT_AG_ANG; ++q) {
                 acc[e][q] = R(0);
-                const int col = G->col[e * PT_AG_ANG + qmap[q]];
-                W[e][q] = (MODE == MODE_ADJ && e < X.n_eta && q < X.n_ang && col >= 0)
-                              ? w[(size_t)c * a.ldw + col]
-                              : R(0);
+                W[e][q] = MODE == MODE_ADJ ? lane_value(wl, kCol + e * PT_AG_ANG + qmap[q]) : R(0);
             }
         }
+        const R zl_l = (R)(G.d * __shfl(G.d, lane + PT_DBL(AG, lam) - PT_DBL(AG, zeta)));   // zeta lambda, in zeta's lanes
         bool z1 = true, p4 = true;
 #pragma unroll
         for (int q = 0; q < PT_AG_ANG; ++q) {
             const bool on = q < X.n_ang;
             const int tq = qmap[q];
-            X.lam[q] = on ? (R)G->lam[tq] : R(0);
-            X.zeta[q] = on ? (R)G->zeta[tq] : R(1);
-            X.pre[q] = on ? (R)G->pre[tq] : R(0);
-            X.izeta[q] = on ? uniform(G->izeta[tq]) : 1;
-            X.zl[q] = on ? (R)(G->zeta[tq] * G->lam[tq]) : R(0);
+            X.lam[q] = on ? lane_value(gr, PT_DBL(AG, lam) + tq) : R(0);
+            X.zeta[q] = on ? lane_value(gr, PT_DBL(AG, zeta) + tq) : R(1);
+            X.pre[q] = on ? lane_value(gr, PT_DBL(AG, pre) + tq) : R(0);
+            X.izeta[q] = on ? lane_word(G.w, PT_WORD(AG, izeta) + tq) : 1;
+            X.zl[q] = on ? lane_value(zl_l, PT_DBL(AG, zeta) + tq) : R(0);
             z1 = z1 && X.izeta[q] == 1;
             p4 = p4 && (X.izeta[q] == 1 || X.izeta[q] == 2 || X.izeta[q] == 4);
         }
@@ -969,70 +1121,92 @@ __device__ __forceinline__ void acsf_centre(const KArgs& a, char* smem) {
                        : (X.cut == PT_CUT_COS ? CUTK_COS : CUTK_GEN);
         const int ak = z14 ? ANGK_Z14
                            : (z1 ? (X.n_ang <= 2 ? ANGK_Z1N2 : ANGK_Z1) : (p4 ? ANGK_P4 : ANGK_GEN));
-        wave_sync();
+        centre_sync<WPC>();   // the previous group's cutoff values are no longer read
         if constexpr (KIND == PT_ACSF_TANH_Z14) {
             if (ck == CUTK_TANH && ak == ANGK_Z14)
-                angular_group<R, MODE, CUTK_TANH, ANGK_Z14>(S, X, W, acc, cap);
+                angular_group<R, MODE, CUTK_TANH, ANGK_Z14, WPC>(S, X, W, acc, cap, sub);
             else
                 bad = true;
         } else if constexpr (KIND == PT_ACSF_TANH_P4) {
             if (ck == CUTK_TANH && ak != ANGK_GEN)
-                angular_group<R, MODE, CUTK_TANH, ANGK_P4>(S, X, W, acc, cap);
+                angular_group<R, MODE, CUTK_TANH, ANGK_P4, WPC>(S, X, W, acc, cap, sub);
             else
                 bad = true;
         } else if constexpr (KIND == PT_ACSF_TANH_Z1N2) {
             if (ck == CUTK_TANH && ak == ANGK_Z1N2)
-                angular_group<R, MODE, CUTK_TANH, ANGK_Z1N2>(S, X, W, acc, cap);
+                angular_group<R, MODE, CUTK_TANH, ANGK_Z1N2, WPC>(S, X, W, acc, cap, sub);
             else
                 bad = true;
         } else if (MODE == MODE_TAN || (sizeof(R) == 8 && ck != CUTK_TANH)) {
-            angular_group<R, MODE, CUTK_GEN, ANGK_GEN>(S, X, W, acc, cap);
+            angular_group<R, MODE, CUTK_GEN, ANGK_GEN, WPC>(S, X, W, acc, cap, sub);
         } else if (sizeof(R) == 8) {
-            if (ak == ANGK_GEN) angular_group<R, MODE, CUTK_TANH, ANGK_GEN>(S, X, W, acc, cap);
-            else angular_group<R, MODE, CUTK_TANH, ANGK_P4>(S, X, W, acc, cap);
+            if (ak == ANGK_GEN) angular_group<R, MODE, CUTK_TANH, ANGK_GEN, WPC>(S, X, W, acc, cap, sub);
+            else angular_group<R, MODE, CUTK_TANH, ANGK_P4, WPC>(S, X, W, acc, cap, sub);
         } else if (ck == CUTK_TANH) {
-            if (ak == ANGK_Z1N2) angular_group<R, MODE, CUTK_TANH, ANGK_Z1N2>(S, X, W, acc, cap);
-            else if (ak == ANGK_Z1) angular_group<R, MODE, CUTK_TANH, ANGK_Z1>(S, X, W, acc, cap);
-            else if (ak == ANGK_P4) angular_group<R, MODE, CUTK_TANH, ANGK_P4>(S, X, W, acc, cap);
-            else angular_group<R, MODE, CUTK_TANH, ANGK_GEN>(S, X, W, acc, cap);
+            if (ak == ANGK_Z1N2) angular_group<R, MODE, CUTK_TANH, ANGK_Z1N2, WPC>(S, X, W, acc, cap, sub);
+            else if (ak == ANGK_Z1) angular_group<R, MODE, CUTK_TANH, ANGK_Z1, WPC>(S, X, W, acc, cap, sub);
+            else if (ak == ANGK_P4) angular_group<R, MODE, CUTK_TANH, ANGK_P4, WPC>(S, X, W, acc, cap, sub);
+            else angular_group<R, MODE, CUTK_TANH, ANGK_GEN, WPC>(S, X, W, acc, cap, sub);
         } else if (ck == CUTK_COS) {
-            if (ak == ANGK_Z1N2) angular_group<R, MODE, CUTK_COS, ANGK_Z1N2>(S, X, W, acc, cap);
-            else if (ak == ANGK_Z1) angular_group<R, MODE, CUTK_COS, ANGK_Z1>(S, X, W, acc, cap);
-            else if (ak == ANGK_P4) angular_group<R, MODE, CUTK_COS, ANGK_P4>(S, X, W, acc, cap);
-            else angular_group<R, MODE, CUTK_COS, ANGK_GEN>(S, X, W, acc, cap);
+            if (ak == ANGK_Z1N2) angular_group<R, MODE, CUTK_COS, ANGK_Z1N2, WPC>(S, X, W, acc, cap, sub);
+            else if (ak == ANGK_Z1) angular_group<R, MODE, CUTK_COS, ANGK_Z1, WPC>(S, X, W, acc, cap, sub);
+            else if (ak == ANGK_P4) angular_group<R, MODE, CUTK_COS, ANGK_P4, WPC>(S, X, W, acc, cap, sub);
+            else angular_group<R, MODE, CUTK_COS, ANGK_GEN, WPC>(S, X, W, acc, cap, sub);
         } else {
-            angular_group<R, MODE, CUTK_GEN, ANGK_GEN>(S, X, W, acc, cap);
+            angular_group<R, MODE, CUTK_GEN, ANGK_GEN, WPC>(S, X, W, acc, cap, sub);
         }
 
         if (MODE != MODE_ADJ) {
             // reduce only the group's cells that own a column (uniform branches
-            // keep all lanes active)
+            // keep all lanes active); a team sums its wavefronts' parts in order
 #pragma unroll
             for (int e = 0; e < PT_AG_ETA; ++e)
 #pragma unroll
                 for (int q = 0; q < PT_AG_ANG; ++q) {
-                    const int col = (e < X.n_eta && q < X.n_ang) ? uniform(G->col[e * PT_AG_ANG + qmap[q]]) : -1;
-                    if (col >= 0) {
+                    const int k = kCol + e * PT_AG_ANG + qmap[q];
+                    if ((owned >> k) & 1ull) {
                         const R v = wave_sum(acc[e][q]);
-                        if (lane == 0) out[(size_t)c * a.ld + col] = v;
+                        wl = lane == k ? v : wl;
                     }
                 }
+            if constexpr (WPC > 1) {
+                if (mine) T.part[sub][cell] = wl;
+                __syncthreads();
+                if (mine && sub == 0) {
+#pragma unroll
+                    for (int k = 1; k < WPC; ++k) wl += T.part[k][cell];
+                }
+            }
+            if (mine && sub == 0) out[(size_t)c * a.ld + G.w] = wl;
         }
-        wave_sync();
+        if constexpr (WPC == 1) wave_sync();
     }
+    centre_sync<WPC>();
 
     const R nan = __builtin_nan("");
-    if (MODE != MODE_ADJ && bad) {
+    if (MODE != MODE_ADJ && bad && sub == 0) {
         for (int q = lane; q < a.ld; q += kWave) out[(size_t)c * a.ld + q] = nan;
     }
     if (MODE == MODE_ADJ) {
+        if constexpr (WPC > 1) {
+            // the wavefronts' accumulators, in order, into those of the first
+            double* D0 = S.DA - 3 * cap * sub;
+            for (int s = threadIdx.x; s < 3 * m; s += WPC * kWave) {
+                double v = D0[s];
+#pragma unroll
+                for (int k = 1; k < WPC; ++k) v += D0[3 * cap * k + s];
+                D0[s] = v;
+            }
+            S.DA = D0;
+            __syncthreads();
+        }
         if (a.edge_grad) {
             R* eg = (R*)a.edge_grad;
             // the staging ballots give each kept row entry its staged slot
             int ms = 0;
             for (int t0 = 0; t0 < len; t0 += kWave) {
                 const unsigned long long bal = S.keep[t0 / kWave];
-                if ((bal >> lane) & 1ull) {
+                if ((WPC == 1 || t0 / kWave % WPC == sub) && ((bal >> lane) & 1ull)) {
                     const int s = ms + lanes_below(bal);
                     const long long e = a.rev ? (long long)a.rev[off + t0 + lane] : off + t0 + lane;
                     if (e >= 0) {
@@ -1044,7 +1218,7 @@ __device__ __forceinline__ void acsf_centre(const KArgs& a, char* smem) {
                 ms += __popcll(bal);
             }
         }
-        if (a.f_self) {
+        if (rn.f_self && sub == 0) {
             // G_i depends on r_i only through R_ij = r_i - r_j, so dE_i/dr_i = -sum_j dE_i/dr_j
             // and F_self = -dE_i/dr_i = sum_j dE_i/dr_j, the per-edge accumulators
             double fx = 0.0, fy = 0.0, fz = 0.0;
@@ -1055,9 +1229,9 @@ __device__ __forceinline__ void acsf_centre(const KArgs& a, char* smem) {
             }
             const double sx = wave_sum(fx), sy = wave_sum(fy), sz = wave_sum(fz);
             if (lane == 0) {
-                a.f_self[3 * c + 0] = bad ? (double)nan : sx;
-                a.f_self[3 * c + 1] = bad ? (double)nan : sy;
-                a.f_self[3 * c + 2] = bad ? (double)nan : sz;
+                rn.f_self[3 * c + 0] = bad ? (double)nan : sx;
+                rn.f_self[3 * c + 1] = bad ? (double)nan : sy;
+                rn.f_self[3 * c + 2] = bad ? (double)nan : sz;
             }
         }
     }
@@ -1070,34 +1244,64 @@ __device__ __forceinline__ void acsf_centre(const KArgs& a, char* smem) {
 template <typename R, int MODE, int KIND>
 __global__ __launch_bounds__(256) void k_acsf(KArgs a) {
     extern __shared__ __align__(32) char smem[];
-    acsf_centre<R, MODE, KIND>(a, smem);
+    Team<R, 1> T;
+    acsf_centre<R, MODE, KIND, 1>(a, smem, T);
 }
 
 template <typename R, int MODE, int KIND>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_acsf_w4(KArgs a) {
     extern __shared__ __align__(32) char smem[];
-    acsf_centre<R, MODE, KIND>(a, smem);
+    Team<R, 1> T;
+    acsf_centre<R, MODE, KIND, 1>(a, smem, T);
 }
 
 template <typename R, int MODE, int KIND>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_acsf_w8(KArgs a) {
     extern __shared__ __align__(32) char smem[];
-    acsf_centre<R, MODE, KIND>(a, smem);
+    Team<R, 1> T;
+    acsf_centre<R, MODE, KIND, 1>(a, smem, T);
 }
+
+// A team of kTeam wavefronts per centre.
+constexpr int kTeam = 4;
+
+template <typename R, int MODE, int KIND>
+__global__ __launch_bounds__(64 * kTeam) void k_acsf_team(KArgs a) {
+    extern __shared__ __align__(32) char smem[];
+    __shared__ Team<R, kTeam> T;
+    acsf_centre<R, MODE, KIND, kTeam>(a, smem, T);
+}
+
+// Launches of at most this many centres run a team per centre; the line lies
+// where a SIMD would get about one wavefront and a half.  Rows of fewer than
+// kTeamRow entries leave a team little to share.  Measured, us per launch, one
+// wavefront | team of 4 (52 functions at 12 Bohr, ~110 neighbours; 34 at 8 Bohr, ~32):
+//   12 Bohr FP64 forward  96 centres 58.2 | 30.6   768 63.2 | 42.9   1,536 76.2 | 74.4   2,048 75.4 | 91.0
+//   12 Bohr FP64 adjoint  96 centres 65.9 | 32.4   768 72.4 | 46.0   1,536 92.4 | 83.3   2,048 93.9 | 98.7
+//   12 Bohr FP32 forward  96 centres 41.5 | 22.2   768 45.6 | 27.0   1,536 49.6 | 37.7   2,048 49.2 | 51.1
+//   8 Bohr FP32 forward   96 centres 16.6 | 15.0   768 17.8 | 17.9   1,536 19.6 | 23.9
+// (teams of 2 win 15 % between 1,500 and 2,000 centres, teams of 8 only below 100.)
+constexpr int kTeamLong = 1536, kTeamShort = 512, kTeamRow = 80;
 
 template <typename R, int MODE, int KIND>
 int launch(KArgs a, hipStream_t stream) {
-    if (a.n_centers <= 0) return PT_OK;
+    if (a.n_items <= 0) return PT_OK;
     a.cap = (std::max(a.cap, 1) + 3) / 4 * 4;
     if (a.cap > 65535) {
         set_error("acsf: neighbour rows longer than 65535 entries are not supported");
         return PT_ERR_UNSUPPORTED;
     }
-    const size_t per_wave = stage_bytes<R, MODE>(a.cap);
+    const size_t per_wave = stage_bytes<R, MODE, 1>(a.cap);
     const size_t lds_budget = lds_limit();
     if (per_wave > lds_budget) {
         set_error("acsf: neighbour row of %d entries exceeds the LDS budget", a.cap);
         return PT_ERR_UNSUPPORTED;
+    }
+    const size_t team = stage_bytes<R, MODE, kTeam>(a.cap);
+    // (a row that only fits the LDS without a team's extra arrays keeps one wavefront)
+    if (a.n_items <= (a.cap >= kTeamRow ? kTeamLong : kTeamShort) && team + sizeof(Team<R, kTeam>) + 512 <= lds_budget) {
+        hipLaunchKernelGGL((k_acsf_team<R, MODE, KIND>), dim3(a.n_items), dim3(64 * kTeam), team, stream, a);
+        return launch_check("k_acsf_team");
     }
     // waves per workgroup: the most resident waves per CU under the LDS limit,
     // ties to the smaller workgroup (a workgroup's LDS is held until its
@@ -1111,7 +1315,7 @@ int launch(KArgs a, hipStream_t stream) {
         const size_t waves = (size_t)w * (cu / ((size_t)w * per_wave));
         if (waves > best) { best = waves; wpb = w; }
     }
-    const int blocks = (a.n_centers + wpb - 1) / wpb;
+    const int blocks = (a.n_items + wpb - 1) / wpb;
     if constexpr (sizeof(R) == 8 && MODE == MODE_FWD && KIND != PT_ACSF_GENERIC)
         hipLaunchKernelGGL((k_acsf_w4<R, MODE, KIND>), dim3(blocks), dim3(64 * wpb), wpb * per_wave, stream, a);
     else if constexpr (sizeof(R) == 4 && MODE == MODE_FWD && (KIND == PT_ACSF_TANH_Z14 || KIND == PT_ACSF_TANH_Z1N2))
@@ -1121,46 +1325,55 @@ int launch(KArgs a, hipStream_t stream) {
     return launch_check("k_acsf");
 }
 
-template <typename R>
-int run_kind(int mode, int kind, KArgs& a, hipStream_t st) {
-    if (mode == MODE_TAN) {
-        switch (kind) {
-        case PT_ACSF_GENERIC: return launch<R, MODE_TAN, PT_ACSF_GENERIC>(a, st);
-        case PT_ACSF_TANH_P4: return launch<R, MODE_TAN, PT_ACSF_TANH_P4>(a, st);
-        case PT_ACSF_TANH_Z1N2: return launch<R, MODE_TAN, PT_ACSF_TANH_Z1N2>(a, st);
-        case PT_ACSF_TANH_Z14: return launch<R, MODE_TAN, PT_ACSF_TANH_Z14>(a, st);
-        }
-        set_error("acsf: unknown kernel kind %d", kind);
-        return PT_ERR_ARG;
-    }
+template <typename R, int MODE>
+int run_kind(int kind, const KArgs& a, hipStream_t st) {
     switch (kind) {
-    case PT_ACSF_GENERIC:
-        return mode == MODE_FWD ? launch<R, MODE_FWD, PT_ACSF_GENERIC>(a, st) : launch<R, MODE_ADJ, PT_ACSF_GENERIC>(a, st);
-    case PT_ACSF_TANH_P4:
-        return mode == MODE_FWD ? launch<R, MODE_FWD, PT_ACSF_TANH_P4>(a, st) : launch<R, MODE_ADJ, PT_ACSF_TANH_P4>(a, st);
-    case PT_ACSF_TANH_Z1N2:
-        return mode == MODE_FWD ? launch<R, MODE_FWD, PT_ACSF_TANH_Z1N2>(a, st)
-                                : launch<R, MODE_ADJ, PT_ACSF_TANH_Z1N2>(a, st);
-    case PT_ACSF_TANH_Z14:
-        return mode == MODE_FWD ? launch<R, MODE_FWD, PT_ACSF_TANH_Z14>(a, st)
-                                : launch<R, MODE_ADJ, PT_ACSF_TANH_Z14>(a, st);
+    case PT_ACSF_GENERIC: return launch<R, MODE, PT_ACSF_GENERIC>(a, st);
+    case PT_ACSF_TANH_P4: return launch<R, MODE, PT_ACSF_TANH_P4>(a, st);
+    case PT_ACSF_TANH_Z1N2: return launch<R, MODE, PT_ACSF_TANH_Z1N2>(a, st);
+    case PT_ACSF_TANH_Z14: return launch<R, MODE, PT_ACSF_TANH_Z14>(a, st);
     }
     set_error("acsf: unknown kernel kind %d", kind);
     return PT_ERR_ARG;
 }
 
-int run(int precision_kind, int mode, KArgs& a, hipStream_t st) {
-    const int precision = precision_kind & ((1 << PT_ACSF_KIND_SHIFT) - 1);
-    const int kind = precision_kind >> PT_ACSF_KIND_SHIFT;
-    if (precision == PT_F64) return run_kind<double>(mode, kind, a, st);
-    if (precision == PT_F32) return run_kind<float>(mode, kind, a, st);
-    set_error("acsf: unknown precision %d", precision);
-    return PT_ERR_ARG;
+// The runs of one table kind go into one launch (kMaxRuns at a time), in order.
+template <int MODE>
+int run_all(int precision, KArgs& a, int n_runs, const pt_acsf_run* runs, hipStream_t st) {
+    PT_REQUIRE(precision == PT_F64 || precision == PT_F32, "acsf: unknown precision %d", precision);
+    for (int r = 0; r < n_runs; ++r) {
+        PT_REQUIRE(runs[r].n_centers >= 0, "acsf: bad sizes");
+        PT_REQUIRE(runs[r].table, "acsf: null argument");
+    }
+    for (int r = 0; r < n_runs;) {
+        const int kind = runs[r].kind;
+        long long items = 0;
+        a.n_runs = 0;
+        for (; r < n_runs && runs[r].kind == kind && a.n_runs < kMaxRuns; ++r) {
+            const pt_acsf_run& q = runs[r];
+            if (q.n_centers == 0) continue;
+            KRun& k = a.run[a.n_runs++];
+            k.table = q.table;
+            k.centers = q.centers;
+            k.out = q.out;
+            k.w = q.w;
+            k.f_self = q.f_self;
+            k.delta = q.delta;
+            k.dir = q.dir;
+            k.n = q.n_centers;
+            k.begin = q.center_begin;
+            k.item0 = (int)items;
+            items += q.n_centers;
+        }
+        PT_REQUIRE(items < (1LL << 31), "acsf: too many centres in one launch");
+        a.n_items = (int)items;
+        const int rc = precision == PT_F64 ? run_kind<double, MODE>(kind, a, st) : run_kind<float, MODE>(kind, a, st);
+        if (rc) return rc;
+    }
+    return PT_OK;
 }
 
-KArgs common_args(const double* pos4, const double* box, const long long* row_off, const int* nbr,
-                  int max_row, int n_centers, int center_begin, const int* centers,
-                  const pt_sf_table* table) {
+KArgs common_args(const double* pos4, const double* box, const long long* row_off, const int* nbr, int max_row) {
     KArgs a{};
     a.pos4 = pos4;
     a.box.periodic = box != nullptr;
@@ -1170,30 +1383,65 @@ KArgs common_args(const double* pos4, const double* box, const long long* row_of
     }
     a.row_off = row_off;
     a.nbr = nbr;
-    a.n_centers = n_centers;
-    a.center_begin = center_begin;
-    a.centers = centers;
-    a.table = table;
     a.cap = max_row;
     return a;
 }
+
+// a run of the single-table entry points (their precision argument carries the table kind)
+pt_acsf_run single_run(int precision_kind, const pt_sf_table* table, int n_centers, int center_begin,
+                       const int* centers) {
+    pt_acsf_run r{};
+    r.table = table;
+    r.kind = precision_kind >> PT_ACSF_KIND_SHIFT;
+    r.n_centers = n_centers;
+    r.center_begin = center_begin;
+    r.centers = centers;
+    return r;
+}
+
+int base_precision(int precision_kind) { return precision_kind & ((1 << PT_ACSF_KIND_SHIFT) - 1); }
 
 }  // namespace
 }  // namespace pt
 
 using namespace pt;
 
+extern "C" int pt_acsf_forward_multi(int precision, const double* pos4, const double* box, const long long* row_off,
+                                     const int* nbr, int max_row, int n_runs, const pt_acsf_run* runs, int ldg,
+                                     pt_stream_t stream) {
+    PT_REQUIRE(pos4 && row_off && n_runs >= 0 && (runs || n_runs == 0), "pt_acsf_forward: null argument");
+    PT_REQUIRE(ldg >= 0, "pt_acsf_forward: bad sizes");
+    for (int r = 0; r < n_runs; ++r)
+        PT_REQUIRE(runs[r].out || runs[r].n_centers == 0, "pt_acsf_forward: null argument");
+    KArgs a = common_args(pos4, box, row_off, nbr, max_row);
+    a.ld = ldg;
+    return run_all<MODE_FWD>(precision, a, n_runs, runs, (hipStream_t)stream);
+}
+
 extern "C" int pt_acsf_forward(int precision, const double* pos4, const double* box,
                                const long long* row_off, const int* nbr, int max_row,
                                int n_centers, int center_begin, const int* centers,
                                const pt_sf_table* table, void* G, int ldg, pt_stream_t stream) {
-    PT_REQUIRE(pos4 && row_off && table && (G || n_centers == 0), "pt_acsf_forward: null argument");
-    PT_REQUIRE(n_centers >= 0 && ldg >= 0, "pt_acsf_forward: bad sizes");
-    hipStream_t st = (hipStream_t)stream;
-    KArgs a = common_args(pos4, box, row_off, nbr, max_row, n_centers, center_begin, centers, table);
-    a.out = G;
-    a.ld = ldg;
-    return run(precision, MODE_FWD, a, st);
+    pt_acsf_run r = single_run(precision, table, n_centers, center_begin, centers);
+    r.out = G;
+    return pt_acsf_forward_multi(base_precision(precision), pos4, box, row_off, nbr, max_row, 1, &r, ldg, stream);
+}
+
+extern "C" int pt_acsf_adjoint_multi(int precision, const double* pos4, const double* box, const double* boxes,
+                                     const int* box_id, const long long* row_off, const int* nbr, const int* rev,
+                                     int max_row, int n_runs, const pt_acsf_run* runs, int ldw, void* edge_grad,
+                                     pt_stream_t stream) {
+    PT_REQUIRE(pos4 && row_off && n_runs >= 0 && (runs || n_runs == 0), "pt_acsf_adjoint: null argument");
+    PT_REQUIRE(!boxes || (box_id && !box), "pt_acsf_adjoint: box table without box indices");
+    for (int r = 0; r < n_runs; ++r)
+        PT_REQUIRE(runs[r].w || runs[r].n_centers == 0, "pt_acsf_adjoint: null argument");
+    KArgs a = common_args(pos4, box, row_off, nbr, max_row);
+    a.boxes = boxes;
+    a.box_id = box_id;
+    a.ld = ldw;
+    a.edge_grad = edge_grad;
+    a.rev = rev;
+    return run_all<MODE_ADJ>(precision, a, n_runs, runs, (hipStream_t)stream);
 }
 
 extern "C" int pt_acsf_adjoint(int precision, const double* pos4, const double* box,
@@ -1201,14 +1449,11 @@ extern "C" int pt_acsf_adjoint(int precision, const double* pos4, const double* 
                                int n_centers, int center_begin, const int* centers,
                                const pt_sf_table* table, const void* w, int ldw, double* f_self,
                                void* edge_grad, pt_stream_t stream) {
-    PT_REQUIRE(pos4 && row_off && table && (w || n_centers == 0), "pt_acsf_adjoint: null argument");
-    hipStream_t st = (hipStream_t)stream;
-    KArgs a = common_args(pos4, box, row_off, nbr, max_row, n_centers, center_begin, centers, table);
-    a.w = w;
-    a.ldw = ldw;
-    a.f_self = f_self;
-    a.edge_grad = edge_grad;
-    return run(precision, MODE_ADJ, a, st);
+    pt_acsf_run r = single_run(precision, table, std::max(n_centers, 0), center_begin, centers);
+    r.w = w;
+    r.f_self = f_self;
+    return pt_acsf_adjoint_multi(base_precision(precision), pos4, box, nullptr, nullptr, row_off, nbr, nullptr,
+                                 max_row, 1, &r, ldw, edge_grad, stream);
 }
 
 extern "C" int pt_acsf_adjoint_transposed(int precision, const double* pos4, const double* box,
@@ -1216,16 +1461,31 @@ extern "C" int pt_acsf_adjoint_transposed(int precision, const double* pos4, con
                                           int n_centers, int center_begin, const int* centers,
                                           const pt_sf_table* table, const void* w, int ldw, double* f_self,
                                           void* edge_grad_t, pt_stream_t stream) {
-    PT_REQUIRE(pos4 && row_off && rev && table && (w || n_centers == 0),
-               "pt_acsf_adjoint_transposed: null argument");
-    hipStream_t st = (hipStream_t)stream;
-    KArgs a = common_args(pos4, box, row_off, nbr, max_row, n_centers, center_begin, centers, table);
-    a.w = w;
-    a.ldw = ldw;
-    a.f_self = f_self;
-    a.edge_grad = edge_grad_t;
-    a.rev = rev;
-    return run(precision, MODE_ADJ, a, st);
+    PT_REQUIRE(rev, "pt_acsf_adjoint_transposed: null argument");
+    pt_acsf_run r = single_run(precision, table, std::max(n_centers, 0), center_begin, centers);
+    r.w = w;
+    r.f_self = f_self;
+    return pt_acsf_adjoint_multi(base_precision(precision), pos4, box, nullptr, nullptr, row_off, nbr, rev, max_row,
+                                 1, &r, ldw, edge_grad_t, stream);
+}
+
+extern "C" int pt_acsf_tangent_multi(int precision, const double* pos4, const double* box, const double* boxes,
+                                     const int* box_id, const long long* row_off, const int* nbr, int max_row,
+                                     int n_runs, const pt_acsf_run* runs, int center_only, int ldt,
+                                     pt_stream_t stream) {
+    PT_REQUIRE(pos4 && row_off && n_runs >= 0 && (runs || n_runs == 0), "pt_acsf_tangent: null argument");
+    PT_REQUIRE(!boxes || (box_id && !box), "pt_acsf_tangent: box table without box indices");
+    for (int r = 0; r < n_runs; ++r) {
+        PT_REQUIRE(runs[r].out || runs[r].n_centers == 0, "pt_acsf_tangent: null argument");
+        PT_REQUIRE(runs[r].delta || (center_only && runs[r].dir >= 0 && runs[r].dir <= 2),
+                   "pt_acsf_tangent: a run without a displacement field needs a direction and center_only");
+    }
+    KArgs a = common_args(pos4, box, row_off, nbr, max_row);
+    a.boxes = boxes;
+    a.box_id = box_id;
+    a.ld = ldt;
+    a.center_only = center_only;
+    return run_all<MODE_TAN>(precision, a, n_runs, runs, (hipStream_t)stream);
 }
 
 extern "C" int pt_acsf_tangent(int precision, const double* pos4, const double* box,
@@ -1233,15 +1493,12 @@ extern "C" int pt_acsf_tangent(int precision, const double* pos4, const double* 
                                int n_centers, int center_begin, const int* centers,
                                const pt_sf_table* table, const double* delta, int center_only,
                                void* T, int ldt, pt_stream_t stream) {
-    PT_REQUIRE(pos4 && row_off && table && delta && (T || n_centers == 0),
-               "pt_acsf_tangent: null argument");
-    hipStream_t st = (hipStream_t)stream;
-    KArgs a = common_args(pos4, box, row_off, nbr, max_row, n_centers, center_begin, centers, table);
-    a.out = T;
-    a.ld = ldt;
-    a.delta = delta;
-    a.center_only = center_only;
-    return run(precision, MODE_TAN, a, st);
+    PT_REQUIRE(delta, "pt_acsf_tangent: null argument");
+    pt_acsf_run r = single_run(precision, table, std::max(n_centers, 0), center_begin, centers);
+    r.out = T;
+    r.delta = delta;
+    return pt_acsf_tangent_multi(base_precision(precision), pos4, box, nullptr, nullptr, row_off, nbr, max_row, 1,
+                                 &r, center_only, ldt, stream);
 }
 
 extern "C" int pt_sf_table_kind(const pt_sf_table* t) {

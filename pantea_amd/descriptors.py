@@ -24,7 +24,7 @@ from typing import Dict, NamedTuple, Optional, Sequence, Tuple
 import numpy as np
 
 from . import _lib
-from .engine import PRECISIONS, DeviceTable, NeighborList, SFRow, acsf_forward, acsf_tangent, gather_rows
+from .engine import PRECISIONS, DeviceTable, NeighborList, SFRow, acsf_forward, acsf_run, acsf_tangent_multi, gather_rows
 
 
 # ---------------------------------------------------------------------------
@@ -215,13 +215,11 @@ class ACSF:
         nl, tab, inv, prec = self._prepare(structure, precision)
         centers = inv[torch.as_tensor(idx, device=inv.device)].contiguous()
         n = int(centers.numel())
-        out = torch.empty((n, self.num_symmetry_functions, 3),
-                          dtype=torch.float64 if prec == _lib.PT_F64 else torch.float32, device=inv.device)
-        for d in range(3):
-            delta = torch.zeros((structure.natoms, 3), dtype=torch.float64, device=inv.device)
-            delta[:, d] = 1.0
-            out[:, :, d] = acsf_tangent(nl, tab, prec, n, delta, center_only=True, centers=centers)
-        return out
+        n_sf = self.num_symmetry_functions
+        T = torch.zeros((3, n, n_sf), dtype=torch.float64 if prec == _lib.PT_F64 else torch.float32, device=inv.device)
+        acsf_tangent_multi(nl, prec, [acsf_run(tab, n, centers=centers, out=T[d], direction=d) for d in range(3)],
+                           center_only=True, ld=n_sf)
+        return T.permute(1, 2, 0).contiguous()
 
     def __repr__(self) -> str:
         return f"ACSF(central_element='{self.central_element}', num_symmetry_functions={self.num_symmetry_functions})"

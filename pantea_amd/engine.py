@@ -356,6 +356,44 @@ def acsf_tangent(nl: NeighborList, table: DeviceTable, precision: int, n_centers
     return out
 
 
+def acsf_run(table: DeviceTable, n_centers: int, center_begin: int = 0, centers=None, out=None, w=None, f_self=None,
+             delta=None, direction: int = -1) -> _lib.AcsfRun:
+    """Centres that share a table in one of the *_multi launches (tensors must outlive the call)."""
+    return _lib.AcsfRun(table.ptr, table.kind, n_centers, center_begin, direction, _vp(centers), _vp(out), _vp(w),
+                        _vp(f_self), _vp(delta))
+
+
+def run_array(runs):
+    """(count, array) arguments of the *_multi calls."""
+    return len(runs), (_lib.AcsfRun * max(1, len(runs)))(*runs)
+
+
+def acsf_forward_multi(nl: NeighborList, precision: int, runs, ld: int) -> None:
+    """acsf_forward of several runs (acsf_run) in one launch."""
+    box_p, _keep = _box_arg(nl.box_lengths)
+    _lib.check(_lib.load().pt_acsf_forward_multi(
+        precision, nl.pos4.data_ptr(), box_p, nl.row_off.data_ptr(), nl.nbr.data_ptr(), nl.max_row, *run_array(runs),
+        ld, _lib.stream_ptr()), "pt_acsf_forward_multi")
+
+
+def acsf_adjoint_multi(nl: NeighborList, precision: int, runs, ldw: int, edge_grad=None,
+                       transposed: bool = False) -> None:
+    """acsf_adjoint of several runs in one launch."""
+    box_p, _keep = _box_arg(nl.box_lengths)
+    _lib.check(_lib.load().pt_acsf_adjoint_multi(
+        precision, nl.pos4.data_ptr(), box_p, None, None, nl.row_off.data_ptr(), nl.nbr.data_ptr(),
+        nl.rev.data_ptr() if transposed else None, nl.max_row, *run_array(runs), ldw, _vp(edge_grad),
+        _lib.stream_ptr()), "pt_acsf_adjoint_multi")
+
+
+def acsf_tangent_multi(nl: NeighborList, precision: int, runs, center_only: bool, ld: int) -> None:
+    """acsf_tangent of several runs in one launch."""
+    box_p, _keep = _box_arg(nl.box_lengths)
+    _lib.check(_lib.load().pt_acsf_tangent_multi(
+        precision, nl.pos4.data_ptr(), box_p, None, None, nl.row_off.data_ptr(), nl.nbr.data_ptr(), nl.max_row,
+        *run_array(runs), int(center_only), ld, _lib.stream_ptr()), "pt_acsf_tangent_multi")
+
+
 def force_gather(nl: NeighborList, edge_grad, precision: int, out=None):
     torch = _torch()
     if out is None:

@@ -35,7 +35,8 @@ from typing import Any, Callable, Dict, List, Optional, Tuple
 import numpy as np
 
 from . import _lib
-from .engine import NeighborList, Reducer, acsf_adjoint, acsf_forward, acsf_tangent, gather_rows
+from .engine import (NeighborList, Reducer, acsf_adjoint_multi, acsf_forward_multi, acsf_run, acsf_tangent_multi,
+                     gather_rows)
 from .models import energy_grad_multi
 from .potential import NNPSettings, NeuralNetworkPotential
 
@@ -164,14 +165,11 @@ class KalmanFilter:
                 b, cnt = nl.type_block(t)
                 if cnt == 0:
                     continue
-                tab = pot.atomic_potentials[e].descriptor.device_table(emap, self.dev)
-                acsf_forward(nl, tab, _lib.PT_F64, cnt, center_begin=b, out=G[b:], ld=ld)
-                for a in range(3):
-                    delta = torch.zeros((n, 3), dtype=torch.float64, device=self.dev)
-                    delta[:, a] = 1.0
-                    acsf_tangent(nl, tab, _lib.PT_F64, cnt, delta, center_only=True, center_begin=b,
-                                 out=T[a, b:], ld=ld)
-                blocks.append((e, b, cnt, tab))
+                blocks.append((e, b, cnt, pot.atomic_potentials[e].descriptor.device_table(emap, self.dev)))
+            acsf_forward_multi(nl, _lib.PT_F64, [acsf_run(tab, cnt, b, out=G[b:]) for _, b, cnt, tab in blocks], ld)
+            acsf_tangent_multi(nl, _lib.PT_F64, [acsf_run(tab, cnt, b, out=T[a, b:], direction=a)
+                                                 for _, b, cnt, tab in blocks for a in range(3)],
+                               center_only=True, ld=ld)
             F_ref = gather_rows(nl.perm, s.forces.to(torch.float64).contiguous())
             nl.release_workspace()
             items.append(_Item(n, nl, blocks, G, T, F_ref, float(s.total_energy)))
@@ -222,8 +220,8 @@ class KalmanFilter:
         self._energy(it)
         f = self.f_self[:it.n]
         f.zero_()
-        for e, b, cnt, tab in it.blocks:
-            acsf_adjoint(it.nl, tab, _lib.PT_F64, cnt, self.dEdG[b:], self.ld, center_begin=b, f_self=f[b:])
+        acsf_adjoint_multi(it.nl, _lib.PT_F64, [acsf_run(tab, cnt, b, w=self.dEdG[b:], f_self=f[b:])
+                                                for _, b, cnt, tab in it.blocks], self.ld)
         m3 = 3 * it.n
         _lib.check(lib.pt_kalman_residual(m3, f.data_ptr(), it.F_ref.data_ptr(), 0.0, 1.0, self.xi.data_ptr(),
                                           self.loss[1:].data_ptr(), _lib.stream_ptr()), "pt_kalman_residual")

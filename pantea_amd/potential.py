@@ -32,7 +32,8 @@ from . import _lib
 from .atoms import ElementMap
 from .descriptors import (ACSF, G1, G2, G3, G9, CutoffFunction, DescriptorScaler, NeighborElements,
                           ScalerParams)
-from .engine import (NeighborList, Reducer, acsf_adjoint, acsf_forward, force_gather, scatter_rows)
+from .engine import (NeighborList, Reducer, acsf_adjoint_multi, acsf_forward_multi, acsf_run, force_gather,
+                     scatter_rows)
 from .models import (MLP_MODES, DeviceMLP, ModelParams, NeuralNetworkModel, UniformInitializer,
                      energy_grad_multi)
 
@@ -240,10 +241,11 @@ class _Evaluation:
                 yield e, b, cnt
 
     def energy(self, pot):
-        for e, b, cnt in self._blocks(pot):
-            acsf_forward(self.nl, self.tables[e], self.g_prec, cnt, center_begin=b, out=self.G[b:], ld=self.ld)
+        blocks = list(self._blocks(pot))
+        acsf_forward_multi(self.nl, self.g_prec, [acsf_run(self.tables[e], cnt, b, out=self.G[b:])
+                                                  for e, b, cnt in blocks], self.ld)
         energy_grad_multi(self.mlp_mode, [(self.mlps[e], cnt, self.G[b:], self.e_atom[b:], self.dEdG[b:])
-                                          for e, b, cnt in self._blocks(pot)], self.ld, self.g_prec)
+                                          for e, b, cnt in blocks], self.ld, self.g_prec)
         return self.reducer.sum(self.e_atom)
 
     def forces(self, pot, full: bool):
@@ -256,9 +258,10 @@ class _Evaluation:
         if full and not self.covered:
             self.edge.zero_()
         self.f_self.zero_()
-        for e, b, cnt in self._blocks(pot):
-            acsf_adjoint(self.nl, self.tables[e], self.g_prec, cnt, self.dEdG[b:], self.ld, center_begin=b,
-                         f_self=self.f_self[b:], edge_grad=self.edge if full else None)
+        acsf_adjoint_multi(self.nl, self.g_prec,
+                           [acsf_run(self.tables[e], cnt, b, w=self.dEdG[b:], f_self=self.f_self[b:])
+                            for e, b, cnt in self._blocks(pot)],
+                           self.ld, edge_grad=self.edge if full else None)
         if full:
             force_gather(self.nl, self.edge, self.g_prec, out=self.f_full)
             return self.f_full

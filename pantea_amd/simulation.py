@@ -37,8 +37,8 @@ import numpy as np
 
 from . import _lib
 from .atoms import ElementMap, host_box
-from .engine import (NeighborList, Reducer, acsf_adjoint, acsf_forward, force_gather, force_gather_transposed,
-                     gather_rows, scatter_rows)
+from .engine import (NeighborList, Reducer, acsf_adjoint_multi, acsf_forward_multi, acsf_run,
+                     force_gather_transposed, gather_rows, scatter_rows)
 from .models import energy_grad_multi
 from .potential import PRECISION_MODES, NeuralNetworkPotential
 from .units import units
@@ -79,7 +79,7 @@ class _ForceField:
         self.tables = {e: pot.atomic_potentials[e].descriptor.device_table(emap, dev)
                        for e in pot.elements if e in emap.element_to_atom_type}
         # descriptor tables hold no centre element: elements whose tables are
-        # byte-identical share one launch (one grid tail instead of several)
+        # byte-identical share one run
         self._table_key = {e: bytes(t.host) for e, t in self.tables.items()}
         self.covered = all(e in pot.atomic_potentials for e in emap.unique_elements)
         self.mlps = pot._device_mlps(dev)
@@ -99,7 +99,7 @@ class _ForceField:
                 yield e, b, cnt
 
     def _desc_runs(self, nl: NeighborList):
-        """(table, first centre, centres) of each descriptor launch: adjacent element
+        """(table, first centre, centres) of each run of a descriptor launch: adjacent element
         blocks (internal order is type-sorted) with identical tables form one run."""
         runs = []
         for e, b, cnt in sorted(self._blocks(nl), key=lambda x: x[1]):
@@ -116,8 +116,7 @@ class _ForceField:
         blocks = list(self._blocks(nl))
         runs = self._desc_runs(nl)
         mark("acsf_forward", True)
-        for tab, b, cnt in runs:
-            acsf_forward(nl, tab, self.g_prec, cnt, center_begin=b, out=self.G[b:], ld=self.ld)
+        acsf_forward_multi(nl, self.g_prec, [acsf_run(tab, cnt, b, out=self.G[b:]) for tab, b, cnt in runs], self.ld)
         mark("acsf_forward", False)
         mark("mlp", True)
         energy_grad_multi(self.mlp_mode, [(self.mlps[e], cnt, self.G[b:], self.e_atom[b:], self.dEdG[b:])
@@ -137,10 +136,10 @@ class _ForceField:
         if not self.covered:
             target.zero_()
         mark("acsf_adjoint", True)
-        for tab, b, cnt in runs:
-            # -grad E: edge gradients in the reverse edges' slots, so the gather reads rows contiguously
-            acsf_adjoint(nl, tab, self.g_prec, cnt, self.dEdG[b:], self.ld, center_begin=b,
-                         f_self=target[b:], edge_grad=self.edge if full else None, transposed=full)
+        # -grad E: edge gradients in the reverse edges' slots, so the gather reads rows contiguously
+        acsf_adjoint_multi(nl, self.g_prec, [acsf_run(tab, cnt, b, w=self.dEdG[b:], f_self=target[b:])
+                                             for tab, b, cnt in runs],
+                           self.ld, edge_grad=self.edge if full else None, transposed=full)
         mark("acsf_adjoint", False)
         if full:
             mark("force_gather", True)

@@ -33,7 +33,8 @@ import numpy as np
 
 from . import _lib
 from .atoms import Structure
-from .engine import NeighborList, Reducer, acsf_adjoint, acsf_forward, acsf_tangent, force_gather, gather_rows
+from .engine import (NeighborList, Reducer, acsf_adjoint_multi, acsf_forward_multi, acsf_run, acsf_tangent_multi,
+                     force_gather, gather_rows)
 from .models import energy_grad_multi
 from .potential import PRECISION_MODES, NeuralNetworkPotential
 from .units import units
@@ -134,14 +135,14 @@ class StudentTrainer:
                 if cnt:
                     blocks.append((el, b, cnt))
             G = torch.zeros((s.natoms, self.ld), dtype=self.fdt, device=self.dev)
+            key = tuple(sorted(emap.element_to_atom_type.items()))
             for el, b, cnt in blocks:
-                tab = pot.atomic_potentials[el].descriptor.device_table(emap, self.dev)
-                self.tables[(el, tuple(sorted(emap.element_to_atom_type.items())))] = tab
-                acsf_forward(nl, tab, self.g_prec, cnt, center_begin=b, out=G[b:], ld=self.ld)
+                self.tables[(el, key)] = pot.atomic_potentials[el].descriptor.device_table(emap, self.dev)
+            acsf_forward_multi(nl, self.g_prec, [acsf_run(self.tables[(el, key)], cnt, b, out=G[b:])
+                                                 for el, b, cnt in blocks], self.ld)
             F_int = gather_rows(nl.perm, f.to(torch.float64).contiguous())
             nl.release_workspace()
-            self.snapshots.append(Snapshot(s.natoms, nl, blocks, G, F_int, e,
-                                           tuple(sorted(emap.element_to_atom_type.items()))))
+            self.snapshots.append(Snapshot(s.natoms, nl, blocks, G, F_int, e, key))
         self._raw = []
         if fit_scaler:
             from .descriptors import DescriptorScaler
@@ -189,9 +190,9 @@ class StudentTrainer:
         energy_grad_multi(self.mlp_mode, [(self.mlps[el], cnt, sn.G[b:], self.e_atom[b:], self.dEdG[b:])
                                           for el, b, cnt in sn.blocks], self.ld, self.g_prec)
         E = self.reducer.sum(self.e_atom[:n])
-        for el, b, cnt in sn.blocks:
-            acsf_adjoint(sn.nl, self._table(sn, el), self.g_prec, cnt, self.dEdG[b:], self.ld, center_begin=b,
-                         f_self=self.f_self[b:], edge_grad=self.edge)
+        acsf_adjoint_multi(sn.nl, self.g_prec, [acsf_run(self._table(sn, el), cnt, b, w=self.dEdG[b:],
+                                                         f_self=self.f_self[b:]) for el, b, cnt in sn.blocks],
+                           self.ld, edge_grad=self.edge)
         force_gather(sn.nl, self.edge, self.g_prec, out=self.F[:n])
         return E, self.F[:n]
 
@@ -202,9 +203,9 @@ class StudentTrainer:
                                               self.w_energy * scale, self.w_force * scale, self.delta.data_ptr(),
                                               self.gy.data_ptr(), self.loss.data_ptr(), _lib.stream_ptr()),
                    "pt_train_seeds")
-        for el, b, cnt in sn.blocks:
-            acsf_tangent(sn.nl, self._table(sn, el), self.g_prec, cnt, self.delta[:n], center_only=False,
-                         center_begin=b, out=self.T[b:], ld=self.ld)
+        acsf_tangent_multi(sn.nl, self.g_prec, [acsf_run(self._table(sn, el), cnt, b, out=self.T[b:],
+                                                         delta=self.delta) for el, b, cnt in sn.blocks],
+                           center_only=False, ld=self.ld)
         for el, b, cnt in sn.blocks:
             self.mlps[el].train_grad(self.mlp_mode, cnt, sn.G[b:], self.T[b:], self.ld, self.g_prec, self.gy[b:],
                                      -1.0, self.grad[el])
