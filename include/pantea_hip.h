@@ -364,6 +364,29 @@ int pt_mlp_train_grad(int mode, int n_atoms, const void *G, const void *T, int l
 int pt_train_seeds(int n, const double *force, const double *force_ref, const double *energy,
                    double energy_ref, double w_energy, double w_force, double *delta, double *gy,
                    double *loss, pt_stream_t stream);
+/* A batch of labelled structures as one list, so that every step of the loss
+ * gradient is one launch.  Segment q = e * n_struct + k of the batch holds the
+ * atoms of element e of structure k.  plan (device, pt_train_batch_words 64-bit
+ * words): per structure the device addresses of pos4, row_off, nbr, rev, the
+ * descriptors G (n x ld) and the labels F* (n x 3), then E* (FP64 bits), the
+ * three box lengths (FP64 bits; 0: not periodic) and the atom count; per
+ * (structure, element) the element block's first atom (past the last atom if
+ * the structure has none) and row_off there; the first batch atom and the first
+ * batch edge of every segment, each closed by the total.  Every atom belongs to
+ * an element block.
+ * pt_train_batch_assemble copies the lists into pos4 .. boxes (n_atoms + 1
+ * row offsets, n_struct x 3 box lengths, a structure index per atom: the box
+ * table of pt_acsf_*_multi).  pt_train_batch_seeds: from f_self and the
+ * transposed edge gradients of the batch and e_atom, per structure delta, gy
+ * and the loss sums of pt_train_seeds (sq: n_atoms doubles of workspace). */
+int pt_train_batch_words(int n_struct, int n_elem);
+int pt_train_batch_assemble(int n_struct, int n_elem, const long long *plan, int n_atoms, int ld, int g_precision,
+                            double *pos4, long long *row_off, int *nbr, int *rev, void *G, double *f_ref,
+                            int *box_id, double *boxes, pt_stream_t stream);
+int pt_train_batch_seeds(int n_struct, int n_elem, const long long *plan, int n_atoms, const long long *row_off,
+                         const double *f_self, const void *edge_grad_t, int edge_precision, const int *box_id,
+                         const double *f_ref, const double *e_atom, double w_energy, double w_force, double *delta,
+                         double *gy, double *sq, double *loss, pt_stream_t stream);
 /* Adam (decoupled weight decay when weight_decay > 0), step counts from 1;
  * optax.adamw semantics (gradient_descent.py:70-76). */
 int pt_adam_step(int n, double *params, const double *grad, double *m, double *v, double lr,

@@ -158,6 +158,11 @@ _SIGS = {
     "pt_mlp_train_grad": (_c_int, [_c_int, _c_int, _vp, _vp, _c_int, _c_int, _vp, _vp, _vp, _vp,
                                    _c_dbl, _vp, _vp]),
     "pt_train_seeds": (_c_int, [_c_int, _vp, _vp, _vp, _c_dbl, _c_dbl, _c_dbl, _vp, _vp, _vp, _vp]),
+    "pt_train_batch_words": (_c_int, [_c_int, _c_int]),
+    "pt_train_batch_assemble": (_c_int, [_c_int, _c_int, _vp, _c_int, _c_int, _c_int, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
+                                         _vp, _vp]),
+    "pt_train_batch_seeds": (_c_int, [_c_int, _c_int, _vp, _c_int, _vp, _vp, _vp, _c_int, _vp, _vp, _vp, _c_dbl, _c_dbl,
+                                      _vp, _vp, _vp, _vp, _vp]),
     "pt_adam_step": (_c_int, [_c_int, _vp, _vp, _vp, _vp, _c_dbl, _c_dbl, _c_dbl, _c_dbl, _c_dbl,
                               _c_int, _vp]),
     "pt_mlp_jacobian": (_c_int, [_c_int, _c_int, _vp, _vp, _c_ll, _c_int, _vp, _vp, _vp, _c_dbl, _vp, _c_ll, _vp]),

@@ -35,7 +35,7 @@ HIPCC_FLAGS = [
     f"-I{CSRC}",
 ]
 
-SOURCES = ["md.hip", "nbr.hip", "acsf.hip", "mlp.hip", "scaler.hip", "kalman.hip"]
+SOURCES = ["md.hip", "nbr.hip", "acsf.hip", "mlp.hip", "train.hip", "scaler.hip", "kalman.hip"]
 
 # the Kalman filter update calls rocBLAS (GEMM, SYRK, TRMM, TRSM, GEMV) and rocSOLVER (dpotrs)
 LINK_FLAGS = ["-L/opt/rocm/lib", "-Wl,-rpath,/opt/rocm/lib", "-lrocsolver", "-lrocblas"]

@@ -13,7 +13,9 @@ Pipeline:
         delta = dL/dF, dL/dE        pt_train_seeds
         T = J delta                 pt_acsf_tangent (forward mode)
         dL/dtheta accumulation      pt_mlp_train_grad (forward-over-reverse)
-     and after each batch one Adam step (pt_adam_step) and a repack.
+     and after each batch one Adam step (pt_adam_step) and a repack.  The
+     structures of a batch are copied into one list (pt_train_batch_assemble),
+     so each of these is one launch per batch (pt_train_batch_seeds).
 Loss per structure: w_E ((E - E*)/N)^2 + w_F / (3N) sum |F - F*|^2,
 averaged over the batch.  The reference's own trainer
 (potentials/nnp/gradient_descent.py:157-233) is broken and never run by its
@@ -34,7 +36,7 @@ import numpy as np
 from . import _lib
 from .atoms import Structure
 from .engine import (NeighborList, Reducer, acsf_adjoint_multi, acsf_forward_multi, acsf_run, acsf_tangent_multi,
-                     force_gather, gather_rows)
+                     force_gather, gather_rows, run_array)
 from .models import energy_grad_multi
 from .potential import PRECISION_MODES, NeuralNetworkPotential
 from .units import units
@@ -51,6 +53,12 @@ class Snapshot:
     F_ref: object                        # (n, 3) FP64 teacher forces, internal order
     E_ref: float
     emap_key: tuple = ()                 # element map (element, type) pairs
+    block_edges: tuple = ()              # list offset at the first atom of each block
+
+    @property
+    def whole(self) -> bool:
+        """Every atom is of an element with a model."""
+        return sum(cnt for _, _, cnt in self.blocks) == self.n
 
 
 def teacher_snapshots(teacher: NeuralNetworkPotential, n_structures: int = 64, n_snapshots: int = 2000,
@@ -86,6 +94,37 @@ def teacher_snapshots(teacher: NeuralNetworkPotential, n_structures: int = 64, n
             yield snap, float(e), f.clone()
         if log:
             log(f"teacher structure {k}: {3 * int(nm)} atoms, {count} snapshots")
+
+
+class _Batch:
+    """Device arrays of a batch of snapshots as one list (grown as needed)."""
+
+    MAX_ATOMS = 65536   # snapshots beyond this many atoms go into a further pass
+
+    def __init__(self, ld: int, fdt, dev):
+        self.ld, self.fdt, self.dev = ld, fdt, dev
+        self.atoms = self.edges = self.structs = 0
+
+    def reserve(self, atoms: int, edges: int, structs: int) -> None:
+        import torch
+
+        f64 = dict(dtype=torch.float64, device=self.dev)
+        if atoms > self.atoms:
+            self.atoms = n = max(atoms, min(2 * self.atoms, self.MAX_ATOMS))
+            self.pos4 = torch.empty((n, 4), **f64)
+            self.row_off = torch.empty(n + 1, dtype=torch.int64, device=self.dev)
+            self.box_id = torch.empty(n, dtype=torch.int32, device=self.dev)
+            self.e_atom, self.gy, self.sq = (torch.empty(n, **f64) for _ in range(3))
+            self.f_ref, self.f_self, self.delta = (torch.empty((n, 3), **f64) for _ in range(3))
+            self.G, self.dEdG, self.T = (torch.zeros((n, self.ld), dtype=self.fdt, device=self.dev) for _ in range(3))
+        if edges > self.edges:
+            self.edges = e = int(1.1 * edges) + 1
+            self.nbr = torch.empty(e, dtype=torch.int32, device=self.dev)
+            self.rev = torch.empty(e, dtype=torch.int32, device=self.dev)
+            self.edge = torch.empty(3 * e, dtype=self.fdt, device=self.dev)
+        if structs > self.structs:
+            self.structs = structs
+            self.boxes = torch.empty((structs, 3), **f64)
 
 
 class StudentTrainer:
@@ -144,6 +183,11 @@ class StudentTrainer:
             nl.release_workspace()
             self.snapshots.append(Snapshot(s.natoms, nl, blocks, G, F_int, e, key))
         self._raw = []
+        new = [sn for sn in self.snapshots if not sn.block_edges and sn.blocks]
+        if new:   # one read for all new lists
+            at = torch.cat([sn.nl.row_off[[b for _, b, _ in sn.blocks]] for sn in new]).cpu().tolist()
+            for sn in new:
+                sn.block_edges, at = tuple(at[:len(sn.blocks)]), at[len(sn.blocks):]
         if fit_scaler:
             from .descriptors import DescriptorScaler
 
@@ -179,14 +223,25 @@ class StudentTrainer:
         self.reducer = Reducer(nmax, self.dev)
         emax = max(sn.nl.n_pairs for sn in self.snapshots)
         self.edge = torch.zeros(3 * max(emax, 1), dtype=self.fdt, device=self.dev)
+        self.batch = _Batch(self.ld, self.fdt, self.dev)
 
     # ---- one structure ------------------------------------------------------------
     def _table(self, sn: Snapshot, el: str):
         return self.tables[(el, sn.emap_key)]
 
+    @staticmethod
+    def _clear_absent(tab, T) -> None:
+        """Functions of elements that a structure does not hold have no row in its table: the
+        tangent kernel leaves their columns as the last structure wrote them."""
+        if len(tab.rows) < tab.n_sf:
+            T.zero_()
+
     def _energy_forces(self, sn: Snapshot):
         """Student E (device scalar) and F (internal order) of a snapshot."""
         n = sn.n
+        if not sn.whole:   # atoms without a model contribute nothing: no kernel writes their entries
+            self.e_atom[:n].zero_()
+            self.edge.zero_()
         energy_grad_multi(self.mlp_mode, [(self.mlps[el], cnt, sn.G[b:], self.e_atom[b:], self.dEdG[b:])
                                           for el, b, cnt in sn.blocks], self.ld, self.g_prec)
         E = self.reducer.sum(self.e_atom[:n])
@@ -203,6 +258,8 @@ class StudentTrainer:
                                               self.w_energy * scale, self.w_force * scale, self.delta.data_ptr(),
                                               self.gy.data_ptr(), self.loss.data_ptr(), _lib.stream_ptr()),
                    "pt_train_seeds")
+        for el, b, cnt in sn.blocks:
+            self._clear_absent(self._table(sn, el), self.T[b:b + cnt])
         acsf_tangent_multi(sn.nl, self.g_prec, [acsf_run(self._table(sn, el), cnt, b, out=self.T[b:],
                                                          delta=self.delta) for el, b, cnt in sn.blocks],
                            center_only=False, ld=self.ld)
@@ -210,14 +267,98 @@ class StudentTrainer:
             self.mlps[el].train_grad(self.mlp_mode, cnt, sn.G[b:], self.T[b:], self.ld, self.g_prec, self.gy[b:],
                                      -1.0, self.grad[el])
 
+    # ---- a batch of structures as one list -------------------------------------------
+    def _passes(self, snaps: Sequence[Snapshot]):
+        """``snaps`` in groups that share an element map and fit one pass."""
+        groups: Dict[tuple, List[Snapshot]] = {}
+        for sn in snaps:
+            groups.setdefault(sn.emap_key, []).append(sn)
+        for group in groups.values():
+            part, n, pairs = [], 0, 0
+            for sn in group:
+                # (batch edges are 32-bit indices)
+                if part and (n + sn.n > _Batch.MAX_ATOMS or pairs + sn.nl.n_pairs >= 2 ** 31 - 1):
+                    yield part
+                    part, n, pairs = [], 0, 0
+                part.append(sn)
+                n, pairs = n + sn.n, pairs + sn.nl.n_pairs
+            yield part
+
+    def _plan(self, snaps: Sequence[Snapshot]):
+        """The plan words of pt_train_batch_*, the atom offsets of the elements, the atom and edge totals."""
+        ns, els = len(snaps), self.pot.elements
+        ne = len(els)
+        rec = np.zeros((ns, 11), dtype=np.int64)
+        real = rec.view(np.float64)
+        begin = np.full((ns, ne), 1 << 30, dtype=np.int64)
+        edge0 = np.zeros((ns, ne), dtype=np.int64)
+        atoms = np.zeros((ne, ns), dtype=np.int64)
+        edges = np.zeros((ne, ns), dtype=np.int64)
+        for k, sn in enumerate(snaps):
+            nl = sn.nl
+            rec[k, :6] = (nl.pos4.data_ptr(), nl.row_off.data_ptr(), nl.nbr.data_ptr(), nl.rev.data_ptr(),
+                          sn.G.data_ptr(), sn.F_ref.data_ptr())
+            real[k, 6] = sn.E_ref
+            if nl.box_lengths is not None:
+                real[k, 7:10] = nl.box_lengths
+            rec[k, 10] = sn.n
+            order = sorted(zip(sn.block_edges, sn.blocks), key=lambda x: x[1][1])
+            ends = [o for o, _ in order[1:]] + [nl.n_pairs]
+            for (o, (el, b, cnt)), end in zip(order, ends):
+                e = els.index(el)
+                begin[k, e], edge0[k, e] = b, o
+                atoms[e, k], edges[e, k] = cnt, end - o
+        first = [np.concatenate([[0], np.cumsum(x.reshape(-1))]) for x in (atoms, edges)]
+        words = np.concatenate([rec.reshape(-1), begin.reshape(-1), edge0.reshape(-1), *first])
+        assert words.size == _lib.load().pt_train_batch_words(ns, ne)
+        return words, first[0][::ns], int(first[0][-1]), int(first[1][-1])
+
+    def _accumulate_batch(self, snaps: Sequence[Snapshot], scale: float) -> None:
+        import torch
+
+        lib, st, B = _lib.load(), _lib.stream_ptr(), self.batch
+        words, at, n, pairs = self._plan(snaps)
+        ns, ne = len(snaps), len(self.pot.elements)
+        B.reserve(n, pairs, ns)
+        plan = torch.from_numpy(words).to(self.dev)
+        _lib.check(lib.pt_train_batch_assemble(
+            ns, ne, plan.data_ptr(), n, self.ld, self.g_prec, B.pos4.data_ptr(), B.row_off.data_ptr(),
+            B.nbr.data_ptr(), B.rev.data_ptr(), B.G.data_ptr(), B.f_ref.data_ptr(), B.box_id.data_ptr(),
+            B.boxes.data_ptr(), st), "pt_train_batch_assemble")
+        blocks = [(el, int(at[e]), int(at[e + 1] - at[e])) for e, el in enumerate(self.pot.elements) if at[e + 1] > at[e]]
+        tab = {el: self._table(snaps[0], el) for el, _, _ in blocks}
+        energy_grad_multi(self.mlp_mode, [(self.mlps[el], cnt, B.G[b:], B.e_atom[b:], B.dEdG[b:])
+                                          for el, b, cnt in blocks], self.ld, self.g_prec)
+        row = max(sn.nl.max_row for sn in snaps)
+        lists = (B.pos4.data_ptr(), None, B.boxes.data_ptr(), B.box_id.data_ptr(), B.row_off.data_ptr(), B.nbr.data_ptr())
+        runs = run_array([acsf_run(tab[el], cnt, b, w=B.dEdG[b:], f_self=B.f_self[b:]) for el, b, cnt in blocks])
+        _lib.check(lib.pt_acsf_adjoint_multi(self.g_prec, *lists, B.rev.data_ptr(), row, *runs, self.ld,
+                                             B.edge.data_ptr(), st), "pt_acsf_adjoint_multi")
+        _lib.check(lib.pt_train_batch_seeds(
+            ns, ne, plan.data_ptr(), n, B.row_off.data_ptr(), B.f_self.data_ptr(), B.edge.data_ptr(), self.g_prec,
+            B.box_id.data_ptr(), B.f_ref.data_ptr(), B.e_atom.data_ptr(), self.w_energy * scale, self.w_force * scale,
+            B.delta.data_ptr(), B.gy.data_ptr(), B.sq.data_ptr(), self.loss.data_ptr(), st), "pt_train_batch_seeds")
+        for el, b, cnt in blocks:
+            self._clear_absent(tab[el], B.T[b:b + cnt])
+        runs = run_array([acsf_run(tab[el], cnt, b, out=B.T[b:], delta=B.delta) for el, b, cnt in blocks])
+        _lib.check(lib.pt_acsf_tangent_multi(self.g_prec, *lists, row, *runs, 0, self.ld, st), "pt_acsf_tangent_multi")
+        for el, b, cnt in blocks:
+            self.mlps[el].train_grad(self.mlp_mode, cnt, B.G[b:], B.T[b:], self.ld, self.g_prec, B.gy[b:], -1.0,
+                                     self.grad[el])
+
     def gradient(self, indices: Sequence[int]):
         """Loss (energy term, force term) and its gradient over ``indices`` (batch mean)."""
         for g in self.grad.values():
             g.zero_()
         self.loss.zero_()
         scale = 1.0 / len(indices)
-        for k in indices:
-            self._accumulate(self.snapshots[k], scale)
+        snaps = [self.snapshots[k] for k in indices]
+        # a structure with atoms of an element without a model has no place in a batch list
+        for part in self._passes([sn for sn in snaps if sn.whole]):
+            self._accumulate_batch(part, scale)
+        for sn in snaps:
+            if not sn.whole:
+                self._accumulate(sn, scale)
         return self.loss.clone(), {e: g.clone() for e, g in self.grad.items()}
 
     def step(self, indices: Sequence[int]):
