@@ -328,12 +328,12 @@ def run_surrogate(teacher, student, s, steps, warmup, args, instrument=False, th
 
 def kalman_flops(n_w: int, m: int) -> float:
     """Algorithmic FP64 flops of one pt_kalman_update in the form it computes.  m <= n_w: X = P H
-    (2 n_w^2 m), A = H^T X (2 m^2 n_w), Cholesky of A (m^3 / 3), the solve for Y = A^-1 X^T (2 m^2 n_w),
-    P -= Y^T X^T (2 n_w^2 m).  m > n_w (n_w x n_w factors): Cholesky of P (n_w^3 / 3), G = L^T H
+    (2 n_w^2 m), A = H^T X (m^2 n_w, one triangle), Cholesky of A (m^3 / 3), Z = X L^-T (m^2 n_w),
+    P -= Z Z^T (n_w^2 m).  m > n_w (n_w x n_w factors): Cholesky of P (n_w^3 / 3), G = L^T H
     (n_w^2 m), S = G G^T (n_w^2 m), Cholesky of S (n_w^3 / 3), M = L Ls^-T (n_w^3), M M^T (n_w^3)."""
     if m > n_w:
         return 2.0 * n_w * n_w * m + 8.0 / 3.0 * n_w ** 3
-    return 4.0 * n_w * n_w * m + 4.0 * m * m * n_w + m ** 3 / 3.0
+    return 3.0 * n_w * n_w * m + 2.0 * m * m * n_w + m ** 3 / 3.0
 
 
 def run_kalman(args):
@@ -395,8 +395,8 @@ def run_kalman(args):
            "update_frac_of_fp64_peak": flops / (upd_ms * 1e-3) / 1e12 / PEAK_FP64_MFMA_TFLOPS,
            "update_form": "n_w x n_w factors (m > n_w)" if m > n_w else "m x m factor",
            "note": "flops of the form computed (kalman_flops in bench.py: m > n_w: 2 n_w^2 m + 8/3 n_w^3, else "
-                   "4 n_w^2 m + 4 m^2 n_w + m^3/3); its two Cholesky factorisations of n_w rows (blocked, one "
-                   "wavefront per 64 x 64 diagonal block) and their many small BLAS calls are latency-bound; "
+                   "3 n_w^2 m + 2 m^2 n_w + m^3/3); its two Cholesky factorisations of n_w rows (blocked, two "
+                   "launches per 64 columns, one after another) are latency-bound; "
                    f"peak = MI355X FP64 matrix {PEAK_FP64_MFMA_TFLOPS} TFLOP/s; HIP events over {reps} calls"}
     if not args.no_cpu_baseline:
         # the same update in numpy on the host, the reference's explicit inverse (one call)

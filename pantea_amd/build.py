@@ -37,10 +37,6 @@ HIPCC_FLAGS = [
 
 SOURCES = ["md.hip", "nbr.hip", "acsf.hip", "mlp.hip", "train.hip", "scaler.hip", "kalman.hip"]
 
-# the Kalman filter update calls rocBLAS (GEMM, SYRK, TRMM, TRSM, GEMV) and rocSOLVER (dpotrs)
-LINK_FLAGS = ["-L/opt/rocm/lib", "-Wl,-rpath,/opt/rocm/lib", "-lrocsolver", "-lrocblas"]
-
-
 def hipcc() -> str:
     exe = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     if not Path(exe).exists():
@@ -51,7 +47,7 @@ def hipcc() -> str:
 def build(verbose: bool = False) -> Path:
     srcs = [str(CSRC / s) for s in SOURCES]
     tmp = LIB.with_suffix(".so.tmp")
-    cmd = [hipcc(), *HIPCC_FLAGS, *srcs, *LINK_FLAGS, "-o", str(tmp)]
+    cmd = [hipcc(), *HIPCC_FLAGS, *srcs, "-o", str(tmp)]
     if verbose:
         print(" ".join(cmd), flush=True)
     res = subprocess.run(cmd, capture_output=True, text=True)

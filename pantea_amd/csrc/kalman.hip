@@ -5,17 +5,15 @@
 // one state vector) and m observations of one structure (m = 1 for the
 // energy, m = 3 N for the force components):
 //
-//   X = P H                           n_w x m    rocBLAS dgemm
-//   A = H^T X + r I                   m x m      rocBLAS dgemm + k_add_diag
-//   A = L L^T                                    chol_lower (below)
-//   Y = A^-1 X^T         (= K^T)      m x n_w    k_transpose + rocSOLVER dpotrs
-//   P = c (P - Y^T X^T) + q I                    rocBLAS dgemm + k_add_diag
-//   W = W + Y^T xi                               rocBLAS dgemv
+//   X = P H                                 n_w x m
+//   A = H^T X + r I = L L^T                 m x m     k_gemm_f64, chol_lower
+//   [Z; z^T] = [X; xi^T] L^-T               rows carried by the factorisation
+//   P = c (P - Z Z^T) + q I,  W = W + Z z   (K = X A^-1, K X^T = Z Z^T, K xi = Z z)
 //
 // r is the measurement noise (1/eta for the filter of type 0, lambda for
 // type 1), c the fading-memory factor (1 or 1/lambda) and q the process
 // noise; the schedules of eta, q and lambda are host scalars.  The
-// reference forms inv(A) and multiplies; the Cholesky solve gives the same
+// reference forms inv(A) and multiplies; the Cholesky factor gives the same
 // K (A is symmetric positive definite: H^T P H is semi-definite and r > 0)
 // without forming the inverse.
 //
@@ -25,32 +23,27 @@
 // push-through identity K = X A^-1 = L S^-1 G with S = G G^T + r I (n_w x n_w),
 // so that P - K X^T = r L S^-1 L^T.  With S = Ls Ls^T and M = L Ls^-T:
 //
-//   L = chol(P)                                  chol_lower (n_w)
-//   G = L^T H                        n_w x m     rocBLAS dtrmm
-//   S = G G^T + r I,  Ls = chol(S)   n_w x n_w   rocBLAS dsyrk + chol_lower
-//   [M; y^T] = [L; (G xi)^T] Ls^-T               dgemv + dtrsm (one solve: y = Ls^-1 G xi)
-//   W = W + M y  (= L S^-1 G xi)                 dgemv
-//   P = c r M M^T + q I                          dsyrk + k_symm_lower
+//   L = chol(P)
+//   G = L^T H                               n_w x m
+//   S = G G^T + r I = Ls Ls^T,  [M; y^T] = [L; (G xi)^T] Ls^-T   (one factorisation)
+//   W = W + M y  (= L S^-1 G xi),  P = c r M M^T + q I
 //
-// about 2 n_w^2 m + 8/3 n_w^3 flops against 4 n_w^2 m + 4 m^2 n_w + m^3 / 3,
+// about 2 n_w^2 m + 8/3 n_w^3 flops against 3 n_w^2 m + 2 m^2 n_w + m^3 / 3,
 // and factorisations of n_w rows instead of m.  All matrices are column-major FP64:
 // P (n_w x n_w, ld n_w) and H (n_w x m, ld ldh) -- H column o is the
 // gradient of observation o, i.e. a row-major (m x n_w) Jacobian.
-#include <mutex>
-#include <vector>
-
-#include <rocblas/rocblas.h>
-#include <rocsolver/rocsolver.h>
+//
+// Every product and factorisation is a kernel of this file: the library's
+// triangular kernels and its many small products per block took most of the
+// update (student network, n_w = 1,698, m = 4,608: 11.0 ms, now 2.8).
+#include <algorithm>
+#include <cmath>
+#include <type_traits>
 
 #include "common.h"
 
 namespace pt {
 namespace {
-
-__global__ void k_add_diag(int n, double* __restrict__ A, long long lda, double v) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) A[(size_t)i * lda + i] += v;
-}
 
 // M ((n + 1) x n, ld ldm > n) = the lower triangle of A (zeros above) with g^T as its last row
 __global__ void k_lower_copy(int n, const double* __restrict__ A, long long lda, const double* __restrict__ g,
@@ -59,15 +52,6 @@ __global__ void k_lower_copy(int n, const double* __restrict__ A, long long lda,
     const int j = blockIdx.y;                             // column
     if (i < n) M[(size_t)j * ldm + i] = i >= j ? A[(size_t)j * lda + i] : 0.0;
     else if (i == n) M[(size_t)j * ldm + n] = g[j];
-}
-
-// A = its lower triangle mirrored into the upper one, plus v on the diagonal
-__global__ void k_symm_lower(int n, double* __restrict__ A, long long lda, double v) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;   // row
-    const int j = blockIdx.y;                             // column
-    if (i >= n) return;
-    if (i > j) A[(size_t)i * lda + j] = A[(size_t)j * lda + i];
-    else if (i == j) A[(size_t)j * lda + i] += v;
 }
 
 // the first of two factorisations' info codes that is not zero
@@ -79,84 +63,511 @@ __global__ void k_zero_int(int* __restrict__ p) {
     if (threadIdx.x == 0) *p = 0;
 }
 
-// ---- Cholesky factorisation A = L L^T (lower, in place), right-looking in
-// blocks of kCholNb columns.  Each diagonal block is factorised by one
-// wavefront (lane i holds row i in registers), which also writes the block's inverse;
-// the panel below is then L_21 = A_21 L_11^-T, a GEMM with that inverse, and
-// the trailing matrix takes A_22 -= L_21 L_21^T (rocBLAS dsyrk).  rocSOLVER's
-// dpotrf factorises its diagonal panels in a kernel of ~156 us each, most of
-// the time of a factorisation of a few thousand rows.
-constexpr int kCholNb = 64;
-
-__device__ __forceinline__ double readlane_f64(double v, int lane) {
-    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(u & 0xffffffffu), lane);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(u >> 32), lane);
-    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+// dst[i * ldd] = src[i]
+__global__ void k_set_row(int n, const double* __restrict__ src, double* __restrict__ dst, long long ldd) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) dst[(size_t)i * ldd] = src[i];
 }
 
-// Lane l holds row l of the block in registers (r[c] = A(k0 + l, k0 + c)); the
-// column entries a step needs from other rows are read with v_readlane, so the
-// factorisation and the inverse run without LDS or barriers.
-__global__ __launch_bounds__(kCholNb) void k_chol_diag(int n, double* __restrict__ A, long long lda, int k0,
-                                                       double* __restrict__ Linv, int* __restrict__ info) {
-    const int l = threadIdx.x;
-    const int nb = min(kCholNb, n - k0);
-    double r[kCholNb];
+// One observation: a = h . x + r with x = P h; x -> x / sqrt(a), z = xi / sqrt(a).  One workgroup.
+__global__ __launch_bounds__(1024) void k_one_obs(int n, const double* __restrict__ h, double* __restrict__ x,
+                                                  const double* __restrict__ xi, double r, double* __restrict__ z,
+                                                  int* __restrict__ info) {
+    __shared__ double part[16];
+    double s = 0.0;
+    for (int i = threadIdx.x; i < n; i += 1024) s += h[i] * x[i];
+    s = wave_sum(s);
+    if (wave_lane() == 0) part[threadIdx.x >> 6] = s;
+    __syncthreads();
+    double a = r;
+    for (int q = 0; q < 16; ++q) a += part[q];
+    const double ir = 1.0 / sqrt(a);
+    for (int i = threadIdx.x; i < n; i += 1024) x[i] *= ir;
+    if (threadIdx.x == 0) {
+        *z = *xi * ir;
+        *info = a > 0.0 ? 0 : 1;
+    }
+}
+
+// ---- FP64 products on the matrix cores -------------------------------------
+//
+// C (M x N) = alpha A B + beta C [+ diag I], column-major, one workgroup of four
+// wavefronts per T x T tile (T = 64: a 2 x 2 block of 16 x 16 MFMA tiles per
+// wavefront; T = 32: one, for products of few tiles).  K runs in chunks of 16
+// through LDS; loads are issued two chunks ahead (a chunk's products take about
+// the latency of a load that misses L2).  Bound: the matrix cores, for 1,698 x
+// 1,698 x 4,608 (lower half) 347 us = 38 TFLOP/s of 70: 378 tiles leave a CU with
+// one or two, so a quarter of the time is the imbalance.  The
+// operands' layouts are compile-time: LA = 0: A(r, k) at r + k lda, 1: at
+// k + r lda; LB = 0: B(k, c) at c + k ldb, 1: at k + c ldb.  LDS holds [k][row]
+// with rows T + 1 doubles apart (both the column-wise stores of a k-contiguous
+// operand and the fragment reads then spread over the banks).
+// lower: only tiles on or below the diagonal, each also written transposed when
+// mirror is set (symmetric results).  tri: A is a lower triangle read
+// transposed (LA = 1): k starts at the tile's first row and entries k < r
+// count as zero.
+constexpr int kKc = 16;
+typedef double mf_d4 __attribute__((ext_vector_type(4)));
+
+struct GemmArgs {
+    int M, N, K;
+    const double* A;
+    long long lda;
+    const double* B;
+    long long ldb;
+    double* C;
+    long long ldc;
+    double alpha, beta, diag;
+    int lower, mirror, tri;
+};
+
+template <int LA, int LB, int T>
+__global__ __launch_bounds__(256) void k_gemm_f64(GemmArgs g) {
+    constexpr int W = T / 32;             // MFMA tiles per wavefront and dimension
+    constexpr int LDP = T + 1;
+    constexpr int PER = T * kKc / 256;    // elements per thread, chunk and operand
+    __shared__ double sA[2][kKc * LDP], sB[2][kKc * LDP];
+    const int r0 = blockIdx.x * T, c0 = blockIdx.y * T;
+    if (g.lower && r0 + T <= c0) return;
+    const int l = wave_lane(), wv = uniform(threadIdx.x >> 6);
+    const int row = l & 15, grp = l >> 4;
+    const int wr = (wv & 1) * 16 * W, wc = (wv >> 1) * 16 * W;
+    const int kb = g.tri ? r0 / kKc * kKc : 0;
+    const int nk = max(0, (g.K - kb) / kKc);      // whole chunks
+    struct Chunk {
+        double a[PER], b[PER];
+    };
+    // the thread's elements of chunk 0 and the way to the next chunk (rows and columns
+    // past the end repeat the last one: their products are not stored)
+    const double *pa[PER], *pb[PER];
 #pragma unroll
-    for (int c = 0; c < kCholNb; ++c)
-        r[c] = (l < nb && c < nb && l >= c) ? A[(size_t)(k0 + c) * lda + k0 + l] : 0.0;
-    int bad = 0;   // 1-based column of the first pivot that is not positive (the same in every lane)
+    for (int i = 0; i < PER; ++i) {
+        const int t = threadIdx.x + 256 * i;
+        const size_t ka = kb + (LA ? t % kKc : t / T), ra = min(r0 + (LA ? t / kKc : t % T), g.M - 1);
+        const size_t kc = kb + (LB ? t % kKc : t / T), cb = min(c0 + (LB ? t / kKc : t % T), g.N - 1);
+        pa[i] = g.A + (LA ? ka + ra * g.lda : ra + ka * g.lda);
+        pb[i] = g.B + (LB ? kc + cb * g.ldb : cb + kc * g.ldb);
+    }
+    // loads a chunk and moves on by `chunks` (the last whole chunk is loaded again past the end)
+    auto fetch = [&](Chunk& v, int chunks) {
+        const long long da = LA ? kKc * chunks : kKc * chunks * g.lda, db = LB ? kKc * chunks : kKc * chunks * g.ldb;
 #pragma unroll
-    for (int j = 0; j < kCholNb; ++j) {
-        if (j < nb) {
-            const double ajj = readlane_f64(r[j], j);
-            if (!(ajj > 0.0) && bad == 0) bad = j + 1;
-            const double d = sqrt(ajj);
-            const double inv = 1.0 / d;
-            if (l == j) r[j] = d;
-            else if (l > j) r[j] *= inv;
-            // A(l, c) -= L(l, j) L(c, j) for j < c <= l
+        for (int i = 0; i < PER; ++i) {
+            v.a[i] = *pa[i];
+            v.b[i] = *pb[i];
+            pa[i] += da;
+            pb[i] += db;
+        }
+    };
+    auto put = [&](const Chunk& v, int s, int k0) {
 #pragma unroll
-            for (int c = j + 1; c < kCholNb; ++c) {
-                const double lcj = readlane_f64(r[j], c);
-                if (l >= c) r[c] -= r[j] * lcj;
+        for (int i = 0; i < PER; ++i) {
+            const int t = threadIdx.x + 256 * i;
+            const int ka = LA ? t % kKc : t / T, ra = LA ? t / kKc : t % T;
+            sA[s][ka * LDP + ra] = LA && g.tri && k0 + ka < r0 + ra ? 0.0 : v.a[i];
+            sB[s][(LB ? t % kKc : t / T) * LDP + (LB ? t / kKc : t % T)] = v.b[i];
+        }
+    };
+    mf_d4 acc[W][W] = {};
+    auto products = [&](int s) {
+        double a[kKc / 4][W], b[kKc / 4][W];
+#pragma unroll
+        for (int k = 0; k < kKc / 4; ++k)
+#pragma unroll
+            for (int i = 0; i < W; ++i) {
+                a[k][i] = sA[s][(4 * k + grp) * LDP + wr + 16 * i + row];
+                b[k][i] = sB[s][(4 * k + grp) * LDP + wc + 16 * i + row];
             }
+#pragma unroll
+        for (int k = 0; k < kKc / 4; ++k)
+#pragma unroll
+            for (int i = 0; i < W; ++i)
+#pragma unroll
+                for (int j = 0; j < W; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[k][j], a[k][i], acc[i][j], 0, 0, 0);
+    };
+    // chunk c: products from LDS buffer c & 1; chunk c + 1 goes from registers to
+    // the other buffer (last read before the barrier), chunk c + 2 is loaded.  No
+    // branch around a load: the wait at its use would cover every later load too.
+    if (nk > 0) {
+        Chunk u, v;
+        fetch(u, nk > 1);
+        put(u, 0, kb);
+        fetch(u, nk > 2);
+        __syncthreads();
+        for (int c = 0;; c += 2) {
+            fetch(v, c + 3 < nk);
+            products(0);
+            put(u, 1, kb + (c + 1) * kKc);
+            __syncthreads();
+            if (c + 1 >= nk) break;
+            fetch(u, c + 4 < nk);
+            products(1);
+            put(v, 0, kb + (c + 2) * kKc);
+            __syncthreads();
+            if (c + 2 >= nk) break;
+        }
+    }
+    const int kr = kb + nk * kKc;
+    if (kr < g.K) {   // the last columns, fewer than a chunk
+        for (int t = threadIdx.x; t < T * kKc; t += 256) {
+            const int ka = kr + t / T, ra = r0 + t % T, cb = c0 + t % T;
+            const bool in = ka < g.K;
+            sA[0][t / T * LDP + t % T] =
+                in && ra < g.M && !(LA && g.tri && ka < ra) ? g.A[LA ? ka + ra * (size_t)g.lda : ra + ka * (size_t)g.lda] : 0.0;
+            sB[0][t / T * LDP + t % T] = in && cb < g.N ? g.B[LB ? ka + cb * (size_t)g.ldb : cb + ka * (size_t)g.ldb] : 0.0;
+        }
+        __syncthreads();
+        products(0);
+    }
+#pragma unroll
+    for (int i = 0; i < W; ++i)
+#pragma unroll
+        for (int j = 0; j < W; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int r = r0 + wr + 16 * i + row, cc = c0 + wc + 16 * j + grp + 4 * q;
+                if (r >= g.M || cc >= g.N || (g.lower && r < cc)) continue;
+                const double p = g.alpha * acc[i][j][q] + (r == cc ? g.diag : 0.0);
+                double* o = g.C + r + (size_t)cc * g.ldc;
+                *o = g.beta != 0.0 ? p + g.beta * *o : p;
+                if (g.mirror && r > cc) {
+                    o = g.C + cc + (size_t)r * g.ldc;
+                    *o = g.beta != 0.0 ? p + g.beta * *o : p;
+                }
+            }
+}
+
+// tiles of 64 x 64 from which on they are used (see gemm_f64)
+constexpr long long kGemmTiles = 256;
+
+template <int LA, int LB>
+int gemm_f64(const GemmArgs& g, hipStream_t st) {
+    // 64 x 64 tiles need about a tile per CU; below that the smaller tiles keep more CUs busy
+    // (1,698 x 288 x 1,698: 85 us in 1,431 -- 32 x 32 -- tiles, 135 larger ones would leave half the chip idle)
+    const long long tiles = (long long)((g.M + 63) / 64) * ((g.N + 63) / 64) / (g.lower ? 2 : 1);
+    if (tiles >= kGemmTiles)
+        hipLaunchKernelGGL((k_gemm_f64<LA, LB, 64>), dim3((g.M + 63) / 64, (g.N + 63) / 64), dim3(256), 0, st, g);
+    else
+        hipLaunchKernelGGL((k_gemm_f64<LA, LB, 32>), dim3((g.M + 31) / 32, (g.N + 31) / 32), dim3(256), 0, st, g);
+    return launch_check("k_gemm_f64");
+}
+
+// ---- Cholesky factorisation A = L L^T (lower, in place), right-looking in
+// blocks of 64 columns, two launches per block.  A may carry further rows below
+// its n x n part (rows n .. rows - 1): they come out as B L^-T, the triangular
+// solve with the factor, at the cost of more tiles in the same launches.
+//
+// k_chol_panel: every workgroup factorises the 64 x 64 diagonal block itself
+// (in LDS; a launch and a round trip through memory cost more than the repeated
+// work) and solves 64 rows of the panel below.  Both go in 16-column steps: two
+// wavefronts factorise the 16 x 16 diagonal block, each with the rows of its own
+// below it (the rest of the block, the panel rows) -- panel16 -- and all
+// subtract the step's products from the columns to the right by MFMA.  What
+// bounds it: the serial chain of the 64 pivots.  Measured at n = 1,698: 15.4 us
+// (27.8 with loads under a condition each, 256 threads and a division per pivot;
+// the single-wavefront block factorisation before it 61, its panel product apart).
+constexpr int kNb = 64, kSb = 16, kLd = kNb + 1;
+
+// lane C's value of each 16-lane row, in every lane of the row
+template <int C>
+__device__ __forceinline__ double row_bcast(double v) {
+    const long long u = __builtin_bit_cast(long long, v);
+    const long long r = __builtin_amdgcn_update_dpp(0LL, u, 0x150 + C, 0xF, 0xF, true);   // row_newbcast:C
+    return __builtin_bit_cast(double, r);
+}
+
+template <int B, int N, typename F>
+__device__ __forceinline__ void static_range(F&& f) {
+    if constexpr (B < N) {
+        f(std::integral_constant<int, B>{});
+        static_range<B + 1, N>(f);
+    }
+}
+
+// 1 / sqrt(p): the hardware estimate with two Newton steps (a third of the latency
+// of a root and a division), on p scaled by an even power of two into [1/2, 2), so
+// that every positive p is in the estimate's range.  Not positive -> NaN.
+__device__ __forceinline__ double pivot_rsqrt(double p) {
+    const int e = __builtin_amdgcn_frexp_exp(p) & ~1;
+    const double m = __builtin_amdgcn_ldexp(p, -e), h = 0.5 * m;
+    double y = __builtin_amdgcn_rsq(m);
+    y = y * fma(-h, y * y, 1.5);
+    y = y * fma(-h, y * y, 1.5);
+    y = __builtin_amdgcn_ldexp(y, -(e >> 1));
+    return p > 1.7976931348623157e308 ? 0.0 : y;
+}
+
+// A 16-column step of one wavefront: a (lane l of each 16-lane row holds row l of
+// the 16 x 16 diagonal block, the same in all four) -> its Cholesky factor, x (a
+// row of the panel per lane) -> x L^-T; the entries of other rows come by a row
+// broadcast, one for both.  The next column and its pivot's chain come before the
+// other columns' products, which then fill that chain's gaps.  Returns the 1-based
+// column of the first pivot that is not positive, else 0.
+__device__ __forceinline__ int panel16(double (&a)[kSb], double (&x)[kSb]) {
+    const int l = wave_lane() & (kSb - 1);
+    double rd = pivot_rsqrt(row_bcast<0>(a[0]));
+    static_range<0, kSb>([&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        a[j] *= rd;                        // (the pivot's own lane: p / sqrt(p))
+        x[j] *= rd;
+        if constexpr (j + 1 < kSb) {
+            const double f = row_bcast<j + 1>(a[j]);
+            a[j + 1] = fma(-a[j], f, a[j + 1]);
+            x[j + 1] = fma(-x[j], f, x[j + 1]);
+            rd = pivot_rsqrt(row_bcast<j + 1>(a[j + 1]));
+            static_range<j + 2, kSb>([&](auto cc) {
+                constexpr int c = decltype(cc)::value;
+                const double g = row_bcast<c>(a[j]);
+                a[c] = fma(-a[j], g, a[c]);
+                x[c] = fma(-x[j], g, x[c]);
+            });
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    });
+    double d = a[0];
+#pragma unroll
+    for (int c = 1; c < kSb; ++c) d = l == c ? a[c] : d;
+    const unsigned long long m = __ballot(!(d > 0.0)) & 0xFFFFull;
+    return m ? __ffsll(m) : 0;
+}
+
+// acc += s * X(16 rows at x, stride ldx) Y(16 rows at y, stride ldy)^T over 16 columns
+__device__ __forceinline__ mf_d4 mul16(const double* x, int ldx, const double* y, int ldy, double s, mf_d4 acc) {
+    const int row = wave_lane() & 15, grp = wave_lane() >> 4;
+#pragma unroll
+    for (int k = 0; k < kSb; k += 4)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(s * x[row * ldx + k + grp], y[row * ldy + k + grp], acc, 0, 0, 0);
+    return acc;
+}
+
+__device__ __forceinline__ mf_d4 tile_load(const double* x) {
+    const int row = wave_lane() & 15, grp = wave_lane() >> 4;
+    mf_d4 v;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = x[(grp + 4 * q) * kLd + row];
+    return v;
+}
+
+__device__ __forceinline__ void tile_store(double* x, const mf_d4& v) {
+    const int row = wave_lane() & 15, grp = wave_lane() >> 4;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) x[(grp + 4 * q) * kLd + row] = v[q];
+}
+
+constexpr size_t kPanelLds = sizeof(double) * 2 * kNb * kLd;   // the diagonal block and the strip
+
+constexpr int kPanelThreads = 512;
+
+__global__ __launch_bounds__(kPanelThreads) void k_chol_panel(int rows, int n, double* __restrict__ A, long long lda, int k0,
+                                                    double* __restrict__ Ldiag, int* __restrict__ info) {
+    extern __shared__ __align__(16) double sm[];
+    double* D = sm;                        // diagonal block, row-major
+    double* X = sm + kNb * kLd;            // this workgroup's 64 rows of the panel
+    const int nb = min(kNb, n - k0);
+    const int wv = uniform(threadIdx.x >> 6);
+    const int R0 = k0 + nb + blockIdx.x * kNb;
+    const int nr = max(0, min(kNb, rows - R0));
+    // (a block of fewer columns is completed with the unit matrix)
+    {
+        constexpr int N = kNb * kNb / kPanelThreads;
+        const int r = threadIdx.x % kNb, c0 = threadIdx.x / kNb;
+        const double* Ad = A + k0 + min(r, nb - 1);
+        const double* Ax = A + min(R0 + r, rows - 1);
+        double vd[N], vx[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const size_t o = (size_t)(k0 + min(c0 + i * (kPanelThreads / kNb), nb - 1)) * lda;
+            vd[i] = Ad[o];
+            vx[i] = Ax[o];
+        }
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const int c = c0 + i * (kPanelThreads / kNb);
+            D[r * kLd + c] = r < nb && c <= r ? vd[i] : (r == c ? 1.0 : 0.0);
+            X[r * kLd + c] = r < nr && c < nb ? vx[i] : 0.0;
+        }
+    }
+    __syncthreads();
+    int bad = 0;
+    const int l = wave_lane();
+#pragma unroll 1
+    for (int b = 0; b < kNb / kSb; ++b) {
+        double a[kSb], x[kSb];
+        const double* dg = D + b * kSb * (kLd + 1) + (l & (kSb - 1)) * kLd;
+        const bool mine = wv == 1 || (wv == 0 && l < kNb - kSb * (b + 1));
+        double* xr = (wv == 0 ? D + (kSb * (b + 1) + (mine ? l : 0)) * kLd : X + l * kLd) + b * kSb;
+        int e = 0;
+        if (wv < 2) {
+            // (a lane without a row of its own works on some row of the buffers and stores nothing)
+#pragma unroll
+            for (int c = 0; c < kSb; ++c) { a[c] = dg[c]; x[c] = xr[c]; }
+            e = panel16(a, x);
+        }
+        __syncthreads();   // both wavefronts have read the diagonal block
+        if (wv < 2) {
+            if (wv == 0 && l < kSb) {
+#pragma unroll
+                for (int c = 0; c < kSb; ++c) D[b * kSb * (kLd + 1) + l * kLd + c] = c <= l ? a[c] : 0.0;
+            }
+            if (mine) {
+#pragma unroll
+                for (int c = 0; c < kSb; ++c) xr[c] = x[c];
+            }
+            if (e != 0 && bad == 0) bad = b * kSb + e;
+        }
+        __syncthreads();
+        // columns to the right: D_t,u -= D_t,b D_u,b^T for b < u <= t, X_t,u -= X_t,b D_u,b^T
+        int q = 0;
+        for (int u = b + 1; u < kNb / kSb; ++u) {
+            const double* Du = D + u * kSb * kLd + b * kSb;
+            for (int t = u; t < kNb / kSb + 4; ++t, ++q)
+                if (q % (kPanelThreads / kWave) == wv) {
+                    double* row = t < kNb / kSb ? D + t * kSb * kLd : X + (t - kNb / kSb) * kSb * kLd;
+                    tile_store(row + u * kSb, mul16(row + b * kSb, kLd, Du, kLd, -1.0, tile_load(row + u * kSb)));
+                }
+        }
+        __syncthreads();
+    }
+    if (blockIdx.x == 0) {
+        for (int t = threadIdx.x; t < kNb * kNb; t += kPanelThreads) Ldiag[t] = D[(t % kNb) * kLd + t / kNb];
+        if (threadIdx.x == 0 && bad != 0 && *info == 0) *info = k0 + bad;
+    }
+    for (int t = threadIdx.x; t < kNb * kNb; t += kPanelThreads) {
+        const int r = t % kNb, c = t / kNb;
+        if (r < nr && c < nb) A[R0 + r + (size_t)(k0 + c) * lda] = X[r * kLd + c];
+    }
+}
+
+// Trailing matrix: A(r, c) -= sum_k A(r, k) A(c, k) over the 64 panel columns,
+// rows k1 .. rows - 1, columns k1 .. n - 1, tiles on or below the diagonal.  The
+// first workgroup also stores the diagonal block's factor (k_chol_panel's
+// workgroups read the unfactorised block).
+__global__ __launch_bounds__(256) void k_chol_update(int rows, int n, double* __restrict__ A, long long lda, int k0,
+                                                     const double* __restrict__ Ldiag) {
+    constexpr int LDP = kNb + 1, KH = kNb / 2;            // the columns in two halves
+    __shared__ double sR[KH * LDP], sC[KH * LDP];         // [k][row]
+    const int nb = min(kNb, n - k0), k1 = k0 + nb;
+    if (blockIdx.x == 0 && blockIdx.y == 0)
+        for (int t = threadIdx.x; t < kNb * kNb; t += 256) {
+            const int r = t % kNb, c = t / kNb;
+            if (r < nb && c <= r) A[k0 + r + (size_t)(k0 + c) * lda] = Ldiag[t];
+        }
+    const int r0 = k1 + blockIdx.x * kNb, c0 = k1 + blockIdx.y * kNb;
+    if (blockIdx.x < blockIdx.y || c0 >= n || r0 >= rows) return;
+    // (a block with columns to its right has all 64 of its own; rows and columns past
+    // the end repeat the last one, their products are not stored)
+    double va[2][KH / 4], vb[2][KH / 4];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < KH / 4; ++i) {
+            const int t = threadIdx.x + 256 * i, r = t % kNb, k = h * KH + t / kNb;
+            va[h][i] = A[min(r0 + r, rows - 1) + (size_t)(k0 + k) * lda];
+            vb[h][i] = A[min(c0 + r, n - 1) + (size_t)(k0 + k) * lda];
+        }
+    const int l = wave_lane(), wv = uniform(threadIdx.x >> 6);
+    const int row = l & 15, grp = l >> 4;
+    const int wr = (wv & 1) * 32, wc = (wv >> 1) * 32;
+    // the tile itself, in flight with the panel rows (a lane's rows are consecutive in memory)
+    double old[2][2][4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int r = r0 + wr + 16 * i + row, c = c0 + wc + 16 * j + grp + 4 * q;
+                old[i][j][q] = A[min(r, rows - 1) + (size_t)min(c, n - 1) * lda];
+            }
+    mf_d4 acc[2][2] = {};
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        if (h) __syncthreads();
+#pragma unroll
+        for (int i = 0; i < KH / 4; ++i) {
+            const int t = threadIdx.x + 256 * i;
+            sR[t / kNb * LDP + t % kNb] = va[h][i];
+            sC[t / kNb * LDP + t % kNb] = vb[h][i];
+        }
+        __syncthreads();
+#pragma unroll 4
+        for (int k = 0; k < KH; k += 4) {
+            double a[2], b[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                a[i] = sR[(k + grp) * LDP + wr + 16 * i + row];
+                b[i] = sC[(k + grp) * LDP + wc + 16 * i + row];
+            }
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[j], a[i], acc[i][j], 0, 0, 0);
         }
     }
 #pragma unroll
-    for (int c = 0; c < kCholNb; ++c)
-        if (l < nb && c < nb && l >= c) A[(size_t)(k0 + c) * lda + k0 + l] = r[c];
-    // inverse: lane l forms column l of X = L^-1 by forward substitution,
-    // x[i] = (delta(i, l) - sum_{k < i} L(i, k) x[k]) / L(i, i)
-    double x[kCholNb];
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int i = 0; i < kCholNb; ++i) {
-        double t = (i == l) ? 1.0 : 0.0;
+        for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int k = 0; k < i; ++k) t -= readlane_f64(r[k], i) * x[k];
-        x[i] = (i < nb) ? t / readlane_f64(r[i], i) : 0.0;
-    }
-#pragma unroll
-    for (int i = 0; i < kCholNb; ++i) Linv[(size_t)l * kCholNb + i] = (l < nb) ? x[i] : 0.0;
-    if (l == 0 && bad != 0 && *info == 0) *info = k0 + bad;
+            for (int q = 0; q < 4; ++q) {
+                const int r = r0 + wr + 16 * i + row, c = c0 + wc + 16 * j + grp + 4 * q;
+                if (r < rows && c < n && r >= c) A[r + (size_t)c * lda] = old[i][j][q] - acc[i][j][q];
+            }
 }
 
-// B (cols x rows, ld ldb) = A^T, A rows x cols (ld lda), 32 x 32 tiles through LDS
-__global__ void k_transpose(int rows, int cols, const double* __restrict__ A, long long lda,
-                            double* __restrict__ B, long long ldb) {
-    __shared__ double t[32][33];
-    const int r0 = blockIdx.x * 32, c0 = blockIdx.y * 32;
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8 threads
-    for (int j = ty; j < 32; j += 8) {
-        const int r = r0 + tx, c = c0 + j;
-        if (r < rows && c < cols) t[j][tx] = A[(size_t)c * lda + r];
+// A (rows x n, rows >= n, ld lda): the lower triangle of its first n rows -> L,
+// the rows below -> B L^-T.  *info = 0 or the 1-based column of the first pivot
+// that is not positive (as dpotrf reports it).  Ldiag: kNb * kNb doubles.
+int chol_lower(hipStream_t st, int rows, int n, double* A, long long lda, double* Ldiag, int* info) {
+    hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, st, info);
+    for (int k0 = 0; k0 < n; k0 += kNb) {
+        const int k1 = std::min(k0 + kNb, n);
+        const int strips = std::max(1, (rows - k1 + kNb - 1) / kNb), cols = std::max(1, (n - k1 + kNb - 1) / kNb);
+        hipLaunchKernelGGL(k_chol_panel, dim3(strips), dim3(kPanelThreads), kPanelLds, st, rows, n, A, lda, k0, Ldiag, info);
+        hipLaunchKernelGGL(k_chol_update, dim3(k1 < n ? strips : 1, cols), dim3(256), 0, st, rows, n, A, lda, k0,
+                           (const double*)Ldiag);
+        if (int e = launch_check("Cholesky block")) return e;
     }
-    __syncthreads();
-    for (int j = ty; j < 32; j += 8) {
-        const int c = c0 + tx, r = r0 + j;
-        if (r < rows && c < cols) B[(size_t)r * ldb + c] = t[tx][j];
-    }
+    return PT_OK;
+}
+
+// y (n) += A (n x m, ld lda) x (stride incx): kGemvCols columns per workgroup and
+// 256 rows, partial sums in part[chunk][n], added in order by k_gemv_sum
+constexpr int kGemvCols = 64;
+
+__global__ __launch_bounds__(256) void k_gemv(int n, int m, const double* __restrict__ A, long long lda,
+                                              const double* __restrict__ x, long long incx,
+                                              double* __restrict__ part) {
+    const int r = blockIdx.x * 256 + threadIdx.x;
+    const int c0 = blockIdx.y * kGemvCols, c1 = min(m, c0 + kGemvCols);
+    if (r >= n) return;
+    double s = 0.0;
+#pragma unroll 8
+    for (int c = c0; c < c1; ++c) s += A[r + (size_t)c * lda] * x[(size_t)c * incx];
+    part[(size_t)blockIdx.y * n + r] = s;
+}
+
+__global__ __launch_bounds__(256) void k_gemv_sum(int n, int chunks, const double* __restrict__ part, double beta,
+                                                  double* __restrict__ y, long long incy) {
+    const int r = blockIdx.x * 256 + threadIdx.x;
+    if (r >= n) return;
+    double s = 0.0;
+    for (int c = 0; c < chunks; ++c) s += part[(size_t)c * n + r];
+    y[(size_t)r * incy] = beta != 0.0 ? y[(size_t)r * incy] + s : s;
+}
+
+size_t gemv_ws_doubles(int n, int m) { return (size_t)n * ((m + kGemvCols - 1) / kGemvCols); }
+
+// y = [y +] A x
+int gemv(hipStream_t st, int n, int m, const double* A, long long lda, const double* x, long long incx, bool add,
+         double* y, long long incy, double* part) {
+    const int chunks = (m + kGemvCols - 1) / kGemvCols;
+    hipLaunchKernelGGL(k_gemv, dim3((n + 255) / 256, chunks), dim3(256), 0, st, n, m, A, lda, x, incx, part);
+    hipLaunchKernelGGL(k_gemv_sum, dim3((n + 255) / 256), dim3(256), 0, st, n, chunks, (const double*)part,
+                       add ? 1.0 : 0.0, y, incy);
+    return launch_check("gemv");
 }
 
 // xi = (ref - pred) * scale, loss += sum xi^2 (one block of 256 per 256 entries)
@@ -175,91 +586,41 @@ __global__ void k_residual(int n, const double* __restrict__ pred, const double*
     if (threadIdx.x == 0) atomicAdd(loss, part[0] + part[1] + part[2] + part[3]);
 }
 
-std::mutex g_mu;
-std::vector<rocblas_handle> g_handles;
-
-rocblas_handle handle_for_current_device(int* rc) {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) {
-        set_error("pt_kalman_update: hipGetDevice failed");
-        *rc = PT_ERR_HIP;
-        return nullptr;
-    }
-    std::lock_guard<std::mutex> lock(g_mu);
-    if ((int)g_handles.size() <= dev) g_handles.resize(dev + 1, nullptr);
-    if (!g_handles[dev]) {
-        rocblas_handle h = nullptr;
-        if (rocblas_create_handle(&h) != rocblas_status_success) {
-            set_error("pt_kalman_update: rocblas_create_handle failed");
-            *rc = PT_ERR_HIP;
-            return nullptr;
-        }
-        rocblas_set_pointer_mode(h, rocblas_pointer_mode_host);
-        g_handles[dev] = h;
-    }
-    return g_handles[dev];
-}
-
 size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
 // the n_w x n_w form when the observations outnumber the weights
 bool factored_form(int n_w, int m) { return m > n_w; }
-
-// workspace of chol_lower for n rows: the block inverse and the panel
-size_t chol_ws_bytes(int n) { return align256(8 * (size_t)kCholNb * kCholNb) + align256(8 * (size_t)n * kCholNb); }
-
-#define PT_BLAS(call, what)                                                            \
-    do {                                                                               \
-        rocblas_status st_ = (call);                                                   \
-        if (st_ != rocblas_status_success) {                                           \
-            set_error("pt_kalman_update: %s failed (%s)", what, rocblas_status_to_string(st_)); \
-            return PT_ERR_HIP;                                                         \
-        }                                                                              \
-    } while (0)
-
-// A (n x n, lower triangle, ld lda) = L L^T in place; *info = 0 or the 1-based
-// column of the first pivot that is not positive (as dpotrf reports it).
-int chol_lower(rocblas_handle h, hipStream_t st, int n, double* A, int lda, char* ws, int* info) {
-    double* Linv = (double*)ws;
-    double* T = (double*)(ws + align256(8 * (size_t)kCholNb * kCholNb));
-    const double one = 1.0, zero = 0.0, mone = -1.0;
-    hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, st, info);
-    if (int e = launch_check("k_zero_int")) return e;
-    for (int k0 = 0; k0 < n; k0 += kCholNb) {
-        const int nb = std::min(kCholNb, n - k0);
-        hipLaunchKernelGGL(k_chol_diag, dim3(1), dim3(kCholNb), 0, st, n, A, (long long)lda, k0, Linv, info);
-        if (int e = launch_check("k_chol_diag")) return e;
-        const int mk = n - k0 - nb;
-        if (mk <= 0) break;
-        double* A21 = A + (size_t)k0 * lda + k0 + nb;
-        double* A22 = A + (size_t)(k0 + nb) * lda + k0 + nb;
-        // T = A_21 L_11^-T, A_22 -= T T^T, A_21 = T
-        PT_BLAS(rocblas_dgemm(h, rocblas_operation_none, rocblas_operation_transpose, mk, nb, nb, &one, A21, lda,
-                              Linv, kCholNb, &zero, T, mk),
-                "dgemm panel");
-        PT_BLAS(rocblas_dsyrk(h, rocblas_fill_lower, rocblas_operation_none, mk, nb, &mone, T, mk, &one, A22, lda),
-                "dsyrk trailing");
-        if (hipMemcpy2DAsync(A21, (size_t)lda * 8, T, (size_t)mk * 8, (size_t)mk * 8, nb, hipMemcpyDeviceToDevice,
-                             st) != hipSuccess) {
-            set_error("pt_kalman_update: panel copy failed");
-            return PT_ERR_HIP;
-        }
-    }
-    return PT_OK;
-}
 
 }  // namespace
 }  // namespace pt
 
 using namespace pt;
 
+namespace {
+// Workspace: the factorised matrix with the rows it carries, G (n_w x n_w form only),
+// partial sums of the products with a vector, a vector, the diagonal block, info.
+struct KalmanWs {
+    size_t aug, G, part, vec, diag, info, total;
+    long long lda;
+    KalmanWs(int n_w, int m) {
+        const size_t nw = (size_t)n_w, mm = (size_t)m;
+        const bool f = factored_form(n_w, m);
+        lda = f ? 2 * (long long)n_w + 1 : (long long)m + n_w + 1;
+        size_t o = 0;
+        aug = o; o += align256(8 * (size_t)lda * (f ? nw : mm));
+        G = o; o += f ? align256(8 * nw * mm) : 0;
+        part = o; o += align256(8 * gemv_ws_doubles(n_w, std::max(n_w, m)));
+        vec = o; o += align256(8 * nw);
+        diag = o; o += align256(8 * (size_t)kNb * kNb);
+        info = o; o += align256(sizeof(int));
+        total = o;
+    }
+};
+}  // namespace
+
 extern "C" size_t pt_kalman_workspace_bytes(int n_w, int m) {
     if (n_w < 1 || m < 1) return 0;
-    const size_t nw = (size_t)n_w, mm = (size_t)m;
-    if (factored_form(n_w, m))   // G, S, [M; y^T], g, info, Cholesky workspace
-        return align256(8 * nw * mm) + align256(8 * nw * nw) + align256(8 * (nw + 1) * nw) + align256(8 * nw) +
-               align256(sizeof(int)) + chol_ws_bytes(n_w);
-    return align256(8 * nw * mm) + align256(8 * mm * mm) + align256(8 * mm * nw) + chol_ws_bytes(m);
+    return KalmanWs(n_w, m).total;
 }
 
 extern "C" int pt_kalman_residual(int n, const double* pred, const double* ref, double ref_scalar, double scale,
@@ -281,85 +642,52 @@ extern "C" int pt_kalman_update(int n_w, int m, double* P, const double* H, long
     PT_REQUIRE((size_t)n_w * n_w < (1ull << 31) && (factored_form(n_w, m) || (size_t)m * m < (1ull << 31)) &&
                    (size_t)n_w * m < (1ull << 31) && ldh < (1LL << 31),
                "pt_kalman_update: matrices beyond 32-bit BLAS indexing");
-    int rc = PT_OK;
-    rocblas_handle h = handle_for_current_device(&rc);
-    if (!h) return rc;
     hipStream_t st = (hipStream_t)stream;
-    PT_BLAS(rocblas_set_stream(h, st), "rocblas_set_stream");
+    const KalmanWs L(n_w, m);
     char* base = (char*)ws;
-    const double one = 1.0, zero = 0.0, mc = -c;
+    double* S = (double*)(base + L.aug);
+    double* G = (double*)(base + L.G);
+    double* part = (double*)(base + L.part);
+    double* vec = (double*)(base + L.vec);
+    double* diag = (double*)(base + L.diag);
+    int* info2 = (int*)(base + L.info);
+    const long long ld = L.lda;
     if (factored_form(n_w, m)) {
-        const size_t sz_g = align256(8 * (size_t)n_w * m), sz_s = align256(8 * (size_t)n_w * n_w);
-        const size_t sz_m = align256(8 * ((size_t)n_w + 1) * n_w);
-        const int ldm = n_w + 1;
-        double* G = (double*)base;
-        double* S = (double*)(base + sz_g);
-        double* M = (double*)(base + sz_g + sz_s);
-        double* g = (double*)(base + sz_g + sz_s + sz_m);
-        int* info2 = (int*)(base + sz_g + sz_s + sz_m + align256(8 * (size_t)n_w));
-        char* cws = base + sz_g + sz_s + sz_m + align256(8 * (size_t)n_w) + align256(sizeof(int));
-        const dim3 grid2((n_w + 256) / 256, n_w);   // rows 0 .. n_w
         // L = chol(P), lower triangle in place
-        if (int e = chol_lower(h, st, n_w, P, n_w, cws, info)) return e;
+        if (int e = chol_lower(st, n_w, n_w, P, n_w, diag, info)) return e;
         // G = L^T H
-        PT_BLAS(rocblas_dtrmm(h, rocblas_side_left, rocblas_fill_lower, rocblas_operation_transpose,
-                              rocblas_diagonal_non_unit, n_w, m, &one, P, n_w, H, (rocblas_int)ldh, G, n_w),
-                "dtrmm L^T H");
-        // S = G G^T + r I = Ls Ls^T
-        PT_BLAS(rocblas_dsyrk(h, rocblas_fill_lower, rocblas_operation_none, n_w, m, &one, G, n_w, &zero, S, n_w),
-                "dsyrk G G^T");
-        hipLaunchKernelGGL(k_add_diag, dim3((n_w + 255) / 256), dim3(256), 0, st, n_w, S, (long long)n_w, r);
-        if (int e = launch_check("k_add_diag")) return e;
-        if (int e = chol_lower(h, st, n_w, S, n_w, cws, info2)) return e;
+        if (int e = gemm_f64<1, 1>({n_w, m, n_w, P, n_w, H, ldh, G, n_w, 1.0, 0.0, 0.0, 0, 0, 1}, st)) return e;
+        // S = G G^T + r I, below it L and (G xi)^T
+        if (int e = gemm_f64<0, 0>({n_w, n_w, m, G, n_w, G, n_w, S, ld, 1.0, 0.0, r, 1, 0, 0}, st)) return e;
+        if (int e = gemv(st, n_w, m, G, n_w, xi, 1, false, vec, 1, part)) return e;
+        hipLaunchKernelGGL(k_lower_copy, dim3((n_w + 256) / 256, n_w), dim3(256), 0, st, n_w, (const double*)P,
+                           (long long)n_w, (const double*)vec, S + n_w, ld);
+        if (int e = launch_check("k_lower_copy")) return e;
+        // S = Ls Ls^T, M = L Ls^-T, y = Ls^-1 G xi
+        if (int e = chol_lower(st, 2 * n_w + 1, n_w, S, ld, diag, info2)) return e;
         hipLaunchKernelGGL(k_merge_info, dim3(1), dim3(64), 0, st, info, (const int*)info2);
         if (int e = launch_check("k_merge_info")) return e;
-        // [M; y^T] = [L; (G xi)^T] Ls^-T: M = L Ls^-T and y = Ls^-1 G xi in one solve
-        PT_BLAS(rocblas_dgemv(h, rocblas_operation_none, n_w, m, &one, G, n_w, xi, 1, &zero, g, 1), "dgemv G xi");
-        hipLaunchKernelGGL(k_lower_copy, grid2, dim3(256), 0, st, n_w, (const double*)P, (long long)n_w,
-                           (const double*)g, M, (long long)ldm);
-        if (int e = launch_check("k_lower_copy")) return e;
-        PT_BLAS(rocblas_dtrsm(h, rocblas_side_right, rocblas_fill_lower, rocblas_operation_transpose,
-                              rocblas_diagonal_non_unit, n_w + 1, n_w, &one, S, n_w, M, ldm),
-                "dtrsm [L; g^T] Ls^-T");
         // W += M y (= L S^-1 G xi), then P = c r M M^T + q I
-        PT_BLAS(rocblas_dgemv(h, rocblas_operation_none, n_w, n_w, &one, M, ldm, M + n_w, ldm, &one, W, 1),
-                "dgemv M y");
-        const double cr = c * r;
-        PT_BLAS(rocblas_dsyrk(h, rocblas_fill_lower, rocblas_operation_none, n_w, n_w, &cr, M, ldm, &zero, P, n_w),
-                "dsyrk M M^T");
-        hipLaunchKernelGGL(k_symm_lower, grid2, dim3(256), 0, st, n_w, P, (long long)n_w, q);
-        return launch_check("k_symm_lower");
+        const double* M = S + n_w;
+        if (int e = gemv(st, n_w, n_w, M, ld, S + 2 * (size_t)n_w, ld, true, W, 1, part)) return e;
+        return gemm_f64<0, 0>({n_w, n_w, n_w, M, ld, M, ld, P, n_w, c * r, 0.0, q, 1, 1, 0}, st);
     }
-    double* X = (double*)base;
-    double* A = (double*)(base + align256(8 * (size_t)n_w * m));
-    double* Y = (double*)(base + align256(8 * (size_t)n_w * m) + align256(8 * (size_t)m * m));
-    // X = P H
-    PT_BLAS(rocblas_dgemm(h, rocblas_operation_none, rocblas_operation_none, n_w, m, n_w, &one, P, n_w, H,
-                          (rocblas_int)ldh, &zero, X, n_w),
-            "dgemm P H");
-    // A = H^T X + r I
-    PT_BLAS(rocblas_dgemm(h, rocblas_operation_transpose, rocblas_operation_none, m, m, n_w, &one, H,
-                          (rocblas_int)ldh, X, n_w, &zero, A, m),
-            "dgemm H^T X");
-    hipLaunchKernelGGL(k_add_diag, dim3((m + 255) / 256), dim3(256), 0, st, m, A, (long long)m, r);
-    if (int e = launch_check("k_add_diag")) return e;
-    if (int e = chol_lower(h, st, m, A, m, base + align256(8 * (size_t)n_w * m) + align256(8 * (size_t)m * m) +
-                                              align256(8 * (size_t)m * n_w), info))
-        return e;
-    // Y = X^T, then A Y = X^T
-    hipLaunchKernelGGL(k_transpose, dim3((n_w + 31) / 32, (m + 31) / 32), dim3(256), 0, st, n_w, m, X,
-                       (long long)n_w, Y, (long long)m);
-    if (int e = launch_check("k_transpose")) return e;
-    PT_BLAS(rocsolver_dpotrs(h, rocblas_fill_lower, m, n_w, A, m, Y, m), "dpotrs");
-    // P = c (P - Y^T X^T) + q I
-    PT_BLAS(rocblas_dgemm(h, rocblas_operation_transpose, rocblas_operation_transpose, n_w, n_w, m, &mc, Y, m, X,
-                          n_w, &c, P, n_w),
-            "dgemm K X^T");
-    if (q != 0.0) {
-        hipLaunchKernelGGL(k_add_diag, dim3((n_w + 255) / 256), dim3(256), 0, st, n_w, P, (long long)n_w, q);
-        if (int e = launch_check("k_add_diag")) return e;
+    double* X = S + m;                       // n_w rows below the m x m matrix
+    double* z = S + m + (size_t)n_w;         // and the row of the residuals
+    if (m == 1) {
+        if (int e = gemv(st, n_w, n_w, P, n_w, H, 1, false, X, 1, part)) return e;
+        hipLaunchKernelGGL(k_one_obs, dim3(1), dim3(1024), 0, st, n_w, H, X, xi, r, z, info);
+        if (int e = launch_check("k_one_obs")) return e;
+    } else {
+        // X = P H, A = H^T X + r I, the residuals as the last row
+        if (int e = gemm_f64<0, 1>({n_w, m, n_w, P, n_w, H, ldh, X, ld, 1.0, 0.0, 0.0, 0, 0, 0}, st)) return e;
+        if (int e = gemm_f64<1, 1>({m, m, n_w, H, ldh, X, ld, S, ld, 1.0, 0.0, r, 1, 0, 0}, st)) return e;
+        hipLaunchKernelGGL(k_set_row, dim3((m + 255) / 256), dim3(256), 0, st, m, xi, z, ld);
+        if (int e = launch_check("k_set_row")) return e;
+        // A = L L^T, Z = X L^-T, z = L^-1 xi
+        if (int e = chol_lower(st, m + n_w + 1, m, S, ld, diag, info)) return e;
     }
-    // W += Y^T xi
-    PT_BLAS(rocblas_dgemv(h, rocblas_operation_transpose, m, n_w, &one, Y, m, xi, 1, &one, W, 1), "dgemv K xi");
-    return PT_OK;
+    // W += Z z, P = c (P - Z Z^T) + q I
+    if (int e = gemv(st, n_w, m, X, ld, z, ld, true, W, 1, part)) return e;
+    return gemm_f64<0, 0>({n_w, n_w, m, X, ld, X, ld, P, n_w, -c, c, q, 1, 1, 0}, st);
 }

@@ -18,7 +18,7 @@ then runs
              H = (1/N) sum_i dE_i/dW           pt_mlp_train_grad
     force:   pt_mlp_energy_grad_multi, pt_acsf_adjoint (self term),
              pt_kalman_residual, H = dF/dW      pt_mlp_jacobian
-    both:    pt_kalman_update (rocBLAS GEMMs + rocSOLVER Cholesky), pt_mlp_pack
+    both:    pt_kalman_update (products and Cholesky on the matrix cores), pt_mlp_pack
 
 with nothing read back to the host inside an epoch.
 """

@@ -1,0 +1,50 @@
+"""pt_kalman_update where its products' and its factorisation's tiles end: fewer rows
+than a tile, a remainder of one, whole tiles, a K remainder, both forms and a leading
+dimension of H beyond n_w, against the oracle's explicit-inverse update.  Tolerance:
+P is 50 I + B B^T and r >= 0.01, so A's condition number stays below 1e4 and the
+inverse's rounding below about 1e4 n eps = 4e-10 relative to the correction, which is
+below 1 % of P: 1e-10 of the largest entry."""
+
+import numpy as np
+import pytest
+
+from oracle import kalman as okf
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+@pytest.mark.parametrize("n_w,m", [(1, 1), (1, 3), (15, 16), (16, 15), (17, 2), (63, 65), (64, 64), (64, 128), (65, 63),
+                                   (129, 130), (190, 97), (270, 31)])
+def test_update_at_tile_edges(n_w, m):
+    from pantea_amd import _lib
+
+    lib = _lib.load()
+    rng = np.random.default_rng(7 * n_w + m)
+    st = okf.FilterState(rng.normal(size=n_w), kalman_type=1)
+    B = rng.normal(size=(n_w, n_w)) * 0.05
+    st.P = np.eye(n_w) * 50.0 + B @ B.T
+    H = rng.normal(size=(n_w, m)) * 0.02
+    xi = rng.normal(size=m)
+    ldh = n_w + 3
+    P_d = torch.as_tensor(st.P.T.copy(), device="cuda")
+    W_d = torch.as_tensor(st.W[:, 0].copy(), device="cuda")
+    H_d = torch.full((m, ldh), float("nan"), dtype=torch.float64, device="cuda")
+    H_d[:, :n_w] = torch.as_tensor(H.T.copy(), device="cuda")
+    x_d = torch.as_tensor(xi, device="cuda")
+    r, c, q = st.lambda0, 1.0 / st.lambda0, st.q
+    okf.ekf_update(st, xi, H)
+    # the workspace holds NaN: nothing of it may reach the result
+    ws = torch.full((lib.pt_kalman_workspace_bytes(n_w, m) // 8,), float("nan"), dtype=torch.float64, device="cuda")
+    info = torch.full((1,), -1, dtype=torch.int32, device="cuda")
+    _lib.check(lib.pt_kalman_update(n_w, m, P_d.data_ptr(), H_d.data_ptr(), ldh, x_d.data_ptr(), W_d.data_ptr(),
+                                    r, c, q, ws.data_ptr(), ws.numel() * 8, info.data_ptr(), _lib.stream_ptr()),
+               "pt_kalman_update")
+    torch.cuda.synchronize()
+    assert int(info.item()) == 0
+    P = P_d.cpu().numpy().T
+    np.testing.assert_array_equal(P, P.T)
+    np.testing.assert_allclose(P, st.P, rtol=0, atol=1e-10 * np.abs(st.P).max())
+    dW = st.W[:, 0] - W_d.cpu().numpy()
+    assert np.abs(dW).max() <= 1e-10 * max(np.abs(st.W[:, 0]).max(), 1.0)
