@@ -358,6 +358,23 @@ int pt_mlp_train_grad(int mode, int n_atoms, const void *G, const void *T, int l
                       int g_precision, const double *scale, const pt_mlp_desc *desc,
                       const void *packed, const double *gy, double tseed, double *grad,
                       pt_stream_t stream);
+/* Several elements' networks in one launch, for the weight gradient and for
+ * the per-row Jacobian below: every job is one call of pt_mlp_train_grad (out:
+ * grad) or pt_mlp_jacobian (out: J; gy unused). */
+typedef struct {
+    int n_atoms;
+    const void *G;
+    const void *T;
+    const double *scale;
+    const pt_mlp_desc *desc;
+    const void *packed;
+    const double *gy;
+    double *out;
+} pt_mlp_train_job;
+int pt_mlp_train_grad_multi(int mode, int n_jobs, const pt_mlp_train_job *jobs, int ldg, int g_precision,
+                            double tseed, pt_stream_t stream);
+int pt_mlp_jacobian_multi(int n_dir, int n_jobs, const pt_mlp_train_job *jobs, long long t_dir, int ldg, double sign,
+                          long long ldj, pt_stream_t stream);
 /* delta = w_F 2 (F - F*) / (3N), gy = w_E 2 (E - E*) / N^2 (per atom), and
  * loss[0] += w_E ((E - E*)/N)^2, loss[1] += w_F / (3N) sum |F - F*|^2.
  * energy: device scalar. */

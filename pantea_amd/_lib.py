@@ -92,6 +92,11 @@ class MlpJob(ctypes.Structure):
                 ("packed", _vp), ("e_atom", _vp), ("dEdG", _vp)]
 
 
+class MlpTrainJob(ctypes.Structure):
+    _fields_ = [("n_atoms", _c_int), ("G", _vp), ("T", _vp), ("scale", _vp), ("desc", ctypes.POINTER(MlpDesc)),
+                ("packed", _vp), ("gy", _vp), ("out", _vp)]
+
+
 class AcsfRun(ctypes.Structure):
     _fields_ = [("table", _vp), ("kind", _c_int), ("n_centers", _c_int), ("center_begin", _c_int), ("dir", _c_int),
                 ("centers", _vp), ("out", _vp), ("w", _vp), ("f_self", _vp), ("delta", _vp)]
@@ -157,6 +162,8 @@ _SIGS = {
     "pt_mlp_param_count": (_c_size, [_vp]),
     "pt_mlp_train_grad": (_c_int, [_c_int, _c_int, _vp, _vp, _c_int, _c_int, _vp, _vp, _vp, _vp,
                                    _c_dbl, _vp, _vp]),
+    "pt_mlp_train_grad_multi": (_c_int, [_c_int, _c_int, ctypes.POINTER(MlpTrainJob), _c_int, _c_int, _c_dbl, _vp]),
+    "pt_mlp_jacobian_multi": (_c_int, [_c_int, _c_int, ctypes.POINTER(MlpTrainJob), _c_ll, _c_int, _c_dbl, _c_ll, _vp]),
     "pt_train_seeds": (_c_int, [_c_int, _vp, _vp, _vp, _c_dbl, _c_dbl, _c_dbl, _vp, _vp, _vp, _vp]),
     "pt_train_batch_words": (_c_int, [_c_int, _c_int]),
     "pt_train_batch_assemble": (_c_int, [_c_int, _c_int, _vp, _c_int, _c_int, _c_int, _vp, _vp, _vp, _vp, _vp, _vp, _vp,

@@ -738,438 +738,301 @@ __device__ __forceinline__ void wgrad_tile(const typename MT<MODE>::T* A, const 
     }
 }
 
-struct TrainArgs {
+// What bounds it: one tile's chain of small products and elementwise passes
+// between barriers; the four wavefronts of a workgroup share a tile (column tiles
+// and halves of the products, cells of the elementwise passes), where one
+// wavefront per tile needed the same LDS and left three of a CU's four SIMDs idle.
+// Measured, student networks of two elements: Jacobian of 4,608 rows 240 -> 58 us
+// (FP64), gradient sums of 26,000 atoms 226 -> 72 us (BF16x3), 123 -> 24 us for one
+// structure (FP64); the elements share the launch.
+struct TrainNet {
     MlpShape s;
     int n_atoms;
+    int block0, nblocks;  // this network's workgroups
+    int nparam;
     const void* G;
-    const void* T;
-    int ldg;
-    int g_f64;
+    const void* T;        // TRAIN: tangents; JACOBIAN: T[d * t_dir + atom * ldg + k]
     const double* scale;
     double scale_add;
     const char* packed;
-    const double* gy;     // per-atom seed of y
-    double tseed;         // seed of ydot (same for every atom)
-    double* grad;         // parameter gradient, FP64, layout of the unpacked params
-    int stride;
-    int nparam;
+    const double* gy;     // TRAIN: per-atom seed of y
+    double* out;          // TRAIN: parameter gradient (FP64, layout of the unpacked params); JACOBIAN: J
 };
 
-__device__ __forceinline__ void wave_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
+struct TrainArgs {
+    TrainNet net[kMlpNets];
+    int n_net;
+    int ldg;
+    int g_f64;
+    double tseed;         // seed of ydot (same for every atom); JACOBIAN: the sign
+    int stride;
+    // JACOBIAN
+    int n_dir;
+    long long t_dir, ldj;
+};
+
+// LDS of a workgroup: layer inputs (H + 1), pre-activations (H) and two reverse
+// buffers of 32 rows, 64 per-row scalars, and the gradient sums (TRAIN)
+inline size_t train_lds(size_t word, int H, int stride, int nparam) {
+    return word * ((size_t)(2 * H + 3) * 32 * stride + 64 + nparam);
 }
 
-template <int MODE>
+// cells of 16 rows x `width` columns (a multiple of 32) over the 256 threads
+template <typename F>
+__device__ __forceinline__ void for_cells(int width, F&& f) {
+    for (int k = threadIdx.x & 31; k < width; k += 32) {
+        f((int)(threadIdx.x >> 5), k);
+        f((int)(threadIdx.x >> 5) + 8, k);
+    }
+}
+
+// JAC = false: sums of the loss gradient over the atoms.  JAC = true (FP64): one
+// row of J per (atom, direction), nothing summed: a dense layer's block of a row
+// is the outer product a[r] (x) zbar[r] + adot[r] (x) zdotbar[r] and a bias block
+// is zbar[r], written to HBM with consecutive threads on consecutive parameters.
+template <int MODE, bool JAC>
 __global__ __launch_bounds__(256) void k_mlp_train(TrainArgs a) {
     typedef typename MT<MODE>::T T;
     extern __shared__ __align__(16) char smem[];
-    const MlpShape& s = a.s;
+    int gi = 0;
+    while (gi + 1 < a.n_net && (int)blockIdx.x >= a.net[gi + 1].block0) ++gi;
+    const TrainNet& net = a.net[gi];
+    const MlpShape& s = net.s;
     const int H = s.n_hidden;
-    const int l = wave_lane();
-    const int wv = threadIdx.x >> 6;
-    const int wpb = blockDim.x >> 6;
+    const int l = wave_lane(), tid = threadIdx.x;
+    const int wv = uniform(tid >> 6);
     const int stride = a.stride;
     const size_t tile = (size_t)32 * stride;
-    const size_t per_wave = (size_t)(2 * H + 3) * tile + 64 + a.nparam;
-    T* base = reinterpret_cast<T*>(smem) + (size_t)wv * per_wave;
-    T* Abuf[kMaxHidden + 1];
-    T* Zbuf[kMaxHidden];
-    for (int h = 0; h <= H; ++h) Abuf[h] = base + h * tile;
-    for (int h = 0; h < H; ++h) Zbuf[h] = base + (H + 1 + h) * tile;
-    T* P[2] = {base + (2 * H + 1) * tile, base + (2 * H + 2) * tile};
-    T* outv = base + (2 * H + 3) * tile;  // [0,16): z_L, [16,32): zdot_L, [32,48): zbar_L, [48,64): zdotbar_L
+    T* base = reinterpret_cast<T*>(smem);
+    auto Abuf = [&](int h) { return base + h * tile; };
+    auto Zbuf = [&](int h) { return base + (H + 1 + h) * tile; };
+    T* P = base + (2 * H + 1) * tile;     // reverse buffers, swapped after each layer
+    T* Q = P + tile;
+    T* outv = Q + tile;                   // [0,16): z_L, [16,32): zdot_L, [32,48): zbar_L, [48,64): zdotbar_L
     T* gacc = outv + 64;
-    for (int k = l; k < a.nparam; k += kWave) gacc[k] = T(0);
+    const char* packed = net.packed;
+    if (!JAC)
+        for (int k = tid; k < net.nparam; k += 256) gacc[k] = T(0);
     const int row = l & 15, grp = l >> 4;
-    const T* wout = (MODE == PT_MLP_F64) ? (const T*)(a.packed + s.wout64) : (const T*)(a.packed + s.wout32);
-    const T bout = (MODE == PT_MLP_F64) ? (T)((const double*)(a.packed + s.bout64))[0]
-                                        : (T)((const float*)(a.packed + s.bout32))[0];
-    const int ntiles = (a.n_atoms + 15) / 16;
-    for (int tl = blockIdx.x * wpb + wv; tl < ntiles; tl += gridDim.x * wpb) {
-        const int a0 = tl * 16;
-        // scaled input and its tangent
-        for (int e = l; e < 16 * s.in_p; e += kWave) {
-            const int r = e / s.in_p, k = e % s.in_p;
-            const int atom = a0 + r;
+    const T* wout = (MODE == PT_MLP_F64) ? (const T*)(packed + s.wout64) : (const T*)(packed + s.wout32);
+    const T bout = (MODE == PT_MLP_F64) ? (T)((const double*)(packed + s.bout64))[0]
+                                        : (T)((const float*)(packed + s.bout32))[0];
+    const int L = H;
+    const int fan_L = H > 0 ? s.w[H - 1] : s.in_dim;
+    const int ndir = JAC ? a.n_dir : 1;
+    const int items = (net.n_atoms + 15) / 16 * ndir;
+    for (int it = blockIdx.x - net.block0; it < items; it += net.nblocks) {
+        const int a0 = it / ndir * 16, d = it % ndir;
+        const int nrows = min(16, net.n_atoms - a0);
+        // row r of this item in J
+        auto Jrow = [&](int r) { return net.out + (size_t)((long long)(a0 + r) * ndir + d) * a.ldj; };
+        // scaled input (rows 0..15) and its tangent (rows 16..31)
+        for_cells(s.in_p, [&](int r, int k) {
             T v = T(0), t = T(0);
-            if (atom < a.n_atoms && k < s.in_dim) {
-                const size_t o = (size_t)atom * a.ldg + k;
-                const double g = a.g_f64 ? ((const double*)a.G)[o] : (double)((const float*)a.G)[o];
-                const double gt = a.g_f64 ? ((const double*)a.T)[o] : (double)((const float*)a.T)[o];
-                v = (T)((g - a.scale[k]) * a.scale[s.in_dim + k] + a.scale_add);
-                t = (T)(gt * a.scale[s.in_dim + k]);
+            if (r < nrows && k < s.in_dim) {
+                const size_t o = (size_t)(a0 + r) * a.ldg + k, ot = o + (JAC ? (size_t)d * a.t_dir : 0);
+                const double g = a.g_f64 ? ((const double*)net.G)[o] : (double)((const float*)net.G)[o];
+                const double gt = a.g_f64 ? ((const double*)net.T)[ot] : (double)((const float*)net.T)[ot];
+                v = (T)((g - net.scale[k]) * net.scale[s.in_dim + k] + net.scale_add);
+                t = (T)(gt * net.scale[s.in_dim + k]);
             }
-            Abuf[0][r * stride + k] = v;
-            Abuf[0][(16 + r) * stride + k] = t;
-        }
-        wave_fence();
-        // forward: primal rows 0..15, tangent rows 16..31
+            Abuf(0)[r * stride + k] = v;
+            Abuf(0)[(16 + r) * stride + k] = t;
+        });
+        __syncthreads();
+        // forward: the products of (column tile, half) units in turn, then the activations
         int kin = s.in_p;
         for (int h = 0; h < H; ++h) {
             const int wp = s.wp[h];
-            for (int n0 = 0; n0 < wp; n0 += 16) {
-                T az[4] = {T(0), T(0), T(0), T(0)}, at[4] = {T(0), T(0), T(0), T(0)};
-                if (MODE == PT_MLP_F64) {
-                    gemm_tile<MODE>(Abuf[h], stride, kin, a.packed, s.W64[h], 0, wp, false, n0, az);
-                    gemm_tile<MODE>(Abuf[h] + 16 * stride, stride, kin, a.packed, s.W64[h], 0, wp, false, n0, at);
-                } else {
-                    gemm_tile<MODE>(Abuf[h], stride, kin, a.packed, s.WTh[h], s.WTl[h], kin, true, n0, az);
-                    gemm_tile<MODE>(Abuf[h] + 16 * stride, stride, kin, a.packed, s.WTh[h], s.WTl[h], kin, true, n0, at);
-                }
+            for (int u = wv; u < wp / 8; u += 4) {
+                const int n0 = (u >> 1) * 16, half = (u & 1) * 16;
                 const int col = n0 + row;
-                const T bias = (MODE == PT_MLP_F64) ? (T)((const double*)(a.packed + s.b64[h]))[col]
-                                                    : (T)((const float*)(a.packed + s.b32[h]))[col];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int r = crow<MODE>(grp, i);
-                    const T z = az[i] + bias, zd = at[i];
-                    T y, dy;
-                    activate<T>(s.act[h], z, y, dy);
-                    const bool pad = col >= s.w[h];
-                    Zbuf[h][r * stride + col] = pad ? T(0) : z;
-                    Zbuf[h][(16 + r) * stride + col] = pad ? T(0) : zd;
-                    Abuf[h + 1][r * stride + col] = pad ? T(0) : y;
-                    Abuf[h + 1][(16 + r) * stride + col] = pad ? T(0) : dy * zd;
+                T z[4] = {T(0), T(0), T(0), T(0)};
+                if (n0 < s.w[h]) {
+                    if (MODE == PT_MLP_F64)
+                        gemm_tile<MODE>(Abuf(h) + half * stride, stride, kin, packed, s.W64[h], 0, wp, false, n0, z);
+                    else
+                        gemm_tile<MODE>(Abuf(h) + half * stride, stride, kin, packed, s.WTh[h], s.WTl[h], kin, true, n0, z);
                 }
+                const T bias = half ? T(0) : (MODE == PT_MLP_F64) ? (T)((const double*)(packed + s.b64[h]))[col]
+                                                                  : (T)((const float*)(packed + s.b32[h]))[col];
+                const bool pad = col >= s.w[h];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    Zbuf(h)[(half + crow<MODE>(grp, i)) * stride + col] = pad ? T(0) : z[i] + bias;
             }
-            wave_fence();
+            __syncthreads();
+            for_cells(wp, [&](int r, int k) {
+                T y, dy;
+                activate<T>(s.act[h], Zbuf(h)[r * stride + k], y, dy);
+                const bool pad = k >= s.w[h];
+                Abuf(h + 1)[r * stride + k] = pad ? T(0) : y;
+                Abuf(h + 1)[(16 + r) * stride + k] = pad ? T(0) : dy * Zbuf(h)[(16 + r) * stride + k];
+            });
+            __syncthreads();
             kin = wp;
         }
-        // output layer and its reverse seeds: 4 lanes per atom
-        {
+        // output layer and its reverse seeds: 4 lanes per atom, one wavefront
+        if (wv == 0) {
             const int r = l >> 2, part = l & 3;
             T z = T(0), zd = T(0);
             for (int k = part; k < kin; k += 4) {
-                z += Abuf[H][r * stride + k] * wout[k];
-                zd += Abuf[H][(16 + r) * stride + k] * wout[k];
+                z += Abuf(H)[r * stride + k] * wout[k];
+                zd += Abuf(H)[(16 + r) * stride + k] * wout[k];
             }
             z += __shfl_xor(z, 1, kWave); z += __shfl_xor(z, 2, kWave);
             zd += __shfl_xor(zd, 1, kWave); zd += __shfl_xor(zd, 2, kWave);
             z += bout;
             T y, dy, ddy;
             activate2<T>(s.act_out, z, y, dy, ddy);
-            const int atom = a0 + r;
-            const bool ok = atom < a.n_atoms;
-            const T gy = ok ? (T)a.gy[atom] : T(0);
+            const bool ok = r < nrows;
+            const T gy = !JAC && ok ? (T)net.gy[a0 + r] : T(0);
             const T gt = ok ? (T)a.tseed : T(0);
             if (part == 0) {
-                outv[r] = z;
-                outv[16 + r] = zd;
                 outv[32 + r] = gy * dy + gt * ddy * zd;  // zbar_L
                 outv[48 + r] = gt * dy;                  // zdotbar_L
             }
         }
-        wave_fence();
-        // gradients of the output layer
-        const int L = H;
-        for (int k = l; k < kin; k += kWave) {
-            T gw = T(0);
-            for (int r = 0; r < 16; ++r)
-                gw += Abuf[H][r * stride + k] * outv[32 + r] + Abuf[H][(16 + r) * stride + k] * outv[48 + r];
-            const int fan_in = H > 0 ? s.w[H - 1] : s.in_dim;
-            if (k < fan_in) gacc[s.pW[L] + k] += gw;
+        __syncthreads();
+        // gradients of the output layer; abar, adotbar of the last hidden output -> P
+        if constexpr (JAC) {
+            for (int k = tid; k < fan_L; k += 256)
+                for (int r = 0; r < nrows; ++r)
+                    Jrow(r)[s.pW[L] + k] = Abuf(H)[r * stride + k] * outv[32 + r] + Abuf(H)[(16 + r) * stride + k] * outv[48 + r];
+            if (tid < nrows) Jrow(tid)[s.pb[L]] = outv[32 + tid];
+        } else {
+            for (int k = tid; k < fan_L; k += 256) {
+                T gw = T(0);
+                for (int r = 0; r < 16; ++r)
+                    gw += Abuf(H)[r * stride + k] * outv[32 + r] + Abuf(H)[(16 + r) * stride + k] * outv[48 + r];
+                gacc[s.pW[L] + k] += gw;
+            }
+            if (tid == 255) {
+                T gb = T(0);
+                for (int r = 0; r < 16; ++r) gb += outv[32 + r];
+                gacc[s.pb[L]] += gb;
+            }
         }
-        if (l == 0) {
-            T gb = T(0);
-            for (int r = 0; r < 16; ++r) gb += outv[32 + r];
-            gacc[s.pb[L]] += gb;
-        }
-        // abar, adotbar of the last hidden output -> P[0]
-        for (int e = l; e < 16 * kin; e += kWave) {
-            const int r = e / kin, k = e % kin;
-            P[0][r * stride + k] = outv[32 + r] * wout[k];
-            P[0][(16 + r) * stride + k] = outv[48 + r] * wout[k];
-        }
-        wave_fence();
-        int cur = 0;
         for (int h = H - 1; h >= 0; --h) {
             const int wp = s.wp[h];
             const int kin_h = h > 0 ? s.wp[h - 1] : s.in_p;
             // zbar = abar f'(z) + adotbar f''(z) zdot ; zdotbar = adotbar f'(z)   (in place)
-            for (int e = l; e < 16 * wp; e += kWave) {
-                const int r = e / wp, k = e % wp;
-                const T z = Zbuf[h][r * stride + k], zd = Zbuf[h][(16 + r) * stride + k];
+            for_cells(wp, [&](int r, int k) {
+                const T z = Zbuf(h)[r * stride + k], zd = Zbuf(h)[(16 + r) * stride + k];
                 T y, dy, ddy;
                 activate2<T>(s.act[h], z, y, dy, ddy);
-                const T ab = P[cur][r * stride + k], adb = P[cur][(16 + r) * stride + k];
+                const T ab = h == H - 1 ? outv[32 + r] * wout[k] : P[r * stride + k];
+                const T adb = h == H - 1 ? outv[48 + r] * wout[k] : P[(16 + r) * stride + k];
                 const bool pad = k >= s.w[h];
-                P[cur][r * stride + k] = pad ? T(0) : ab * dy + adb * ddy * zd;
-                P[cur][(16 + r) * stride + k] = pad ? T(0) : adb * dy;
-            }
-            wave_fence();
-            // dW_h += A_h^T [zbar; zdotbar]  (K = 32 rows)
+                P[r * stride + k] = pad ? T(0) : ab * dy + adb * ddy * zd;
+                P[(16 + r) * stride + k] = pad ? T(0) : adb * dy;
+            });
+            __syncthreads();
             const int fan_in = h > 0 ? s.w[h - 1] : s.in_dim;
-            for (int i0 = 0; i0 < kin_h; i0 += 16) {
-                for (int o0 = 0; o0 < wp; o0 += 16) {
+            const int wo = s.w[h];
+            const T* A = Abuf(h);
+            if constexpr (JAC) {
+                // rows of J: W_h[in][out], q = in * wo + out (in and out advance without a division)
+                const int nW = fan_in * wo, dq = 256 / wo, rq = 256 - dq * wo;
+                int in = tid / wo, out = tid - in * wo;
+                for (int q = tid; q < nW; q += 256) {
+                    for (int r = 0; r < nrows; ++r)
+                        Jrow(r)[s.pW[h] + q] = A[r * stride + in] * P[r * stride + out] +
+                                               A[(16 + r) * stride + in] * P[(16 + r) * stride + out];
+                    in += dq; out += rq;
+                    if (out >= wo) { out -= wo; ++in; }
+                }
+                for (int k = tid; k < wo; k += 256)
+                    for (int r = 0; r < nrows; ++r) Jrow(r)[s.pb[h] + k] = P[r * stride + k];
+            } else {
+                // dW_h += A_h^T [zbar; zdotbar]  (K = 32 rows), tiles in turn over the wavefronts
+                const int to = (wo + 15) / 16, ti = (fan_in + 15) / 16;
+                for (int u = wv; u < ti * to; u += 4) {
+                    const int i0 = u / to * 16, o0 = u % to * 16;
                     T c[4];
-                    wgrad_tile<MODE>(Abuf[h], P[cur], stride, i0, o0, c);
+                    wgrad_tile<MODE>(A, P, stride, i0, o0, c);
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         const int in = i0 + crow<MODE>(grp, i), out = o0 + row;
-                        if (in < fan_in && out < s.w[h]) gacc[s.pW[h] + (size_t)in * s.w[h] + out] += c[i];
+                        if (in < fan_in && out < wo) gacc[s.pW[h] + (size_t)in * wo + out] += c[i];
                     }
                 }
-            }
-            for (int k = l; k < s.w[h]; k += kWave) {
-                T gb = T(0);
-                for (int r = 0; r < 16; ++r) gb += P[cur][r * stride + k];
-                gacc[s.pb[h] + k] += gb;
+                for (int k = tid; k < wo; k += 256) {
+                    T gb = T(0);
+                    for (int r = 0; r < 16; ++r) gb += P[r * stride + k];
+                    gacc[s.pb[h] + k] += gb;
+                }
             }
             if (h > 0) {
-                // [abar; adotbar] of layer h's input = [zbar; zdotbar] W_h^T  -> P[cur ^ 1]
-                for (int n0 = 0; n0 < kin_h; n0 += 16) {
-                    T c0[4] = {T(0), T(0), T(0), T(0)}, c1[4] = {T(0), T(0), T(0), T(0)};
-                    if (MODE == PT_MLP_F64) {
-                        gemm_tile<MODE>(P[cur], stride, wp, a.packed, s.W64[h], 0, wp, true, n0, c0);
-                        gemm_tile<MODE>(P[cur] + 16 * stride, stride, wp, a.packed, s.W64[h], 0, wp, true, n0, c1);
-                    } else {
-                        gemm_tile<MODE>(P[cur], stride, wp, a.packed, s.Wh[h], s.Wl[h], wp, true, n0, c0);
-                        gemm_tile<MODE>(P[cur] + 16 * stride, stride, wp, a.packed, s.Wh[h], s.Wl[h], wp, true, n0, c1);
+                // [abar; adotbar] of layer h's input = [zbar; zdotbar] W_h^T  -> Q
+                for (int u = wv; u < kin_h / 8; u += 4) {
+                    const int n0 = (u >> 1) * 16, half = (u & 1) * 16;
+                    T c[4] = {T(0), T(0), T(0), T(0)};
+                    if (n0 < s.w[h - 1]) {
+                        if (MODE == PT_MLP_F64)
+                            gemm_tile<MODE>(P + half * stride, stride, wp, packed, s.W64[h], 0, wp, true, n0, c);
+                        else
+                            gemm_tile<MODE>(P + half * stride, stride, wp, packed, s.Wh[h], s.Wl[h], wp, true, n0, c);
                     }
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const int r = crow<MODE>(grp, i);
-                        P[cur ^ 1][r * stride + n0 + row] = c0[i];
-                        P[cur ^ 1][(16 + r) * stride + n0 + row] = c1[i];
-                    }
+                    for (int i = 0; i < 4; ++i) Q[(half + crow<MODE>(grp, i)) * stride + n0 + row] = c[i];
                 }
-                cur ^= 1;
+                T* t = P; P = Q; Q = t;
             }
-            wave_fence();
+            __syncthreads();
         }
+        __syncthreads();
     }
-    wave_fence();
-    for (int k = l; k < a.nparam; k += kWave) {
-        const double v = (double)gacc[k];
-        if (v != 0.0) atomicAdd(&a.grad[k], v);
+    if constexpr (!JAC) {
+        __syncthreads();
+        for (int k = tid; k < net.nparam; k += 256) {
+            const double v = (double)gacc[k];
+            if (v != 0.0) atomicAdd(&net.out[k], v);
+        }
     }
 }
 
-template <int MODE>
-int launch_train(TrainArgs a, hipStream_t st) {
+constexpr int kTrainBlocks = 4096;   // of the sums: each ends with an atomic per parameter
+
+// Workgroups of a launch's networks: an item each, shared out by items beyond
+// kTrainBlocks.  Networks whose widest, deepest and largest need more LDS together
+// than a workgroup has are launched one by one.
+template <int MODE, bool JAC>
+int launch_train(TrainArgs& a, hipStream_t st) {
     typedef typename MT<MODE>::T T;
-    const int H = a.s.n_hidden;
-    a.stride = a.s.wmax + (sizeof(T) == 8 ? 1 : 4);
-    const size_t per_wave = sizeof(T) * ((size_t)(2 * H + 3) * 32 * a.stride + 64 + a.nparam);
-    const size_t budget = lds_limit();
-    if (per_wave > budget) {
-        set_error("mlp training: %zu bytes of LDS per wavefront exceed the device limit", per_wave);
+    int wmax = 0, hid = 0, np = 0;
+    long long total = 0;
+    for (int g = 0; g < a.n_net; ++g) {
+        wmax = std::max(wmax, a.net[g].s.wmax);
+        hid = std::max(hid, a.net[g].s.n_hidden);
+        np = std::max(np, a.net[g].nparam);
+        total += (long long)((a.net[g].n_atoms + 15) / 16) * (JAC ? a.n_dir : 1);
+    }
+    a.stride = wmax + (sizeof(T) == 8 ? 1 : 4);
+    const size_t bytes = train_lds(sizeof(T), hid, a.stride, JAC ? 0 : np);
+    if (bytes > lds_limit() && a.n_net > 1) {
+        TrainArgs one = a;
+        one.n_net = 1;
+        for (int g = 0; g < a.n_net; ++g) {
+            one.net[0] = a.net[g];
+            if (int rc = launch_train<MODE, JAC>(one, st)) return rc;
+        }
+        return PT_OK;
+    }
+    if (bytes > lds_limit()) {
+        set_error("mlp training: %zu bytes of LDS per workgroup exceed the device limit", bytes);
         return PT_ERR_UNSUPPORTED;
     }
-    const int wpb = (int)std::min<size_t>(4, budget / per_wave);
-    const int ntiles = (a.n_atoms + 15) / 16;
-    const int blocks = std::max(1, std::min((ntiles + wpb - 1) / wpb, 1024));
-    hipLaunchKernelGGL(k_mlp_train<MODE>, dim3(blocks), dim3(64 * wpb), wpb * per_wave, st, a);
-    return launch_check("k_mlp_train");
-}
-
-// ---- per-row Jacobian of the input-gradient projection (FP64) -----------------
-//
-// Row (atom r, direction d) of J is  sign * d(ydot_d)/dtheta,  with
-// ydot_d = grad_x' MLP . (T_d * mul) the MLP output's derivative along the
-// scaled tangent of direction d.  The forward-over-reverse sweep is the one of
-// k_mlp_train (primal rows 0..15 once per tile, tangent rows 16..31 once per
-// direction), but nothing is summed over atoms: a dense layer's block of a
-// row is the outer product  a[r] (x) zbar[r] + adot[r] (x) zdotbar[r]  and a
-// bias block is zbar[r], written straight to HBM with consecutive lanes on
-// consecutive parameters of one row.
-struct JacArgs {
-    MlpShape s;
-    int n_atoms;
-    const double* G;
-    const double* T;      // T[d * t_dir + atom * ldg + k]
-    long long t_dir;
-    int n_dir;
-    int ldg;
-    const double* scale;
-    double scale_add;
-    const char* packed;
-    double sign;
-    double* J;            // row (atom * n_dir + d), unpacked parameter layout
-    long long ldj;
-    int stride;
-};
-
-__global__ __launch_bounds__(256) void k_mlp_jacobian(JacArgs a) {
-    typedef double T;
-    constexpr int MODE = PT_MLP_F64;
-    extern __shared__ __align__(16) char smem[];
-    const MlpShape& s = a.s;
-    const int H = s.n_hidden;
-    const int l = wave_lane();
-    const int wv = threadIdx.x >> 6;
-    const int wpb = blockDim.x >> 6;
-    const int stride = a.stride;
-    const size_t tile = (size_t)32 * stride;
-    const size_t per_wave = (size_t)(2 * H + 3) * tile + 64;
-    T* base = reinterpret_cast<T*>(smem) + (size_t)wv * per_wave;
-    T* Abuf[kMaxHidden + 1];
-    T* Zbuf[kMaxHidden];
-    for (int h = 0; h <= H; ++h) Abuf[h] = base + h * tile;
-    for (int h = 0; h < H; ++h) Zbuf[h] = base + (H + 1 + h) * tile;
-    T* P[2] = {base + (2 * H + 1) * tile, base + (2 * H + 2) * tile};
-    T* outv = base + (2 * H + 3) * tile;  // [0,16): z_L, [32,48): zbar_L, [48,64): zdotbar_L
-    const int row = l & 15, grp = l >> 4;
-    const T* wout = (const T*)(a.packed + s.wout64);
-    const T bout = ((const double*)(a.packed + s.bout64))[0];
-    const int L = H;
-    const int fan_L = H > 0 ? s.w[H - 1] : s.in_dim;
-    const int ntiles = (a.n_atoms + 15) / 16;
-    // one work item = (16-atom tile, direction): the primal sweep is redone per direction
-    for (int it = blockIdx.x * wpb + wv; it < ntiles * a.n_dir; it += gridDim.x * wpb) {
-        const int a0 = (it / a.n_dir) * 16;
-        const int d = it % a.n_dir;
-        const int nrows = min(16, a.n_atoms - a0);
-        for (int e = l; e < 16 * s.in_p; e += kWave) {
-            const int r = e / s.in_p, k = e % s.in_p;
-            T v = T(0);
-            if (r < nrows && k < s.in_dim)
-                v = (a.G[(size_t)(a0 + r) * a.ldg + k] - a.scale[k]) * a.scale[s.in_dim + k] + a.scale_add;
-            Abuf[0][r * stride + k] = v;
-        }
-        wave_fence();
-        // primal forward, rows 0..15 (kept for every direction)
-        int kin = s.in_p;
-        for (int h = 0; h < H; ++h) {
-            const int wp = s.wp[h];
-            for (int n0 = 0; n0 < wp; n0 += 16) {
-                T az[4] = {T(0), T(0), T(0), T(0)};
-                gemm_tile<MODE>(Abuf[h], stride, kin, a.packed, s.W64[h], 0, wp, false, n0, az);
-                const int col = n0 + row;
-                const T bias = ((const double*)(a.packed + s.b64[h]))[col];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int r = crow<MODE>(grp, i);
-                    T y, dy;
-                    const T z = az[i] + bias;
-                    activate<T>(s.act[h], z, y, dy);
-                    const bool pad = col >= s.w[h];
-                    Zbuf[h][r * stride + col] = pad ? T(0) : z;
-                    Abuf[h + 1][r * stride + col] = pad ? T(0) : y;
-                }
-            }
-            wave_fence();
-            kin = wp;
-        }
-        {
-            const int r = l >> 2, part = l & 3;
-            T z = T(0);
-            for (int k = part; k < kin; k += 4) z += Abuf[H][r * stride + k] * wout[k];
-            z += __shfl_xor(z, 1, kWave);
-            z += __shfl_xor(z, 2, kWave);
-            if (part == 0) outv[r] = z + bout;
-        }
-        wave_fence();
-        {
-            // tangent input, rows 16..31
-            for (int e = l; e < 16 * s.in_p; e += kWave) {
-                const int r = e / s.in_p, k = e % s.in_p;
-                T t = T(0);
-                if (r < nrows && k < s.in_dim)
-                    t = a.T[(size_t)d * a.t_dir + (size_t)(a0 + r) * a.ldg + k] * a.scale[s.in_dim + k];
-                Abuf[0][(16 + r) * stride + k] = t;
-            }
-            wave_fence();
-            kin = s.in_p;
-            for (int h = 0; h < H; ++h) {
-                const int wp = s.wp[h];
-                for (int n0 = 0; n0 < wp; n0 += 16) {
-                    T at[4] = {T(0), T(0), T(0), T(0)};
-                    gemm_tile<MODE>(Abuf[h] + 16 * stride, stride, kin, a.packed, s.W64[h], 0, wp, false, n0, at);
-                    const int col = n0 + row;
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const int r = crow<MODE>(grp, i);
-                        T y, dy;
-                        activate<T>(s.act[h], Zbuf[h][r * stride + col], y, dy);
-                        const bool pad = col >= s.w[h];
-                        Zbuf[h][(16 + r) * stride + col] = pad ? T(0) : at[i];
-                        Abuf[h + 1][(16 + r) * stride + col] = pad ? T(0) : dy * at[i];
-                    }
-                }
-                wave_fence();
-                kin = wp;
-            }
-            // output layer: seeds of the projection's reverse sweep
-            {
-                const int r = l >> 2, part = l & 3;
-                T zd = T(0);
-                for (int k = part; k < kin; k += 4) zd += Abuf[H][(16 + r) * stride + k] * wout[k];
-                zd += __shfl_xor(zd, 1, kWave);
-                zd += __shfl_xor(zd, 2, kWave);
-                T y, dy, ddy;
-                activate2<T>(s.act_out, outv[r], y, dy, ddy);
-                const T gt = r < nrows ? (T)a.sign : T(0);
-                if (part == 0) {
-                    outv[32 + r] = gt * ddy * zd;  // zbar_L
-                    outv[48 + r] = gt * dy;        // zdotbar_L
-                }
-            }
-            wave_fence();
-            // rows of J: output layer
-            for (int e = l; e < 16 * fan_L; e += kWave) {
-                const int r = e / fan_L, k = e % fan_L;
-                if (r < nrows)
-                    a.J[(size_t)((a0 + r) * a.n_dir + d) * a.ldj + s.pW[L] + k] =
-                        Abuf[H][r * stride + k] * outv[32 + r] + Abuf[H][(16 + r) * stride + k] * outv[48 + r];
-            }
-            if (l < nrows) a.J[(size_t)((a0 + l) * a.n_dir + d) * a.ldj + s.pb[L]] = outv[32 + l];
-            for (int e = l; e < 16 * kin; e += kWave) {
-                const int r = e / kin, k = e % kin;
-                P[0][r * stride + k] = outv[32 + r] * wout[k];
-                P[0][(16 + r) * stride + k] = outv[48 + r] * wout[k];
-            }
-            wave_fence();
-            int cur = 0;
-            for (int h = H - 1; h >= 0; --h) {
-                const int wp = s.wp[h];
-                const int kin_h = h > 0 ? s.wp[h - 1] : s.in_p;
-                for (int e = l; e < 16 * wp; e += kWave) {
-                    const int r = e / wp, k = e % wp;
-                    const T z = Zbuf[h][r * stride + k], zd = Zbuf[h][(16 + r) * stride + k];
-                    T y, dy, ddy;
-                    activate2<T>(s.act[h], z, y, dy, ddy);
-                    const T ab = P[cur][r * stride + k], adb = P[cur][(16 + r) * stride + k];
-                    const bool pad = k >= s.w[h];
-                    P[cur][r * stride + k] = pad ? T(0) : ab * dy + adb * ddy * zd;
-                    P[cur][(16 + r) * stride + k] = pad ? T(0) : adb * dy;
-                }
-                wave_fence();
-                // rows of J: W_h[in][out] and b_h[out]
-                const int fan_in = h > 0 ? s.w[h - 1] : s.in_dim;
-                const int wo = s.w[h];
-                const int nW = fan_in * wo;
-                for (int e = l; e < 16 * nW; e += kWave) {
-                    const int r = e / nW, q = e % nW;
-                    const int in = q / wo, out = q % wo;
-                    if (r < nrows)
-                        a.J[(size_t)((a0 + r) * a.n_dir + d) * a.ldj + s.pW[h] + q] =
-                            Abuf[h][r * stride + in] * P[cur][r * stride + out] +
-                            Abuf[h][(16 + r) * stride + in] * P[cur][(16 + r) * stride + out];
-                }
-                for (int e = l; e < 16 * wo; e += kWave) {
-                    const int r = e / wo, out = e % wo;
-                    if (r < nrows) a.J[(size_t)((a0 + r) * a.n_dir + d) * a.ldj + s.pb[h] + out] = P[cur][r * stride + out];
-                }
-                if (h > 0) {
-                    for (int n0 = 0; n0 < kin_h; n0 += 16) {
-                        T c0[4] = {T(0), T(0), T(0), T(0)}, c1[4] = {T(0), T(0), T(0), T(0)};
-                        gemm_tile<MODE>(P[cur], stride, wp, a.packed, s.W64[h], 0, wp, true, n0, c0);
-                        gemm_tile<MODE>(P[cur] + 16 * stride, stride, wp, a.packed, s.W64[h], 0, wp, true, n0, c1);
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const int r = crow<MODE>(grp, i);
-                            P[cur ^ 1][r * stride + n0 + row] = c0[i];
-                            P[cur ^ 1][(16 + r) * stride + n0 + row] = c1[i];
-                        }
-                    }
-                    cur ^= 1;
-                }
-                wave_fence();
-            }
-        }
+    const long long most = JAC ? 1 << 20 : kTrainBlocks;
+    int blocks = 0;
+    for (int g = 0; g < a.n_net; ++g) {
+        const long long items = (long long)((a.net[g].n_atoms + 15) / 16) * (JAC ? a.n_dir : 1);
+        a.net[g].block0 = blocks;
+        a.net[g].nblocks = (int)std::max<long long>(1, std::min(items, items * most / std::max(total, 1LL) + 1));
+        blocks += a.net[g].nblocks;
     }
+    hipLaunchKernelGGL((k_mlp_train<MODE, JAC>), dim3(blocks), dim3(256), bytes, st, a);
+    return launch_check("k_mlp_train");
 }
 
 // ---- loss seeds and Adam --------------------------------------------------------
@@ -1337,37 +1200,88 @@ extern "C" size_t pt_mlp_param_count(const pt_mlp_desc* desc) {
     return s.pb[s.n_hidden] + 1;
 }
 
+// a job of pt_mlp_train_grad_multi / pt_mlp_jacobian_multi as a network of the launch
+static int train_net(const pt_mlp_train_job& q, int ldg, const char* what, pt::TrainNet& t) {
+    PT_REQUIRE(q.n_atoms >= 0, "%s: n_atoms < 0", what);
+    if (q.n_atoms == 0) return PT_OK;
+    PT_REQUIRE(q.G && q.T && q.scale && q.desc && q.packed && q.out, "%s: null argument", what);
+    if (int rc = make_shape(q.desc, t.s)) return rc;
+    PT_REQUIRE(ldg >= q.desc->in_dim, "%s: ldg < in_dim", what);
+    t.n_atoms = q.n_atoms;
+    t.G = q.G;
+    t.T = q.T;
+    t.scale = q.scale;
+    t.scale_add = q.desc->scale_add;
+    t.packed = (const char*)q.packed;
+    t.gy = q.gy;
+    t.out = q.out;
+    t.nparam = (int)(t.s.pb[t.s.n_hidden] + 1);
+    return PT_OK;
+}
+
+extern "C" int pt_mlp_train_grad_multi(int mode, int n_jobs, const pt_mlp_train_job* jobs, int ldg, int g_precision,
+                                       double tseed, pt_stream_t stream) {
+    PT_REQUIRE(n_jobs >= 0 && (jobs || n_jobs == 0), "pt_mlp_train_grad: bad job list");
+    PT_REQUIRE(g_precision == PT_F64 || g_precision == PT_F32, "pt_mlp_train_grad: bad precision");
+    PT_REQUIRE(mode == PT_MLP_F64 || mode == PT_MLP_BF16 || mode == PT_MLP_BF16X3, "pt_mlp_train_grad: unknown mode %d",
+               mode);
+    hipStream_t st = (hipStream_t)stream;
+    TrainArgs a{};
+    a.ldg = ldg;
+    a.g_f64 = g_precision == PT_F64;
+    a.tseed = tseed;
+    for (int j = 0; j < n_jobs; ++j) {
+        PT_REQUIRE(jobs[j].gy || jobs[j].n_atoms == 0, "pt_mlp_train_grad: null argument");
+        if (int rc = train_net(jobs[j], ldg, "pt_mlp_train_grad", a.net[a.n_net])) return rc;
+        if (jobs[j].n_atoms > 0) ++a.n_net;
+        if (a.n_net == kMlpNets || (j == n_jobs - 1 && a.n_net > 0)) {
+            const int rc = mode == PT_MLP_F64    ? launch_train<PT_MLP_F64, false>(a, st)
+                           : mode == PT_MLP_BF16 ? launch_train<PT_MLP_BF16, false>(a, st)
+                                                 : launch_train<PT_MLP_BF16X3, false>(a, st);
+            if (rc) return rc;
+            a.n_net = 0;
+        }
+    }
+    return PT_OK;
+}
+
 extern "C" int pt_mlp_train_grad(int mode, int n_atoms, const void* G, const void* T, int ldg,
                                  int g_precision, const double* scale, const pt_mlp_desc* desc,
                                  const void* packed, const double* gy, double tseed, double* grad,
                                  pt_stream_t stream) {
     PT_REQUIRE(n_atoms >= 0, "pt_mlp_train_grad: n_atoms < 0");
     if (n_atoms == 0) return PT_OK;
-    PT_REQUIRE(G && T && scale && desc && packed && gy && grad, "pt_mlp_train_grad: null argument");
-    PT_REQUIRE(g_precision == PT_F64 || g_precision == PT_F32, "pt_mlp_train_grad: bad precision");
+    const pt_mlp_train_job job{n_atoms, G, T, scale, desc, packed, gy, grad};
+    return pt_mlp_train_grad_multi(mode, 1, &job, ldg, g_precision, tseed, stream);
+}
+
+extern "C" int pt_mlp_jacobian_multi(int n_dir, int n_jobs, const pt_mlp_train_job* jobs, long long t_dir, int ldg,
+                                     double sign, long long ldj, pt_stream_t stream) {
+    PT_REQUIRE(n_dir >= 1, "pt_mlp_jacobian: n_atoms < 0 or n_dir < 1");
+    PT_REQUIRE(n_jobs >= 0 && (jobs || n_jobs == 0), "pt_mlp_jacobian: bad job list");
     TrainArgs a{};
-    if (int rc = make_shape(desc, a.s)) return rc;
-    PT_REQUIRE(ldg >= desc->in_dim, "pt_mlp_train_grad: ldg < in_dim");
-    a.n_atoms = n_atoms;
-    a.G = G;
-    a.T = T;
     a.ldg = ldg;
-    a.g_f64 = g_precision == PT_F64;
-    a.scale = scale;
-    a.scale_add = desc->scale_add;
-    a.packed = (const char*)packed;
-    a.gy = gy;
-    a.tseed = tseed;
-    a.grad = grad;
-    a.nparam = (int)(a.s.pb[a.s.n_hidden] + 1);
-    hipStream_t st = (hipStream_t)stream;
-    switch (mode) {
-    case PT_MLP_F64: return launch_train<PT_MLP_F64>(a, st);
-    case PT_MLP_BF16: return launch_train<PT_MLP_BF16>(a, st);
-    case PT_MLP_BF16X3: return launch_train<PT_MLP_BF16X3>(a, st);
+    a.g_f64 = 1;
+    a.tseed = sign;
+    a.n_dir = n_dir;
+    a.t_dir = t_dir;
+    a.ldj = ldj;
+    for (int j = 0; j < n_jobs; ++j) {
+        TrainNet& t = a.net[a.n_net];
+        if (int rc = train_net(jobs[j], ldg, "pt_mlp_jacobian", t)) return rc;
+        if (jobs[j].n_atoms > 0) {
+            PT_REQUIRE(t_dir >= (long long)(t.n_atoms - 1) * ldg + jobs[j].desc->in_dim || n_dir == 1,
+                       "pt_mlp_jacobian: tangent directions overlap");
+            PT_REQUIRE(ldj >= t.nparam, "pt_mlp_jacobian: ldj below the parameter count");
+            PT_REQUIRE((long long)t.n_atoms * n_dir < (1LL << 31), "pt_mlp_jacobian: too many rows");
+            ++a.n_net;
+        }
+        if (a.n_net == kMlpNets || (j == n_jobs - 1 && a.n_net > 0)) {
+            if (int rc = launch_train<PT_MLP_F64, true>(a, (hipStream_t)stream)) return rc;
+            a.n_net = 0;
+        }
     }
-    set_error("pt_mlp_train_grad: unknown mode %d", mode);
-    return PT_ERR_ARG;
+    return PT_OK;
 }
 
 extern "C" int pt_mlp_jacobian(int n_atoms, int n_dir, const double* G, const double* T, long long t_dir, int ldg,
@@ -1375,39 +1289,8 @@ extern "C" int pt_mlp_jacobian(int n_atoms, int n_dir, const double* G, const do
                                double* J, long long ldj, pt_stream_t stream) {
     PT_REQUIRE(n_atoms >= 0 && n_dir >= 1, "pt_mlp_jacobian: n_atoms < 0 or n_dir < 1");
     if (n_atoms == 0) return PT_OK;
-    PT_REQUIRE(G && T && scale && desc && packed && J, "pt_mlp_jacobian: null argument");
-    JacArgs a{};
-    if (int rc = make_shape(desc, a.s)) return rc;
-    PT_REQUIRE(ldg >= desc->in_dim, "pt_mlp_jacobian: ldg < in_dim");
-    PT_REQUIRE(t_dir >= (long long)(n_atoms - 1) * ldg + desc->in_dim || n_dir == 1,
-               "pt_mlp_jacobian: tangent directions overlap");
-    const long long np = (long long)(a.s.pb[a.s.n_hidden] + 1);
-    PT_REQUIRE(ldj >= np, "pt_mlp_jacobian: ldj below the parameter count");
-    PT_REQUIRE((long long)n_atoms * n_dir < (1LL << 31), "pt_mlp_jacobian: too many rows");
-    a.n_atoms = n_atoms;
-    a.n_dir = n_dir;
-    a.G = G;
-    a.T = T;
-    a.t_dir = t_dir;
-    a.ldg = ldg;
-    a.scale = scale;
-    a.scale_add = desc->scale_add;
-    a.packed = (const char*)packed;
-    a.sign = sign;
-    a.J = J;
-    a.ldj = ldj;
-    a.stride = a.s.wmax + 1;
-    const size_t per_wave = sizeof(double) * ((size_t)(2 * a.s.n_hidden + 3) * 32 * a.stride + 64);
-    const size_t budget = lds_limit();
-    if (per_wave > budget) {
-        set_error("pt_mlp_jacobian: %zu bytes of LDS per wavefront exceed the device limit", per_wave);
-        return PT_ERR_UNSUPPORTED;
-    }
-    const int wpb = (int)std::min<size_t>(4, budget / per_wave);
-    const long long items = (long long)((n_atoms + 15) / 16) * n_dir;
-    const int blocks = (int)std::max<long long>(1, std::min<long long>((items + wpb - 1) / wpb, 8192));
-    hipLaunchKernelGGL(k_mlp_jacobian, dim3(blocks), dim3(64 * wpb), wpb * per_wave, (hipStream_t)stream, a);
-    return launch_check("k_mlp_jacobian");
+    const pt_mlp_train_job job{n_atoms, G, T, scale, desc, packed, nullptr, J};
+    return pt_mlp_jacobian_multi(n_dir, 1, &job, t_dir, ldg, sign, ldj, stream);
 }
 
 extern "C" int pt_train_seeds(int n, const double* force, const double* force_ref, const double* energy,

@@ -15,9 +15,9 @@ Per structure the descriptors G and the centre-only tangents T_a = dG_i/dr_ia
 then runs
 
     energy:  pt_mlp_energy_grad_multi, pt_reduce_sum_f64, pt_kalman_residual,
-             H = (1/N) sum_i dE_i/dW           pt_mlp_train_grad
+             H = (1/N) sum_i dE_i/dW           pt_mlp_train_grad_multi
     force:   pt_mlp_energy_grad_multi, pt_acsf_adjoint (self term),
-             pt_kalman_residual, H = dF/dW      pt_mlp_jacobian
+             pt_kalman_residual, H = dF/dW      pt_mlp_jacobian_multi
     both:    pt_kalman_update (products and Cholesky on the matrix cores), pt_mlp_pack
 
 with nothing read back to the host inside an epoch.
@@ -25,7 +25,6 @@ with nothing read back to the host inside an epoch.
 
 from __future__ import annotations
 
-import ctypes
 import math
 import random
 from collections import defaultdict
@@ -37,7 +36,7 @@ import numpy as np
 from . import _lib
 from .engine import (NeighborList, Reducer, acsf_adjoint_multi, acsf_forward_multi, acsf_run, acsf_tangent_multi,
                      gather_rows)
-from .models import energy_grad_multi
+from .models import energy_grad_multi, jacobian_multi, train_grad_multi
 from .potential import NNPSettings, NeuralNetworkPotential
 
 
@@ -208,10 +207,9 @@ class KalmanFilter:
         H = self.H[:1]
         H.zero_()
         self.gy[:it.n].fill_(1.0 / it.n)
-        for e, b, cnt, _ in it.blocks:
-            m = self.mlps[e]
-            m.train_grad(_lib.PT_MLP_F64, cnt, it.G[b:], it.G[b:], self.ld, _lib.PT_F64, self.gy[b:], 0.0,
-                         H[0, self.offsets[e]:])
+        train_grad_multi(_lib.PT_MLP_F64, [(self.mlps[e], cnt, it.G[b:], it.G[b:], self.gy[b:],
+                                            H[0, self.offsets[e]:]) for e, b, cnt, _ in it.blocks],
+                         self.ld, _lib.PT_F64, 0.0)
         return self.xi[:1], H
 
     def calculate_loss_force(self, it: _Item):
@@ -228,13 +226,9 @@ class KalmanFilter:
         H = self.H[:m3]
         H.zero_()
         n_w = self.num_states
-        for e, b, cnt, _ in it.blocks:
-            m = self.mlps[e]
-            J = H[3 * b:]
-            _lib.check(lib.pt_mlp_jacobian(cnt, 3, it.G[b:].data_ptr(), it.T[:, b:].data_ptr(), it.n * self.ld,
-                                           self.ld, m.scale.data_ptr(), ctypes.byref(m.desc), m.packed.data_ptr(),
-                                           -1.0, J.data_ptr() + 8 * self.offsets[e], n_w, _lib.stream_ptr()),
-                       "pt_mlp_jacobian")
+        jacobian_multi(3, [(self.mlps[e], cnt, it.G[b:], it.T[:, b:],
+                            H[3 * b:].data_ptr() + 8 * self.offsets[e]) for e, b, cnt, _ in it.blocks],
+                       it.n * self.ld, self.ld, -1.0, n_w)
         return self.xi[:m3], H
 
     # ---- the filter ----------------------------------------------------------------------------

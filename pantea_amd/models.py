@@ -188,3 +188,23 @@ def energy_grad_multi(mode: int, jobs, ldg: int, g_precision: int) -> None:
                     None if d is None else d.data_ptr()) for m, n, G, e, d in jobs])
     _lib.check(_lib.load().pt_mlp_energy_grad_multi(mode, len(jobs), arr, ldg, g_precision, _lib.stream_ptr()),
                "pt_mlp_energy_grad_multi")
+
+
+def _train_jobs(jobs):
+    return (_lib.MlpTrainJob * len(jobs))(*[
+        _lib.MlpTrainJob(n, G, T, m.scale.data_ptr(), ctypes.pointer(m.desc), m.packed.data_ptr(), gy, out)
+        for m, n, G, T, gy, out in jobs])
+
+
+def train_grad_multi(mode: int, jobs, ldg: int, g_precision: int, tseed: float) -> None:
+    """train_grad of several elements in one launch: ``jobs`` are (mlp, n_atoms, G, T, gy, grad)."""
+    arr = _train_jobs([(m, n, G.data_ptr(), T.data_ptr(), gy.data_ptr(), g.data_ptr()) for m, n, G, T, gy, g in jobs])
+    _lib.check(_lib.load().pt_mlp_train_grad_multi(mode, len(jobs), arr, ldg, g_precision, float(tseed),
+                                                   _lib.stream_ptr()), "pt_mlp_train_grad_multi")
+
+
+def jacobian_multi(n_dir: int, jobs, t_dir: int, ldg: int, sign: float, ldj: int) -> None:
+    """pt_mlp_jacobian of several elements in one launch: ``jobs`` are (mlp, n_atoms, G, T, address of J)."""
+    arr = _train_jobs([(m, n, G.data_ptr(), T.data_ptr(), None, J) for m, n, G, T, J in jobs])
+    _lib.check(_lib.load().pt_mlp_jacobian_multi(n_dir, len(jobs), arr, t_dir, ldg, float(sign), ldj,
+                                                 _lib.stream_ptr()), "pt_mlp_jacobian_multi")

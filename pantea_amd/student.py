@@ -12,7 +12,7 @@ Pipeline:
         F = -J^T dE/dG              pt_acsf_adjoint + pt_force_gather
         delta = dL/dF, dL/dE        pt_train_seeds
         T = J delta                 pt_acsf_tangent (forward mode)
-        dL/dtheta accumulation      pt_mlp_train_grad (forward-over-reverse)
+        dL/dtheta accumulation      pt_mlp_train_grad_multi (forward-over-reverse)
      and after each batch one Adam step (pt_adam_step) and a repack.  The
      structures of a batch are copied into one list (pt_train_batch_assemble),
      so each of these is one launch per batch (pt_train_batch_seeds).
@@ -37,7 +37,7 @@ from . import _lib
 from .atoms import Structure
 from .engine import (NeighborList, Reducer, acsf_adjoint_multi, acsf_forward_multi, acsf_run, acsf_tangent_multi,
                      force_gather, gather_rows, run_array)
-from .models import energy_grad_multi
+from .models import energy_grad_multi, train_grad_multi
 from .potential import PRECISION_MODES, NeuralNetworkPotential
 from .units import units
 
@@ -263,9 +263,8 @@ class StudentTrainer:
         acsf_tangent_multi(sn.nl, self.g_prec, [acsf_run(self._table(sn, el), cnt, b, out=self.T[b:],
                                                          delta=self.delta) for el, b, cnt in sn.blocks],
                            center_only=False, ld=self.ld)
-        for el, b, cnt in sn.blocks:
-            self.mlps[el].train_grad(self.mlp_mode, cnt, sn.G[b:], self.T[b:], self.ld, self.g_prec, self.gy[b:],
-                                     -1.0, self.grad[el])
+        train_grad_multi(self.mlp_mode, [(self.mlps[el], cnt, sn.G[b:], self.T[b:], self.gy[b:], self.grad[el])
+                                         for el, b, cnt in sn.blocks], self.ld, self.g_prec, -1.0)
 
     # ---- a batch of structures as one list -------------------------------------------
     def _passes(self, snaps: Sequence[Snapshot]):
@@ -342,9 +341,8 @@ class StudentTrainer:
             self._clear_absent(tab[el], B.T[b:b + cnt])
         runs = run_array([acsf_run(tab[el], cnt, b, out=B.T[b:], delta=B.delta) for el, b, cnt in blocks])
         _lib.check(lib.pt_acsf_tangent_multi(self.g_prec, *lists, row, *runs, 0, self.ld, st), "pt_acsf_tangent_multi")
-        for el, b, cnt in blocks:
-            self.mlps[el].train_grad(self.mlp_mode, cnt, B.G[b:], B.T[b:], self.ld, self.g_prec, B.gy[b:], -1.0,
-                                     self.grad[el])
+        train_grad_multi(self.mlp_mode, [(self.mlps[el], cnt, B.G[b:], B.T[b:], B.gy[b:], self.grad[el])
+                                         for el, b, cnt in blocks], self.ld, self.g_prec, -1.0)
 
     def gradient(self, indices: Sequence[int]):
         """Loss (energy term, force term) and its gradient over ``indices`` (batch mean)."""
