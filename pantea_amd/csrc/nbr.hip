@@ -23,6 +23,7 @@
 // row exceeds kStageW takes a second candidate pass instead.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 #include <cstdio>
 #include <cstring>
 
@@ -99,17 +100,20 @@ __global__ void k_bbox(int n, const double* pos, int ps, double* out) {
 // the order and the positions stay those of the last build.
 __device__ __forceinline__ bool gated_off(const int* gate) { return gate != nullptr && *gate == 0; }
 
+__device__ __forceinline__ int bin_key(const double* pos, int ps, const int* types, const Grid& g, int i) {
+    const int c0 = cell_coord(pos[(size_t)ps * i + 0], g.lo[0], g.inv_w[0], g.nc[0], g.periodic);
+    const int c1 = cell_coord(pos[(size_t)ps * i + 1], g.lo[1], g.inv_w[1], g.nc[1], g.periodic);
+    const int c2 = cell_coord(pos[(size_t)ps * i + 2], g.lo[2], g.inv_w[2], g.nc[2], g.periodic);
+    return (types[i] - 1) * g.ncell + (c2 * g.nc[1] + c1) * g.nc[0] + c0;
+}
+
 __global__ void k_bin(const int* __restrict__ gate, int n, const double* pos, int ps, const int* types, Grid g,
                       int* keys, int* vals, unsigned long long* bmax) {
     if (gated_off(gate)) return;
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     if (i == 0) *bmax = 0ull;   // max |coordinate|, raised by k_gather_pos4
-    int c0 = cell_coord(pos[(size_t)ps * i + 0], g.lo[0], g.inv_w[0], g.nc[0], g.periodic);
-    int c1 = cell_coord(pos[(size_t)ps * i + 1], g.lo[1], g.inv_w[1], g.nc[1], g.periodic);
-    int c2 = cell_coord(pos[(size_t)ps * i + 2], g.lo[2], g.inv_w[2], g.nc[2], g.periodic);
-    int cell = (c2 * g.nc[1] + c1) * g.nc[0] + c0;
-    keys[i] = (types[i] - 1) * g.ncell + cell;
+    keys[i] = bin_key(pos, ps, types, g, i);
     vals[i] = i;
 }
 
@@ -245,6 +249,28 @@ __global__ void k_cell_start(const int* __restrict__ gate, int nkeys, int n, con
     cell_start[k] = lo;
 }
 
+// atom v -> internal position i; returns its max |coordinate| as ordered bits
+__device__ __forceinline__ unsigned long long gather_one(int i, int v, const double* pos, int ps, const int* types,
+                                                         double* pos4, float4* pos4f) {
+    double4 p;
+    p.x = pos[(size_t)ps * v]; p.y = pos[(size_t)ps * v + 1]; p.z = pos[(size_t)ps * v + 2];
+    p.w = (double)types[v];
+    reinterpret_cast<double4*>(pos4)[i] = p;
+    pos4f[i] = make_float4((float)p.x, (float)p.y, (float)p.z, 0.0f);
+    // a NaN coordinate makes the bound NaN: every candidate then takes the exact test
+    double m = fmax(fmax(fabs(p.x), fabs(p.y)), fabs(p.z));
+    if (p.x != p.x || p.y != p.y || p.z != p.z) m = __builtin_nan("");
+    return __builtin_bit_cast(unsigned long long, m) & ~(1ull << 63);
+}
+
+__device__ __forceinline__ unsigned long long wave_max(unsigned long long b) {
+    for (int off = 1; off < kWave; off <<= 1) {
+        const unsigned long long o = __shfl_xor(b, off, kWave);
+        b = o > b ? o : b;
+    }
+    return b;
+}
+
 // Internal-order positions: FP64 (x, y, z, type) and an FP32 copy for the
 // candidate screen; bmax gets the bit pattern of max |coordinate| (the bit
 // patterns of non-negative doubles order like the values).
@@ -254,23 +280,9 @@ __global__ __launch_bounds__(256) void k_gather_pos4(const int* __restrict__ gat
     if (gated_off(gate)) return;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) perm_out[i] = perm[i];
-    double m = 0.0;
-    if (i < n) {
-        const int v = perm[i];
-        double4 p;
-        p.x = pos[(size_t)ps * v]; p.y = pos[(size_t)ps * v + 1]; p.z = pos[(size_t)ps * v + 2];
-        p.w = (double)types[v];
-        reinterpret_cast<double4*>(pos4)[i] = p;
-        pos4f[i] = make_float4((float)p.x, (float)p.y, (float)p.z, 0.0f);
-        // a NaN coordinate makes the bound NaN: every candidate then takes the exact test
-        m = fmax(fmax(fabs(p.x), fabs(p.y)), fabs(p.z));
-        if (p.x != p.x || p.y != p.y || p.z != p.z) m = __builtin_nan("");
-    }
-    unsigned long long b = __builtin_bit_cast(unsigned long long, m) & ~(1ull << 63);
-    for (int off = 1; off < kWave; off <<= 1) {
-        const unsigned long long o = __shfl_xor(b, off, kWave);
-        b = o > b ? o : b;
-    }
+    unsigned long long b = 0ull;
+    if (i < n) b = gather_one(i, perm[i], pos, ps, types, pos4, pos4f);
+    b = wave_max(b);
     // one atomic per block, and only when it raises the bound
     __shared__ unsigned long long wmax[256 / kWave];
     if ((threadIdx.x & (kWave - 1)) == 0) wmax[threadIdx.x >> 6] = b;
@@ -278,6 +290,133 @@ __global__ __launch_bounds__(256) void k_gather_pos4(const int* __restrict__ gat
     if (threadIdx.x == 0) {
         for (int q = 1; q < (int)(blockDim.x >> 6); ++q) b = wmax[q] > b ? wmax[q] : b;
         if (b > __hip_atomic_load(bmax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(bmax, b);
+    }
+}
+
+// ---- up to kSortSmall atoms: all of the above in one workgroup --------------
+//
+// Keys, stable radix sort, cell starts and the gather, with keys and order in
+// LDS: what bounds a small build is its launches (6 to 9 of them, each a few us
+// of start and end for work of less).  Wavefront w owns the items
+// [64 w rounds, 64 (w + 1) rounds) in order, so a pass counts digits per wavefront
+// without workgroup barriers and is stable.
+// Measured, a whole build at a cutoff of 12: 96 atoms 33 -> 25 us, 4,096 atoms 57 -> 50,
+// 6,000 atoms 81 -> 72, 8,192 (not taken) the same either way.
+// R: rounds of 1,024 items, as few as hold n (unused ones of 8 cost 3 us at 1,200 atoms).
+constexpr int kSortSmall = 6144;
+
+// exclusive sum over the 1024 threads of v; total: the sum of all
+template <typename T>
+__device__ __forceinline__ T block_exclusive(T v, T* wtot, T& total) {
+    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x >> 6;
+    T incl = v;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+        const T o = __shfl_up(incl, off, kWave);
+        if (lane >= off) incl += o;
+    }
+    if (lane == kWave - 1) wtot[w] = incl;
+    __syncthreads();
+    T before = 0, all = 0;
+    for (int q = 0; q < 1024 / kWave; ++q) {
+        const T o = wtot[q];
+        before += q < w ? o : 0;
+        all += o;
+    }
+    __syncthreads();   // wtot is free again
+    total = all;
+    return before + incl - v;
+}
+
+template <int R>
+__global__ __launch_bounds__(1024) void k_sort_small(const int* __restrict__ gate, int n, const double* pos, int ps,
+                                                     const int* types, Grid g, int nkeys, int bits,
+                                                     int* __restrict__ cell_start, int* __restrict__ perm,
+                                                     double* __restrict__ pos4, float4* __restrict__ pos4f,
+                                                     unsigned long long* __restrict__ bmax) {
+    if (gated_off(gate)) return;
+    __shared__ int skey[1024 * R], sval[1024 * R];
+    __shared__ int count[256 * 16];          // [digit][wavefront]
+    __shared__ int wtot[16];
+    __shared__ unsigned long long wmax[16];
+    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x >> 6;
+    const int rounds = (n + 1023) / 1024;
+    int key[R], val[R], rank[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int idx = (w * rounds + r) * kWave + lane;
+        const bool in = r < rounds && idx < n;
+        key[r] = in ? bin_key(pos, ps, types, g, idx) : 0;
+        val[r] = idx;
+    }
+    for (int shift = 0; shift < bits; shift += 8) {
+        if (shift) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int idx = (w * rounds + r) * kWave + lane;
+                if (r < rounds && idx < n) { key[r] = skey[idx]; val[r] = sval[idx]; }
+            }
+        }
+        for (int k = threadIdx.x; k < 256 * 16; k += 1024) count[k] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int idx = (w * rounds + r) * kWave + lane;
+            const bool in = r < rounds && idx < n;
+            const int d = (key[r] >> shift) & 255;
+            unsigned long long peers = __ballot(in);   // lanes with the same digit
+#pragma unroll
+            for (int b = 0; b < 8; ++b) {
+                const unsigned long long bal = __ballot((d >> b) & 1);
+                peers &= ((d >> b) & 1) ? bal : ~bal;
+            }
+            const int below = lanes_below(peers);
+            const int base = count[d * 16 + w];
+            rank[r] = base + below;
+            wave_sync();
+            if (in && below == 0) count[d * 16 + w] = base + __popcll(peers);
+            wave_sync();
+        }
+        __syncthreads();
+        int c[4], sum = 0, all;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) { c[q] = count[4 * threadIdx.x + q]; sum += c[q]; }
+        int run = block_exclusive(sum, wtot, all);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) { count[4 * threadIdx.x + q] = run; run += c[q]; }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int idx = (w * rounds + r) * kWave + lane;
+            if (r < rounds && idx < n) {
+                const int dst = count[((key[r] >> shift) & 255) * 16 + w] + rank[r];
+                skey[dst] = key[r];
+                sval[dst] = val[r];
+            }
+        }
+        __syncthreads();
+    }
+    for (int k = threadIdx.x; k <= nkeys; k += 1024) {
+        int lo = 0, hi = n;
+        while (lo < hi) {
+            const int mid = (lo + hi) >> 1;
+            if (skey[mid] < k) lo = mid + 1; else hi = mid;
+        }
+        cell_start[k] = lo;
+    }
+    unsigned long long b = 0ull;
+    for (int i = threadIdx.x; i < n; i += 1024) {
+        const int v = sval[i];
+        perm[i] = v;
+        const unsigned long long o = gather_one(i, v, pos, ps, types, pos4, pos4f);
+        b = o > b ? o : b;
+    }
+    b = wave_max(b);
+    if (lane == 0) wmax[w] = b;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int q = 1; q < 16; ++q) b = wmax[q] > b ? wmax[q] : b;
+        *bmax = b;
     }
 }
 
@@ -345,12 +484,19 @@ __device__ __forceinline__ Screen make_screen(double thr, double bmax, const Box
     return sc;
 }
 
+// Workgroups of the candidate pass up to which cells are split over several: a whole
+// build at a cutoff of 12 takes 68 -> 25 us for 96 atoms (1 cell), 65 -> 50 for 4,096,
+// 107 -> 102 for 12,288 (343 cells, 2 each); 16,384 (512 cells, 2 each) took 119 -> 123.
+constexpr int kCellGroups = 960;
 constexpr int kCand = 1536;   // candidates of one cell staged in LDS, large configuration (a multiple of 64)
 
 // One workgroup per cell: the candidate ranges of the cell's stencil (the
 // same for all its centres) are built once, the candidates (FP32 position and
 // index) staged in LDS when they fit, and the workgroup's wavefronts take
-// the cell's centres in turn, 64 candidates per step.  A cell with more than
+// the cell's centres in turn, 256 candidates per step (four tests side by side:
+// one wavefront's chain of LDS read, distance and ballot is what bounds a cell;
+// 46 -> 29 us at 12,288 atoms together with the split), the last ones 64 at a
+// time.  Few cells are split over workgroups (kCellGroups).  A cell with more than
 // kCand candidates reads them from global memory instead (index by binary
 // search over the ranges).  Rows come out in candidate order: type-major,
 // stencil cells ascending, i.e. ascending internal index.
@@ -364,7 +510,7 @@ __global__ __launch_bounds__(THREADS) void k_nbr_cell(const int* __restrict__ ga
                                                   const float4* __restrict__ pos4f,
                                                   const unsigned long long* __restrict__ bmax,
                                                   const int* __restrict__ cell_start, Grid g,
-                                                  BoxArg box, int n_types, double thr,
+                                                  BoxArg box, int n_types, double thr, int split,
                                                   int* __restrict__ counts,
                                                   const long long* __restrict__ row_off,
                                                   int* __restrict__ out_idx,
@@ -388,7 +534,8 @@ __global__ __launch_bounds__(THREADS) void k_nbr_cell(const int* __restrict__ ga
     __shared__ int s_nr;
     const int lane = threadIdx.x & (kWave - 1);
     const int w = threadIdx.x >> 6;
-    const int cell = xcd_block();
+    const int blk = xcd_block();
+    const int cell = blk / split, part = blk - cell * split;
 
     if (threadIdx.x == 0) {
         int acc = 0;
@@ -512,7 +659,7 @@ __global__ __launch_bounds__(THREADS) void k_nbr_cell(const int* __restrict__ ga
     // (a candidate with a larger component takes the FP64 test)
     const float3 ib = make_float3(1.0f / bf.x, 1.0f / bf.y, 1.0f / bf.z);
     const float3 lim = make_float3(1.45f * bf.x, 1.45f * bf.y, 1.45f * bf.z);
-    for (int k = w; k < ncent; k += THREADS / kWave) {
+    for (int k = part * (THREADS / kWave) + w; k < ncent; k += split * (THREADS / kWave)) {
         int t0 = 0;
         while (t0 + 1 < n_types && s_cpre[t0 + 1] <= k) ++t0;
         const int i = uniform(s_cbeg[t0] + (k - s_cpre[t0]));
@@ -520,52 +667,80 @@ __global__ __launch_bounds__(THREADS) void k_nbr_cell(const int* __restrict__ ga
         const float4 pif = pos4f[i];
         const long long out = FILL ? row_off[i] : 0;
         int count = 0;
-        for (int base = 0; base < total; base += kWave) {
-            const int t = base + lane;
-            int j = i;
-            float4 pj = pif;
-            if (staged) {
-                // t < CAND: total <= CAND and CAND is a multiple of the wave size
-                const int4 c = s_cand[t];
-                pj = make_float4(__builtin_bit_cast(float, c.x), __builtin_bit_cast(float, c.y),
-                                 __builtin_bit_cast(float, c.z), 0.0f);
-                j = c.w;
-            } else if (t < total) {
-                int lo = 0, hi = nr;
-                while (hi - lo > 1) {
-                    const int mid = (lo + hi) >> 1;
-                    if (s_rpre[mid] <= t) lo = mid; else hi = mid;
-                }
-                j = s_rstart[lo] + (t - s_rpre[lo]);
-                pj = pos4f[j];
-            }
-            const bool ok = (t < total) & (j != i);   // r_ii = 0 is never a neighbour
-            float dx = pif.x - pj.x, dy = pif.y - pj.y, dz = pif.z - pj.z;
-            bool img = true;
-            if (box.periodic && !direct) {
-                img = (fabsf(dx) < lim.x) & (fabsf(dy) < lim.y) & (fabsf(dz) < lim.z);
-                dx = fmaf(-bf.x, rintf(dx * ib.x), dx);
-                dy = fmaf(-bf.y, rintf(dy * ib.y), dy);
-                dz = fmaf(-bf.z, rintf(dz * ib.z), dz);
-            }
-            const float s32 = dx * dx + dy * dy + dz * dz;
-            bool hit = ok & img & (s32 > sc.hit_lo) & (s32 < sc.hit_hi);
-            if (ok & !hit & (!img | !(s32 >= sc.miss))) {
-                const double4 pd = reinterpret_cast<const double4*>(pos4)[j];
-                const double s = mic_dist2(pi.x - pd.x, pi.y - pd.y, pi.z - pd.z, box);
-                hit = (s <= thr) && (s > 0.0);   // r <= rc and r > 0
-            }
-            const unsigned long long bal = __ballot(hit);
-            if (hit) {
-                const int slot = count + lanes_below(bal);
-                if (FILL) out_idx[out + slot] = j;
-                if (PASS == PASS_STAGE && slot < kStageW) {
-                    out_idx[(size_t)i * kStageW + slot] = j;
-                    if (slot % kBucket == 0) heads[(size_t)i * kNBucket + slot / kBucket] = j;
+        // 64 U candidates: their tests side by side, the hits stored in candidate order
+        auto step = [&](auto U_, int base) {
+            constexpr int U = decltype(U_)::value;
+            int j[U];
+            float x[U], y[U], z[U];
+            bool hit[U], check[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int t = base + u * kWave + lane;
+                if (staged) {
+                    // t < CAND: base + 64 U <= total rounded up to 64 <= CAND
+                    const int4 c = s_cand[t];
+                    x[u] = __builtin_bit_cast(float, c.x);
+                    y[u] = __builtin_bit_cast(float, c.y);
+                    z[u] = __builtin_bit_cast(float, c.z);
+                    j[u] = c.w;
+                } else {
+                    j[u] = i;
+                    if (t < total) {
+                        int lo = 0, hi = nr;
+                        while (hi - lo > 1) {
+                            const int mid = (lo + hi) >> 1;
+                            if (s_rpre[mid] <= t) lo = mid; else hi = mid;
+                        }
+                        j[u] = s_rstart[lo] + (t - s_rpre[lo]);
+                    }
+                    const float4 p = pos4f[j[u]];
+                    x[u] = p.x; y[u] = p.y; z[u] = p.z;
                 }
             }
-            count += __popcll(bal);
-        }
+            bool any = false;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const bool ok = (base + u * kWave + lane < total) & (j[u] != i);   // r_ii = 0 is never a neighbour
+                float dx = pif.x - x[u], dy = pif.y - y[u], dz = pif.z - z[u];
+                bool img = true;
+                if (box.periodic && !direct) {
+                    img = (fabsf(dx) < lim.x) & (fabsf(dy) < lim.y) & (fabsf(dz) < lim.z);
+                    dx = fmaf(-bf.x, rintf(dx * ib.x), dx);
+                    dy = fmaf(-bf.y, rintf(dy * ib.y), dy);
+                    dz = fmaf(-bf.z, rintf(dz * ib.z), dz);
+                }
+                const float s32 = dx * dx + dy * dy + dz * dz;
+                hit[u] = ok & img & (s32 > sc.hit_lo) & (s32 < sc.hit_hi);
+                check[u] = ok & !hit[u] & (!img | !(s32 >= sc.miss));
+                any |= check[u];
+            }
+            if (__ballot(any) != 0ull) {
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (check[u]) {
+                        const double4 pd = reinterpret_cast<const double4*>(pos4)[j[u]];
+                        const double d2 = mic_dist2(pi.x - pd.x, pi.y - pd.y, pi.z - pd.z, box);
+                        hit[u] = (d2 <= thr) && (d2 > 0.0);   // r <= rc and r > 0
+                    }
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const unsigned long long bal = __ballot(hit[u]);
+                if (hit[u]) {
+                    const int slot = count + lanes_below(bal);
+                    if (FILL) out_idx[out + slot] = j[u];
+                    if (PASS == PASS_STAGE && slot < kStageW) {
+                        out_idx[(size_t)i * kStageW + slot] = j[u];
+                        if (slot % kBucket == 0) heads[(size_t)i * kNBucket + slot / kBucket] = j[u];
+                    }
+                }
+                count += __popcll(bal);
+            }
+        };
+        int base = 0;
+        if (staged)
+            for (; base + 3 * kWave < total; base += 4 * kWave) step(std::integral_constant<int, 4>{}, base);
+        for (; base < total; base += kWave) step(std::integral_constant<int, 1>{}, base);
         if (!FILL && lane == 0) counts[i] = count;
         if (PASS == PASS_STAGE && count <= kStageW) {
             // INT_MAX past the row end, to the end of its last bucket, and in
@@ -607,6 +782,18 @@ __global__ __launch_bounds__(256) void k_scan_reduce(const int* __restrict__ gat
 // totals (when set): the running totals of an asynchronous build: [0] pairs of the last
 // build, [1] largest row and [2] largest pair count since the caller cleared them,
 // [3] builds done
+__device__ __forceinline__ void store_totals(long long pairs, int max_row, long long* total_and_max,
+                                             long long* totals) {
+    total_and_max[0] = pairs;
+    total_and_max[1] = max_row;
+    if (totals) {
+        totals[0] = pairs;
+        totals[1] = max_row > totals[1] ? max_row : totals[1];
+        totals[2] = pairs > totals[2] ? pairs : totals[2];
+        totals[3] += 1;
+    }
+}
+
 __global__ __launch_bounds__(1024) void k_scan_top(const int* __restrict__ gate, int nb, long long* psum,
                                                    const int* pmax, long long* total_and_max,
                                                    long long* __restrict__ totals) {
@@ -640,16 +827,7 @@ __global__ __launch_bounds__(1024) void k_scan_top(const int* __restrict__ gate,
         if ((int)threadIdx.x < o) mx[threadIdx.x] = max(mx[threadIdx.x], mx[threadIdx.x + o]);
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        total_and_max[0] = carry;
-        total_and_max[1] = mx[0];
-        if (totals) {
-            totals[0] = carry;
-            totals[1] = mx[0] > totals[1] ? mx[0] : totals[1];
-            totals[2] = carry > totals[2] ? carry : totals[2];
-            totals[3] += 1;
-        }
-    }
+    if (threadIdx.x == 0) store_totals(carry, mx[0], total_and_max, totals);
 }
 
 __global__ __launch_bounds__(256) void k_scan_down(const int* __restrict__ gate, int n, const int* counts,
@@ -680,6 +858,45 @@ __global__ __launch_bounds__(256) void k_scan_down(const int* __restrict__ gate,
         if (idx < n) row_off[idx] = pre + loc[k];
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) row_off[n] = total_and_max[0];
+}
+
+// Up to kOffsetsSmall rows in one workgroup (a contiguous piece per thread): one launch
+// for three.  Measured, a whole build: 96 atoms 30 -> 25 us, 8,192 95 -> 94, 16,384 115 -> 122.
+constexpr int kOffsetsSmall = 8192;
+
+__global__ __launch_bounds__(1024) void k_offsets_small(const int* __restrict__ gate, int n,
+                                                        const int* __restrict__ counts,
+                                                        long long* __restrict__ row_off,
+                                                        long long* __restrict__ total_and_max,
+                                                        long long* __restrict__ totals) {
+    if (gated_off(gate)) return;
+    constexpr int PER = kOffsetsSmall / 1024;
+    __shared__ long long wtot[16];
+    __shared__ int wmax[16];
+    const int per = (n + 1023) / 1024, b = threadIdx.x * per;
+    int c[PER], m = 0;
+    long long sum = 0, all;
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        c[q] = q < per && b + q < n ? counts[b + q] : 0;
+        sum += c[q];
+        m = max(m, c[q]);
+    }
+    long long run = block_exclusive(sum, wtot, all);
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        if (q < per && b + q < n) row_off[b + q] = run;
+        run += c[q];
+    }
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) m = max(m, __shfl_xor(m, off, kWave));
+    if ((threadIdx.x & (kWave - 1)) == 0) wmax[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int q = 1; q < 16; ++q) m = max(m, wmax[q]);
+        row_off[n] = all;
+        store_totals(all, m, total_and_max, totals);
+    }
 }
 
 // ---- reverse edge index: rev[e(i->j)] = e(j->i) ------------------------------
@@ -978,31 +1195,38 @@ int build_impl(int n, const double* pos, int pos_stride, const int* types, int n
     }
     const int nkeys = n_types * g.ncell;
 
-    // bin + sort
+    // bin + sort, cell starts, positions in the sorted order
     const int tb = 256;
-    hipLaunchKernelGGL(k_bin, dim3((n + tb - 1) / tb), dim3(tb), 0, stream, gate, n, pos, pos_stride, types,
-                       g, keys_a, vals_a, bmax);
-    if (int rcode = launch_check("k_bin")) return rcode;
     int bits = 1;
     while ((1 << bits) < nkeys) ++bits;
-    const int nblocks = (n + kTile - 1) / kTile;
-    int* kin = keys_a; int* kout = keys_b; int* vin = vals_a; int* vout = vals_b;
-    for (int shift = 0; shift < bits; shift += 8) {
-        hipLaunchKernelGGL(k_radix_hist, dim3(nblocks), dim3(kSortThreads), 0, stream, gate, n, kin,
-                           shift, nblocks, ghist);
-        hipLaunchKernelGGL(k_scan_small, dim3(1), dim3(1024), 0, stream, gate, 256 * nblocks, ghist);
-        hipLaunchKernelGGL(k_radix_scatter, dim3(nblocks), dim3(kSortThreads), 0, stream, gate, n, kin,
-                           vin, shift, nblocks, ghist, kout, vout);
-        if (int rcode = launch_check("radix sort")) return rcode;
-        std::swap(kin, kout);
-        std::swap(vin, vout);
+    if (n <= kSortSmall && nkeys <= kSortSmall) {
+        auto kern = n <= 1024 ? k_sort_small<1> : n <= 2048 ? k_sort_small<2> : n <= 4096 ? k_sort_small<4> : k_sort_small<6>;
+        hipLaunchKernelGGL(kern, dim3(1), dim3(1024), 0, stream, gate, n, pos, pos_stride, types, g, nkeys, bits,
+                           cell_start, o.perm, o.pos4, pos4f, bmax);
+        if (int rcode = launch_check("k_sort_small")) return rcode;
+    } else {
+        hipLaunchKernelGGL(k_bin, dim3((n + tb - 1) / tb), dim3(tb), 0, stream, gate, n, pos, pos_stride, types,
+                           g, keys_a, vals_a, bmax);
+        if (int rcode = launch_check("k_bin")) return rcode;
+        const int nblocks = (n + kTile - 1) / kTile;
+        int* kin = keys_a; int* kout = keys_b; int* vin = vals_a; int* vout = vals_b;
+        for (int shift = 0; shift < bits; shift += 8) {
+            hipLaunchKernelGGL(k_radix_hist, dim3(nblocks), dim3(kSortThreads), 0, stream, gate, n, kin,
+                               shift, nblocks, ghist);
+            hipLaunchKernelGGL(k_scan_small, dim3(1), dim3(1024), 0, stream, gate, 256 * nblocks, ghist);
+            hipLaunchKernelGGL(k_radix_scatter, dim3(nblocks), dim3(kSortThreads), 0, stream, gate, n, kin,
+                               vin, shift, nblocks, ghist, kout, vout);
+            if (int rcode = launch_check("radix sort")) return rcode;
+            std::swap(kin, kout);
+            std::swap(vin, vout);
+        }
+        // kin/vin now hold the sorted keys / permutation (copied to perm by k_gather_pos4)
+        hipLaunchKernelGGL(k_cell_start, dim3((nkeys + 1 + tb - 1) / tb), dim3(tb), 0, stream, gate, nkeys, n,
+                           kin, cell_start);
+        hipLaunchKernelGGL(k_gather_pos4, dim3((n + tb - 1) / tb), dim3(tb), 0, stream, gate, n, vin, pos,
+                           pos_stride, types, o.pos4, pos4f, bmax, o.perm);
+        if (int rcode = launch_check("cell start / gather")) return rcode;
     }
-    // kin/vin now hold the sorted keys / permutation (copied to perm by k_gather_pos4)
-    hipLaunchKernelGGL(k_cell_start, dim3((nkeys + 1 + tb - 1) / tb), dim3(tb), 0, stream, gate, nkeys, n,
-                       kin, cell_start);
-    hipLaunchKernelGGL(k_gather_pos4, dim3((n + tb - 1) / tb), dim3(tb), 0, stream, gate, n, vin, pos,
-                       pos_stride, types, o.pos4, pos4f, bmax, o.perm);
-    if (int rcode = launch_check("cell start / gather")) return rcode;
 
     // count + stage, scan, then compact (or a second pass for rows > kStageW)
     const int nwb = (n + 3) / 4;
@@ -1012,9 +1236,13 @@ int build_impl(int n, const double* pos, int pos_stride, const int* types, int n
     const int ccfg = avg_cand * 1.6 <= 512 ? 0 : (avg_cand * 1.6 <= 1024 ? 1 : 2);
     auto launch_cell = [&](bool fill, const long long* tm, const long long* roff, int* out, int* hd) {
         auto go = [&](auto kern, int threads) {
-            hipLaunchKernelGGL(kern, dim3(g.ncell), dim3(threads), 0, stream, gate, tm, o.cap, o.pos4,
+            // few cells: a cell's centres go to several workgroups, down to a centre per wavefront
+            const int per_wg = threads / kWave;
+            const int most = std::max(1, (int)std::ceil((double)n / g.ncell / per_wg));
+            const int split = std::max(1, std::min(most, kCellGroups / g.ncell));
+            hipLaunchKernelGGL(kern, dim3(g.ncell * split), dim3(threads), 0, stream, gate, tm, o.cap, o.pos4,
                                (const float4*)pos4f, (const unsigned long long*)bmax, cell_start, g, ba, n_types,
-                               thr, counts, roff, out, hd);
+                               thr, split, counts, roff, out, hd);
         };
         if (ccfg == 0) {
             if (fill) go(k_nbr_cell<PASS_FILL, 512, 128>, 128); else go(k_nbr_cell<PASS_STAGE, 512, 128>, 128);
@@ -1029,9 +1257,14 @@ int build_impl(int n, const double* pos, int pos_stride, const int* types, int n
     if (int rcode = launch_check("k_nbr_cell<stage>")) return rcode;
     const int nsb = (n + kScanBlock - 1) / kScanBlock;
     long long* tot_max = (long long*)misc;
-    hipLaunchKernelGGL(k_scan_reduce, dim3(nsb), dim3(256), 0, stream, gate, n, counts, psum, pmax);
-    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, stream, gate, nsb, psum, pmax, tot_max, dev_totals);
-    hipLaunchKernelGGL(k_scan_down, dim3(nsb), dim3(256), 0, stream, gate, n, counts, psum, tot_max, o.row_off);
+    if (n <= kOffsetsSmall) {
+        hipLaunchKernelGGL(k_offsets_small, dim3(1), dim3(1024), 0, stream, gate, n, (const int*)counts, o.row_off,
+                           tot_max, dev_totals);
+    } else {
+        hipLaunchKernelGGL(k_scan_reduce, dim3(nsb), dim3(256), 0, stream, gate, n, counts, psum, pmax);
+        hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, stream, gate, nsb, psum, pmax, tot_max, dev_totals);
+        hipLaunchKernelGGL(k_scan_down, dim3(nsb), dim3(256), 0, stream, gate, n, counts, psum, tot_max, o.row_off);
+    }
     if (int rcode = launch_check("row offsets")) return rcode;
     // the compaction checks the totals itself, so it is queued before the host
     // reads them (the GPU does not idle through the round trip)
