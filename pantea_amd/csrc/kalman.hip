@@ -35,7 +35,7 @@
 //
 // Every product and factorisation is a kernel of this file: the library's
 // triangular kernels and its many small products per block took most of the
-// update (student network, n_w = 1,698, m = 4,608: 11.0 ms, now 2.8).
+// update (student network, n_w = 1,698, m = 4,608: 11.0 ms, now 2.6).
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
@@ -57,10 +57,6 @@ __global__ void k_lower_copy(int n, const double* __restrict__ A, long long lda,
 // the first of two factorisations' info codes that is not zero
 __global__ void k_merge_info(int* __restrict__ info, const int* __restrict__ info2) {
     if (threadIdx.x == 0 && *info == 0) *info = *info2;
-}
-
-__global__ void k_zero_int(int* __restrict__ p) {
-    if (threadIdx.x == 0) *p = 0;
 }
 
 // dst[i * ldd] = src[i]
@@ -254,19 +250,25 @@ int gemm_f64(const GemmArgs& g, hipStream_t st) {
 }
 
 // ---- Cholesky factorisation A = L L^T (lower, in place), right-looking in
-// blocks of 64 columns, two launches per block.  A may carry further rows below
-// its n x n part (rows n .. rows - 1): they come out as B L^-T, the triangular
-// solve with the factor, at the cost of more tiles in the same launches.
+// blocks of 64 columns, one launch per block (k_chol_step).  A may carry further
+// rows below its n x n part (rows n .. rows - 1): they come out as B L^-T, the
+// triangular solve with the factor, at the cost of more tiles in the same launches.
 //
-// k_chol_panel: every workgroup factorises the 64 x 64 diagonal block itself
-// (in LDS; a launch and a round trip through memory cost more than the repeated
-// work) and solves 64 rows of the panel below.  Both go in 16-column steps: two
-// wavefronts factorise the 16 x 16 diagonal block, each with the rows of its own
-// below it (the rest of the block, the panel rows) -- panel16 -- and all
-// subtract the step's products from the columns to the right by MFMA.  What
-// bounds it: the serial chain of the 64 pivots.  Measured at n = 1,698: 15.4 us
-// (27.8 with loads under a condition each, 256 threads and a division per pivot;
-// the single-wavefront block factorisation before it 61, its panel product apart).
+// The launch of block k holds two kinds of workgroups, both starting from the
+// finished columns of block k - 1:
+//  * a strip: 64 rows of block k's own columns.  It applies block k - 1 to them and
+//    to the 64 x 64 diagonal block (MFMA),
+//    factorises the diagonal block itself (in LDS; a launch and a round trip
+//    through memory cost more than the repeated work) and solves its rows.  The last
+//    two go in 16-column steps: two wavefronts factorise the 16 x 16 diagonal
+//    block, each with the rows of its own below it (the rest of the block, the
+//    strip's rows) -- panel16 -- and all subtract the step's products from the
+//    columns to the right by MFMA;
+//  * a tile: 64 x 64 entries further right, from which block k - 1 is subtracted.
+// Nothing that a workgroup writes is read by another of the same launch.  What
+// bounds it: the serial chain of the 64 pivots; the tiles run beside it.  Measured per
+// block at n = 1,698: 22.4 us, with 1,699 rows carried 25.6 (as two launches, panel
+// and trailing update, 15.4 + 8 to 20 and a launch more); 16.5 without a block before it.
 constexpr int kNb = 64, kSb = 16, kLd = kNb + 1;
 
 // lane C's value of each 16-lane row, in every lane of the row
@@ -355,37 +357,100 @@ __device__ __forceinline__ void tile_store(double* x, const mf_d4& v) {
     for (int q = 0; q < 4; ++q) x[(grp + 4 * q) * kLd + row] = v[q];
 }
 
-constexpr size_t kPanelLds = sizeof(double) * 2 * kNb * kLd;   // the diagonal block and the strip
+constexpr size_t kStepLds = sizeof(double) * 2 * kNb * kLd;   // a strip's diagonal block and rows; a tile's operands
 
-constexpr int kPanelThreads = 512;
+constexpr int kStepThreads = 512;
 
-__global__ __launch_bounds__(kPanelThreads) void k_chol_panel(int rows, int n, double* __restrict__ A, long long lda, int k0,
-                                                    double* __restrict__ Ldiag, int* __restrict__ info) {
-    extern __shared__ __align__(16) double sm[];
-    double* D = sm;                        // diagonal block, row-major
-    double* X = sm + kNb * kLd;            // this workgroup's 64 rows of the panel
+// Rows x0 .. x0 + 63 (the last one xmax repeated past the end) of the 64 columns from kp,
+// one thread's part: entry i is row t % 64 of column t / 64, t = thread + kStepThreads i
+constexpr int kStepPer = kNb * kNb / kStepThreads;
+
+__device__ __forceinline__ void block_fetch(const double* __restrict__ A, long long lda, int kp, int x0, int xmax,
+                                            double (&v)[kStepPer]) {
+    const double* p = A + min(x0 + (int)(threadIdx.x % kNb), xmax) + (size_t)(kp + threadIdx.x / kNb) * lda;
+#pragma unroll
+    for (int i = 0; i < kStepPer; ++i) v[i] = p[(size_t)(i * (kStepThreads / kNb)) * lda];
+}
+
+// into LDS as [column][row]
+__device__ __forceinline__ void block_put(double* s, const double (&v)[kStepPer]) {
+#pragma unroll
+    for (int i = 0; i < kStepPer; ++i) {
+        const int t = threadIdx.x + kStepThreads * i;
+        s[t / kNb * kLd + t % kNb] = v[i];
+    }
+}
+
+// acc[j] += sum over the 64 columns of x(row) y(16 j + row): x, y point at the first row of such a block's tiles
+template <int N, int M>
+__device__ __forceinline__ void block_products(const double* x, const double* y, mf_d4 (&acc)[M]) {
+    const int row = wave_lane() & 15, grp = wave_lane() >> 4;
+#pragma unroll 4
+    for (int k = 0; k < kNb; k += 4) {
+        const double a = x[(k + grp) * kLd + row];
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+            acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(y[(k + grp) * kLd + 16 * j + row], a, acc[j], 0, 0, 0);
+    }
+}
+
+__device__ __forceinline__ void chol_strip(int rows, int n, double* __restrict__ A, long long lda, int k0, int strip,
+                                           double* __restrict__ Ldiag, int* __restrict__ info, double* sm) {
+    double* D = sm;                        // diagonal block, row-major (lower 16 x 16 tiles)
+    double* X = sm + kNb * kLd;            // this workgroup's 64 rows of the block's columns
     const int nb = min(kNb, n - k0);
     const int wv = uniform(threadIdx.x >> 6);
-    const int R0 = k0 + nb + blockIdx.x * kNb;
+    const int R0 = k0 + nb + strip * kNb;
     const int nr = max(0, min(kNb, rows - R0));
-    // (a block of fewer columns is completed with the unit matrix)
-    {
-        constexpr int N = kNb * kNb / kPanelThreads;
-        const int r = threadIdx.x % kNb, c0 = threadIdx.x / kNb;
-        const double* Ad = A + k0 + min(r, nb - 1);
-        const double* Ax = A + min(R0 + r, rows - 1);
-        double vd[N], vx[N];
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-            const size_t o = (size_t)(k0 + min(c0 + i * (kPanelThreads / kNb), nb - 1)) * lda;
-            vd[i] = Ad[o];
-            vx[i] = Ax[o];
+    if (strip == 0 && k0 > 0) {
+        // the factor of the previous diagonal block goes to its place (until now other
+        // workgroups read the unfactorised one); thread t reads what it overwrites below
+        for (int t = threadIdx.x; t < kNb * kNb; t += kStepThreads) {
+            const int r = t % kNb, c = t / kNb;
+            if (c <= r) A[k0 - kNb + r + (size_t)(k0 - kNb + c) * lda] = Ldiag[t];
         }
+    }
+    {
+        // wavefront w < 4: row tile w of the diagonal block, column tiles 0 .. w; w >= 4: row tile w - 4 of the strip
+        const bool diag = wv < 4;
+        const int t = wv & 3, nu = diag ? t + 1 : 4;
+        const int x = (diag ? k0 : R0) + 16 * t, xmax = diag ? k0 + nb - 1 : rows - 1;
+        const int l = wave_lane(), row = l & 15, grp = l >> 4;
+        double old[4][4], vd[kStepPer], vx[kStepPer];
+        if (k0 > 0) {
+            block_fetch(A, lda, k0 - kNb, k0, k0 + nb - 1, vd);
+            block_fetch(A, lda, k0 - kNb, R0, rows - 1, vx);
+        }
+        const double* px = A + min(x + row, xmax);
 #pragma unroll
-        for (int i = 0; i < N; ++i) {
-            const int c = c0 + i * (kPanelThreads / kNb);
-            D[r * kLd + c] = r < nb && c <= r ? vd[i] : (r == c ? 1.0 : 0.0);
-            X[r * kLd + c] = r < nr && c < nb ? vx[i] : 0.0;
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) old[u][q] = px[(size_t)min(k0 + 16 * u + grp + 4 * q, n - 1) * lda];
+        mf_d4 acc[4] = {};
+        if (k0 > 0) {
+            block_put(D, vd);
+            block_put(X, vx);
+            __syncthreads();
+            const double* xo = (diag ? D : X) + 16 * t;
+            if (nu == 4) block_products<4>(xo, D, acc);
+            else if (nu == 3) block_products<3>(xo, D, acc);
+            else if (nu == 2) block_products<2>(xo, D, acc);
+            else block_products<1>(xo, D, acc);
+            __syncthreads();   // the operands' LDS becomes the block's and the strip's
+        }
+        // (a block of fewer columns is completed with the unit matrix)
+        const int r = 16 * t + row;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (u < nu) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int c = 16 * u + grp + 4 * q;
+                    const double v = old[u][q] - acc[u][q];
+                    if (diag) D[r * kLd + c] = r < nb && c <= r ? v : (r == c ? 1.0 : 0.0);
+                    else X[r * kLd + c] = r < nr && c < nb ? v : 0.0;
+                }
+            }
         }
     }
     __syncthreads();
@@ -422,115 +487,102 @@ __global__ __launch_bounds__(kPanelThreads) void k_chol_panel(int rows, int n, d
         for (int u = b + 1; u < kNb / kSb; ++u) {
             const double* Du = D + u * kSb * kLd + b * kSb;
             for (int t = u; t < kNb / kSb + 4; ++t, ++q)
-                if (q % (kPanelThreads / kWave) == wv) {
+                if (q % (kStepThreads / kWave) == wv) {
                     double* row = t < kNb / kSb ? D + t * kSb * kLd : X + (t - kNb / kSb) * kSb * kLd;
                     tile_store(row + u * kSb, mul16(row + b * kSb, kLd, Du, kLd, -1.0, tile_load(row + u * kSb)));
                 }
         }
         __syncthreads();
     }
-    if (blockIdx.x == 0) {
-        for (int t = threadIdx.x; t < kNb * kNb; t += kPanelThreads) Ldiag[t] = D[(t % kNb) * kLd + t / kNb];
-        if (threadIdx.x == 0 && bad != 0 && *info == 0) *info = k0 + bad;
+    if (strip == 0) {
+        for (int t = threadIdx.x; t < kNb * kNb; t += kStepThreads) Ldiag[t] = D[(t % kNb) * kLd + t / kNb];
+        if (threadIdx.x == 0) {
+            if (k0 == 0) *info = bad;
+            else if (bad != 0 && *info == 0) *info = k0 + bad;
+        }
     }
-    for (int t = threadIdx.x; t < kNb * kNb; t += kPanelThreads) {
+    for (int t = threadIdx.x; t < kNb * kNb; t += kStepThreads) {
         const int r = t % kNb, c = t / kNb;
         if (r < nr && c < nb) A[R0 + r + (size_t)(k0 + c) * lda] = X[r * kLd + c];
     }
 }
 
-// Trailing matrix: A(r, c) -= sum_k A(r, k) A(c, k) over the 64 panel columns,
-// rows k1 .. rows - 1, columns k1 .. n - 1, tiles on or below the diagonal.  The
-// first workgroup also stores the diagonal block's factor (k_chol_panel's
-// workgroups read the unfactorised block).
-__global__ __launch_bounds__(256) void k_chol_update(int rows, int n, double* __restrict__ A, long long lda, int k0,
-                                                     const double* __restrict__ Ldiag) {
-    constexpr int LDP = kNb + 1, KH = kNb / 2;            // the columns in two halves
-    __shared__ double sR[KH * LDP], sC[KH * LDP];         // [k][row]
-    const int nb = min(kNb, n - k0), k1 = k0 + nb;
-    if (blockIdx.x == 0 && blockIdx.y == 0)
-        for (int t = threadIdx.x; t < kNb * kNb; t += 256) {
-            const int r = t % kNb, c = t / kNb;
-            if (r < nb && c <= r) A[k0 + r + (size_t)(k0 + c) * lda] = Ldiag[t];
-        }
-    const int r0 = k1 + blockIdx.x * kNb, c0 = k1 + blockIdx.y * kNb;
-    if (blockIdx.x < blockIdx.y || c0 >= n || r0 >= rows) return;
-    // (a block with columns to its right has all 64 of its own; rows and columns past
-    // the end repeat the last one, their products are not stored)
-    double va[2][KH / 4], vb[2][KH / 4];
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int i = 0; i < KH / 4; ++i) {
-            const int t = threadIdx.x + 256 * i, r = t % kNb, k = h * KH + t / kNb;
-            va[h][i] = A[min(r0 + r, rows - 1) + (size_t)(k0 + k) * lda];
-            vb[h][i] = A[min(c0 + r, n - 1) + (size_t)(k0 + k) * lda];
-        }
+// A(r, c) -= sum_k A(r, k) A(c, k) over the 64 columns of block kp, rows from r0, columns
+// from c0 (entries on or below the diagonal)
+__device__ __forceinline__ void chol_tile(int rows, int n, double* __restrict__ A, long long lda, int kp, int r0, int c0,
+                                          double* sm) {
+    double *sR = sm, *sC = sm + kNb * kLd;
+    // (rows and columns past the end repeat the last one, their products are not stored)
+    double va[kStepPer], vb[kStepPer];
+    block_fetch(A, lda, kp, r0, rows - 1, va);
+    block_fetch(A, lda, kp, c0, n - 1, vb);
     const int l = wave_lane(), wv = uniform(threadIdx.x >> 6);
     const int row = l & 15, grp = l >> 4;
-    const int wr = (wv & 1) * 32, wc = (wv >> 1) * 32;
-    // the tile itself, in flight with the panel rows (a lane's rows are consecutive in memory)
-    double old[2][2][4];
+    const int wr = (wv & 3) * 16, wc = (wv >> 2) * 32;
+    // the tile itself, in flight with the block's rows (a lane's rows are consecutive in memory)
+    double old[2][4];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int q = 0; q < 4; ++q)
+            old[j][q] = A[min(r0 + wr + row, rows - 1) + (size_t)min(c0 + wc + 16 * j + grp + 4 * q, n - 1) * lda];
+    block_put(sR, va);
+    block_put(sC, vb);
+    __syncthreads();
+    mf_d4 acc[2] = {};
+    block_products<2>(sR + wr, sC + wc, acc);
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int r = r0 + wr + 16 * i + row, c = c0 + wc + 16 * j + grp + 4 * q;
-                old[i][j][q] = A[min(r, rows - 1) + (size_t)min(c, n - 1) * lda];
-            }
-    mf_d4 acc[2][2] = {};
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        if (h) __syncthreads();
-#pragma unroll
-        for (int i = 0; i < KH / 4; ++i) {
-            const int t = threadIdx.x + 256 * i;
-            sR[t / kNb * LDP + t % kNb] = va[h][i];
-            sC[t / kNb * LDP + t % kNb] = vb[h][i];
+        for (int q = 0; q < 4; ++q) {
+            const int r = r0 + wr + row, c = c0 + wc + 16 * j + grp + 4 * q;
+            if (r < rows && c < n && r >= c) A[r + (size_t)c * lda] = old[j][q] - acc[j][q];
         }
-        __syncthreads();
-#pragma unroll 4
-        for (int k = 0; k < KH; k += 4) {
-            double a[2], b[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                a[i] = sR[(k + grp) * LDP + wr + 16 * i + row];
-                b[i] = sC[(k + grp) * LDP + wc + 16 * i + row];
-            }
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[j], a[i], acc[i][j], 0, 0, 0);
-        }
+}
+
+// Block k0: workgroups 0 .. strips - 1 are its strips (the longest work, started first),
+// the others the tiles to its right, column by column.
+__global__ __launch_bounds__(kStepThreads) void k_chol_step(int rows, int n, double* __restrict__ A, long long lda, int k0,
+                                                            int strips, double* __restrict__ Ldiag,
+                                                            int* __restrict__ info) {
+    extern __shared__ __align__(16) double sm[];
+    if ((int)blockIdx.x < strips) {
+        chol_strip(rows, n, A, lda, k0, blockIdx.x, Ldiag, info, sm);
+        return;
     }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int r = r0 + wr + 16 * i + row, c = c0 + wc + 16 * j + grp + 4 * q;
-                if (r < rows && c < n && r >= c) A[r + (size_t)c * lda] = old[i][j][q] - acc[i][j][q];
-            }
+    const int k1 = k0 + kNb;               // (a block with tiles to its right has all 64 columns)
+    int t = blockIdx.x - strips, j = 0;
+    while (t >= strips - j) { t -= strips - j; ++j; }
+    chol_tile(rows, n, A, lda, k0 - kNb, k1 + (j + t) * kNb, k1 + j * kNb, sm);
+}
+
+// the factor of the last diagonal block to its place
+__global__ __launch_bounds__(256) void k_chol_last(int nb, double* __restrict__ A, long long lda,
+                                                   const double* __restrict__ Ldiag) {
+    for (int t = threadIdx.x; t < kNb * kNb; t += 256) {
+        const int r = t % kNb, c = t / kNb;
+        if (r < nb && c <= r) A[r + (size_t)c * lda] = Ldiag[t];
+    }
 }
 
 // A (rows x n, rows >= n, ld lda): the lower triangle of its first n rows -> L,
 // the rows below -> B L^-T.  *info = 0 or the 1-based column of the first pivot
 // that is not positive (as dpotrf reports it).  Ldiag: kNb * kNb doubles.
 int chol_lower(hipStream_t st, int rows, int n, double* A, long long lda, double* Ldiag, int* info) {
-    hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, st, info);
-    for (int k0 = 0; k0 < n; k0 += kNb) {
+    int k0 = 0;
+    for (; k0 < n; k0 += kNb) {
         const int k1 = std::min(k0 + kNb, n);
-        const int strips = std::max(1, (rows - k1 + kNb - 1) / kNb), cols = std::max(1, (n - k1 + kNb - 1) / kNb);
-        hipLaunchKernelGGL(k_chol_panel, dim3(strips), dim3(kPanelThreads), kPanelLds, st, rows, n, A, lda, k0, Ldiag, info);
-        hipLaunchKernelGGL(k_chol_update, dim3(k1 < n ? strips : 1, cols), dim3(256), 0, st, rows, n, A, lda, k0,
-                           (const double*)Ldiag);
-        if (int e = launch_check("Cholesky block")) return e;
+        const int strips = std::max(1, (rows - k1 + kNb - 1) / kNb);
+        // the first block has nothing before it to subtract
+        const int cols = k0 == 0 ? 0 : (n - k1 + kNb - 1) / kNb;
+        const int tiles = cols * strips - cols * (cols - 1) / 2;
+        hipLaunchKernelGGL(k_chol_step, dim3(strips + tiles), dim3(kStepThreads), kStepLds, st, rows, n, A, lda, k0,
+                           strips, Ldiag, info);
+        if (int e = launch_check("k_chol_step")) return e;
     }
-    return PT_OK;
+    k0 -= kNb;
+    hipLaunchKernelGGL(k_chol_last, dim3(1), dim3(256), 0, st, n - k0, A + k0 + (size_t)k0 * lda, lda, (const double*)Ldiag);
+    return launch_check("k_chol_last");
 }
 
 // y (n) += A (n x m, ld lda) x (stride incx): kGemvCols columns per workgroup and
