@@ -530,6 +530,31 @@ int pt_max_displacement(int n, const double *pos4, const double *ref, const doub
  * as the out array of pt_max_displacement.  No host read. */
 int pt_skin_check(int n, const double *pos4, const double *ref, const double *box, double skin,
                   double *scratch, int *flag, pt_stream_t stream);
+/* The work of an MD step around its rebuild and forces in three calls, with
+ * the results of the separate calls above bit for bit:
+ * pt_md_positions: pt_verlet_positions, the new pos4 also to pos_out (n x 4);
+ * ref != NULL (n x 4): *flag as pt_skin_check(pos4, ref, box, skin, scratch).
+ * pt_md_velocities: unless gate (device, optional) holds 0, the new state of
+ * atom i follows from the old one of atom perm[i] (the order of a gated
+ * rebuild; f_old is in the old order, f_new in the new one), else from that
+ * of atom i: velocities as pt_verlet_velocities (with_mass: a = F / m), the
+ * rest moved.  in and out share no array.  ref_pos (optional): takes pos4
+ * under the same gate.  ke_part (optional): ceil(n / 1024) partial sums of
+ * the kinetic energy, as pt_reduce_workspace_bytes(n) holds.
+ * pt_md_berendsen: pt_berendsen_rescale from those partial sums. */
+typedef struct {
+    double *vel;       /* (device) n x 3 */
+    double *mass, *inv_mass;
+    int *orig, *types;
+} pt_md_state;
+int pt_md_positions(int n, double *pos4, const double *vel, const double *force, const double *inv_mass,
+                    double dt, const double *box, double *pos_out, const double *ref, double skin,
+                    double *scratch, int *flag, pt_stream_t stream);
+int pt_md_velocities(int n, const int *gate, const int *perm, const pt_md_state *in, const pt_md_state *out,
+                     const double *f_old, const double *f_new, int with_mass, double dt, const double *pos4,
+                     double *ref_pos, double *ke_part, pt_stream_t stream);
+int pt_md_berendsen(int n, double *vel, const double *ke_part, double dt, double tau, double t0, double kb,
+                    pt_stream_t stream);
 /* dst <- src (n_words words of word_bytes = 4 or 8), unless gate (device,
  * optional) holds 0. */
 int pt_copy_gated(long long n_words, int word_bytes, const void *src, void *dst, const int *gate,

@@ -102,6 +102,13 @@ class AcsfRun(ctypes.Structure):
                 ("centers", _vp), ("out", _vp), ("w", _vp), ("f_self", _vp), ("delta", _vp)]
 
 
+class MDState(ctypes.Structure):
+    """pt_md_state: an MD state's arrays in one atom order."""
+
+    _fields_ = [("vel", ctypes.c_void_p), ("mass", ctypes.c_void_p), ("inv_mass", ctypes.c_void_p),
+                ("orig", ctypes.c_void_p), ("types", ctypes.c_void_p)]
+
+
 class PermuteArray(ctypes.Structure):
     _fields_ = [("buf", _vp), ("width", _c_int), ("word_bytes", _c_int)]
 
@@ -119,6 +126,10 @@ _SIGS = {
     "pt_nbr_build_async": (_c_int, [_c_int, _vp, _c_int, _vp, _c_int, _vp, _c_dbl, _vp, _vp, _vp, _vp, _vp,
                                     _c_ll, _vp, _vp, _c_int, _vp, _c_size, _vp]),
     "pt_nbr_mark_rows": (_c_int, [_c_int, _vp, _vp, _vp, _vp, _vp]),
+    "pt_md_positions": (_c_int, [_c_int, _vp, _vp, _vp, _vp, _c_dbl, _vp, _vp, _vp, _c_dbl, _vp, _vp, _vp]),
+    "pt_md_velocities": (_c_int, [_c_int, _vp, _vp, ctypes.POINTER(MDState), ctypes.POINTER(MDState), _vp, _vp, _c_int,
+                                  _c_dbl, _vp, _vp, _vp, _vp]),
+    "pt_md_berendsen": (_c_int, [_c_int, _vp, _vp, _c_dbl, _c_dbl, _c_dbl, _c_dbl, _vp]),
     "pt_skin_check": (_c_int, [_c_int, _vp, _vp, _vp, _c_dbl, _vp, _vp, _vp]),
     "pt_copy_gated": (_c_int, [_c_ll, _c_int, _vp, _vp, _vp, _vp]),
     "pt_permute_rows_gated": (_c_int, [_c_int, _c_int, _c_int, _vp, _vp, _vp, _vp, _vp]),

@@ -5,11 +5,11 @@ simulation/simulate.py:31-88).
 The state of a System lives on the device in the neighbour list's internal
 order (atoms grouped by type and cell).  One MD step is
 
-  pt_verlet_positions  x <- wrap(x + v dt + 1/2 a dt^2)
-  [pt_nbr_build         when the list is stale]
+  pt_md_positions      x <- wrap(x + v dt + 1/2 a dt^2)
+  [pt_nbr_build_async   when the list is stale]
   descriptors -> MLP -> adjoint -> force gather   (the potential's kernels)
-  pt_verlet_velocities v <- v + 1/2 (a + a') dt
-  [pt_kinetic_energy + pt_berendsen_rescale]
+  pt_md_velocities     v <- v + 1/2 (a + a') dt, the state into the list's order
+  [pt_md_berendsen]
 
 Two integrator modes: ``"reference"`` (a = F, the reference's update that
 never divides by the mass, molecular_dynamics.py:16-30) and ``"physical"``
@@ -21,8 +21,8 @@ two largest atom displacements since the last build sum to more than the
 skin (no pair can have moved by more); the descriptor kernels re-apply the
 exact mask (r <= rc, r > 0), so every step sees exactly the reference's
 neighbour set.  In a periodic box that decision is taken on the device
-(pt_skin_check; without a skin every step rebuilds) and the rebuild runs
-behind its flag (pt_nbr_build_async, pt_permute_state_gated), so a step
+(as pt_skin_check; without a skin every step rebuilds) and the rebuild runs
+behind its flag (pt_nbr_build_async, the reorder of the state too), so a step
 never waits for the GPU; the list's totals are verified whenever the host
 reads the state.
 """
@@ -220,6 +220,7 @@ class _DeviceMD:
         self.ref_pos = nl.pos4.clone()
         self.force = torch.zeros((n, 3), dtype=torch.float64, device=self.dev)
         self.force_new = torch.zeros_like(self.force)
+        self._other = None    # the state arrays that an eager gated step writes (allocated by the first)
         self._size_bounds()
 
     # ---- list bounds of the gated step ------------------------------------------
@@ -333,8 +334,22 @@ class _DeviceMD:
         self._builds += 1
         self.row_bound = max(getattr(self, "row_bound", 0), nl.max_row)
 
+    def _build_gated(self, box_p, st) -> None:
+        """The list for the positions in pos_in, behind the device flag: no host read."""
+        lib = _lib.load()
+        nl = self._nl
+        _lib.check(lib.pt_nbr_build_async(self.n, self.pos_in.data_ptr(), 4, self.types.data_ptr(), nl.n_types,
+                                          box_p, nl.r_cutoff, nl.perm.data_ptr(), nl.pos4.data_ptr(),
+                                          nl.row_off.data_ptr(), nl.nbr.data_ptr(), nl.rev.data_ptr(), nl.cap,
+                                          self.flag.data_ptr(), self.totals.data_ptr(), int(self.row_bound),
+                                          nl.ws.data_ptr(), nl.ws.numel(), st),
+                   "pt_nbr_build_async")
+        # the descriptor kernels stage rows up to the bound; buffers are sized for the capacity
+        nl.max_row = self.row_bound
+        nl.n_pairs = nl.cap
+
     def _rebuild_gated(self) -> None:
-        """Skin check, then (behind its device flag) rebuild and reorder the state: no host read."""
+        """Skin check, then (behind its device flag) rebuild and reorder the state in place: no host read."""
         lib = _lib.load()
         nl = self._nl
         st = _lib.stream_ptr()
@@ -348,12 +363,7 @@ class _DeviceMD:
         # neither the displacement check nor the reference positions are needed
         _lib.check(lib.pt_copy_gated(4 * self.n, 8, nl.pos4.data_ptr(), self.pos_in.data_ptr(), g, st),
                    "pt_copy_gated")
-        _lib.check(lib.pt_nbr_build_async(self.n, self.pos_in.data_ptr(), 4, self.types.data_ptr(), nl.n_types,
-                                          box_p, nl.r_cutoff, nl.perm.data_ptr(), nl.pos4.data_ptr(),
-                                          nl.row_off.data_ptr(), nl.nbr.data_ptr(), nl.rev.data_ptr(), nl.cap, g,
-                                          self.totals.data_ptr(), int(self.row_bound), nl.ws.data_ptr(),
-                                          nl.ws.numel(), st),
-                   "pt_nbr_build_async")
+        self._build_gated(box_p, st)
         arrays = (_lib.PermuteArray * 6)(*[_lib.PermuteArray(b.data_ptr(), w, wb) for b, w, wb in (
             (self.vel, 3, 8), (self.force, 3, 8), (self.mass, 1, 8), (self.inv_mass, 1, 8), (self.orig, 1, 4),
             (self.types, 1, 4))])
@@ -362,9 +372,6 @@ class _DeviceMD:
         if self.skin > 0.0:
             _lib.check(lib.pt_copy_gated(4 * self.n, 8, nl.pos4.data_ptr(), self.ref_pos.data_ptr(), g, st),
                        "pt_copy_gated")
-        # the descriptor kernels stage rows up to the bound; buffers are sized for the capacity
-        nl.max_row = self.row_bound
-        nl.n_pairs = nl.cap
 
     def lists_ok(self) -> bool:
         """Whether every gated build since the last check fitted the row bound and the
@@ -431,7 +438,10 @@ class _DeviceMD:
         args = (dt, integrator, force_mode, thermostat)
         if not (self.gated and self.use_graph) or self.timers is not None:
             self._graph = None
-            self._step_body(*args, swap=True)
+            if self.gated:
+                self._step_fused(*args)
+            else:
+                self._step_body(*args, swap=True)
             return
         import torch
 
@@ -456,8 +466,52 @@ class _DeviceMD:
         return (args[:3], id(args[3]), id(ff), id(ff.mlps), nl.cap, self.row_bound,
                 tuple(0 if b is None else b.data_ptr() for b in bufs))
 
+    def _state(self, *arrays) -> "_lib.MDState":
+        return _lib.MDState(*(a.data_ptr() for a in arrays))
+
+    def _step_fused(self, dt: float, integrator: str, force_mode: str,
+                    thermostat: Optional[BrendsenThermostat]) -> None:
+        """A gated step with its own work in three calls (pt_md_positions, pt_md_velocities,
+        pt_md_berendsen): the reordered state goes to a second set of arrays, which then
+        changes places with the first."""
+        import torch
+
+        lib = _lib.load()
+        nl = self._nl
+        st = _lib.stream_ptr()
+        box = host_box(self.box)
+        box_p = ctypes.cast(box, ctypes.c_void_p)
+        physical = integrator == "physical"
+        skin = self.skin > 0.0
+        self._mark("nbr_build", True)
+        # without a skin the flag keeps the 1 it was created with: every step rebuilds
+        _lib.check(lib.pt_md_positions(self.n, nl.pos4.data_ptr(), self.vel.data_ptr(), self.force.data_ptr(),
+                                       self.inv_mass.data_ptr() if physical else None, dt, box_p,
+                                       self.pos_in.data_ptr(), self.ref_pos.data_ptr() if skin else None, self.skin,
+                                       self.disp.data_ptr(), self.flag.data_ptr(), st), "pt_md_positions")
+        self._build_gated(box_p, st)
+        self._mark("nbr_build", False)
+        self.compute(self.force_new, force_mode)
+        now = (self.vel, self.mass, self.inv_mass, self.orig, self.types)
+        if self._other is None:
+            self._other = tuple(torch.empty_like(a) for a in now)
+        new = self._other
+        ke = self.reducer.ws.data_ptr() if thermostat is not None else None
+        _lib.check(lib.pt_md_velocities(self.n, self.flag.data_ptr(), nl.perm.data_ptr(), self._state(*now),
+                                        self._state(*new), self.force.data_ptr(), self.force_new.data_ptr(),
+                                        int(physical), dt, nl.pos4.data_ptr(),
+                                        self.ref_pos.data_ptr() if skin else None, ke, st), "pt_md_velocities")
+        self.vel, self.mass, self.inv_mass, self.orig, self.types = new
+        self._other = now
+        self.force, self.force_new = self.force_new, self.force
+        if thermostat is not None:
+            _lib.check(lib.pt_md_berendsen(self.n, self.vel.data_ptr(), ke, dt, thermostat.time_constant,
+                                           thermostat.target_temperature, KB, st), "pt_md_berendsen")
+
     def _step_body(self, dt: float, integrator: str, force_mode: str, thermostat: Optional[BrendsenThermostat],
                    swap: bool):
+        """The step in place: structures without a box (swap), and captured steps (a replayed
+        step keeps its buffers)."""
         lib = _lib.load()
         inv_m = self.inv_mass.data_ptr() if integrator == "physical" else None
         box = host_box(self.box)
