@@ -271,6 +271,18 @@ __device__ __forceinline__ unsigned long long wave_max(unsigned long long b) {
     return b;
 }
 
+// the largest of a workgroup's bounds into *bmax: one atomic per block, and only when it raises the bound
+__device__ __forceinline__ void raise_bmax(unsigned long long b, unsigned long long* bmax) {
+    b = wave_max(b);
+    __shared__ unsigned long long wmax[256 / kWave];
+    if ((threadIdx.x & (kWave - 1)) == 0) wmax[threadIdx.x >> 6] = b;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int q = 1; q < (int)(blockDim.x >> 6); ++q) b = wmax[q] > b ? wmax[q] : b;
+        if (b > __hip_atomic_load(bmax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(bmax, b);
+    }
+}
+
 // Internal-order positions: FP64 (x, y, z, type) and an FP32 copy for the
 // candidate screen; bmax gets the bit pattern of max |coordinate| (the bit
 // patterns of non-negative doubles order like the values).
@@ -282,28 +294,8 @@ __global__ __launch_bounds__(256) void k_gather_pos4(const int* __restrict__ gat
     if (i < n) perm_out[i] = perm[i];
     unsigned long long b = 0ull;
     if (i < n) b = gather_one(i, perm[i], pos, ps, types, pos4, pos4f);
-    b = wave_max(b);
-    // one atomic per block, and only when it raises the bound
-    __shared__ unsigned long long wmax[256 / kWave];
-    if ((threadIdx.x & (kWave - 1)) == 0) wmax[threadIdx.x >> 6] = b;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int q = 1; q < (int)(blockDim.x >> 6); ++q) b = wmax[q] > b ? wmax[q] : b;
-        if (b > __hip_atomic_load(bmax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(bmax, b);
-    }
+    raise_bmax(b, bmax);
 }
-
-// ---- up to kSortSmall atoms: all of the above in one workgroup --------------
-//
-// Keys, stable radix sort, cell starts and the gather, with keys and order in
-// LDS: what bounds a small build is its launches (6 to 9 of them, each a few us
-// of start and end for work of less).  Wavefront w owns the items
-// [64 w rounds, 64 (w + 1) rounds) in order, so a pass counts digits per wavefront
-// without workgroup barriers and is stable.
-// Measured, a whole build at a cutoff of 12: 96 atoms 33 -> 25 us, 4,096 atoms 57 -> 50,
-// 6,000 atoms 81 -> 72, 8,192 (not taken) the same either way.
-// R: rounds of 1,024 items, as few as hold n (unused ones of 8 cost 3 us at 1,200 atoms).
-constexpr int kSortSmall = 6144;
 
 // exclusive sum over the 1024 threads of v; total: the sum of all
 template <typename T>
@@ -327,6 +319,101 @@ __device__ __forceinline__ T block_exclusive(T v, T* wtot, T& total) {
     total = all;
     return before + incl - v;
 }
+
+// ---- counting sort by (type, cell) ------------------------------------------
+//
+// Five launches where the radix sort, the cell starts and the gather take nine (each
+// a few us of start and end around 1 to 5 us of work: 65 us at 98,304 atoms): atoms per
+// cell by atomics (one per cell and wavefront), the cells' starts, the atoms to
+// their cells in any order, and a last pass that puts each atom at its rank by index
+// among its cell's atoms, which is the stable order, and gathers its position there.
+// That pass reads the cell once per atom (wavefronts share the reads).  The starts'
+// workgroups add up the counts before them themselves, which is why the number of cells is bounded.
+// Measured, these passes: 98,304 atoms 65 -> 29 us at a cutoff of 12 (6,750 cells of a
+// type) and 31 at 8 (24,334); 12,288 atoms 43 -> 18.
+constexpr int kCountKeys = 1 << 18;
+
+__global__ void k_count_zero(const int* __restrict__ gate, int nkeys, int* __restrict__ cnt, unsigned long long* bmax) {
+    if (gated_off(gate)) return;
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < nkeys) cnt[k] = 0;
+    if (k == 0) *bmax = 0ull;   // max |coordinate|, raised by k_rank_gather
+}
+
+// keys[i], and slots[i]: a place of atom i of its own among its cell's atoms
+__global__ __launch_bounds__(256) void k_bin_count(const int* __restrict__ gate, int n, const double* pos, int ps,
+                                                   const int* types, Grid g, int nkeys, int bits,
+                                                   int* __restrict__ cnt, int* __restrict__ keys,
+                                                   int* __restrict__ slots) {
+    if (gated_off(gate)) return;
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool in = i < n;
+    // (a type outside 1 .. n_types has no cell: the counts must stay in their array)
+    const int key = in ? min(max(bin_key(pos, ps, types, g, i), 0), nkeys - 1) : 0;
+    unsigned long long peers = __ballot(in);   // lanes with the same key
+    for (int b = 0; b < bits; ++b) {
+        const unsigned long long bal = __ballot((key >> b) & 1);
+        peers &= ((key >> b) & 1) ? bal : ~bal;
+    }
+    const int below = lanes_below(peers);
+    int base = 0;
+    if (in && below == 0) base = atomicAdd(&cnt[key], __popcll(peers));
+    base = __shfl(base, in ? __ffsll(peers) - 1 : 0, kWave);
+    if (in) {
+        keys[i] = key;
+        slots[i] = base + below;
+    }
+}
+
+__global__ __launch_bounds__(1024) void k_cell_scan(const int* __restrict__ gate, int nkeys,
+                                                    const int* __restrict__ cnt, int* __restrict__ cell_start) {
+    if (gated_off(gate)) return;
+    __shared__ int wtot[16];
+    int s = 0, before, all;
+    for (int k = threadIdx.x; k < (int)blockIdx.x * 1024; k += 1024) s += cnt[k];
+    block_exclusive(s, wtot, before);
+    const int k = blockIdx.x * 1024 + threadIdx.x;
+    const int excl = block_exclusive(k < nkeys ? cnt[k] : 0, wtot, all);
+    if (k <= nkeys) cell_start[k] = before + excl;
+}
+
+__global__ __launch_bounds__(256) void k_cell_scatter(const int* __restrict__ gate, int n, const int* __restrict__ keys,
+                                                      const int* __restrict__ slots, const int* __restrict__ cell_start,
+                                                      int* __restrict__ order) {
+    if (gated_off(gate)) return;
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) order[cell_start[keys[i]] + slots[i]] = i;
+}
+
+__global__ __launch_bounds__(256) void k_rank_gather(const int* __restrict__ gate, int n, const int* __restrict__ keys,
+                                                     const int* __restrict__ cell_start, const int* __restrict__ order,
+                                                     const double* pos, int ps, const int* types, double* pos4,
+                                                     float4* pos4f, unsigned long long* bmax, int* __restrict__ perm_out) {
+    if (gated_off(gate)) return;
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    unsigned long long b = 0ull;
+    if (p < n) {
+        const int v = order[p], key = keys[v];
+        const int s = cell_start[key], e = cell_start[key + 1];
+        int i = s;
+        for (int q = s; q < e; ++q) i += order[q] < v ? 1 : 0;
+        perm_out[i] = v;
+        b = gather_one(i, v, pos, ps, types, pos4, pos4f);
+    }
+    raise_bmax(b, bmax);
+}
+
+// ---- up to kSortSmall atoms: all of the above in one workgroup --------------
+//
+// Keys, stable radix sort, cell starts and the gather, with keys and order in
+// LDS: what bounds a small build is its launches (6 to 9 of them, each a few us
+// of start and end for work of less).  Wavefront w owns the items
+// [64 w rounds, 64 (w + 1) rounds) in order, so a pass counts digits per wavefront
+// without workgroup barriers and is stable.
+// Measured, a whole build at a cutoff of 12: 96 atoms 33 -> 25 us, 4,096 atoms 57 -> 50,
+// 6,000 atoms 81 -> 72, 8,192 (not taken) the same either way.
+// R: rounds of 1,024 items, as few as hold n (unused ones of 8 cost 3 us at 1,200 atoms).
+constexpr int kSortSmall = 6144;
 
 template <int R>
 __global__ __launch_bounds__(1024) void k_sort_small(const int* __restrict__ gate, int n, const double* pos, int ps,
@@ -1204,6 +1291,20 @@ int build_impl(int n, const double* pos, int pos_stride, const int* types, int n
         hipLaunchKernelGGL(kern, dim3(1), dim3(1024), 0, stream, gate, n, pos, pos_stride, types, g, nkeys, bits,
                            cell_start, o.perm, o.pos4, pos4f, bmax);
         if (int rcode = launch_check("k_sort_small")) return rcode;
+    } else if (nkeys <= kCountKeys && nkeys <= 4LL * n) {
+        // (few atoms in very many cells: zeroing and adding up the cells costs more than sorting the atoms)
+        int* cnt = stage;   // free until the candidate pass: n * kStageW ints
+        const dim3 ab((n + tb - 1) / tb);
+        hipLaunchKernelGGL(k_count_zero, dim3((nkeys + tb - 1) / tb), dim3(tb), 0, stream, gate, nkeys, cnt, bmax);
+        hipLaunchKernelGGL(k_bin_count, ab, dim3(tb), 0, stream, gate, n, pos, pos_stride, types, g, nkeys, bits, cnt, keys_a,
+                           vals_a);
+        hipLaunchKernelGGL(k_cell_scan, dim3((nkeys + 1024) / 1024), dim3(1024), 0, stream, gate, nkeys,
+                           (const int*)cnt, cell_start);
+        hipLaunchKernelGGL(k_cell_scatter, ab, dim3(tb), 0, stream, gate, n, (const int*)keys_a, (const int*)vals_a,
+                           (const int*)cell_start, vals_b);
+        hipLaunchKernelGGL(k_rank_gather, ab, dim3(tb), 0, stream, gate, n, (const int*)keys_a, (const int*)cell_start,
+                           (const int*)vals_b, pos, pos_stride, types, o.pos4, pos4f, bmax, o.perm);
+        if (int rcode = launch_check("counting sort")) return rcode;
     } else {
         hipLaunchKernelGGL(k_bin, dim3((n + tb - 1) / tb), dim3(tb), 0, stream, gate, n, pos, pos_stride, types,
                            g, keys_a, vals_a, bmax);
