@@ -34,6 +34,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstddef>
+#include <type_traits>
 
 #include "common.h"
 
@@ -815,6 +816,32 @@ struct Team {
 template <typename R>
 struct Team<R, 1> {};
 
+// Sums of a group's first N cells over the wavefront (a team adds its wavefronts' parts in
+// order) into their columns; gw: the group's words (GroupWords).
+template <int N, typename R, int WPC>
+__device__ __forceinline__ void store_cells(const R (&acc)[PT_AG_ETA][PT_AG_ANG], const int (&qmap)[PT_AG_ANG], int gw,
+                                            int n_eta, int n_ang, Team<R, WPC>& T, int sub, R* row) {
+    R flat[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) flat[k] = acc[k / PT_AG_ANG][k % PT_AG_ANG];
+    R v = wave_sums<N>(flat);
+    const int slot = sum_of_lane<N>(), q = slot & (PT_AG_ANG - 1);
+    // (the map packed: indexed by lane the array would live in scratch)
+    const unsigned packed = (unsigned)(qmap[0] | qmap[1] << 8 | qmap[2] << 16 | qmap[3] << 24);
+    const int tq = (int)((packed >> (8 * q)) & 3u);
+    const int col = __shfl(gw, PT_WORD(pt_angular_group, col) + max(slot - q, 0) + tq, kWave);
+    const bool own = slot >= 0 && slot / PT_AG_ANG < n_eta && q < n_ang && col >= 0;
+    if constexpr (WPC > 1) {
+        if (own) T.part[sub][slot] = v;
+        __syncthreads();
+        if (own && sub == 0) {
+#pragma unroll
+            for (int k = 1; k < WPC; ++k) v += T.part[k][slot];
+        }
+    }
+    if (own && sub == 0) row[col] = v;
+}
+
 template <typename R, int MODE, int KIND, int WPC>
 __device__ __forceinline__ void acsf_centre(const KArgs& a, char* smem, Team<R, WPC>& T) {
     if (sizeof(R) == 8) exp2_tab_load();
@@ -1003,7 +1030,7 @@ __device__ __forceinline__ void acsf_centre(const KArgs& a, char* smem, Team<R, 
         const R rc = lane_value(gr, kRc), irc = lane_value((R)(1.0 / G.d), kRc);
         const bool mine = lane >= kCol && lane < kCol + nfun;   // lane kCol + q: function q's column
         R wl = R(0);
-        if (MODE == MODE_ADJ && mine) wl = w[(size_t)c * a.ld + G.w];
+        if (MODE == MODE_ADJ && mine) wl = w[(size_t)c * a.ld + G.w];   // its dE/dG
         R wgt[PT_RG_MAX], acc[PT_RG_MAX], keta[PT_RG_MAX], eta[PT_RG_MAX], rs[PT_RG_MAX];
 #pragma unroll
         for (int q = 0; q < PT_RG_MAX; ++q) {
@@ -1043,13 +1070,10 @@ __device__ __forceinline__ void acsf_centre(const KArgs& a, char* smem, Team<R, 
             }
         }
         if (MODE != MODE_ADJ) {
-#pragma unroll
-            for (int q = 0; q < PT_RG_MAX; ++q)
-                if (q < nfun) {
-                    const R v = wave_sum(acc[q]);
-                    wl = lane == kCol + q ? v : wl;
-                }
-            if (mine) out[(size_t)c * a.ld + G.w] = wl;
+            const R v = wave_sums<PT_RG_MAX>(acc);
+            const int f = sum_of_lane<PT_RG_MAX>();
+            const int col = __shfl(G.w, kCol + max(f, 0), kWave);
+            if (f >= 0 && f < nfun) out[(size_t)c * a.ld + col] = v;
         }
         wave_sync();
     }
@@ -1086,12 +1110,11 @@ __device__ __forceinline__ void acsf_centre(const KArgs& a, char* smem, Team<R, 
 #pragma unroll
             for (int q = 0; q < PT_AG_ANG; ++q) qmap[q] = q;
         }
-        // lane kCol + cell holds the cell's column, its weight (adjoint) and its sum (forward, tangent)
+        // lane kCol + cell holds the cell's column and its weight (adjoint)
         const int cell = lane - kCol;
         const bool mine = cell >= 0 && cell < kCells && cell / PT_AG_ANG < X.n_eta && cell % PT_AG_ANG < X.n_ang && G.w >= 0;
         R wl = R(0);
         if (MODE == MODE_ADJ && mine) wl = w[(size_t)c * a.ld + G.w];
-        const unsigned long long owned = __ballot(mine);
         R W[PT_AG_ETA][PT_AG_ANG], acc[PT_AG_ETA][PT_AG_ANG];
         const R keta_l = (R)(-G.d * M<R>::kexp);
 #pragma unroll
@@ -1157,27 +1180,10 @@ __device__ __forceinline__ void acsf_centre(const KArgs& a, char* smem, Team<R, 
         }
 
         if (MODE != MODE_ADJ) {
-            // reduce only the group's cells that own a column (uniform branches
-            // keep all lanes active); a team sums its wavefronts' parts in order
-#pragma unroll
-            for (int e = 0; e < PT_AG_ETA; ++e)
-#pragma unroll
-                for (int q = 0; q < PT_AG_ANG; ++q) {
-                    const int k = kCol + e * PT_AG_ANG + qmap[q];
-                    if ((owned >> k) & 1ull) {
-                        const R v = wave_sum(acc[e][q]);
-                        wl = lane == k ? v : wl;
-                    }
-                }
-            if constexpr (WPC > 1) {
-                if (mine) T.part[sub][cell] = wl;
-                __syncthreads();
-                if (mine && sub == 0) {
-#pragma unroll
-                    for (int k = 1; k < WPC; ++k) wl += T.part[k][cell];
-                }
-            }
-            if (mine && sub == 0) out[(size_t)c * a.ld + G.w] = wl;
+            // three eta values and fewer leave the last row of cells out
+            R* row = out + (size_t)c * a.ld;
+            if (X.n_eta < PT_AG_ETA) store_cells<kCells - PT_AG_ANG>(acc, qmap, G.w, X.n_eta, X.n_ang, T, sub, row);
+            else store_cells<kCells>(acc, qmap, G.w, X.n_eta, X.n_ang, T, sub, row);
         }
         if constexpr (WPC == 1) wave_sync();
     }
@@ -1265,8 +1271,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
 // A team of kTeam wavefronts per centre.
 constexpr int kTeam = 4;
 
+// (the FP64 tangent of the table classes is held to three waves per SIMD: with two, 768
+// items took 73 us, not 59)
 template <typename R, int MODE, int KIND>
-__global__ __launch_bounds__(64 * kTeam) void k_acsf_team(KArgs a) {
+__global__ __launch_bounds__(64 * kTeam, sizeof(R) == 8 && MODE == MODE_TAN && KIND != PT_ACSF_GENERIC ? 3 : 1)
+void k_acsf_team(KArgs a) {
     extern __shared__ __align__(32) char smem[];
     __shared__ Team<R, kTeam> T;
     acsf_centre<R, MODE, KIND, kTeam>(a, smem, T);
