@@ -1,6 +1,6 @@
 // (b) ACSF descriptors, their adjoint and their tangent on gfx950.
 //
-// One wavefront (64 lanes) per centre, or kTeam wavefronts per centre when a
+// One wavefront (64 lanes) per centre, or a team of 4 or 8 when a
 // launch has too few centres to fill the chip.  The centre's neighbour row is staged
 // in LDS (relative vectors R_ij = r_i - r_j under the minimum image with r_ij
 // or 1/r_ij, and per mode the cutoff values), compacted to r_ij <= rc_max and
@@ -282,13 +282,13 @@ __host__ __device__ constexpr size_t stage_bytes_per_nbr() {
 // cap is a multiple of 4 and >= the row length; the per-wave area is a
 // multiple of 32 bytes
 // (WPC wavefronts share the stage: each has a queue and, in the adjoint,
-// accumulators of its own -- added in a fixed order at the end, so that the
+// weights and accumulators of its own -- added in a fixed order at the end, so that the
 // result does not depend on the wavefronts' timing -- and the staging ballots
 // are kept in every mode)
 template <typename R, int MODE, int WPC>
 __host__ __device__ constexpr size_t stage_bytes(int cap) {
     return ((size_t)cap * stage_bytes_per_nbr<R, MODE, WPC>() + WPC * queue_len<MODE>() * sizeof(unsigned) +
-            (MODE == MODE_ADJ ? PT_AG_ETA * PT_AG_ANG * sizeof(R) : 0) +
+            (MODE == MODE_ADJ ? WPC * PT_AG_ETA * PT_AG_ANG * sizeof(R) : 0) +
             (MODE == MODE_ADJ || WPC > 1 ? (size_t)((cap + kWave - 1) / kWave) * sizeof(unsigned long long) : 0) +
             31) / 32 * 32;
 }
@@ -314,8 +314,8 @@ __device__ __forceinline__ Stage<R> carve(char* base, int cap, int sub) {
     s.W = nullptr;
     s.keep = nullptr;
     if (MODE == MODE_ADJ) {
-        s.W = reinterpret_cast<R*>(p);
-        p += PT_AG_ETA * PT_AG_ANG * sizeof(R);
+        s.W = reinterpret_cast<R*>(p) + sub * PT_AG_ETA * PT_AG_ANG;
+        p += WPC * PT_AG_ETA * PT_AG_ANG * sizeof(R);
     }
     if (MODE == MODE_ADJ || WPC > 1) s.keep = reinterpret_cast<unsigned long long*>(p);
     return s;
@@ -475,11 +475,12 @@ __device__ __forceinline__ void ang_eval(const AngGroup<R>& X, R cs, R (&v)[PT_A
 
 // All unordered pairs {j, k} of one angular group: screening on r_jk, a
 // per-wave queue of live pairs, and the pair body in full-wave batches.
-// The WPC wavefronts of a centre (sub: this one) take the screening steps in turn.
+// The WPC wavefronts of a centre take the screening steps in turn (turn: this one's
+// first).  have_cut: the stage holds the cutoff values already.  Returns the number of steps.
 template <typename R, int MODE, int CUT, int ANG, int WPC>
-__device__ __forceinline__ void angular_group(const Stage<R>& S, const AngGroup<R>& X,
-                                              const R (&Win)[PT_AG_ETA][PT_AG_ANG],
-                                              R (&acc)[PT_AG_ETA][PT_AG_ANG], int cap, int sub) {
+__device__ __forceinline__ int angular_group(const Stage<R>& S, const AngGroup<R>& X,
+                                             const R (&Win)[PT_AG_ETA][PT_AG_ANG],
+                                             R (&acc)[PT_AG_ETA][PT_AG_ANG], int cap, int sub, int turn, bool have_cut) {
     const int lane = wave_lane();
     constexpr int NA = ang_terms<ANG>();
     constexpr bool kPreOut = ANG != ANGK_GEN;   // pre applied outside the pair loop
@@ -511,7 +512,7 @@ __device__ __forceinline__ void angular_group(const Stage<R>& S, const AngGroup<
         }
     }
     if (kWLds) {
-        if (lane == 0 && sub == 0) {
+        if (lane == 0) {
 #pragma unroll
             for (int e = 0; e < PT_AG_ETA; ++e)
 #pragma unroll
@@ -519,27 +520,31 @@ __device__ __forceinline__ void angular_group(const Stage<R>& S, const AngGroup<
         }
     }
     // cutoff values of the group's neighbours
-    for (int pass = 0; pass < (X.same ? 1 : 2); ++pass) {
-        const int sb = pass == 0 ? X.bj : X.bk, sn = pass == 0 ? X.nj : X.nk;
-        for (int s = sb + lane + sub * kWave; s < sb + sn; s += WPC * kWave) {
-            R f, df;
-            if constexpr ((MODE == MODE_ADJ)) {
-                const R ir = S.P[s].w;
-                cutoff_k<R, CUT>(X.cut, X.rc, X.irc, X.cpre, X.tanh_pre, M<R>::rcp(ir), f, df);
-                V2<R> fv;
-                fv.x = f; fv.y = df * ir;   // dfc / r
-                S.QF[s] = fv;
-            } else if constexpr (MODE == MODE_FWD) {
-                cutoff_k<R, CUT>(X.cut, X.rc, X.irc, X.cpre, X.tanh_pre, S.Q2[s].x, f, df);
-                S.Q2[s].y = f;
-            } else {
-                cutoff_k<R, CUT>(X.cut, X.rc, X.irc, X.cpre, X.tanh_pre, S.Q[s].x, f, df);
-                S.Q[s].z = f;
-                S.Q[s].w = df;
+    if (have_cut) {
+        wave_sync();
+    } else {
+        for (int pass = 0; pass < (X.same ? 1 : 2); ++pass) {
+            const int sb = pass == 0 ? X.bj : X.bk, sn = pass == 0 ? X.nj : X.nk;
+            for (int s = sb + lane + sub * kWave; s < sb + sn; s += WPC * kWave) {
+                R f, df;
+                if constexpr ((MODE == MODE_ADJ)) {
+                    const R ir = S.P[s].w;
+                    cutoff_k<R, CUT>(X.cut, X.rc, X.irc, X.cpre, X.tanh_pre, M<R>::rcp(ir), f, df);
+                    V2<R> fv;
+                    fv.x = f; fv.y = df * ir;   // dfc / r
+                    S.QF[s] = fv;
+                } else if constexpr (MODE == MODE_FWD) {
+                    cutoff_k<R, CUT>(X.cut, X.rc, X.irc, X.cpre, X.tanh_pre, S.Q2[s].x, f, df);
+                    S.Q2[s].y = f;
+                } else {
+                    cutoff_k<R, CUT>(X.cut, X.rc, X.irc, X.cpre, X.tanh_pre, S.Q[s].x, f, df);
+                    S.Q[s].z = f;
+                    S.Q[s].w = df;
+                }
             }
         }
+        centre_sync<WPC>();
     }
-    centre_sync<WPC>();
 
     // one live pair (ia, ib)
     auto body = [&](const int ia, const int ib) {
@@ -699,18 +704,18 @@ __device__ __forceinline__ void angular_group(const Stage<R>& S, const AngGroup<
     // q < n/2 is taken there
     const int h = X.same ? X.nj / 2 : ncol;
     const int npairs = nrow * h;
-    if (npairs <= 0) return;   // (the same for every wavefront of the centre)
+    if (npairs <= 0) return 0;   // (the same for every wavefront of the centre)
     const int half_d = (X.same && X.nj % 2 == 0) ? h - 1 : -1;   // the doubled diagonal
     const int half_q = X.nj / 2;
     constexpr int kStep = kWave * WPC;
     const int d64 = uniform(kStep / nrow), r64 = uniform(kStep - d64 * nrow);
-    const int p0 = WPC == 1 ? lane : lane + sub * kWave;
+    const int p0 = WPC == 1 ? lane : lane + turn * kWave;
     int d = p0 / nrow, q = p0 - (p0 / nrow) * nrow;
     // screen r_jk^2 < rc^2 (loosened by 1e-4 relative); the exact r_jk < rc
     // test is the cutoff's own (it is 0 beyond rc)
     const R rc2 = X.g3 ? X.rc * X.rc * R(1.0001) : R(INFINITY);
     const int sk = X.same ? 1 : 0;
-    int qn = 0, base = WPC == 1 ? 0 : sub * kWave;
+    int qn = 0, base = WPC == 1 ? 0 : turn * kWave;
     // one batch of up to 64 queued pairs through the body; the rest moves up
     auto drain = [&]() {
         wave_sync();
@@ -785,6 +790,7 @@ __device__ __forceinline__ void angular_group(const Stage<R>& S, const AngGroup<
             for (int q = 0; q < PT_AG_ANG; ++q) acc[e][q] *= X.pre[q];
     }
     wave_sync();
+    return (npairs2 + kWave - 1) / kWave;
 }
 
 // 1 when the group's terms are exactly zeta {1, 4} x lambda {+1, -1} (any
@@ -810,36 +816,40 @@ __device__ __forceinline__ int z14_order(const GroupWords& G, int n_ang, int (&q
 // Shared between the wavefronts of a centre (beyond the stage).
 template <typename R, int WPC>
 struct Team {
-    R part[WPC][PT_AG_ETA * PT_AG_ANG];   // a group's sums of each wavefront
-    int seg[WPC][16];                     // segment counts of each wavefront's row chunks
+    static constexpr int kPending = 4;                   // groups whose parts wait for the other wavefronts'
+    static_assert(WPC >= kPending, "a wavefront per pending group adds its parts");
+    R part[WPC][kPending][PT_AG_ETA * PT_AG_ANG];        // groups' sums of each wavefront
+    int seg[WPC][16];                               // segment counts of each wavefront's row chunks
 };
 template <typename R>
-struct Team<R, 1> {};
+struct Team<R, 1> {
+    static constexpr int kPending = 1;
+};
 
-// Sums of a group's first N cells over the wavefront (a team adds its wavefronts' parts in
-// order) into their columns; gw: the group's words (GroupWords).
+// Sums of a group's first N cells over the wavefront.  One wavefront per centre: into their
+// columns.  A team: into its part of pending group `slot`, whose lane's column
+// (or -1) and cell wavefront `slot` keeps.
+// gw: the group's words (GroupWords).
 template <int N, typename R, int WPC>
 __device__ __forceinline__ void store_cells(const R (&acc)[PT_AG_ETA][PT_AG_ANG], const int (&qmap)[PT_AG_ANG], int gw,
-                                            int n_eta, int n_ang, Team<R, WPC>& T, int sub, R* row) {
+                                            int n_eta, int n_ang, Team<R, WPC>& T, int sub, int slot, int& pending_col, int& pending_cell,
+                                            R* row) {
     R flat[N];
 #pragma unroll
     for (int k = 0; k < N; ++k) flat[k] = acc[k / PT_AG_ANG][k % PT_AG_ANG];
-    R v = wave_sums<N>(flat);
-    const int slot = sum_of_lane<N>(), q = slot & (PT_AG_ANG - 1);
+    const R v = wave_sums<N>(flat);
+    const int cell = sum_of_lane<N>(), q = cell & (PT_AG_ANG - 1);
     // (the map packed: indexed by lane the array would live in scratch)
     const unsigned packed = (unsigned)(qmap[0] | qmap[1] << 8 | qmap[2] << 16 | qmap[3] << 24);
     const int tq = (int)((packed >> (8 * q)) & 3u);
-    const int col = __shfl(gw, PT_WORD(pt_angular_group, col) + max(slot - q, 0) + tq, kWave);
-    const bool own = slot >= 0 && slot / PT_AG_ANG < n_eta && q < n_ang && col >= 0;
+    const int k = __shfl(gw, PT_WORD(pt_angular_group, col) + max(cell - q, 0) + tq, kWave);
+    const bool own = cell >= 0 && cell / PT_AG_ANG < n_eta && q < n_ang && k >= 0;
     if constexpr (WPC > 1) {
-        if (own) T.part[sub][slot] = v;
-        __syncthreads();
-        if (own && sub == 0) {
-#pragma unroll
-            for (int k = 1; k < WPC; ++k) v += T.part[k][slot];
-        }
+        if (own) T.part[sub][slot][cell] = v;
+        if (sub == slot) { pending_col = own ? k : -1; pending_cell = cell; }
+    } else if (own) {
+        row[k] = v;
     }
-    if (own && sub == 0) row[col] = v;
 }
 
 template <typename R, int MODE, int KIND, int WPC>
@@ -912,6 +922,29 @@ __device__ __forceinline__ void acsf_centre(const KArgs& a, char* smem, Team<R, 
     const int n_rg = uniform(tab->n_rg), n_ag = uniform(tab->n_ag);
     int tg = lane < n_rg ? tab->rg[lane].elem : 0;
     if (lane < n_ag) tg = max(tg, max(tab->ag[lane].ej, tab->ag[lane].ek));
+    // Tables whose angular groups share one tanh cutoff (and whose radial groups do too:
+    // cut_r): its values are computed as the row is staged, once per neighbour, where
+    // every group computed them for its own segments (two elements: five times)
+    bool cut_a = false, cut_r = false;
+    R rc0 = R(0), irc0 = R(0), cpre0 = R(1);
+    int cut0 = 0;
+    if constexpr (KIND != PT_ACSF_GENERIC) {
+        const int ca = lane < n_ag ? tab->ag[lane].cut : -1, cr = lane < n_rg ? tab->rg[lane].cut : -1;
+        const double ra = lane < n_ag ? tab->ag[lane].rc : 0.0, rr = lane < n_rg ? tab->rg[lane].rc : 0.0;
+        cut0 = lane_word(ca, 0);
+        const double r0 = lane_value(ra, 0);
+        cut_a = (cut0 == PT_CUT_TANH || cut0 == PT_CUT_TANHU) && __ballot(lane < n_ag && (ca != cut0 || ra != r0)) == 0ull;
+        cut_r = cut_a && __ballot(lane < n_rg && (cr != cut0 || rr != r0)) == 0ull;
+        rc0 = (R)r0;
+        irc0 = (R)(1.0 / r0);
+        cpre0 = cut0 == PT_CUT_TANH ? tanh_pre : R(1);
+    }
+    // a team's next angular group, loaded while the one before is worked on
+    GroupWords Gn{0, 0.0};
+    if (WPC > 1 && n_ag > 0) Gn = group_words(&tab->ag[0]);
+    // and the adjoint's weights by column
+    R wrow = R(0);
+    if (MODE == MODE_ADJ && WPC > 1 && lane < a.ld) wrow = ((const R*)rn.w)[(size_t)c * a.ld + lane];
     int tmax = 0;
     while (tmax < kSegTypes && __ballot(tg > tmax) != 0ull) ++tmax;
     const int nseg = min(tmax + 1, kSegTypes);
@@ -945,13 +978,20 @@ __device__ __forceinline__ void acsf_centre(const KArgs& a, char* smem, Team<R, 
             pv.w = (R)(1.0 / e.r);
             qv.x = (R)e.r; qv.y = (R)e.r * (R)e.r; qv.z = R(0); qv.w = R(0);
             S.P[s] = pv;
+            R f = R(0), df = R(0);
+            if (cut_a) cutoff_k<R, CUTK_TANH>(cut0, rc0, irc0, cpre0, tanh_pre, qv.x, f, df);
             if constexpr ((MODE == MODE_ADJ)) {
-                // (fc, dfc) are written per group
+                if (cut_a) {   // (else written per group)
+                    V2<R> fv;
+                    fv.x = f; fv.y = df * pv.w;
+                    S.QF[s] = fv;
+                }
             } else if constexpr (MODE == MODE_FWD) {
                 V2<R> uv;
-                uv.x = qv.x; uv.y = R(0);
+                uv.x = qv.x; uv.y = f;
                 S.Q2[s] = uv;
             } else {
+                qv.z = f; qv.w = df;
                 S.Q[s] = qv;
             }
             if (MODE == MODE_ADJ && WPC == 1) { S.DA[3 * s] = 0.0; S.DA[3 * s + 1] = 0.0; S.DA[3 * s + 2] = 0.0; }
@@ -1017,36 +1057,45 @@ __device__ __forceinline__ void acsf_centre(const KArgs& a, char* smem, Team<R, 
     const R* w = (const R*)rn.w;
 
     // ---- radial groups -----------------------------------------------------
-    // (a team takes whole groups in turn: no sums across wavefronts)
-    for (int g = sub; g < n_rg; g += WPC) {
+    // (a team takes halves of groups in turn: no sums across wavefronts)
+    constexpr int kHalves = WPC > 1 ? 2 : 1, kFun = PT_RG_MAX / kHalves;
+    for (int g2 = sub; g2 < n_rg * kHalves; g2 += WPC) {
+        const int g = g2 / kHalves, f0 = g2 % kHalves * kFun;
         constexpr int kCol = PT_WORD(pt_radial_group, col), kEta = PT_DBL(pt_radial_group, eta),
                       kRs = PT_DBL(pt_radial_group, rs), kRc = PT_DBL(pt_radial_group, rc);
         const GroupWords G = group_words(&tab->rg[g]);
         const int el = lane_word(G.w, PT_WORD(pt_radial_group, elem));
         const int cut = lane_word(G.w, PT_WORD(pt_radial_group, cut));
-        const int nfun = lane_word(G.w, PT_WORD(pt_radial_group, n));
+        const int nfun = lane_word(G.w, PT_WORD(pt_radial_group, n)) - f0;   // from f0 on
+        if (nfun <= 0) continue;
         const int b = seg_below(seg, el), e = seg_below(seg, el + 1);
         const R gr = (R)G.d;
         const R rc = lane_value(gr, kRc), irc = lane_value((R)(1.0 / G.d), kRc);
-        const bool mine = lane >= kCol && lane < kCol + nfun;   // lane kCol + q: function q's column
+        const bool mine = lane >= kCol + f0 && lane < kCol + f0 + nfun;   // lane kCol + q: function q's column
         R wl = R(0);
         if (MODE == MODE_ADJ && mine) wl = w[(size_t)c * a.ld + G.w];   // its dE/dG
-        R wgt[PT_RG_MAX], acc[PT_RG_MAX], keta[PT_RG_MAX], eta[PT_RG_MAX], rs[PT_RG_MAX];
+        R wgt[kFun], acc[kFun], keta[kFun], eta[kFun], rs[kFun];
 #pragma unroll
-        for (int q = 0; q < PT_RG_MAX; ++q) {
+        for (int q = 0; q < kFun; ++q) {
             acc[q] = R(0);
-            eta[q] = (q < nfun) ? lane_value(gr, kEta + q) : R(0);
+            eta[q] = (q < nfun) ? lane_value(gr, kEta + f0 + q) : R(0);
             keta[q] = -eta[q] * M<R>::kexp;
-            rs[q] = (q < nfun) ? lane_value(gr, kRs + q) : R(0);
-            wgt[q] = MODE == MODE_ADJ ? lane_value(wl, kCol + q) : R(0);
+            rs[q] = (q < nfun) ? lane_value(gr, kRs + f0 + q) : R(0);
+            wgt[q] = MODE == MODE_ADJ ? lane_value(wl, kCol + f0 + q) : R(0);
         }
         for (int s = b + lane; s < e; s += kWave) {
             R r;
             if constexpr ((MODE == MODE_ADJ)) r = M<R>::rcp(S.P[s].w);
             else if constexpr (MODE == MODE_FWD) r = S.Q2[s].x;
             else r = S.Q[s].x;
-            R f, df;
-            cutoff<R>(cut, rc, irc, tanh_pre, r, f, df);
+            R f, df = R(0);
+            if (cut_r) {
+                if constexpr (MODE == MODE_ADJ) { f = S.QF[s].x; df = S.QF[s].y * r; }
+                else if constexpr (MODE == MODE_FWD) f = S.Q2[s].y;
+                else { f = S.Q[s].z; df = S.Q[s].w; }
+            } else {
+                cutoff<R>(cut, rc, irc, tanh_pre, r, f, df);
+            }
             R rdot = R(0);
             V4<R> pv;
             if (MODE != MODE_FWD) pv = S.P[s];
@@ -1054,7 +1103,7 @@ __device__ __forceinline__ void acsf_centre(const KArgs& a, char* smem, Team<R, 
                 rdot = (pv.x * S.D[s] + pv.y * S.D[cap + s] + pv.z * S.D[2 * cap + s]) * pv.w;
             R dsum = R(0);
 #pragma unroll
-            for (int q = 0; q < PT_RG_MAX; ++q) {
+            for (int q = 0; q < kFun; ++q) {
                 if (q < nfun) {
                     const R d = r - rs[q];
                     const R ex = M<R>::ex2k(keta[q] * d * d);
@@ -1070,9 +1119,9 @@ __device__ __forceinline__ void acsf_centre(const KArgs& a, char* smem, Team<R, 
             }
         }
         if (MODE != MODE_ADJ) {
-            const R v = wave_sums<PT_RG_MAX>(acc);
-            const int f = sum_of_lane<PT_RG_MAX>();
-            const int col = __shfl(G.w, kCol + max(f, 0), kWave);
+            const R v = wave_sums<kFun>(acc);
+            const int f = sum_of_lane<kFun>();
+            const int col = __shfl(G.w, kCol + f0 + max(f, 0), kWave);
             if (f >= 0 && f < nfun) out[(size_t)c * a.ld + col] = v;
         }
         wave_sync();
@@ -1080,10 +1129,13 @@ __device__ __forceinline__ void acsf_centre(const KArgs& a, char* smem, Team<R, 
 
     // ---- angular groups ----------------------------------------------------
     bool bad = false;   // a group outside this kernel's table class
+    int turn = sub;              // a team's wavefronts take the steps of all groups in turn
+    int pending_col = -1, pending_cell = 0;   // this wavefront's pending group: the lane's column and cell
     for (int g = 0; g < n_ag; ++g) {
         typedef pt_angular_group AG;
         constexpr int kCol = PT_WORD(AG, col), kCells = PT_AG_ETA * PT_AG_ANG;
-        const GroupWords G = group_words(&tab->ag[g]);
+        const GroupWords G = WPC > 1 ? Gn : group_words(&tab->ag[g]);
+        if (WPC > 1 && g + 1 < n_ag) Gn = group_words(&tab->ag[g + 1]);
         const R gr = (R)G.d;
         AngGroup<R> X;
         const int ej = lane_word(G.w, PT_WORD(AG, ej)), ek = lane_word(G.w, PT_WORD(AG, ek));
@@ -1114,7 +1166,14 @@ __device__ __forceinline__ void acsf_centre(const KArgs& a, char* smem, Team<R, 
         const int cell = lane - kCol;
         const bool mine = cell >= 0 && cell < kCells && cell / PT_AG_ANG < X.n_eta && cell % PT_AG_ANG < X.n_ang && G.w >= 0;
         R wl = R(0);
-        if (MODE == MODE_ADJ && mine) wl = w[(size_t)c * a.ld + G.w];
+        if (MODE == MODE_ADJ) {
+            if (WPC > 1 && a.ld <= kWave) {
+                const R v = __shfl(wrow, mine ? G.w : 0, kWave);
+                wl = mine ? v : R(0);
+            } else if (mine) {
+                wl = w[(size_t)c * a.ld + G.w];
+            }
+        }
         R W[PT_AG_ETA][PT_AG_ANG], acc[PT_AG_ETA][PT_AG_ANG];
         const R keta_l = (R)(-G.d * M<R>::kexp);
 #pragma unroll
@@ -1144,48 +1203,67 @@ __device__ __forceinline__ void acsf_centre(const KArgs& a, char* smem, Team<R, 
                        : (X.cut == PT_CUT_COS ? CUTK_COS : CUTK_GEN);
         const int ak = z14 ? ANGK_Z14
                            : (z1 ? (X.n_ang <= 2 ? ANGK_Z1N2 : ANGK_Z1) : (p4 ? ANGK_P4 : ANGK_GEN));
-        centre_sync<WPC>();   // the previous group's cutoff values are no longer read
+        if (!cut_a) centre_sync<WPC>();   // the previous group's cutoff values are no longer read
+        int steps = 0;
         if constexpr (KIND == PT_ACSF_TANH_Z14) {
             if (ck == CUTK_TANH && ak == ANGK_Z14)
-                angular_group<R, MODE, CUTK_TANH, ANGK_Z14, WPC>(S, X, W, acc, cap, sub);
+                steps = angular_group<R, MODE, CUTK_TANH, ANGK_Z14, WPC>(S, X, W, acc, cap, sub, turn, cut_a);
             else
                 bad = true;
         } else if constexpr (KIND == PT_ACSF_TANH_P4) {
             if (ck == CUTK_TANH && ak != ANGK_GEN)
-                angular_group<R, MODE, CUTK_TANH, ANGK_P4, WPC>(S, X, W, acc, cap, sub);
+                steps = angular_group<R, MODE, CUTK_TANH, ANGK_P4, WPC>(S, X, W, acc, cap, sub, turn, cut_a);
             else
                 bad = true;
         } else if constexpr (KIND == PT_ACSF_TANH_Z1N2) {
             if (ck == CUTK_TANH && ak == ANGK_Z1N2)
-                angular_group<R, MODE, CUTK_TANH, ANGK_Z1N2, WPC>(S, X, W, acc, cap, sub);
+                steps = angular_group<R, MODE, CUTK_TANH, ANGK_Z1N2, WPC>(S, X, W, acc, cap, sub, turn, cut_a);
             else
                 bad = true;
         } else if (MODE == MODE_TAN || (sizeof(R) == 8 && ck != CUTK_TANH)) {
-            angular_group<R, MODE, CUTK_GEN, ANGK_GEN, WPC>(S, X, W, acc, cap, sub);
+            steps = angular_group<R, MODE, CUTK_GEN, ANGK_GEN, WPC>(S, X, W, acc, cap, sub, turn, cut_a);
         } else if (sizeof(R) == 8) {
-            if (ak == ANGK_GEN) angular_group<R, MODE, CUTK_TANH, ANGK_GEN, WPC>(S, X, W, acc, cap, sub);
-            else angular_group<R, MODE, CUTK_TANH, ANGK_P4, WPC>(S, X, W, acc, cap, sub);
+            if (ak == ANGK_GEN) steps = angular_group<R, MODE, CUTK_TANH, ANGK_GEN, WPC>(S, X, W, acc, cap, sub, turn, cut_a);
+            else steps = angular_group<R, MODE, CUTK_TANH, ANGK_P4, WPC>(S, X, W, acc, cap, sub, turn, cut_a);
         } else if (ck == CUTK_TANH) {
-            if (ak == ANGK_Z1N2) angular_group<R, MODE, CUTK_TANH, ANGK_Z1N2, WPC>(S, X, W, acc, cap, sub);
-            else if (ak == ANGK_Z1) angular_group<R, MODE, CUTK_TANH, ANGK_Z1, WPC>(S, X, W, acc, cap, sub);
-            else if (ak == ANGK_P4) angular_group<R, MODE, CUTK_TANH, ANGK_P4, WPC>(S, X, W, acc, cap, sub);
-            else angular_group<R, MODE, CUTK_TANH, ANGK_GEN, WPC>(S, X, W, acc, cap, sub);
+            if (ak == ANGK_Z1N2) steps = angular_group<R, MODE, CUTK_TANH, ANGK_Z1N2, WPC>(S, X, W, acc, cap, sub, turn, cut_a);
+            else if (ak == ANGK_Z1) steps = angular_group<R, MODE, CUTK_TANH, ANGK_Z1, WPC>(S, X, W, acc, cap, sub, turn, cut_a);
+            else if (ak == ANGK_P4) steps = angular_group<R, MODE, CUTK_TANH, ANGK_P4, WPC>(S, X, W, acc, cap, sub, turn, cut_a);
+            else steps = angular_group<R, MODE, CUTK_TANH, ANGK_GEN, WPC>(S, X, W, acc, cap, sub, turn, cut_a);
         } else if (ck == CUTK_COS) {
-            if (ak == ANGK_Z1N2) angular_group<R, MODE, CUTK_COS, ANGK_Z1N2, WPC>(S, X, W, acc, cap, sub);
-            else if (ak == ANGK_Z1) angular_group<R, MODE, CUTK_COS, ANGK_Z1, WPC>(S, X, W, acc, cap, sub);
-            else if (ak == ANGK_P4) angular_group<R, MODE, CUTK_COS, ANGK_P4, WPC>(S, X, W, acc, cap, sub);
-            else angular_group<R, MODE, CUTK_COS, ANGK_GEN, WPC>(S, X, W, acc, cap, sub);
+            if (ak == ANGK_Z1N2) steps = angular_group<R, MODE, CUTK_COS, ANGK_Z1N2, WPC>(S, X, W, acc, cap, sub, turn, cut_a);
+            else if (ak == ANGK_Z1) steps = angular_group<R, MODE, CUTK_COS, ANGK_Z1, WPC>(S, X, W, acc, cap, sub, turn, cut_a);
+            else if (ak == ANGK_P4) steps = angular_group<R, MODE, CUTK_COS, ANGK_P4, WPC>(S, X, W, acc, cap, sub, turn, cut_a);
+            else steps = angular_group<R, MODE, CUTK_COS, ANGK_GEN, WPC>(S, X, W, acc, cap, sub, turn, cut_a);
         } else {
-            angular_group<R, MODE, CUTK_GEN, ANGK_GEN, WPC>(S, X, W, acc, cap, sub);
+            steps = angular_group<R, MODE, CUTK_GEN, ANGK_GEN, WPC>(S, X, W, acc, cap, sub, turn, cut_a);
         }
 
         if (MODE != MODE_ADJ) {
             // three eta values and fewer leave the last row of cells out
             R* row = out + (size_t)c * a.ld;
-            if (X.n_eta < PT_AG_ETA) store_cells<kCells - PT_AG_ANG>(acc, qmap, G.w, X.n_eta, X.n_ang, T, sub, row);
-            else store_cells<kCells>(acc, qmap, G.w, X.n_eta, X.n_ang, T, sub, row);
+            constexpr int kPending = Team<R, WPC>::kPending;
+            const int slot = g % kPending;
+            if (X.n_eta < PT_AG_ETA)
+                store_cells<kCells - PT_AG_ANG>(acc, qmap, G.w, X.n_eta, X.n_ang, T, sub, slot, pending_col, pending_cell, row);
+            else
+                store_cells<kCells>(acc, qmap, G.w, X.n_eta, X.n_ang, T, sub, slot, pending_col, pending_cell, row);
+            if constexpr (WPC > 1) {
+                if (slot == kPending - 1 || g + 1 == n_ag) {
+                    // each pending group's parts, in order, by one wavefront
+                    __syncthreads();
+                    if (sub <= slot && pending_col >= 0) {
+                        R v = T.part[0][sub][pending_cell];
+#pragma unroll
+                        for (int k = 1; k < WPC; ++k) v += T.part[k][sub][pending_cell];
+                        row[pending_col] = v;
+                    }
+                    if (g + 1 < n_ag) __syncthreads();
+                }
+            }
         }
         if constexpr (WPC == 1) wave_sync();
+        else turn = (turn + WPC - steps % WPC) % WPC;
     }
     centre_sync<WPC>();
 
@@ -1268,29 +1346,33 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
     acsf_centre<R, MODE, KIND, 1>(a, smem, T);
 }
 
-// A team of kTeam wavefronts per centre.
-constexpr int kTeam = 4;
-
+// A team of WPC wavefronts per centre.
 // (the FP64 tangent of the table classes is held to three waves per SIMD: with two, 768
 // items took 73 us, not 59)
-template <typename R, int MODE, int KIND>
-__global__ __launch_bounds__(64 * kTeam, sizeof(R) == 8 && MODE == MODE_TAN && KIND != PT_ACSF_GENERIC ? 3 : 1)
+template <typename R, int MODE, int KIND, int WPC>
+__global__ __launch_bounds__(64 * WPC, sizeof(R) == 8 && MODE == MODE_TAN && KIND != PT_ACSF_GENERIC ? 3 : 1)
 void k_acsf_team(KArgs a) {
     extern __shared__ __align__(32) char smem[];
-    __shared__ Team<R, kTeam> T;
-    acsf_centre<R, MODE, KIND, kTeam>(a, smem, T);
+    __shared__ Team<R, WPC> T;
+    acsf_centre<R, MODE, KIND, WPC>(a, smem, T);
 }
 
-// Launches of at most this many centres run a team per centre; the line lies
-// where a SIMD would get about one wavefront and a half.  Rows of fewer than
-// kTeamRow entries leave a team little to share.  Measured, us per launch, one
-// wavefront | team of 4 (52 functions at 12 Bohr, ~110 neighbours; 34 at 8 Bohr, ~32):
-//   12 Bohr FP64 forward  96 centres 58.2 | 30.6   768 63.2 | 42.9   1,536 76.2 | 74.4   2,048 75.4 | 91.0
-//   12 Bohr FP64 adjoint  96 centres 65.9 | 32.4   768 72.4 | 46.0   1,536 92.4 | 83.3   2,048 93.9 | 98.7
-//   12 Bohr FP32 forward  96 centres 41.5 | 22.2   768 45.6 | 27.0   1,536 49.6 | 37.7   2,048 49.2 | 51.1
-//   8 Bohr FP32 forward   96 centres 16.6 | 15.0   768 17.8 | 17.9   1,536 19.6 | 23.9
-// (teams of 2 win 15 % between 1,500 and 2,000 centres, teams of 8 only below 100.)
-constexpr int kTeamLong = 1536, kTeamShort = 512, kTeamRow = 80;
+// Launches of at most this many centres run a team per centre: of 8 wavefronts while all
+// teams are resident at two to a CU (one, for the FP64 tangent's registers), of 4 until a
+// wavefront per centre fills the chip as well.  Rows of fewer than kTeamRow entries leave
+// a team little to share; teams of 8 gain them nothing.  A centre's wavefronts meet only where the
+// row is staged and where sums are added: radial groups go by halves, the pair steps of
+// all angular groups in turn, and a group's table words are loaded while the one before
+// runs.  (With barriers around every group FP64 took 31 and 37 us at 96 centres, FP32 27 and 33 at 384.)
+// Measured, us per launch, wavefronts per centre 1 | 4 | 8 (52 functions at 12 Bohr,
+// ~110 neighbours; 34 at 8 Bohr, ~32):
+//   12 Bohr FP64 forward  96 centres 53.4 | 23.9 | 18.8   512 57.4 | 28.3 | 27.7   640 57.9 | 32.6 | 38.0   1,536 68.6 | 55.4   2,048 69.2 | 69.7
+//   12 Bohr FP64 adjoint  96 centres 65.8 | 29.8 | 24.5   512 70.5 | 37.0 | 35.8   640 70.9 | 43.5 | 49.8   1,792 89.4 | 83.0   2,048 90.3 | 92.5
+//   12 Bohr FP64 tangent  96 centres 63.3 | 28.3 | 23.0   300 67.2 | 33.9 | 42.5   1,536 85.4 | 75.9
+//   12 Bohr FP32 adjoint  96 centres 48.2 | 22.5 | 18.5   512 51.4 | 26.0 | 23.8   640 51.9 | 28.5 | 34.5   1,792 58.1 | 52.5   2,048 58.5 | 57.7
+//   8 Bohr FP32 forward   96 centres 14.8 | 12.0 | 11.9   768 15.9 | 15.2          1,024 16.1 | 16.6
+// (teams of 2 win 5 to 15 % between 1,536 and 2,048 centres: not worth a third set of kernels.)
+constexpr int kTeam8 = 512, kTeam8Tan64 = 256, kTeamLong = 1792, kTeamShort = 768, kTeamRow = 80;
 
 template <typename R, int MODE, int KIND>
 int launch(KArgs a, hipStream_t stream) {
@@ -1306,12 +1388,23 @@ int launch(KArgs a, hipStream_t stream) {
         set_error("acsf: neighbour row of %d entries exceeds the LDS budget", a.cap);
         return PT_ERR_UNSUPPORTED;
     }
-    const size_t team = stage_bytes<R, MODE, kTeam>(a.cap);
     // (a row that only fits the LDS without a team's extra arrays keeps one wavefront)
-    if (a.n_items <= (a.cap >= kTeamRow ? kTeamLong : kTeamShort) && team + sizeof(Team<R, kTeam>) + 512 <= lds_budget) {
-        hipLaunchKernelGGL((k_acsf_team<R, MODE, KIND>), dim3(a.n_items), dim3(64 * kTeam), team, stream, a);
+    auto team = [&](auto wpc, int most) {
+        constexpr int W = decltype(wpc)::value;
+        const size_t bytes = stage_bytes<R, MODE, W>(a.cap);
+        if (a.n_items > most || bytes + sizeof(Team<R, W>) + 512 > lds_budget) return false;
+        hipLaunchKernelGGL((k_acsf_team<R, MODE, KIND, W>), dim3(a.n_items), dim3(64 * W), bytes, stream, a);
+        return true;
+    };
+    auto some_team = [&]() {
+        constexpr std::integral_constant<int, 4> w4{};
+        if (a.cap < kTeamRow) return team(w4, kTeamShort);
+        if constexpr (KIND != PT_ACSF_GENERIC)
+            if (team(std::integral_constant<int, 8>{}, sizeof(R) == 8 && MODE == MODE_TAN ? kTeam8Tan64 : kTeam8)) return true;
+        return team(w4, kTeamLong);
+    };
+    if (some_team())
         return launch_check("k_acsf_team");
-    }
     // waves per workgroup: the most resident waves per CU under the LDS limit,
     // ties to the smaller workgroup (a workgroup's LDS is held until its
     // slowest wave ends; one-wave groups ran the FP32 adjoint 2.5 % faster
