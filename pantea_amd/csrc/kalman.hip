@@ -35,7 +35,7 @@
 //
 // Every product and factorisation is a kernel of this file: the library's
 // triangular kernels and its many small products per block took most of the
-// update (student network, n_w = 1,698, m = 4,608: 11.0 ms, now 2.6).
+// update (student network, n_w = 1,698, m = 4,608: 11.0 ms, now 2.2).
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
@@ -88,12 +88,15 @@ __global__ __launch_bounds__(1024) void k_one_obs(int n, const double* __restric
 // ---- FP64 products on the matrix cores -------------------------------------
 //
 // C (M x N) = alpha A B + beta C [+ diag I], column-major, one workgroup of four
-// wavefronts per T x T tile (T = 64: a 2 x 2 block of 16 x 16 MFMA tiles per
-// wavefront; T = 32: one, for products of few tiles).  K runs in chunks of 16
+// wavefronts per 64 x 64 tile (a 2 x 2 block of 16 x 16 MFMA tiles per
+// wavefront).  K runs in chunks of 16
 // through LDS; loads are issued two chunks ahead (a chunk's products take about
-// the latency of a load that misses L2).  Bound: the matrix cores, for 1,698 x
-// 1,698 x 4,608 (lower half) 347 us = 38 TFLOP/s of 70: 378 tiles leave a CU with
-// one or two, so a quarter of the time is the imbalance.  The
+// the latency of a load that misses L2).  Bound: the matrix cores.  A CU needs four
+// workgroups to keep them fed (one wavefront per SIMD each), so products of fewer
+// tiles split K over blockIdx.z: every part goes to its slice of `part`, k_gemm_sum adds them in
+// order.  Measured, one part | split: 1,698 x 1,698 x 4,608 (lower half) 503 | 313 + 11 us
+// = 41 TFLOP/s of the 64 that a large product reaches, x 1,698 188 | 120 + 13, 1,698 x 576 x 1,698
+// 91 (in 32 x 32 tiles) | 75 + 10.  The
 // operands' layouts are compile-time: LA = 0: A(r, k) at r + k lda, 1: at
 // k + r lda; LB = 0: B(k, c) at c + k ldb, 1: at k + c ldb.  LDS holds [k][row]
 // with rows T + 1 doubles apart (both the column-wise stores of a k-contiguous
@@ -115,21 +118,27 @@ struct GemmArgs {
     long long ldc;
     double alpha, beta, diag;
     int lower, mirror, tri;
+    int split;       // parts of K (a slice of part each, M x N)
+    double* part;
 };
 
-template <int LA, int LB, int T>
+template <int LA, int LB>
 __global__ __launch_bounds__(256) void k_gemm_f64(GemmArgs g) {
-    constexpr int W = T / 32;             // MFMA tiles per wavefront and dimension
+    constexpr int T = 64, W = T / 32;             // MFMA tiles per wavefront and dimension
     constexpr int LDP = T + 1;
     constexpr int PER = T * kKc / 256;    // elements per thread, chunk and operand
     __shared__ double sA[2][kKc * LDP], sB[2][kKc * LDP];
-    const int r0 = blockIdx.x * T, c0 = blockIdx.y * T;
+    // (a triangle's longest rows, the first ones, start first)
+    const int r0 = (g.tri ? blockIdx.y : blockIdx.x) * T, c0 = (g.tri ? blockIdx.x : blockIdx.y) * T;
     if (g.lower && r0 + T <= c0) return;
     const int l = wave_lane(), wv = uniform(threadIdx.x >> 6);
     const int row = l & 15, grp = l >> 4;
     const int wr = (wv & 1) * 16 * W, wc = (wv >> 1) * 16 * W;
-    const int kb = g.tri ? r0 / kKc * kKc : 0;
-    const int nk = max(0, (g.K - kb) / kKc);      // whole chunks
+    // this part's columns: whole chunks, the last part takes the remainder
+    const int k_begin = g.tri ? r0 / kKc * kKc : 0, chunks = max(0, (g.K - k_begin) / kKc);
+    const int per = (chunks + g.split - 1) / g.split, first = min((int)blockIdx.z * per, chunks);
+    const int kb = k_begin + first * kKc, nk = min(per, chunks - first);
+    const bool last_part = (int)blockIdx.z == g.split - 1;
     struct Chunk {
         double a[PER], b[PER];
     };
@@ -205,7 +214,7 @@ __global__ __launch_bounds__(256) void k_gemm_f64(GemmArgs g) {
         }
     }
     const int kr = kb + nk * kKc;
-    if (kr < g.K) {   // the last columns, fewer than a chunk
+    if (last_part && kr < g.K) {   // the last columns, fewer than a chunk
         for (int t = threadIdx.x; t < T * kKc; t += 256) {
             const int ka = kr + t / T, ra = r0 + t % T, cb = c0 + t % T;
             const bool in = ka < g.K;
@@ -224,6 +233,10 @@ __global__ __launch_bounds__(256) void k_gemm_f64(GemmArgs g) {
             for (int q = 0; q < 4; ++q) {
                 const int r = r0 + wr + 16 * i + row, cc = c0 + wc + 16 * j + grp + 4 * q;
                 if (r >= g.M || cc >= g.N || (g.lower && r < cc)) continue;
+                if (g.split > 1) {
+                    g.part[((size_t)blockIdx.z * g.N + cc) * g.M + r] = acc[i][j][q];
+                    continue;
+                }
                 const double p = g.alpha * acc[i][j][q] + (r == cc ? g.diag : 0.0);
                 double* o = g.C + r + (size_t)cc * g.ldc;
                 *o = g.beta != 0.0 ? p + g.beta * *o : p;
@@ -234,18 +247,68 @@ __global__ __launch_bounds__(256) void k_gemm_f64(GemmArgs g) {
             }
 }
 
-// tiles of 64 x 64 from which on they are used (see gemm_f64)
-constexpr long long kGemmTiles = 256;
+// The parts' sums into C, as the single-part kernel stores its products: 32 x 32 entries per
+// workgroup, the mirrored ones through LDS so that both go to consecutive addresses (written
+// straight from the lower triangle they took 49 us at 1,698 x 1,698, not 17).
+__global__ __launch_bounds__(256) void k_gemm_sum(GemmArgs g) {
+    __shared__ double tile[32][33];
+    const int r0 = blockIdx.x * 32, c0 = blockIdx.y * 32, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    if (g.lower && r0 + 32 <= c0) return;
+    const int r = r0 + tx;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int cc = c0 + ty + 8 * q;
+        if (r >= g.M || cc >= g.N || (g.lower && r < cc)) continue;
+        double s = 0.0;
+        for (int z = 0; z < g.split; ++z) s += g.part[((size_t)z * g.N + cc) * g.M + r];
+        const double p = g.alpha * s + (r == cc ? g.diag : 0.0);
+        double* o = g.C + r + (size_t)cc * g.ldc;
+        *o = g.beta != 0.0 ? p + g.beta * *o : p;
+        tile[ty + 8 * q][tx] = p;
+    }
+    if (!g.mirror) return;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int rr = r0 + ty + 8 * q, cc = c0 + tx;   // entry (rr, cc) of the triangle to (cc, rr)
+        if (rr >= g.M || cc >= g.N || rr <= cc) continue;
+        const double p = tile[tx][ty + 8 * q];
+        double* o = g.C + cc + (size_t)rr * g.ldc;
+        *o = g.beta != 0.0 ? p + g.beta * *o : p;
+    }
+}
+
+// Workgroups that fill the chip (four per CU), most parts of a product, chunks of K that a
+// part has at least (below that its start and its part's way through memory cost more than it saves)
+constexpr int kGemmFill = 1024, kGemmParts = 8, kGemmChunks = 12;
+
+long long gemm_tiles(const GemmArgs& g) {
+    const long long r = (g.M + 63) / 64, c = (g.N + 63) / 64;
+    return g.lower ? r * (r + 1) / 2 : r * c;
+}
+
+int gemm_parts(const GemmArgs& g) {
+    if (g.tri) return 1;
+    const long long want = (kGemmFill + gemm_tiles(g) - 1) / gemm_tiles(g);
+    return (int)std::max(1LL, std::min({want, (long long)kGemmParts, (long long)(g.K / kKc / kGemmChunks)}));
+}
+
+// Doubles that the parts of any product of at most n x n results take: gemm_parts < fill /
+// tiles + 1, and a result has at most 2 x 64 x 64 entries per tile (lower: half the tiles of
+// a full one).  Not less for a smaller product, so a workspace serves all up to its size.
+size_t gemm_part_doubles(int n) {
+    const long long r = (n + 63) / 64;
+    const long long by_tiles = 2LL * 64 * 64 * (kGemmFill + std::min<long long>(kGemmFill, r * r));
+    return (size_t)std::min<long long>((long long)kGemmParts * n * n, by_tiles);
+}
 
 template <int LA, int LB>
-int gemm_f64(const GemmArgs& g, hipStream_t st) {
-    // 64 x 64 tiles need about a tile per CU; below that the smaller tiles keep more CUs busy
-    // (1,698 x 288 x 1,698: 85 us in 1,431 -- 32 x 32 -- tiles, 135 larger ones would leave half the chip idle)
-    const long long tiles = (long long)((g.M + 63) / 64) * ((g.N + 63) / 64) / (g.lower ? 2 : 1);
-    if (tiles >= kGemmTiles)
-        hipLaunchKernelGGL((k_gemm_f64<LA, LB, 64>), dim3((g.M + 63) / 64, (g.N + 63) / 64), dim3(256), 0, st, g);
-    else
-        hipLaunchKernelGGL((k_gemm_f64<LA, LB, 32>), dim3((g.M + 31) / 32, (g.N + 31) / 32), dim3(256), 0, st, g);
+int gemm_f64(GemmArgs g, double* part, hipStream_t st) {
+    g.split = gemm_parts(g);
+    g.part = part;
+    const dim3 rc((g.M + 63) / 64, (g.N + 63) / 64, g.split), cr((g.N + 63) / 64, (g.M + 63) / 64, 1);
+    hipLaunchKernelGGL((k_gemm_f64<LA, LB>), g.tri ? cr : rc, dim3(256), 0, st, g);
+    if (g.split > 1) hipLaunchKernelGGL(k_gemm_sum, dim3((g.M + 31) / 32, (g.N + 31) / 32), dim3(256), 0, st, g);
     return launch_check("k_gemm_f64");
 }
 
@@ -650,9 +713,9 @@ using namespace pt;
 
 namespace {
 // Workspace: the factorised matrix with the rows it carries, G (n_w x n_w form only),
-// partial sums of the products with a vector, a vector, the diagonal block, info.
+// partial sums of the products with a vector and of those split over K, a vector, the diagonal block, info.
 struct KalmanWs {
-    size_t aug, G, part, vec, diag, info, total;
+    size_t aug, G, part, gpart, vec, diag, info, total;
     long long lda;
     KalmanWs(int n_w, int m) {
         const size_t nw = (size_t)n_w, mm = (size_t)m;
@@ -662,6 +725,7 @@ struct KalmanWs {
         aug = o; o += align256(8 * (size_t)lda * (f ? nw : mm));
         G = o; o += f ? align256(8 * nw * mm) : 0;
         part = o; o += align256(8 * gemv_ws_doubles(n_w, std::max(n_w, m)));
+        gpart = o; o += align256(8 * gemm_part_doubles(n_w));
         vec = o; o += align256(8 * nw);
         diag = o; o += align256(8 * (size_t)kNb * kNb);
         info = o; o += align256(sizeof(int));
@@ -700,6 +764,7 @@ extern "C" int pt_kalman_update(int n_w, int m, double* P, const double* H, long
     double* S = (double*)(base + L.aug);
     double* G = (double*)(base + L.G);
     double* part = (double*)(base + L.part);
+    double* gpart = (double*)(base + L.gpart);
     double* vec = (double*)(base + L.vec);
     double* diag = (double*)(base + L.diag);
     int* info2 = (int*)(base + L.info);
@@ -708,9 +773,9 @@ extern "C" int pt_kalman_update(int n_w, int m, double* P, const double* H, long
         // L = chol(P), lower triangle in place
         if (int e = chol_lower(st, n_w, n_w, P, n_w, diag, info)) return e;
         // G = L^T H
-        if (int e = gemm_f64<1, 1>({n_w, m, n_w, P, n_w, H, ldh, G, n_w, 1.0, 0.0, 0.0, 0, 0, 1}, st)) return e;
+        if (int e = gemm_f64<1, 1>({n_w, m, n_w, P, n_w, H, ldh, G, n_w, 1.0, 0.0, 0.0, 0, 0, 1}, gpart, st)) return e;
         // S = G G^T + r I, below it L and (G xi)^T
-        if (int e = gemm_f64<0, 0>({n_w, n_w, m, G, n_w, G, n_w, S, ld, 1.0, 0.0, r, 1, 0, 0}, st)) return e;
+        if (int e = gemm_f64<0, 0>({n_w, n_w, m, G, n_w, G, n_w, S, ld, 1.0, 0.0, r, 1, 0, 0}, gpart, st)) return e;
         if (int e = gemv(st, n_w, m, G, n_w, xi, 1, false, vec, 1, part)) return e;
         hipLaunchKernelGGL(k_lower_copy, dim3((n_w + 256) / 256, n_w), dim3(256), 0, st, n_w, (const double*)P,
                            (long long)n_w, (const double*)vec, S + n_w, ld);
@@ -722,7 +787,7 @@ extern "C" int pt_kalman_update(int n_w, int m, double* P, const double* H, long
         // W += M y (= L S^-1 G xi), then P = c r M M^T + q I
         const double* M = S + n_w;
         if (int e = gemv(st, n_w, n_w, M, ld, S + 2 * (size_t)n_w, ld, true, W, 1, part)) return e;
-        return gemm_f64<0, 0>({n_w, n_w, n_w, M, ld, M, ld, P, n_w, c * r, 0.0, q, 1, 1, 0}, st);
+        return gemm_f64<0, 0>({n_w, n_w, n_w, M, ld, M, ld, P, n_w, c * r, 0.0, q, 1, 1, 0}, gpart, st);
     }
     double* X = S + m;                       // n_w rows below the m x m matrix
     double* z = S + m + (size_t)n_w;         // and the row of the residuals
@@ -732,8 +797,8 @@ extern "C" int pt_kalman_update(int n_w, int m, double* P, const double* H, long
         if (int e = launch_check("k_one_obs")) return e;
     } else {
         // X = P H, A = H^T X + r I, the residuals as the last row
-        if (int e = gemm_f64<0, 1>({n_w, m, n_w, P, n_w, H, ldh, X, ld, 1.0, 0.0, 0.0, 0, 0, 0}, st)) return e;
-        if (int e = gemm_f64<1, 1>({m, m, n_w, H, ldh, X, ld, S, ld, 1.0, 0.0, r, 1, 0, 0}, st)) return e;
+        if (int e = gemm_f64<0, 1>({n_w, m, n_w, P, n_w, H, ldh, X, ld, 1.0, 0.0, 0.0, 0, 0, 0}, gpart, st)) return e;
+        if (int e = gemm_f64<1, 1>({m, m, n_w, H, ldh, X, ld, S, ld, 1.0, 0.0, r, 1, 0, 0}, gpart, st)) return e;
         hipLaunchKernelGGL(k_set_row, dim3((m + 255) / 256), dim3(256), 0, st, m, xi, z, ld);
         if (int e = launch_check("k_set_row")) return e;
         // A = L L^T, Z = X L^-T, z = L^-1 xi
@@ -741,5 +806,5 @@ extern "C" int pt_kalman_update(int n_w, int m, double* P, const double* H, long
     }
     // W += Z z, P = c (P - Z Z^T) + q I
     if (int e = gemv(st, n_w, m, X, ld, z, ld, true, W, 1, part)) return e;
-    return gemm_f64<0, 0>({n_w, n_w, m, X, ld, X, ld, P, n_w, -c, c, q, 1, 1, 0}, st);
+    return gemm_f64<0, 0>({n_w, n_w, m, X, ld, X, ld, P, n_w, -c, c, q, 1, 1, 0}, gpart, st);
 }
