@@ -240,9 +240,11 @@ def require_device() -> "object":
 
 
 def stream_ptr() -> int:
+    """The current stream of the current device (the raw handle: building a Stream object for
+    it took 3 us of every launch)."""
     import torch
 
-    return torch.cuda.current_stream().cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def ptr(t) -> Optional[int]:

@@ -129,7 +129,9 @@ class _ForceField:
             need = nl.n_pairs * 3
             edt = torch.float64 if self.g_prec == _lib.PT_F64 else torch.float32
             if self.edge is None or self.edge.numel() < need:
-                self.edge = torch.zeros(int(need * 1.2) + 3, dtype=edt, device=self.dev)
+                # for the list's capacity at once (a gated step's pair count is its capacity); every edge of a
+                # row is written by its centre, or cleared below where an element has no model
+                self.edge = torch.empty(int(max(need, 3 * nl.cap) * 1.2) + 3, dtype=edt, device=self.dev)
             if not self.covered:
                 self.edge.zero_()
         target = self.f_self if full else out
@@ -239,11 +241,13 @@ class _DeviceMD:
         self.row_bound = int(f * nl.max_row) + self.ROW_MARGIN
         cap = int(f * self.PAIR_MARGIN * nl.n_pairs) + 1024
         if cap > nl.cap:
+            # larger arrays; the list moves over (it was built a second time for them: 250 us of a small box's start)
             nl.cap = cap
-            nl.nbr = torch.empty(cap, dtype=torch.int32, device=self.dev)
-            nl.rev = torch.empty(cap, dtype=torch.int32, device=self.dev)
-            # the list content was lost with the arrays: build it again
-            self._rebuild_sync(nl.pos4.clone())
+            for name in ("nbr", "rev"):
+                old = getattr(nl, name)
+                new = torch.empty(cap, dtype=torch.int32, device=self.dev)
+                new[:nl.n_pairs] = old[:nl.n_pairs]
+                setattr(nl, name, new)
         self.totals.zero_()
 
     def add_field(self, pot, precision: str) -> _ForceField:
