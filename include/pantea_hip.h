@@ -555,6 +555,22 @@ int pt_md_velocities(int n, const int *gate, const int *perm, const pt_md_state 
                      double *ref_pos, double *ke_part, pt_stream_t stream);
 int pt_md_berendsen(int n, double *vel, const double *ke_part, double dt, double tau, double t0, double kb,
                     pt_stream_t stream);
+/* The state of atom i from input-order arrays: atom perm[i]'s velocity, mass,
+ * 1 / mass, perm[i] itself and type. */
+int pt_md_start(int n, const int *perm, const double *vel, const double *mass, const int *types,
+                const pt_md_state *out, pt_stream_t stream);
+/* Up to PT_COPY_MAX copies (device, a multiple of 4 bytes each, ranges that do
+ * not overlap) in one launch. */
+#define PT_COPY_MAX 8
+typedef struct {
+    const void *src;
+    void *dst;
+    long long bytes;
+} pt_copy_array;
+int pt_copy_arrays(int n, const pt_copy_array *arrays, pt_stream_t stream);
+/* dst[idx[i]] (n x 3) = the first three of row i of src (rows src_stride apart). */
+int pt_scatter_rows3_f64(int n, const int *idx, const double *src, int src_stride, double *dst,
+                         pt_stream_t stream);
 /* dst <- src (n_words words of word_bytes = 4 or 8), unless gate (device,
  * optional) holds 0. */
 int pt_copy_gated(long long n_words, int word_bytes, const void *src, void *dst, const int *gate,

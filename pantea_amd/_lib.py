@@ -109,6 +109,10 @@ class MDState(ctypes.Structure):
                 ("orig", ctypes.c_void_p), ("types", ctypes.c_void_p)]
 
 
+class CopyArray(ctypes.Structure):
+    _fields_ = [("src", _vp), ("dst", _vp), ("bytes", ctypes.c_longlong)]
+
+
 class PermuteArray(ctypes.Structure):
     _fields_ = [("buf", _vp), ("width", _c_int), ("word_bytes", _c_int)]
 
@@ -126,6 +130,9 @@ _SIGS = {
     "pt_nbr_build_async": (_c_int, [_c_int, _vp, _c_int, _vp, _c_int, _vp, _c_dbl, _vp, _vp, _vp, _vp, _vp,
                                     _c_ll, _vp, _vp, _c_int, _vp, _c_size, _vp]),
     "pt_nbr_mark_rows": (_c_int, [_c_int, _vp, _vp, _vp, _vp, _vp]),
+    "pt_md_start": (_c_int, [_c_int, _vp, _vp, _vp, _vp, ctypes.POINTER(MDState), _vp]),
+    "pt_copy_arrays": (_c_int, [_c_int, _vp, _vp]),
+    "pt_scatter_rows3_f64": (_c_int, [_c_int, _vp, _vp, _c_int, _vp, _vp]),
     "pt_md_positions": (_c_int, [_c_int, _vp, _vp, _vp, _vp, _c_dbl, _vp, _vp, _vp, _c_dbl, _vp, _vp, _vp]),
     "pt_md_velocities": (_c_int, [_c_int, _vp, _vp, ctypes.POINTER(MDState), ctypes.POINTER(MDState), _vp, _vp, _c_int,
                                   _c_dbl, _vp, _vp, _vp, _vp]),

@@ -3,6 +3,8 @@
 //
 // Reductions are deterministic: fixed-size blocks reduce in a fixed tree
 // order into per-block partials, and one block sums the partials in order.
+#include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -418,6 +420,53 @@ __global__ __launch_bounds__(kRedThreads) void k_md_berendsen(int n, double* __r
     vel[3 * i] *= lam; vel[3 * i + 1] *= lam; vel[3 * i + 2] *= lam;
 }
 
+// ---- an MD state's start, checkpoints and read-out: one launch each -------------
+//
+// What bounds them is their launches: a run of a few steps spent 7 on each checkpoint, 8 on
+// the state's start and two per read-out, each under 2 us of work at 384 atoms.
+
+// the internal-order state from input-order arrays (atom perm[i] becomes atom i)
+__global__ void k_md_start(int n, const int* __restrict__ perm, const double* __restrict__ vel,
+                           const double* __restrict__ mass, const int* __restrict__ types, pt_md_state out) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int j = perm[i];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) out.vel[3 * i + d] = vel[3 * j + d];
+    out.mass[i] = mass[j];
+    out.inv_mass[i] = 1.0 / mass[j];
+    out.orig[i] = j;
+    out.types[i] = types[j];
+}
+
+struct CopyArgs {
+    int n;
+    const char* src[PT_COPY_MAX];
+    char* dst[PT_COPY_MAX];
+    long long bytes[PT_COPY_MAX];
+    int wide[PT_COPY_MAX];        // both ends on 16-byte addresses
+};
+
+// array blockIdx.y; 16 bytes per thread and step where the addresses allow, else and at the end 4
+__global__ __launch_bounds__(256) void k_copy_arrays(CopyArgs a) {
+    const int k = blockIdx.y;
+    const long long first = (long long)blockIdx.x * 256 + threadIdx.x, step = (long long)gridDim.x * 256;
+    const long long whole = a.wide[k] ? a.bytes[k] / 16 : 0;
+    for (long long t = first; t < whole; t += step)
+        reinterpret_cast<int4*>(a.dst[k])[t] = reinterpret_cast<const int4*>(a.src[k])[t];
+    for (long long t = 4 * whole + first; t < a.bytes[k] / 4; t += step)
+        reinterpret_cast<int*>(a.dst[k])[t] = reinterpret_cast<const int*>(a.src[k])[t];
+}
+
+// dst[idx[i]] (3 wide) = the first 3 of row i of src
+__global__ void k_scatter3(int n, const int* __restrict__ idx, const double* __restrict__ src, int stride,
+                           double* __restrict__ dst) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= 3 * n) return;
+    const int i = t / 3, d = t - 3 * i;
+    dst[3 * (size_t)idx[i] + d] = src[(size_t)i * stride + d];
+}
+
 struct PermuteArgs {
     int n_arrays;
     char* buf[PT_PERMUTE_MAX];
@@ -702,6 +751,44 @@ extern "C" int pt_md_berendsen(int n, double* vel, const double* ke_part, double
     hipLaunchKernelGGL(k_md_berendsen, dim3(nblocks(n, kRedThreads)), dim3(kRedThreads), 0, (hipStream_t)stream, n, vel,
                        nblocks(n, kRedTile), ke_part, dt, tau, t0, kb);
     return launch_check("pt_md_berendsen");
+}
+
+extern "C" int pt_md_start(int n, const int* perm, const double* vel, const double* mass, const int* types,
+                           const pt_md_state* out, pt_stream_t stream) {
+    PT_REQUIRE(n >= 0 && perm && vel && mass && types && out && out->vel && out->mass && out->inv_mass && out->orig &&
+                   out->types, "pt_md_start: bad arguments");
+    if (n == 0) return PT_OK;
+    hipLaunchKernelGGL(k_md_start, dim3(nblocks(n, 256)), dim3(256), 0, (hipStream_t)stream, n, perm, vel, mass, types, *out);
+    return launch_check("pt_md_start");
+}
+
+extern "C" int pt_copy_arrays(int n, const pt_copy_array* arrays, pt_stream_t stream) {
+    PT_REQUIRE(n >= 0 && n <= PT_COPY_MAX && (n == 0 || arrays), "pt_copy_arrays: bad arguments");
+    if (n == 0) return PT_OK;
+    CopyArgs a{};
+    a.n = n;
+    long long most = 0;
+    for (int k = 0; k < n; ++k) {
+        const pt_copy_array& c = arrays[k];
+        PT_REQUIRE(c.bytes >= 0 && c.bytes % 4 == 0 && (c.bytes == 0 || (c.src && c.dst)), "pt_copy_arrays: bad array %d", k);
+        PT_REQUIRE(((size_t)c.src | (size_t)c.dst) % 4 == 0, "pt_copy_arrays: misaligned array %d", k);
+        a.src[k] = (const char*)c.src;
+        a.dst[k] = (char*)c.dst;
+        a.bytes[k] = c.bytes;
+        a.wide[k] = ((size_t)c.src | (size_t)c.dst) % 16 == 0;
+        most = std::max(most, c.bytes);
+    }
+    const int blocks = std::max(1, std::min(1024, nblocks(most / 16, 256)));
+    hipLaunchKernelGGL(k_copy_arrays, dim3(blocks, n), dim3(256), 0, (hipStream_t)stream, a);
+    return launch_check("pt_copy_arrays");
+}
+
+extern "C" int pt_scatter_rows3_f64(int n, const int* idx, const double* src, int src_stride, double* dst,
+                                    pt_stream_t stream) {
+    PT_REQUIRE(n >= 0 && n <= (INT_MAX - 255) / 3 && src_stride >= 3 && idx && src && dst, "pt_scatter_rows3_f64: bad arguments");
+    if (n == 0) return PT_OK;
+    hipLaunchKernelGGL(k_scatter3, dim3(nblocks(3LL * n, 256)), dim3(256), 0, (hipStream_t)stream, n, idx, src, src_stride, dst);
+    return launch_check("pt_scatter_rows3_f64");
 }
 
 extern "C" int pt_copy_gated(long long n_words, int word_bytes, const void* src, void* dst, const int* gate,

@@ -442,6 +442,16 @@ def scatter_rows(idx, src, out):
     return out
 
 
+def clone_all(tensors):
+    """Copies of contiguous tensors (at most 8, of 4- or 8-byte words), one launch for all."""
+    torch = _torch()
+    out = [torch.empty_like(t) for t in tensors]
+    arrays = (_lib.CopyArray * len(out))(*[_lib.CopyArray(t.data_ptr(), o.data_ptr(), t.numel() * t.element_size())
+                                           for t, o in zip(tensors, out)])
+    _lib.check(_lib.load().pt_copy_arrays(len(out), arrays, _lib.stream_ptr()), "pt_copy_arrays")
+    return out
+
+
 class Reducer:
     """Deterministic FP64 sums on the device (pt_reduce_sum_f64)."""
 

@@ -37,7 +37,7 @@ import numpy as np
 
 from . import _lib
 from .atoms import ElementMap, host_box
-from .engine import (NeighborList, Reducer, acsf_adjoint_multi, acsf_forward_multi, acsf_run,
+from .engine import (NeighborList, Reducer, acsf_adjoint_multi, acsf_forward_multi, acsf_run, clone_all,
                      force_gather_transposed, gather_rows, scatter_rows)
 from .models import energy_grad_multi
 from .potential import PRECISION_MODES, NeuralNetworkPotential
@@ -213,12 +213,19 @@ class _DeviceMD:
         nl = self._nl.build(s.positions, s.atom_types, self.box, self.type_counts, with_rev=True)
         self._builds += 1
         perm = nl.perm
-        self.orig = perm.clone()                                     # internal -> input index
-        self.types = gather_rows(perm, s.atom_types.to(torch.int32).reshape(-1, 1)).reshape(-1).contiguous()
-        self.vel = gather_rows(perm, system.velocities.contiguous())
-        mass = system.masses.reshape(-1, 1).contiguous()
-        self.mass = gather_rows(perm, mass).reshape(-1).contiguous()
-        self.inv_mass = (1.0 / self.mass).contiguous()
+        f64 = dict(dtype=torch.float64, device=self.dev)
+        i32 = dict(dtype=torch.int32, device=self.dev)
+        self.vel, self.mass, self.inv_mass = torch.empty((n, 3), **f64), torch.empty(n, **f64), torch.empty(n, **f64)
+        self.orig, self.types = torch.empty(n, **i32), torch.empty(n, **i32)   # orig: internal -> input index
+        vel, mass, types = system.velocities, system.masses, s.atom_types.to(torch.int32).contiguous()
+        if vel.dtype != torch.float64 or mass.dtype != torch.float64:
+            raise TypeError(f"velocities and masses must be FP64, got {vel.dtype} and {mass.dtype}")
+        if vel.dim() != 2 or vel.shape[0] < n or vel.shape[1] != 3 or mass.numel() < n:
+            raise ValueError(f"velocities {tuple(vel.shape)} and masses {tuple(mass.shape)} do not fit {n} atoms")
+        vel, mass = vel.contiguous(), mass.contiguous()
+        _lib.check(_lib.load().pt_md_start(n, perm.data_ptr(), vel.data_ptr(), mass.data_ptr(), types.data_ptr(),
+                                           self._state(self.vel, self.mass, self.inv_mass, self.orig, self.types),
+                                           _lib.stream_ptr()), "pt_md_start")
         self.ref_pos = nl.pos4.clone()
         self.force = torch.zeros((n, 3), dtype=torch.float64, device=self.dev)
         self.force_new = torch.zeros_like(self.force)
@@ -406,9 +413,9 @@ class _DeviceMD:
 
     # ---- state snapshots (rewind) -------------------------------------------------
     def save_state(self) -> dict:
-        return {"pos": self._nl.pos4.clone(), "vel": self.vel.clone(), "force": self.force.clone(),
-                "orig": self.orig.clone(), "types": self.types.clone(), "mass": self.mass.clone(),
-                "inv_mass": self.inv_mass.clone()}
+        names = ("pos", "vel", "force", "orig", "types", "mass", "inv_mass")
+        return dict(zip(names, clone_all((self._nl.pos4, self.vel, self.force, self.orig, self.types, self.mass,
+                                          self.inv_mass))))
 
     def restore_state(self, st: dict) -> None:
         self.orig = st["orig"].clone()
@@ -585,7 +592,12 @@ class _DeviceMD:
         return scatter_rows(self.orig, internal.reshape(internal.shape[0], -1), out.reshape(out.shape[0], -1))
 
     def positions(self):
-        return self.to_input(self._nl.pos4[:, :3].contiguous())
+        import torch
+
+        out = torch.empty((self.n, 3), dtype=torch.float64, device=self.dev)
+        _lib.check(_lib.load().pt_scatter_rows3_f64(self.n, self.orig.data_ptr(), self._nl.pos4.data_ptr(), 4,
+                                                    out.data_ptr(), _lib.stream_ptr()), "pt_scatter_rows3_f64")
+        return out
 
 
 class System:
