@@ -559,6 +559,8 @@ int pt_md_berendsen(int n, double *vel, const double *ke_part, double dt, double
  * 1 / mass, perm[i] itself and type. */
 int pt_md_start(int n, const int *perm, const double *vel, const double *mass, const int *types,
                 const pt_md_state *out, pt_stream_t stream);
+/* inv[perm[i]] = i: the internal index of each input atom. */
+int pt_invert_perm(int n, const int *perm, int *inv, pt_stream_t stream);
 /* Up to PT_COPY_MAX copies (device, a multiple of 4 bytes each, ranges that do
  * not overlap) in one launch. */
 #define PT_COPY_MAX 8

@@ -131,6 +131,7 @@ _SIGS = {
                                     _c_ll, _vp, _vp, _c_int, _vp, _c_size, _vp]),
     "pt_nbr_mark_rows": (_c_int, [_c_int, _vp, _vp, _vp, _vp, _vp]),
     "pt_md_start": (_c_int, [_c_int, _vp, _vp, _vp, _vp, ctypes.POINTER(MDState), _vp]),
+    "pt_invert_perm": (_c_int, [_c_int, _vp, _vp, _vp]),
     "pt_copy_arrays": (_c_int, [_c_int, _vp, _vp]),
     "pt_scatter_rows3_f64": (_c_int, [_c_int, _vp, _vp, _c_int, _vp, _vp]),
     "pt_md_positions": (_c_int, [_c_int, _vp, _vp, _vp, _vp, _c_dbl, _vp, _vp, _vp, _c_dbl, _vp, _vp, _vp]),

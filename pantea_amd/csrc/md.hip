@@ -439,6 +439,12 @@ __global__ void k_md_start(int n, const int* __restrict__ perm, const double* __
     out.types[i] = types[j];
 }
 
+// inv[perm[i]] = i
+__global__ void k_invert(int n, const int* __restrict__ perm, int* __restrict__ inv) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) inv[perm[i]] = i;
+}
+
 struct CopyArgs {
     int n;
     const char* src[PT_COPY_MAX];
@@ -760,6 +766,13 @@ extern "C" int pt_md_start(int n, const int* perm, const double* vel, const doub
     if (n == 0) return PT_OK;
     hipLaunchKernelGGL(k_md_start, dim3(nblocks(n, 256)), dim3(256), 0, (hipStream_t)stream, n, perm, vel, mass, types, *out);
     return launch_check("pt_md_start");
+}
+
+extern "C" int pt_invert_perm(int n, const int* perm, int* inv, pt_stream_t stream) {
+    PT_REQUIRE(n >= 0 && perm && inv && perm != inv, "pt_invert_perm: bad arguments");
+    if (n == 0) return PT_OK;
+    hipLaunchKernelGGL(k_invert, dim3(nblocks(n, 256)), dim3(256), 0, (hipStream_t)stream, n, perm, inv);
+    return launch_check("pt_invert_perm");
 }
 
 extern "C" int pt_copy_arrays(int n, const pt_copy_array* arrays, pt_stream_t stream) {

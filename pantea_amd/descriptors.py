@@ -191,8 +191,7 @@ class ACSF:
         nl.build(structure.positions, structure.atom_types, structure.box_lengths,
                  structure.type_counts(), with_rev=False)
         tab = self.device_table(structure.element_map, dev)
-        inv = torch.as_tensor(nl.inverse_perm_host().astype(np.int32), device=dev)
-        return nl, tab, inv, PRECISIONS[precision]
+        return nl, tab, nl.inverse_perm(), PRECISIONS[precision]
 
     def __call__(self, structure, atom_index=None, precision: str = "float64"):
         """Descriptor values (n, n_sf) of the selected central atoms (acsf.py:47-86)."""

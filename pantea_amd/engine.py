@@ -134,6 +134,13 @@ class NeighborList:
         inv[self.perm_host] = np.arange(self.n)
         return inv
 
+    def inverse_perm(self):
+        """The internal index of each input atom (device)."""
+        inv = _torch().empty_like(self.perm)
+        _lib.check(_lib.load().pt_invert_perm(self.n, self.perm.data_ptr(), inv.data_ptr(), _lib.stream_ptr()),
+                   "pt_invert_perm")
+        return inv
+
     def type_block(self, t: int) -> Tuple[int, int]:
         """(begin, count) of the internal block of atom type t (1-based)."""
         b = self.type_offsets[t - 1]
@@ -442,13 +449,18 @@ def scatter_rows(idx, src, out):
     return out
 
 
-def clone_all(tensors):
+def copy_all(sources, targets) -> None:
     """Copies of contiguous tensors (at most 8, of 4- or 8-byte words), one launch for all."""
+    arrays = (_lib.CopyArray * len(sources))(*[_lib.CopyArray(t.data_ptr(), o.data_ptr(), t.numel() * t.element_size())
+                                               for t, o in zip(sources, targets)])
+    _lib.check(_lib.load().pt_copy_arrays(len(sources), arrays, _lib.stream_ptr()), "pt_copy_arrays")
+
+
+def clone_all(tensors):
+    """Clones of contiguous tensors by copy_all."""
     torch = _torch()
     out = [torch.empty_like(t) for t in tensors]
-    arrays = (_lib.CopyArray * len(out))(*[_lib.CopyArray(t.data_ptr(), o.data_ptr(), t.numel() * t.element_size())
-                                           for t, o in zip(tensors, out)])
-    _lib.check(_lib.load().pt_copy_arrays(len(out), arrays, _lib.stream_ptr()), "pt_copy_arrays")
+    copy_all(tensors, out)
     return out
 
 

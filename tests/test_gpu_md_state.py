@@ -41,3 +41,7 @@ def test_state_moves_equal_indexing(n):
     want = torch.empty_like(got)
     want[i] = pos4[:, :3]
     assert torch.equal(got, want)
+
+    inv = torch.full_like(perm, -1)
+    _lib.check(lib.pt_invert_perm(n, perm.data_ptr(), inv.data_ptr(), st), "invert")
+    assert torch.equal(inv[i], torch.arange(n, dtype=torch.int32, device="cuda"))
