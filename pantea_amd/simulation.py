@@ -37,7 +37,7 @@ import numpy as np
 
 from . import _lib
 from .atoms import ElementMap, host_box
-from .engine import (NeighborList, Reducer, acsf_adjoint_multi, acsf_forward_multi, acsf_run, clone_all,
+from .engine import (NeighborList, Reducer, acsf_adjoint_multi, acsf_forward_multi, acsf_run, clone_all, copy_all,
                      force_gather_transposed, gather_rows, scatter_rows)
 from .models import energy_grad_multi
 from .potential import PRECISION_MODES, NeuralNetworkPotential
@@ -239,11 +239,6 @@ class _DeviceMD:
 
         nl = self._nl
         self.pos_in = torch.empty_like(nl.pos4)
-        self.tmp3 = torch.empty((self.n, 3), dtype=torch.float64, device=self.dev)
-        self.tmp1 = torch.empty(self.n, dtype=torch.float64, device=self.dev)
-        self.tmpi = torch.empty(self.n, dtype=torch.int32, device=self.dev)
-        # the gated rebuild's permutation of v, F, m, 1/m, input index, type: 72 bytes per atom
-        self.tmp_state = torch.empty(self.n * 72, dtype=torch.uint8, device=self.dev)
         f = 2.0 if grow else 1.0
         self.row_bound = int(f * nl.max_row) + self.ROW_MARGIN
         cap = int(f * self.PAIR_MARGIN * nl.n_pairs) + 1024
@@ -359,31 +354,6 @@ class _DeviceMD:
         nl.max_row = self.row_bound
         nl.n_pairs = nl.cap
 
-    def _rebuild_gated(self) -> None:
-        """Skin check, then (behind its device flag) rebuild and reorder the state in place: no host read."""
-        lib = _lib.load()
-        nl = self._nl
-        st = _lib.stream_ptr()
-        box = host_box(self.box)
-        box_p = ctypes.cast(box, ctypes.c_void_p)
-        g = self.flag.data_ptr()
-        if self.skin > 0.0:
-            _lib.check(lib.pt_skin_check(self.n, nl.pos4.data_ptr(), self.ref_pos.data_ptr(), box_p, self.skin,
-                                         self.disp.data_ptr(), g, st), "pt_skin_check")
-        # without a skin the flag keeps the 1 it was created with: every step rebuilds, and
-        # neither the displacement check nor the reference positions are needed
-        _lib.check(lib.pt_copy_gated(4 * self.n, 8, nl.pos4.data_ptr(), self.pos_in.data_ptr(), g, st),
-                   "pt_copy_gated")
-        self._build_gated(box_p, st)
-        arrays = (_lib.PermuteArray * 6)(*[_lib.PermuteArray(b.data_ptr(), w, wb) for b, w, wb in (
-            (self.vel, 3, 8), (self.force, 3, 8), (self.mass, 1, 8), (self.inv_mass, 1, 8), (self.orig, 1, 4),
-            (self.types, 1, 4))])
-        _lib.check(lib.pt_permute_state_gated(self.n, nl.perm.data_ptr(), 6, arrays, self.tmp_state.data_ptr(),
-                                              self.tmp_state.numel(), g, st), "pt_permute_state_gated")
-        if self.skin > 0.0:
-            _lib.check(lib.pt_copy_gated(4 * self.n, 8, nl.pos4.data_ptr(), self.ref_pos.data_ptr(), g, st),
-                       "pt_copy_gated")
-
     def lists_ok(self) -> bool:
         """Whether every gated build since the last check fitted the row bound and the
         list arrays (a host read: call where the host synchronises anyway)."""
@@ -450,9 +420,9 @@ class _DeviceMD:
         if not (self.gated and self.use_graph) or self.timers is not None:
             self._graph = None
             if self.gated:
-                self._step_fused(*args)
+                self._step_gated(*args, swap=True)
             else:
-                self._step_body(*args, swap=True)
+                self._step_sync(*args)
             return
         import torch
 
@@ -460,10 +430,10 @@ class _DeviceMD:
             self._graph.replay()
             return
         self._graph = None
-        self._step_body(*args, swap=False)      # this step, run eagerly (sizes every buffer)
+        self._step_gated(*args, swap=False)     # this step, run eagerly (sizes every buffer)
         g = torch.cuda.CUDAGraph()
         with torch.cuda.graph(g):
-            self._step_body(*args, swap=False)  # recorded, not run
+            self._step_gated(*args, swap=False)  # recorded, not run
         self._graph, self._graph_key = g, self._key(args)
 
     def _key(self, args) -> tuple:
@@ -471,20 +441,20 @@ class _DeviceMD:
         ff = self.ff
         nl = self._nl
         bufs = (nl.pos4, nl.perm, nl.row_off, nl.nbr, nl.rev, nl.ws, self.vel, self.force, self.force_new,
-                self.mass, self.inv_mass, self.orig, self.types, self.ref_pos, self.pos_in, self.tmp3, self.tmp1,
-                self.tmpi, self.tmp_state, self.flag, self.totals, self.disp, self.reducer.ws, self.reducer.out, ff.G, ff.dEdG,
-                ff.e_atom, ff.f_self, ff.edge)
+                self.mass, self.inv_mass, self.orig, self.types, *(self._other or ()), self.ref_pos, self.pos_in,
+                self.flag, self.totals, self.disp, self.reducer.ws, ff.G, ff.dEdG, ff.e_atom, ff.f_self, ff.edge)
         return (args[:3], id(args[3]), id(ff), id(ff.mlps), nl.cap, self.row_bound,
                 tuple(0 if b is None else b.data_ptr() for b in bufs))
 
     def _state(self, *arrays) -> "_lib.MDState":
         return _lib.MDState(*(a.data_ptr() for a in arrays))
 
-    def _step_fused(self, dt: float, integrator: str, force_mode: str,
-                    thermostat: Optional[BrendsenThermostat]) -> None:
+    def _step_gated(self, dt: float, integrator: str, force_mode: str,
+                    thermostat: Optional[BrendsenThermostat], swap: bool) -> None:
         """A gated step with its own work in three calls (pt_md_positions, pt_md_velocities,
         pt_md_berendsen): the reordered state goes to a second set of arrays, which then
-        changes places with the first."""
+        changes places with the first (swap) or is copied back (captured steps: a replayed
+        step keeps its buffers)."""
         import torch
 
         lib = _lib.load()
@@ -512,17 +482,18 @@ class _DeviceMD:
                                         self._state(*new), self.force.data_ptr(), self.force_new.data_ptr(),
                                         int(physical), dt, nl.pos4.data_ptr(),
                                         self.ref_pos.data_ptr() if skin else None, ke, st), "pt_md_velocities")
-        self.vel, self.mass, self.inv_mass, self.orig, self.types = new
-        self._other = now
-        self.force, self.force_new = self.force_new, self.force
         if thermostat is not None:
-            _lib.check(lib.pt_md_berendsen(self.n, self.vel.data_ptr(), ke, dt, thermostat.time_constant,
+            _lib.check(lib.pt_md_berendsen(self.n, new[0].data_ptr(), ke, dt, thermostat.time_constant,
                                            thermostat.target_temperature, KB, st), "pt_md_berendsen")
+        if swap:
+            self.vel, self.mass, self.inv_mass, self.orig, self.types = new
+            self._other = now
+            self.force, self.force_new = self.force_new, self.force
+        else:
+            copy_all((*new, self.force_new), (*now, self.force))
 
-    def _step_body(self, dt: float, integrator: str, force_mode: str, thermostat: Optional[BrendsenThermostat],
-                   swap: bool):
-        """The step in place: structures without a box (swap), and captured steps (a replayed
-        step keeps its buffers)."""
+    def _step_sync(self, dt: float, integrator: str, force_mode: str, thermostat: Optional[BrendsenThermostat]) -> None:
+        """A step that decides on the rebuild on the host (structures without a box, sync_free=False)."""
         lib = _lib.load()
         inv_m = self.inv_mass.data_ptr() if integrator == "physical" else None
         box = host_box(self.box)
@@ -531,10 +502,7 @@ class _DeviceMD:
                                            self.force.data_ptr(), inv_m, dt, box_p, _lib.stream_ptr()),
                    "pt_verlet_positions")
         self._mark("nbr_build", True)
-        if self.gated:
-            self._rebuild_gated()
-            inv_m = self.inv_mass.data_ptr() if integrator == "physical" else None
-        elif self._stale():
+        if self._stale():
             self._rebuild_sync()
             inv_m = self.inv_mass.data_ptr() if integrator == "physical" else None
         self._mark("nbr_build", False)
@@ -542,10 +510,7 @@ class _DeviceMD:
         _lib.check(lib.pt_verlet_velocities(self.n, self.vel.data_ptr(), self.force.data_ptr(),
                                             self.force_new.data_ptr(), inv_m, dt, _lib.stream_ptr()),
                    "pt_verlet_velocities")
-        if swap:
-            self.force, self.force_new = self.force_new, self.force
-        else:   # a replayed step keeps its buffers
-            self.force.copy_(self.force_new)
+        self.force, self.force_new = self.force_new, self.force
         if thermostat is not None:
             ke = self.reducer.kinetic(self.vel, self.mass)
             _lib.check(lib.pt_berendsen_rescale(self.n, self.vel.data_ptr(), ke.data_ptr(), dt,
