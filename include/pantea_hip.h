@@ -173,11 +173,20 @@ int pt_nbr_build(int n, const double *pos, int pos_stride, const int *types, int
  *    read, i.e. the max_row it passes them) exceeds 256: a list with a row
  *    over row_limit is unusable either way, and totals[1] reports it.
  * No synchronisation and no host read: every launch is enqueued whatever the
- * data, so the sequence can be replayed or captured. */
+ * data, so the sequence can be replayed or captured.
+ * A list that does not fit (more pairs than cap, or a row over 256 entries
+ * without the second pass) is not written, while row_off holds the offsets it
+ * would have: read the totals before the rows.  pt_nbr_build_async_or_empty
+ * is for callers whose kernels walk the list before the totals are known (the
+ * MD step): the rows of such a list are all empty (row_off holds zeros). */
 int pt_nbr_build_async(int n, const double *pos, int pos_stride, const int *types, int n_types,
                        const double *box, double rc, int *perm, double *pos4, long long *row_off,
                        int *nbr, int *rev, long long cap, const int *gate, long long *totals,
                        int row_limit, void *ws, size_t ws_bytes, pt_stream_t stream);
+int pt_nbr_build_async_or_empty(int n, const double *pos, int pos_stride, const int *types, int n_types,
+                                const double *box, double rc, int *perm, double *pos4, long long *row_off,
+                                int *nbr, int *rev, long long cap, const int *gate, long long *totals,
+                                int row_limit, void *ws, size_t ws_bytes, pt_stream_t stream);
 
 /* Mark the closed neighbourhoods of n_sel atoms: flags[s] = 1 and
  * flags[j] = 1 for every j in the row of s (flags: device, n entries, not

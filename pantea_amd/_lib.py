@@ -129,6 +129,8 @@ _SIGS = {
                               _c_ll, ctypes.POINTER(_c_ll), ctypes.POINTER(_c_int), _vp, _c_size, _vp]),
     "pt_nbr_build_async": (_c_int, [_c_int, _vp, _c_int, _vp, _c_int, _vp, _c_dbl, _vp, _vp, _vp, _vp, _vp,
                                     _c_ll, _vp, _vp, _c_int, _vp, _c_size, _vp]),
+    "pt_nbr_build_async_or_empty": (_c_int, [_c_int, _vp, _c_int, _vp, _c_int, _vp, _c_dbl, _vp, _vp, _vp, _vp, _vp,
+                                             _c_ll, _vp, _vp, _c_int, _vp, _c_size, _vp]),
     "pt_nbr_mark_rows": (_c_int, [_c_int, _vp, _vp, _vp, _vp, _vp]),
     "pt_md_start": (_c_int, [_c_int, _vp, _vp, _vp, _vp, ctypes.POINTER(MDState), _vp]),
     "pt_invert_perm": (_c_int, [_c_int, _vp, _vp, _vp]),

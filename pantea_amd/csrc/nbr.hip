@@ -22,6 +22,7 @@
 // the CSR arrays and pairs every edge with its reverse.  A list whose longest
 // row exceeds kStageW takes a second candidate pass instead.
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <type_traits>
 #include <cstdio>
@@ -917,11 +918,20 @@ __global__ __launch_bounds__(1024) void k_scan_top(const int* __restrict__ gate,
     if (threadIdx.x == 0) store_totals(carry, mx[0], total_and_max, totals);
 }
 
+// A build that nobody waits for may not write its list: more pairs than the arrays hold, or a
+// row beyond the stage without a second pass.  With keep_cap and keep_row set to those
+// bounds, such a build's rows are all empty, so that what is launched after it reads and writes
+// nothing; the totals still tell.
+__device__ __forceinline__ bool rows_kept(long long pairs, int max_row, long long keep_cap, int keep_row) {
+    return pairs <= keep_cap && max_row <= keep_row;
+}
+
 __global__ __launch_bounds__(256) void k_scan_down(const int* __restrict__ gate, int n, const int* counts,
                                                    const long long* psum, const long long* total_and_max,
-                                                   long long* row_off) {
+                                                   long long keep_cap, int keep_row, long long* row_off) {
     if (gated_off(gate)) return;
     __shared__ long long buf[256];
+    const bool kept = rows_kept(total_and_max[0], (int)total_and_max[1], keep_cap, keep_row);
     constexpr int kPer = kScanBlock / 256;
     int base = blockIdx.x * kScanBlock + threadIdx.x * kPer;
     long long loc[kPer];
@@ -942,9 +952,9 @@ __global__ __launch_bounds__(256) void k_scan_down(const int* __restrict__ gate,
     long long pre = psum[blockIdx.x] + buf[threadIdx.x] - s;
     for (int k = 0; k < kPer; ++k) {
         int idx = base + k;
-        if (idx < n) row_off[idx] = pre + loc[k];
+        if (idx < n) row_off[idx] = kept ? pre + loc[k] : 0;
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) row_off[n] = total_and_max[0];
+    if (blockIdx.x == 0 && threadIdx.x == 0) row_off[n] = kept ? total_and_max[0] : 0;
 }
 
 // Up to kOffsetsSmall rows in one workgroup (a contiguous piece per thread): one launch
@@ -952,8 +962,8 @@ __global__ __launch_bounds__(256) void k_scan_down(const int* __restrict__ gate,
 constexpr int kOffsetsSmall = 8192;
 
 __global__ __launch_bounds__(1024) void k_offsets_small(const int* __restrict__ gate, int n,
-                                                        const int* __restrict__ counts,
-                                                        long long* __restrict__ row_off,
+                                                        const int* __restrict__ counts, long long keep_cap,
+                                                        int keep_row, long long* __restrict__ row_off,
                                                         long long* __restrict__ total_and_max,
                                                         long long* __restrict__ totals) {
     if (gated_off(gate)) return;
@@ -971,17 +981,18 @@ __global__ __launch_bounds__(1024) void k_offsets_small(const int* __restrict__ 
     }
     long long run = block_exclusive(sum, wtot, all);
 #pragma unroll
-    for (int q = 0; q < PER; ++q) {
-        if (q < per && b + q < n) row_off[b + q] = run;
-        run += c[q];
-    }
-#pragma unroll
     for (int off = 1; off < kWave; off <<= 1) m = max(m, __shfl_xor(m, off, kWave));
     if ((threadIdx.x & (kWave - 1)) == 0) wmax[threadIdx.x >> 6] = m;
     __syncthreads();
+    for (int q = 0; q < 16; ++q) m = max(m, wmax[q]);
+    const bool kept = rows_kept(all, m, keep_cap, keep_row);
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        if (q < per && b + q < n) row_off[b + q] = kept ? run : 0;
+        run += c[q];
+    }
     if (threadIdx.x == 0) {
-        for (int q = 1; q < 16; ++q) m = max(m, wmax[q]);
-        row_off[n] = all;
+        row_off[n] = kept ? all : 0;
         store_totals(all, m, total_and_max, totals);
     }
 }
@@ -1214,10 +1225,11 @@ struct BuildOut {
 // The whole build.  host_totals != nullptr: synchronous (the host reads the
 // pair count and the longest row and decides on the second pass); otherwise
 // every launch is enqueued unconditionally, behind `gate`, and the totals go
-// to dev_totals.
+// to dev_totals; empty_rows: a list that it does not write has empty rows.
 int build_impl(int n, const double* pos, int pos_stride, const int* types, int n_types, const double* box,
                double rc, const BuildOut& o, void* ws, size_t ws_bytes, const int* gate,
-               long long* host_totals, long long* dev_totals, int row_limit, hipStream_t stream) {
+               long long* host_totals, long long* dev_totals, int row_limit, bool empty_rows,
+               hipStream_t stream) {
     WsLayout L = ws_layout(n, n_types);
     PT_REQUIRE(ws_bytes >= L.total, "pt_nbr_build: workspace too small (%zu < %zu)", ws_bytes, L.total);
     char* w = (char*)ws;
@@ -1358,13 +1370,16 @@ int build_impl(int n, const double* pos, int pos_stride, const int* types, int n
     if (int rcode = launch_check("k_nbr_cell<stage>")) return rcode;
     const int nsb = (n + kScanBlock - 1) / kScanBlock;
     long long* tot_max = (long long*)misc;
+    const long long keep_cap = empty_rows ? o.cap : LLONG_MAX;
+    const int keep_row = empty_rows && row_limit <= kStageW ? kStageW : INT_MAX;
     if (n <= kOffsetsSmall) {
-        hipLaunchKernelGGL(k_offsets_small, dim3(1), dim3(1024), 0, stream, gate, n, (const int*)counts, o.row_off,
-                           tot_max, dev_totals);
+        hipLaunchKernelGGL(k_offsets_small, dim3(1), dim3(1024), 0, stream, gate, n, (const int*)counts, keep_cap,
+                           keep_row, o.row_off, tot_max, dev_totals);
     } else {
         hipLaunchKernelGGL(k_scan_reduce, dim3(nsb), dim3(256), 0, stream, gate, n, counts, psum, pmax);
         hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, stream, gate, nsb, psum, pmax, tot_max, dev_totals);
-        hipLaunchKernelGGL(k_scan_down, dim3(nsb), dim3(256), 0, stream, gate, n, counts, psum, tot_max, o.row_off);
+        hipLaunchKernelGGL(k_scan_down, dim3(nsb), dim3(256), 0, stream, gate, n, counts, psum, tot_max, keep_cap,
+                           keep_row, o.row_off);
     }
     if (int rcode = launch_check("row offsets")) return rcode;
     // the compaction checks the totals itself, so it is queued before the host
@@ -1428,7 +1443,7 @@ extern "C" int pt_nbr_build(int n, const double* pos, int pos_stride, const int*
     BuildOut o{perm, pos4, row_off, nbr, rev, cap};
     long long tm[2] = {0, 0};
     const int rc_ = build_impl(n, pos, pos_stride, types, n_types, box, rc, o, ws, ws_bytes, nullptr, tm,
-                               nullptr, INT_MAX, (hipStream_t)stream_);
+                               nullptr, INT_MAX, false, (hipStream_t)stream_);
     if (rc_ == PT_OK || rc_ == PT_ERR_CAPACITY) {
         *n_pairs = tm[0];
         *max_row = (int)tm[1];
@@ -1436,10 +1451,10 @@ extern "C" int pt_nbr_build(int n, const double* pos, int pos_stride, const int*
     return rc_;
 }
 
-extern "C" int pt_nbr_build_async(int n, const double* pos, int pos_stride, const int* types, int n_types,
-                                  const double* box, double rc, int* perm, double* pos4, long long* row_off,
-                                  int* nbr, int* rev, long long cap, const int* gate, long long* totals,
-                                  int row_limit, void* ws, size_t ws_bytes, pt_stream_t stream_) {
+static int build_async(int n, const double* pos, int pos_stride, const int* types, int n_types, const double* box,
+                       double rc, int* perm, double* pos4, long long* row_off, int* nbr, int* rev, long long cap,
+                       const int* gate, long long* totals, int row_limit, bool empty_rows, void* ws, size_t ws_bytes,
+                       pt_stream_t stream_) {
     PT_REQUIRE(n >= 1, "pt_nbr_build_async: n must be >= 1 (got %d)", n);
     PT_REQUIRE(n_types >= 1 && n_types <= kMaxTypes, "pt_nbr_build_async: n_types must be in [1, %d]",
                kMaxTypes);
@@ -1451,7 +1466,23 @@ extern "C" int pt_nbr_build_async(int n, const double* pos, int pos_stride, cons
     PT_REQUIRE((const void*)pos != (const void*)pos4, "pt_nbr_build_async: pos and pos4 must not alias");
     BuildOut o{perm, pos4, row_off, nbr, rev, cap};
     return build_impl(n, pos, pos_stride, types, n_types, box, rc, o, ws, ws_bytes, gate, nullptr, totals,
-                      row_limit, (hipStream_t)stream_);
+                      row_limit, empty_rows, (hipStream_t)stream_);
+}
+
+extern "C" int pt_nbr_build_async(int n, const double* pos, int pos_stride, const int* types, int n_types,
+                                  const double* box, double rc, int* perm, double* pos4, long long* row_off,
+                                  int* nbr, int* rev, long long cap, const int* gate, long long* totals,
+                                  int row_limit, void* ws, size_t ws_bytes, pt_stream_t stream) {
+    return build_async(n, pos, pos_stride, types, n_types, box, rc, perm, pos4, row_off, nbr, rev, cap, gate, totals,
+                       row_limit, false, ws, ws_bytes, stream);
+}
+
+extern "C" int pt_nbr_build_async_or_empty(int n, const double* pos, int pos_stride, const int* types, int n_types,
+                                           const double* box, double rc, int* perm, double* pos4, long long* row_off,
+                                           int* nbr, int* rev, long long cap, const int* gate, long long* totals,
+                                           int row_limit, void* ws, size_t ws_bytes, pt_stream_t stream) {
+    return build_async(n, pos, pos_stride, types, n_types, box, rc, perm, pos4, row_off, nbr, rev, cap, gate, totals,
+                       row_limit, true, ws, ws_bytes, stream);
 }
 
 extern "C" int pt_nbr_mark_rows(int n_sel, const int* sel, const long long* row_off, const int* nbr,

@@ -6,7 +6,7 @@ The state of a System lives on the device in the neighbour list's internal
 order (atoms grouped by type and cell).  One MD step is
 
   pt_md_positions      x <- wrap(x + v dt + 1/2 a dt^2)
-  [pt_nbr_build_async   when the list is stale]
+  [pt_nbr_build_async_or_empty  when the list is stale]
   descriptors -> MLP -> adjoint -> force gather   (the potential's kernels)
   pt_md_velocities     v <- v + 1/2 (a + a') dt, the state into the list's order
   [pt_md_berendsen]
@@ -22,7 +22,7 @@ skin (no pair can have moved by more); the descriptor kernels re-apply the
 exact mask (r <= rc, r > 0), so every step sees exactly the reference's
 neighbour set.  In a periodic box that decision is taken on the device
 (as pt_skin_check; without a skin every step rebuilds) and the rebuild runs
-behind its flag (pt_nbr_build_async, the reorder of the state too), so a step
+behind its flag (pt_nbr_build_async_or_empty, the reorder of the state too), so a step
 never waits for the GPU; the list's totals are verified whenever the host
 reads the state.
 """
@@ -160,7 +160,7 @@ class _DeviceMD:
     list switches cutoff when the driver does (``use``).
 
     Periodic boxes run the step without any host read ("gated" step): the
-    skin check sets a device flag, and the rebuild (pt_nbr_build_async) and
+    skin check sets a device flag, and the rebuild (pt_nbr_build_async_or_empty) and
     the permutation of the state into the new order are launched every step
     behind that flag, so the host never waits for the GPU.  The list's
     totals stay on the device; they are checked when the host synchronises
@@ -341,15 +341,15 @@ class _DeviceMD:
         self.row_bound = max(getattr(self, "row_bound", 0), nl.max_row)
 
     def _build_gated(self, box_p, st) -> None:
-        """The list for the positions in pos_in, behind the device flag: no host read."""
+        """The list for the positions in pos_in, behind the device flag: no host read.  The step's
+        kernels walk it before its totals are checked, so one that does not fit has empty rows."""
         lib = _lib.load()
         nl = self._nl
-        _lib.check(lib.pt_nbr_build_async(self.n, self.pos_in.data_ptr(), 4, self.types.data_ptr(), nl.n_types,
-                                          box_p, nl.r_cutoff, nl.perm.data_ptr(), nl.pos4.data_ptr(),
-                                          nl.row_off.data_ptr(), nl.nbr.data_ptr(), nl.rev.data_ptr(), nl.cap,
-                                          self.flag.data_ptr(), self.totals.data_ptr(), int(self.row_bound),
-                                          nl.ws.data_ptr(), nl.ws.numel(), st),
-                   "pt_nbr_build_async")
+        _lib.check(lib.pt_nbr_build_async_or_empty(
+            self.n, self.pos_in.data_ptr(), 4, self.types.data_ptr(), nl.n_types, box_p, nl.r_cutoff,
+            nl.perm.data_ptr(), nl.pos4.data_ptr(), nl.row_off.data_ptr(), nl.nbr.data_ptr(), nl.rev.data_ptr(), nl.cap,
+            self.flag.data_ptr(), self.totals.data_ptr(), int(self.row_bound), nl.ws.data_ptr(), nl.ws.numel(), st),
+            "pt_nbr_build_async_or_empty")
         # the descriptor kernels stage rows up to the bound; buffers are sized for the capacity
         nl.max_row = self.row_bound
         nl.n_pairs = nl.cap
