@@ -103,7 +103,8 @@ class _Batch:
 
     def __init__(self, ld: int, fdt, dev):
         self.ld, self.fdt, self.dev = ld, fdt, dev
-        self.atoms = self.edges = self.structs = 0
+        self.atoms = self.structs = 0
+        self.edges = -1   # (arrays for a batch without any edge too)
 
     def reserve(self, atoms: int, edges: int, structs: int) -> None:
         import torch
