@@ -285,9 +285,11 @@ class StudentTrainer:
             yield part
 
     def _plan(self, snaps: Sequence[Snapshot]):
-        """The plan words of pt_train_batch_*, the atom offsets of the elements, the atom and edge totals."""
-        ns, els = len(snaps), self.pot.elements
-        ne = len(els)
+        """The elements that the snapshots hold (a list has at most 8 types, the potential may have
+        more), the plan words of pt_train_batch_*, the atom offsets of the elements, the atom and edge totals."""
+        held = {el for sn in snaps for el, _, _ in sn.blocks}
+        els = [el for el in self.pot.elements if el in held]
+        ns, ne = len(snaps), len(els)
         rec = np.zeros((ns, 11), dtype=np.int64)
         real = rec.view(np.float64)
         begin = np.full((ns, ne), 1 << 30, dtype=np.int64)
@@ -311,21 +313,21 @@ class StudentTrainer:
         first = [np.concatenate([[0], np.cumsum(x.reshape(-1))]) for x in (atoms, edges)]
         words = np.concatenate([rec.reshape(-1), begin.reshape(-1), edge0.reshape(-1), *first])
         assert words.size == _lib.load().pt_train_batch_words(ns, ne)
-        return words, first[0][::ns], int(first[0][-1]), int(first[1][-1])
+        return els, words, first[0][::ns], int(first[0][-1]), int(first[1][-1])
 
     def _accumulate_batch(self, snaps: Sequence[Snapshot], scale: float) -> None:
         import torch
 
         lib, st, B = _lib.load(), _lib.stream_ptr(), self.batch
-        words, at, n, pairs = self._plan(snaps)
-        ns, ne = len(snaps), len(self.pot.elements)
+        els, words, at, n, pairs = self._plan(snaps)
+        ns, ne = len(snaps), len(els)
         B.reserve(n, pairs, ns)
         plan = torch.from_numpy(words).to(self.dev)
         _lib.check(lib.pt_train_batch_assemble(
             ns, ne, plan.data_ptr(), n, self.ld, self.g_prec, B.pos4.data_ptr(), B.row_off.data_ptr(),
             B.nbr.data_ptr(), B.rev.data_ptr(), B.G.data_ptr(), B.f_ref.data_ptr(), B.box_id.data_ptr(),
             B.boxes.data_ptr(), st), "pt_train_batch_assemble")
-        blocks = [(el, int(at[e]), int(at[e + 1] - at[e])) for e, el in enumerate(self.pot.elements) if at[e + 1] > at[e]]
+        blocks = [(el, int(at[e]), int(at[e + 1] - at[e])) for e, el in enumerate(els)]
         tab = {el: self._table(snaps[0], el) for el, _, _ in blocks}
         energy_grad_multi(self.mlp_mode, [(self.mlps[el], cnt, B.G[b:], B.e_atom[b:], B.dEdG[b:])
                                           for el, b, cnt in blocks], self.ld, self.g_prec)
