@@ -31,7 +31,7 @@ from __future__ import annotations
 
 import ctypes
 from pathlib import Path
-from typing import Optional
+from typing import NamedTuple, Optional
 
 import numpy as np
 
@@ -52,6 +52,17 @@ class BrendsenThermostat:
     def __init__(self, target_temperature: float, time_constant: float):
         self.target_temperature = float(target_temperature)
         self.time_constant = float(time_constant)
+
+
+class _Rescale(NamedTuple):
+    """A thermostat's values as a step is given them (its object may change afterwards)."""
+
+    target_temperature: float
+    time_constant: float
+
+    @classmethod
+    def of(cls, thermostat) -> Optional["_Rescale"]:
+        return None if thermostat is None else cls(thermostat.target_temperature, thermostat.time_constant)
 
 
 class _ForceField:
@@ -416,7 +427,7 @@ class _DeviceMD:
         """One MD step.  With ``use_graph`` (gated steps only), the step's launch sequence is
         captured once into a HIP graph and replayed; it is captured again whenever a buffer
         or a parameter of the step changes."""
-        args = (dt, integrator, force_mode, thermostat)
+        args = (dt, integrator, force_mode, _Rescale.of(thermostat))
         if not (self.gated and self.use_graph) or self.timers is not None:
             self._graph = None
             if self.gated:
@@ -443,14 +454,14 @@ class _DeviceMD:
         bufs = (nl.pos4, nl.perm, nl.row_off, nl.nbr, nl.rev, nl.ws, self.vel, self.force, self.force_new,
                 self.mass, self.inv_mass, self.orig, self.types, *(self._other or ()), self.ref_pos, self.pos_in,
                 self.flag, self.totals, self.disp, self.reducer.ws, ff.G, ff.dEdG, ff.e_atom, ff.f_self, ff.edge)
-        return (args[:3], id(args[3]), id(ff), id(ff.mlps), nl.cap, self.row_bound,
+        return (args, id(ff), id(ff.mlps), nl.cap, self.row_bound,
                 tuple(0 if b is None else b.data_ptr() for b in bufs))
 
     def _state(self, *arrays) -> "_lib.MDState":
         return _lib.MDState(*(a.data_ptr() for a in arrays))
 
     def _step_gated(self, dt: float, integrator: str, force_mode: str,
-                    thermostat: Optional[BrendsenThermostat], swap: bool) -> None:
+                    thermostat: Optional[_Rescale], swap: bool) -> None:
         """A gated step with its own work in three calls (pt_md_positions, pt_md_velocities,
         pt_md_berendsen): the reordered state goes to a second set of arrays, which then
         changes places with the first (swap) or is copied back (captured steps: a replayed
@@ -492,7 +503,7 @@ class _DeviceMD:
         else:
             copy_all((*new, self.force_new), (*now, self.force))
 
-    def _step_sync(self, dt: float, integrator: str, force_mode: str, thermostat: Optional[BrendsenThermostat]) -> None:
+    def _step_sync(self, dt: float, integrator: str, force_mode: str, thermostat: Optional[_Rescale]) -> None:
         """A step that decides on the rebuild on the host (structures without a box, sync_free=False)."""
         lib = _lib.load()
         inv_m = self.inv_mass.data_ptr() if integrator == "physical" else None
@@ -522,7 +533,7 @@ class _DeviceMD:
         """``steps`` steps.  Gated steps are verified every ``check_every`` steps (and
         whenever the host reads the state): a stretch whose lists overflowed is redone
         from its checkpoint with larger bounds."""
-        args = (dt, integrator, force_mode, thermostat)
+        args = (dt, integrator, force_mode, _Rescale.of(thermostat))
         for _ in range(int(steps)):
             if self._args is not None and self._args != args:
                 self.verify()
