@@ -454,8 +454,9 @@ class _DeviceMD:
         bufs = (nl.pos4, nl.perm, nl.row_off, nl.nbr, nl.rev, nl.ws, self.vel, self.force, self.force_new,
                 self.mass, self.inv_mass, self.orig, self.types, *(self._other or ()), self.ref_pos, self.pos_in,
                 self.flag, self.totals, self.disp, self.reducer.ws, ff.G, ff.dEdG, ff.e_atom, ff.f_self, ff.edge)
-        return (args, id(ff), id(ff.mlps), nl.cap, self.row_bound,
-                tuple(0 if b is None else b.data_ptr() for b in bufs))
+        # (a field lives as long as this state; its networks may be replaced)
+        nets = tuple((m.packed.data_ptr(), m.scale.data_ptr(), bytes(m.desc)) for m in ff.mlps.values())
+        return (args, id(ff), nets, nl.cap, self.row_bound, tuple(0 if b is None else b.data_ptr() for b in bufs))
 
     def _state(self, *arrays) -> "_lib.MDState":
         return _lib.MDState(*(a.data_ptr() for a in arrays))
