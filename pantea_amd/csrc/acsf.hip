@@ -1364,15 +1364,28 @@ void k_acsf_team(KArgs a) {
 // row is staged and where sums are added: radial groups go by halves, the pair steps of
 // all angular groups in turn, and a group's table words are loaded while the one before
 // runs.  (With barriers around every group FP64 took 31 and 37 us at 96 centres, FP32 27 and 33 at 384.)
-// Measured, us per launch, wavefronts per centre 1 | 4 | 8 (52 functions at 12 Bohr,
-// ~110 neighbours; 34 at 8 Bohr, ~32):
-//   12 Bohr FP64 forward  96 centres 53.4 | 23.9 | 18.8   512 57.4 | 28.3 | 27.7   640 57.9 | 32.6 | 38.0   1,536 68.6 | 55.4   2,048 69.2 | 69.7
-//   12 Bohr FP64 adjoint  96 centres 65.8 | 29.8 | 24.5   512 70.5 | 37.0 | 35.8   640 70.9 | 43.5 | 49.8   1,792 89.4 | 83.0   2,048 90.3 | 92.5
-//   12 Bohr FP64 tangent  96 centres 63.3 | 28.3 | 23.0   300 67.2 | 33.9 | 42.5   1,536 85.4 | 75.9
-//   12 Bohr FP32 adjoint  96 centres 48.2 | 22.5 | 18.5   512 51.4 | 26.0 | 23.8   640 51.9 | 28.5 | 34.5   1,792 58.1 | 52.5   2,048 58.5 | 57.7
-//   8 Bohr FP32 forward   96 centres 14.8 | 12.0 | 11.9   768 15.9 | 15.2          1,024 16.1 | 16.6
+// Measured, us per launch (HIP events over 40 launches in a row), wavefronts per centre
+// 1 | 4 | 8 (52 functions at 12 Bohr, ~110 neighbours; 34 at 8 Bohr, ~32):
+//   12 Bohr FP64 forward  96 centres 60.0 | 24.9 | 19.8   512 66.0 | 30.5 | 29.7   640 66.1 | 34.5 | 38.4   1,792 78.7 | 66.5
+//   12 Bohr FP64 adjoint  96 centres 73.3 | 31.7 | 25.0   512 81.4 | 40.7 | 38.1   640 81.7 | 46.6 | 50.8   1,792 102 | 92.1
+//   12 Bohr FP64 tangent  96 centres 70.8 | 30.1 | 23.6   256 75.2 | 31.1 | 25.4   512 78.3 | 39.2 | 46.4   1,792 98.1 | 93.8   2,048 102 | 106
+//   12 Bohr FP32 forward  96 centres 43.1 | 18.8 | 14.8   512 47.4 | 21.3 | 19.7   640 47.4 | 22.8 | 23.6   1,792 50.7 | 40.6
+//   12 Bohr FP32 adjoint  96 centres 53.4 | 23.5 | 18.6   512 58.8 | 27.5 | 25.1   640 59.1 | 29.7 | 35.3   1,792 66.5 | 55.7
+//   12 Bohr FP32 tangent  96 centres 54.2 | 22.7 | 17.5   512 60.3 | 26.1 | 23.8   640 59.7 | 28.3 | 32.9   1,792 64.2 | 54.6
+//   8 Bohr FP32 forward   96 centres 13.0 | 10.1 | 9.3    768 13.8 | 12.4          1,280 15.5 | 15.6
+//   8 Bohr FP64 adjoint   96 centres 21.2 | 15.0 | 14.1   768 22.5 | 19.5          1,280 26.3 | 29.7
 // (teams of 2 win 5 to 15 % between 1,536 and 2,048 centres: not worth a third set of kernels.)
+// The general table class has no teams of 8, and its FP64 kernels' registers leave two teams of 4
+// to a CU, not four: long rows gain up to 1,280 centres, short ones while all teams are
+// resident.  Cosine cutoff, 1 | 4:
+//   12 Bohr FP64 forward  512 centres 104 | 49.7   640 104 | 73.4   1,280 122 | 116   1,536 124 | 130
+//   12 Bohr FP64 adjoint  512 centres 146 | 72.1   640 146 | 107    1,280 176 | 170   1,536 180 | 191
+//   12 Bohr FP32 adjoint  512 centres 65.3 | 32.9                   1,792 74.0 | 67.9
+//   8 Bohr FP64 forward   512 centres 28.2 | 25.5  640 27.8 | 40.7
+//   8 Bohr FP64 adjoint   512 centres 39.0 | 34.8  640 38.6 | 56.3
+//   8 Bohr FP32 adjoint   768 centres 18.6 | 18.2
 constexpr int kTeam8 = 512, kTeam8Tan64 = 256, kTeamLong = 1792, kTeamShort = 768, kTeamRow = 80;
+constexpr int kTeamLongGeneral64 = 1280, kTeamShortGeneral64 = 512;
 
 template <typename R, int MODE, int KIND>
 int launch(KArgs a, hipStream_t stream) {
@@ -1398,10 +1411,11 @@ int launch(KArgs a, hipStream_t stream) {
     };
     auto some_team = [&]() {
         constexpr std::integral_constant<int, 4> w4{};
-        if (a.cap < kTeamRow) return team(w4, kTeamShort);
+        constexpr bool general64 = KIND == PT_ACSF_GENERIC && sizeof(R) == 8;
+        if (a.cap < kTeamRow) return team(w4, general64 ? kTeamShortGeneral64 : kTeamShort);
         if constexpr (KIND != PT_ACSF_GENERIC)
             if (team(std::integral_constant<int, 8>{}, sizeof(R) == 8 && MODE == MODE_TAN ? kTeam8Tan64 : kTeam8)) return true;
-        return team(w4, kTeamLong);
+        return team(w4, general64 ? kTeamLongGeneral64 : kTeamLong);
     };
     if (some_team())
         return launch_check("k_acsf_team");
