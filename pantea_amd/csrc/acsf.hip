@@ -485,8 +485,11 @@ __device__ __forceinline__ int angular_group(const Stage<R>& S, const AngGroup<R
     constexpr int NA = ang_terms<ANG>();
     constexpr bool kPreOut = ANG != ANGK_GEN;   // pre applied outside the pair loop
     // FP64 adjoint: the weights live in LDS (broadcast reads), which frees
-    // 32 VGPRs in the pair loop
-    constexpr bool kWLds = MODE == MODE_ADJ && sizeof(R) == 8;
+    // 32 VGPRs in the pair loop.  So they do in FP32 where the angular terms take a
+    // power each: their values fill the scalar registers, and 16 weights more were
+    // spilled and read back lane by lane (12 Bohr, 12,288 centres 1,320 -> 1,260 us).
+    constexpr bool kPowers = ANG == ANGK_GEN && CUT != CUTK_GEN && WPC == 1;
+    constexpr bool kWLds = MODE == MODE_ADJ && (sizeof(R) == 8 || kPowers);
     R W[PT_AG_ETA][PT_AG_ANG];
 #pragma unroll
     for (int e = 0; e < PT_AG_ETA; ++e)
