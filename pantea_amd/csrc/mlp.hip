@@ -504,8 +504,8 @@ __global__ __launch_bounds__(256) void k_mlp(MlpArgs a) {
         return a.g_f64 ? ((const double*)net.G)[o] : (double)((const float*)net.G)[o];
     };
 
-    // 1. scaled input, zero padded: 32 columns x 8 rows per step
-    for (int k0 = 0; k0 < s.in_p; k0 += 32) {
+    // 1. scaled input, zero padded: 32 columns x 8 rows per step (a linear model reads it where it is)
+    for (int k0 = 0; H > 0 && k0 < s.in_p; k0 += 32) {
         const int k = k0 + (threadIdx.x & 31);
         const bool ok = k < s.in_dim;
         const double sub = ok ? net.scale[k] : 0.0, mul = ok ? net.scale[s.in_dim + k] : 0.0;
@@ -1102,6 +1102,7 @@ int launch_mlp_cfg(MlpArgs& a, hipStream_t st) {
 //   52-64-64-1 BF16x3    12,288 rows 12.2 | 14.6   32,768 rows 23.0 | 19.2   98,304 rows 58.8 | 50.0
 //   34-16-16-1 FP64      12,288 rows 12.8 | 17.8   32,768 rows 29.4 | 24.5   98,304 rows 78.3 | 65.0
 //   34-16-16-1 BF16x3    32,768 rows 11.4 | 15.7   65,536 rows 21.0 | 19.6   98,304 rows 29.6 | 33.8 (16 rows stay)
+//   linear, 120 inputs FP64, 30,000 rows 17.0 | 38.3   98,304 rows 47.1 | 109 (one wavefront for all columns: 16 rows stay)
 // (64 rows per workgroup for the wide networks, 54.7 us at 98,304 rows in
 // BF16x3, never won.)  One wavefront per 16 rows took 66 / 28 / 32 / 17 us for
 // any size up to 12,288 rows and 245 / 85 / 117 / 42 us at 98,304.
@@ -1118,7 +1119,7 @@ int launch_mlp(MlpArgs& a, hipStream_t st) {
         n += a.net[g].n_atoms;
     }
     if (wp > 64) return launch_mlp_cfg<MODE, 2, 4, 1, 3>(a, st);
-    if (MODE == PT_MLP_F64 && wp <= 32 && n >= kMlpNarrowRows) return launch_mlp_cfg<PT_MLP_F64, 2, 1, 1, 3>(a, st);
+    if (MODE == PT_MLP_F64 && hid > 0 && wp <= 32 && n >= kMlpNarrowRows) return launch_mlp_cfg<PT_MLP_F64, 2, 1, 1, 3>(a, st);
     if (hid <= 2 && wp > 32 && n >= kMlpWideRows) return launch_mlp_cfg<MODE, 1, 4, 2, 2>(a, st);
     return launch_mlp_cfg<MODE, 1, 4, 1, 3>(a, st);
 }
