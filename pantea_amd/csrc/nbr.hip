@@ -981,15 +981,19 @@ __global__ __launch_bounds__(1024) void k_offsets_small(const int* __restrict__ 
     }
     long long run = block_exclusive(sum, wtot, all);
 #pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        if (q < per && b + q < n) row_off[b + q] = run;
+        run += c[q];
+    }
+#pragma unroll
     for (int off = 1; off < kWave; off <<= 1) m = max(m, __shfl_xor(m, off, kWave));
     if ((threadIdx.x & (kWave - 1)) == 0) wmax[threadIdx.x >> 6] = m;
     __syncthreads();
     for (int q = 0; q < 16; ++q) m = max(m, wmax[q]);
     const bool kept = rows_kept(all, m, keep_cap, keep_row);
-#pragma unroll
-    for (int q = 0; q < PER; ++q) {
-        if (q < per && b + q < n) row_off[b + q] = kept ? run : 0;
-        run += c[q];
+    if (!kept) {   // (rare: the offsets above are on their way before the longest row is known)
+        for (int q = 0; q < per; ++q)
+            if (b + q < n) row_off[b + q] = 0;
     }
     if (threadIdx.x == 0) {
         row_off[n] = kept ? all : 0;
