@@ -135,8 +135,8 @@ typedef struct {
  * (a) Neighbour list.  Replaces the dense cutoff masks of
  * atoms/neighbor.py:47-64,102-107 (mask (r <= rc) & (r > 0) over the
  * minimum-image distances of atoms/distance.py:63-78).
- * Cell binning, stable LSD radix sort of (type, cell) keys, then a CSR list
- * whose rows hold internal neighbour indices in ascending order.
+ * Atoms are sorted stably by (type, cell), then a CSR list is built whose rows
+ * hold internal neighbour indices in ascending order.
  *  pos      (device) n rows of pos_stride (>= 3) FP64, x y z first, input
  *           order (pos_stride 4 lets a previous pos4 be the input);
  *           types (device) n, 1-based

@@ -757,7 +757,7 @@ extern "C" int pt_kalman_update(int n_w, int m, double* P, const double* H, long
     PT_REQUIRE(ws_bytes >= pt_kalman_workspace_bytes(n_w, m), "pt_kalman_update: workspace too small");
     PT_REQUIRE((size_t)n_w * n_w < (1ull << 31) && (factored_form(n_w, m) || (size_t)m * m < (1ull << 31)) &&
                    (size_t)n_w * m < (1ull << 31) && ldh < (1LL << 31),
-               "pt_kalman_update: matrices beyond 32-bit BLAS indexing");
+               "pt_kalman_update: matrices of 2^31 entries and more");
     hipStream_t st = (hipStream_t)stream;
     const KalmanWs L(n_w, m);
     char* base = (char*)ws;

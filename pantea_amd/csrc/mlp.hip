@@ -772,9 +772,9 @@ struct TrainArgs {
 };
 
 // LDS of a workgroup: layer inputs (H + 1), pre-activations (H) and two reverse
-// buffers of 32 rows, 64 per-row scalars, and the gradient sums (TRAIN)
+// buffers of 32 rows, 32 per-row scalars, and the gradient sums (TRAIN)
 inline size_t train_lds(size_t word, int H, int stride, int nparam) {
-    return word * ((size_t)(2 * H + 3) * 32 * stride + 64 + nparam);
+    return word * ((size_t)(2 * H + 3) * 32 * stride + 32 + nparam);
 }
 
 // cells of 16 rows x `width` columns (a multiple of 32) over the 256 threads
@@ -808,8 +808,8 @@ __global__ __launch_bounds__(256) void k_mlp_train(TrainArgs a) {
     auto Zbuf = [&](int h) { return base + (H + 1 + h) * tile; };
     T* P = base + (2 * H + 1) * tile;     // reverse buffers, swapped after each layer
     T* Q = P + tile;
-    T* outv = Q + tile;                   // [0,16): z_L, [16,32): zdot_L, [32,48): zbar_L, [48,64): zdotbar_L
-    T* gacc = outv + 64;
+    T* outv = Q + tile;                   // [0,16): zbar_L, [16,32): zdotbar_L
+    T* gacc = outv + 32;
     const char* packed = net.packed;
     if (!JAC)
         for (int k = tid; k < net.nparam; k += 256) gacc[k] = T(0);
@@ -889,8 +889,8 @@ __global__ __launch_bounds__(256) void k_mlp_train(TrainArgs a) {
             const T gy = !JAC && ok ? (T)net.gy[a0 + r] : T(0);
             const T gt = ok ? (T)a.tseed : T(0);
             if (part == 0) {
-                outv[32 + r] = gy * dy + gt * ddy * zd;  // zbar_L
-                outv[48 + r] = gt * dy;                  // zdotbar_L
+                outv[r] = gy * dy + gt * ddy * zd;  // zbar_L
+                outv[16 + r] = gt * dy;                  // zdotbar_L
             }
         }
         __syncthreads();
@@ -898,18 +898,18 @@ __global__ __launch_bounds__(256) void k_mlp_train(TrainArgs a) {
         if constexpr (JAC) {
             for (int k = tid; k < fan_L; k += 256)
                 for (int r = 0; r < nrows; ++r)
-                    Jrow(r)[s.pW[L] + k] = Abuf(H)[r * stride + k] * outv[32 + r] + Abuf(H)[(16 + r) * stride + k] * outv[48 + r];
-            if (tid < nrows) Jrow(tid)[s.pb[L]] = outv[32 + tid];
+                    Jrow(r)[s.pW[L] + k] = Abuf(H)[r * stride + k] * outv[r] + Abuf(H)[(16 + r) * stride + k] * outv[16 + r];
+            if (tid < nrows) Jrow(tid)[s.pb[L]] = outv[tid];
         } else {
             for (int k = tid; k < fan_L; k += 256) {
                 T gw = T(0);
                 for (int r = 0; r < 16; ++r)
-                    gw += Abuf(H)[r * stride + k] * outv[32 + r] + Abuf(H)[(16 + r) * stride + k] * outv[48 + r];
+                    gw += Abuf(H)[r * stride + k] * outv[r] + Abuf(H)[(16 + r) * stride + k] * outv[16 + r];
                 gacc[s.pW[L] + k] += gw;
             }
             if (tid == 255) {
                 T gb = T(0);
-                for (int r = 0; r < 16; ++r) gb += outv[32 + r];
+                for (int r = 0; r < 16; ++r) gb += outv[r];
                 gacc[s.pb[L]] += gb;
             }
         }
@@ -921,8 +921,8 @@ __global__ __launch_bounds__(256) void k_mlp_train(TrainArgs a) {
                 const T z = Zbuf(h)[r * stride + k], zd = Zbuf(h)[(16 + r) * stride + k];
                 T y, dy, ddy;
                 activate2<T>(s.act[h], z, y, dy, ddy);
-                const T ab = h == H - 1 ? outv[32 + r] * wout[k] : P[r * stride + k];
-                const T adb = h == H - 1 ? outv[48 + r] * wout[k] : P[(16 + r) * stride + k];
+                const T ab = h == H - 1 ? outv[r] * wout[k] : P[r * stride + k];
+                const T adb = h == H - 1 ? outv[16 + r] * wout[k] : P[(16 + r) * stride + k];
                 const bool pad = k >= s.w[h];
                 P[r * stride + k] = pad ? T(0) : ab * dy + adb * ddy * zd;
                 P[(16 + r) * stride + k] = pad ? T(0) : adb * dy;

@@ -1,5 +1,6 @@
-// (a) Neighbour list on gfx950: cell binning, stable LSD radix sort of
-// (type, cell) keys, and a CSR list built by one wavefront per centre.
+// (a) Neighbour list on gfx950: atoms sorted stably by (type, cell) (in one
+// workgroup up to 6,144 atoms, by counting above, by an LSD radix sort where cells
+// far outnumber atoms), and a CSR list built by one wavefront per centre.
 //
 // Replaces the dense masks of atoms/neighbor.py:47-64,102-107: row i holds
 // every j with r_ij <= rc and r_ij > 0, r_ij being the single-shift

@@ -129,11 +129,6 @@ class NeighborList:
             self._perm_host = self.perm.cpu().numpy()
         return self._perm_host
 
-    def inverse_perm_host(self) -> np.ndarray:
-        inv = np.empty(self.n, dtype=np.int64)
-        inv[self.perm_host] = np.arange(self.n)
-        return inv
-
     def inverse_perm(self):
         """The internal index of each input atom (device)."""
         inv = _torch().empty_like(self.perm)
